@@ -1,9 +1,11 @@
 """MI355X (gfx950) kernels behind the XLA custom calls of the reference PJRT plugin.
 
 The product is ``libxmk.so`` (``include/xmk.h``): hand-written HIP kernels behind a
-C ABI.  This module is the thin ctypes binding the tests and the benchmark use;
-torch only supplies device memory and the stream.  There is no CPU fallback: if
-the library is missing or a call fails, the wrappers raise.
+C ABI.  This module gives the entry points their Python names and defaults; the calls on
+torch tensors go through a small native module (``csrc/python/native.cc``), the rest
+(descriptors, queries) through ctypes.  torch only supplies device memory and the
+stream.  There is no CPU fallback: if the library is missing or a call fails, the
+wrappers raise.
 
 Function names follow the reference's host entry points:
 ``run_gemm`` <-> RunGemm (xla/service/gpu/onednn_matmul_utils.h:58-73),
@@ -52,11 +54,12 @@ class GemmDesc(ctypes.Structure):
 
 
 _lib = None
+_native = None  # the module of native.cc, bound to LIB_PATH by lib()
 
 
 def lib():
     """Loads libxmk.so; raises if it has not been built (no fallback)."""
-    global _lib
+    global _lib, _native
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(f"{LIB_PATH} is missing: run `python {_HERE}/build.py` "
@@ -73,8 +76,20 @@ def lib():
                               ("xmk_int4_gemm_workspace_bytes", ctypes.c_size_t)):
             if hasattr(L, name):
                 getattr(L, name).restype = restype
+        try:
+            from . import _xmk_native
+        except ImportError as e:
+            raise RuntimeError(f"the native binding is missing or does not load ({e}): run `python {_HERE}/build.py`") from e
+        _xmk_native.bind(LIB_PATH)
+        _native = _xmk_native
         _lib = L
     return _lib
+
+
+def _bound():
+    """The native module (loads the library on the first call)."""
+    lib()
+    return _native
 
 
 def _check(code):
@@ -117,16 +132,8 @@ def run_gemm(lhs, rhs, out, *, lhs_transpose=False, rhs_transpose=False, out_tra
     """out = act(alpha * op(lhs) op(rhs) + beta * c + bias).  Tensors are the *stored*
     row-major matrices; ``*_transpose`` marks the operand as the transpose of what is
     stored (a column-major XLA layout)."""
-    batch = lhs.shape[0] if lhs.dim() == 3 else 1
-    d = GemmDesc(matrix(lhs, lhs_transpose), matrix(rhs, rhs_transpose),
-                 matrix(out, out_transpose), None if c is None else c.data_ptr(),
-                 None if bias is None else bias.data_ptr(), dtype_code(lhs), dtype_code(out),
-                 batch, alpha, beta, epilogue)
-    if workspace is not None:
-        _check(lib().xmk_gemm_ws(ctypes.byref(d), _ptr(workspace), ctypes.c_size_t(workspace.numel() * workspace.element_size()),
-                                 _stream(stream)))
-    else:
-        run_gemm_desc(d, stream)
+    _check((_native or _bound()).gemm(lhs, rhs, out, lhs_transpose, rhs_transpose, out_transpose, c, bias, alpha, beta, epilogue,
+                                      stream, workspace))
     return out
 
 
@@ -140,11 +147,7 @@ def run_gemm_qkv(lhs, weights, out_q, out_k, out_v, *, rhs_transpose=False, bias
                  stream=None):
     """out_i = act(lhs @ weights[i] + bias[i]) for the three stacked weights [3, k, n] (or [3, n, k] with
     ``rhs_transpose``) in one launch; bias is [3, n] or None."""
-    rhs = matrix(weights[0], rhs_transpose)
-    rhs.batch_stride = weights.stride(0)
-    d = GemmDesc(matrix(lhs, False), rhs, matrix(out_q, False), None,
-                 None if bias is None else bias.data_ptr(), dtype_code(lhs), dtype_code(out_q), 1, 1.0, 0.0, epilogue)
-    _check(lib().xmk_gemm_qkv(ctypes.byref(d), _ptr(out_k), _ptr(out_v), _stream(stream)))
+    _check((_native or _bound()).gemm_qkv(lhs, weights, out_q, out_k, out_v, rhs_transpose, bias, epilogue, stream))
     return out_q, out_k, out_v
 
 
@@ -158,32 +161,16 @@ def gemm_policy_name(m, n, k, rhs_transpose=False, dtype_in=BF16, dtype_out=BF16
 def fmha_forward(query, key, value, out, *, bias=None, lse=None, head_scale=None, causal=False,
                  stream=None):
     """query [B,N,F,H], key/value [B,N,T,H], out [B,N,F,H]; bias [B,N,F,T]; lse fp32 [B*N,F]."""
-    B, N, F, H = query.shape
-    T = key.shape[2]
-    scale = (H ** -0.5) if head_scale is None else head_scale
-    _check(lib().xmk_fmha_fwd(_ptr(query), _ptr(key), _ptr(value), _ptr(bias), _ptr(out),
-                              _ptr(lse), ctypes.c_int32(dtype_code(query)), ctypes.c_uint32(B),
-                              ctypes.c_uint32(N), ctypes.c_uint32(H), ctypes.c_uint32(F),
-                              ctypes.c_uint32(T), ctypes.c_float(scale),
-                              ctypes.c_int32(int(causal)), _stream(stream)))
+    _check((_native or _bound()).fmha_forward(query, key, value, out, bias, lse, head_scale, causal, stream))
     return out
 
 
 def fmha_backward(query, key, value, out, grad_out, lse, *, bias=None, head_scale=None, causal=False, stream=None):
     """Gradients (dq, dk, dv) of fmha_forward's output with respect to query, key, value."""
-    B, N, F, H = query.shape
-    T = key.shape[2]
-    scale = (H ** -0.5) if head_scale is None else head_scale
-    nbytes = lib().xmk_fmha_bwd_workspace_bytes(ctypes.c_uint32(B), ctypes.c_uint32(N), ctypes.c_uint32(H),
-                                                ctypes.c_uint32(F), ctypes.c_uint32(T))
-    ws = torch.empty((max(nbytes, 256),), dtype=torch.uint8, device=query.device)
-    dq, dk, dv = torch.empty_like(query), torch.empty_like(key), torch.empty_like(value)
-    _check(lib().xmk_fmha_bwd(_ptr(query), _ptr(key), _ptr(value), _ptr(bias), _ptr(out), _ptr(grad_out), _ptr(lse),
-                              _ptr(dq), _ptr(dk), _ptr(dv), ctypes.c_int32(dtype_code(query)), ctypes.c_uint32(B),
-                              ctypes.c_uint32(N), ctypes.c_uint32(H), ctypes.c_uint32(F), ctypes.c_uint32(T),
-                              ctypes.c_float(scale), ctypes.c_int32(int(causal)), _ptr(ws), ctypes.c_size_t(nbytes),
-                              _stream(stream)))
-    return dq, dk, dv
+    grads = (_native or _bound()).fmha_backward(query, key, value, out, grad_out, lse, bias, head_scale, causal, stream)
+    if type(grads) is int:
+        _check(grads)
+    return grads
 
 
 def fmha_decode_workspace_bytes(B, N, H, T):
@@ -201,17 +188,7 @@ def fmha_decode(query, key, value, out, workspace, *, num_keys=None, kv_head_str
                 head_scale=None, stream=None):
     """query/out [B,N,1,H] (or [B,N,H]); key/value [B,N,Tcap,H] caches of which the first
     ``num_keys`` rows are attended."""
-    B, N = query.shape[0], query.shape[1]
-    H = query.shape[-1]
-    T = key.shape[2] if num_keys is None else num_keys
-    stride = key.stride(1) if kv_head_stride is None else kv_head_stride
-    scale = (H ** -0.5) if head_scale is None else head_scale
-    _check(lib().xmk_fmha_decode(_ptr(query), _ptr(key), _ptr(value), _ptr(out),
-                                 ctypes.c_int32(dtype_code(query)), ctypes.c_uint32(B),
-                                 ctypes.c_uint32(N), ctypes.c_uint32(H), ctypes.c_uint32(T),
-                                 ctypes.c_int64(stride), ctypes.c_float(scale), _ptr(workspace),
-                                 ctypes.c_size_t(workspace.numel() * workspace.element_size()),
-                                 _stream(stream)))
+    _check((_native or _bound()).fmha_decode(query, key, value, out, workspace, num_keys, kv_head_stride, head_scale, stream))
     return out
 
 
@@ -219,15 +196,7 @@ def fmha_decode_static(query, key, value, out, *, num_keys=None, kv_head_stride=
                        stream=None):
     """fmha_decode without a workspace argument: the key splits' partial results go to an array
     inside the library image (xmk_fmha_decode_static: it allocates nothing)."""
-    B, N = query.shape[0], query.shape[1]
-    H = query.shape[-1]
-    T = key.shape[2] if num_keys is None else num_keys
-    stride = key.stride(1) if kv_head_stride is None else kv_head_stride
-    scale = (H ** -0.5) if head_scale is None else head_scale
-    _check(lib().xmk_fmha_decode_static(_ptr(query), _ptr(key), _ptr(value), _ptr(out),
-                                        ctypes.c_int32(dtype_code(query)), ctypes.c_uint32(B),
-                                        ctypes.c_uint32(N), ctypes.c_uint32(H), ctypes.c_uint32(T),
-                                        ctypes.c_int64(stride), ctypes.c_float(scale), _stream(stream)))
+    _check((_native or _bound()).fmha_decode(query, key, value, out, None, num_keys, kv_head_stride, head_scale, stream))
     return out
 
 
@@ -242,11 +211,7 @@ def fmha_decode_static_init():
 
 # ----------------------------------------------------------------------- int4
 def int4_gemm(act, qweight, scales, zeros, out, *, group=128, bias=None, stream=None):
-    m, k = act.shape
-    n = qweight.shape[1]
-    _check(lib().xmk_int4_gemm(_ptr(act), _ptr(qweight), _ptr(scales), _ptr(zeros), _ptr(bias),
-                               _ptr(out), ctypes.c_int64(m), ctypes.c_int64(k), ctypes.c_int64(n),
-                               ctypes.c_int64(group), _stream(stream)))
+    _check((_native or _bound()).int4_gemm(act, qweight, scales, zeros, out, None, group, bias, stream))
     return out
 
 
@@ -256,13 +221,7 @@ def int4_gemm_workspace_bytes(m, k, n):
 
 def int4_gemm_ws(act, qweight, scales, zeros, out, workspace, *, group=128, bias=None, stream=None):
     """xmk_int4_gemm_ws: with enough scratch and rows, dequantise once and run the dense fp16 GEMM."""
-    m, k = act.shape
-    n = qweight.shape[1]
-    nbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    _check(lib().xmk_int4_gemm_ws(_ptr(act), _ptr(qweight), _ptr(scales), _ptr(zeros), _ptr(bias),
-                                  _ptr(out), ctypes.c_int64(m), ctypes.c_int64(k), ctypes.c_int64(n),
-                                  ctypes.c_int64(group), _ptr(workspace), ctypes.c_size_t(nbytes),
-                                  _stream(stream)))
+    _check((_native or _bound()).int4_gemm(act, qweight, scales, zeros, out, workspace, group, bias, stream))
     return out
 
 
@@ -277,16 +236,7 @@ def int4_dequant(qweight, scales, zeros, w_out, *, group=128, stream=None):
 # ------------------------------------------------------------------------ fp8
 def fp8_gemm(a, b, a_scale, b_scale, out, *, rhs_transpose=False, d_scale=None, bias=None, stream=None):
     """out = bf16(d_scale * (a_scale * b_scale * a b + bias)); d_scale / bias given: xmk_fp8_gemm_ex."""
-    m, k = a.shape
-    n = b.shape[0] if rhs_transpose else b.shape[1]
-    if d_scale is None and bias is None:
-        _check(lib().xmk_fp8_gemm(_ptr(a), _ptr(b), _ptr(a_scale), _ptr(b_scale), _ptr(out),
-                                  ctypes.c_int64(m), ctypes.c_int64(n), ctypes.c_int64(k),
-                                  ctypes.c_int32(int(rhs_transpose)), _stream(stream)))
-    else:
-        _check(lib().xmk_fp8_gemm_ex(_ptr(a), _ptr(b), _ptr(a_scale), _ptr(b_scale), _ptr(d_scale), _ptr(bias),
-                                     _ptr(out), ctypes.c_int64(m), ctypes.c_int64(n), ctypes.c_int64(k),
-                                     ctypes.c_int32(int(rhs_transpose)), _stream(stream)))
+    _check((_native or _bound()).fp8_gemm(a, b, a_scale, b_scale, out, rhs_transpose, d_scale, bias, stream))
     return out
 
 
@@ -341,8 +291,7 @@ class GptjDecoder:
         self.workspace = torch.empty((nbytes,), dtype=torch.uint8, device=lnf_gamma.device)
 
     def step(self, hidden_in, position, logits, stream=None):
-        _check(lib().xmk_gptj_decode_step(ctypes.byref(self.cfg), self.layers, _ptr(self.lnf[0]),
-                                          _ptr(self.lnf[1]), ctypes.byref(self.lm_head), _ptr(hidden_in),
-                                          ctypes.c_int32(position), _ptr(logits), _ptr(self.workspace),
-                                          ctypes.c_size_t(self.workspace.numel()), _stream(stream)))
+        _check((_native or _bound()).gptj_decode_step(ctypes.addressof(self.cfg), ctypes.addressof(self.layers), self.lnf[0], self.lnf[1],
+                                                      ctypes.addressof(self.lm_head), hidden_in, position, logits, self.workspace,
+                                                      stream))
         return logits

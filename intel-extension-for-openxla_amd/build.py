@@ -1,4 +1,5 @@
-"""Builds libxmk.so (the C-ABI kernel library) for gfx950 with hipcc, in-tree.
+"""Builds libxmk.so (the C-ABI kernel library) for gfx950 with hipcc and _xmk_native.so (its torch binding)
+with the host compiler, in-tree.
 
 Usage: python build.py [-j N] [--force]   (without --force: incremental)
 Each translation unit under csrc/ is compiled to an object file and the objects
@@ -8,12 +9,15 @@ import concurrent.futures
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libxmk.so")
+NATIVE_SRC = os.path.join(CSRC, "python", "native.cc")
+NATIVE = os.path.join(HERE, "_xmk_native.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-I", INCLUDE, "-I", CSRC,
@@ -52,18 +56,37 @@ def _compile(args):
     return src, obj, r.returncode, out
 
 
+def _compile_native(force):
+    """The host-only module between torch tensors and the C ABI.  It links to nothing of libxmk.so (bound by
+    path when the package loads it)."""
+    if not force and os.path.exists(NATIVE) and os.path.getmtime(NATIVE) > max(os.path.getmtime(NATIVE_SRC), _deps_mtime()):
+        return 0, ""
+    import torch
+    t = os.path.dirname(torch.__file__)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
+           "-DUSE_ROCM", "-I", INCLUDE, "-isystem", "/opt/rocm/include", "-isystem", os.path.join(t, "include"),
+           "-isystem", sysconfig.get_paths()["include"], NATIVE_SRC, "-o", NATIVE, "-L", os.path.join(t, "lib"),
+           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    return r.returncode, r.stdout + r.stderr
+
+
 def build(jobs=None, verbose=False, force=True):
     """force=False recompiles only sources newer than their object file."""
     os.makedirs(OBJ, exist_ok=True)
     jobs = jobs or min(8, os.cpu_count() or 1)
     objs = []
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
+        native = pool.submit(_compile_native, force)
         for src, obj, rc, out in pool.map(_compile, [(s, force) for s in sources()]):
             if out and (verbose or rc != 0):
                 print(f"--- {src}\n{out}", file=sys.stderr)
             if rc != 0:
                 raise RuntimeError(f"hipcc failed on {src}")
             objs.append(obj)
+        rc, out = native.result()
+        if rc != 0:
+            raise RuntimeError(f"the native binding does not compile:\n{out}")
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs
     subprocess.check_call(cmd)
     return LIB
