@@ -45,13 +45,27 @@ struct Fp8Params {
 struct Fp8Epilogue {
   float scale, post;
   const __bf16* bias;
+  float b[8];  // the bias of the lane's columns (gemm_impl::store_tile)
   __device__ __forceinline__ explicit Fp8Epilogue(const Fp8Params& p)
       : scale(p.a_scale[0] * p.b_scale[0]), post(p.d_scale ? p.d_scale[0] : 1.0f), bias(p.bias) {}
-  __device__ __forceinline__ bool plain() const { return !bias && post == 1.0f; }
   __device__ __forceinline__ __bf16 operator()(float acc, int n) const {
     float v = acc * scale;
     if (bias) v += (float)bias[n];
     return (__bf16)(v * post);
+  }
+  __device__ __forceinline__ void columns(int n, int count) {
+    if (bias && count > 0) gemm_impl::GemmEpilogue<__bf16, false>::fetch<false>(bias, n, count, b);
+  }
+  template <int U>
+  __device__ __forceinline__ void apply(float (&v)[U][8], const int (&)[U], int, int) const {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        v[u][e] *= scale;
+        if (bias) v[u][e] += b[e];
+        v[u][e] *= post;
+      }
   }
 };
 
@@ -240,43 +254,10 @@ __global__ __launch_bounds__(WGM * WGN * 64) void fp8_gemm_kernel(Fp8Params p) {
   __builtin_amdgcn_s_waitcnt(gemm_impl::vmcnt_imm(0));  // drain the zero-fill loads before LDS is released
 
   // acc[i][j][e] is out[m][n], m = m0 + wm WTM + 32 i + lane%32, n = n0 + wn WTN + 32 j + 8 (e/4) + 4 (lane/32) + e%4.
-  const Fp8Epilogue epi(p);
-  const float scale = epi.scale;
-  static_assert(NSTAGE * STAGE >= BM * BN * 2, "the output tile is staged in the operand stages");
-  // A bias or an output scale (both rare with a bf16 result) take the direct stores below.
-  if (epi.plain() && m0 + BM <= p.M && n0 + BN <= p.N && p.N % 8 == 0 && reinterpret_cast<uintptr_t>(p.out) % 16 == 0) {
-    // Tile fully inside (uniform over the work-group): round, lay out row-major in LDS and copy out
-    // in whole row segments.
-    gemm_impl::GemmParams q{};
-    q.out = p.out;
-    q.ldc = p.N;
-    q.alpha = scale;
-    q.act = gemm_impl::ACT_NONE;
-    __builtin_amdgcn_s_barrier();  // every wave has read its last fragments
-    gemm_impl::store_tile_via_lds<__bf16, false, WTM, WTN, TM, TN>(q, acc, lds + wave * (WTM * WTN * 2),
-                                                                   m0 + wm * WTM, n0 + wn * WTN, 0, lane);
-    return;
-  }
-  static_for<TM>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    const int m = m0 + wm * WTM + i * 32 + (lane & 31);
-    static_for<TN>([&](auto J) {
-      constexpr int j = decltype(J)::value;
-      const floatx16 t = acc[i][j];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = n0 + wn * WTN + j * 32 + q * 8 + (lane >> 5) * 4;
-        if (m < p.M && n < p.N) {  // N % 4 == 0: the four columns are all in range
-          union { __bf16 e[4]; u32x2 w; } o;
-          o.e[0] = epi(t[4 * q + 0], n);
-          o.e[1] = epi(t[4 * q + 1], n + 1);
-          o.e[2] = epi(t[4 * q + 2], n + 2);
-          o.e[3] = epi(t[4 * q + 3], n + 3);
-          *reinterpret_cast<u32x2*>(p.out + (int64_t)m * p.N + n) = o.w;
-        }
-      }
-    });
-  });
+  Fp8Epilogue epi(p);
+  static_assert(NSTAGE * STAGE >= NWAVES * TN * 4096, "a slab per wave is staged in the operand stages");
+  __builtin_amdgcn_s_barrier();  // every wave has read its last fragments
+  gemm_impl::store_tile<__bf16, false>(epi, acc, lds + wave * (TN * 4096), p.out, p.N, 0, p.M, p.N, m0 + wm * WTM, n0 + wn * WTN, lane);
 }
 
 // Any layout, size and alignment on the matrix cores: the operands are gathered (gemm_gather8.h) into
@@ -361,35 +342,10 @@ __global__ __launch_bounds__(256) void fp8_gemm_gather_kernel(Fp8Params p) {
   }
 
   // acc[i][j][e] is out[m][n], m = m0 + 32 TW wm + 32 i + lane % 32, n = n0 + 32 TW wn + 32 j + 8 (e/4) + 4 (lane/32) + e%4.
-  const Fp8Epilogue epi(p);
-  gemm_impl::GemmParams q{};
-  q.out = p.out;
-  q.M = p.M;
-  q.N = p.N;
-  q.ldc = p.N;
-  q.alpha = epi.scale;
-  q.act = gemm_impl::ACT_NONE;
-#pragma unroll
-  for (int i = 0; i < TW; ++i) {
-    const int m = m0 + wm * 32 * TW + i * 32 + l32;
-#pragma unroll
-    for (int j = 0; j < TW; ++j) {
-      const floatx16 t = acc[i][j];
-      const int nb = n0 + wn * 32 * TW + j * 32 + g * 4;
-      if (epi.plain()) {
-        gemm_impl::store_quad<__bf16, false>(q, gemm_impl::floatx4{t[0], t[1], t[2], t[3]}, m, nb, 0);
-        gemm_impl::store_quad<__bf16, false>(q, gemm_impl::floatx4{t[4], t[5], t[6], t[7]}, m, nb + 8, 0);
-        gemm_impl::store_quad<__bf16, false>(q, gemm_impl::floatx4{t[8], t[9], t[10], t[11]}, m, nb + 16, 0);
-        gemm_impl::store_quad<__bf16, false>(q, gemm_impl::floatx4{t[12], t[13], t[14], t[15]}, m, nb + 24, 0);
-      } else if (m < p.M) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int n = nb + 8 * (e / 4) + e % 4;
-          if (n < p.N) p.out[(int64_t)m * p.N + n] = epi(t[e], n);
-        }
-      }
-    }
-  }
+  Fp8Epilogue epi(p);
+  static_assert(NSTAGE * STAGE >= 4 * TW * 4096, "a slab per wave is staged in the operand stages");
+  gemm_impl::store_tile<__bf16, false>(epi, acc, lds + wave * (TW * 4096), p.out, p.N, 0, p.M, p.N, m0 + wm * 32 * TW,
+                                       n0 + wn * 32 * TW, lane);
 }
 
 template <int TW, int AMODE>

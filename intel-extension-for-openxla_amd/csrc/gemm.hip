@@ -16,13 +16,15 @@
 // The products are issued with the operands swapped (D^T = B^T A^T) so that a lane ends up
 // holding four consecutive output columns of one row.
 //
-// 16-bit operands whose strides or sizes the direct loads cannot take run the same kernel with a
-// gathering loader, fp32 operands the fp32 MFMA kernel (gemm_f32.hip), int8 operands the int8 MFMA
+// 16-bit operands whose strides or sizes the direct loads cannot take run gemm_ragged_kernel (gemm_ragged.h), fp32 operands the fp32 MFMA kernel (gemm_f32.hip), int8 operands the int8 MFMA
 // kernel (gemm_s8.hip); what is left (outputs that are not 16-byte aligned) runs
 // gemm_generic_kernel, a plain LDS-tiled kernel.  This is where
 // the reference falls back to oneDNN (onednn_matmul_utils.cc:394-491).
+#include <algorithm>
+
 #include "gemm_f32.h"
 #include "gemm_kernel.h"
+#include "gemm_ragged.h"
 #include "gemm_rows.h"
 #include "gemm_s8.h"
 
@@ -134,37 +136,41 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(GenericParams p) {
 }
 
 // Second pass of a K-split GEMM: out = act(alpha * sum_z partial[z] + beta * c + bias), one rounding.
-// partial: fp32 [ks][M][N] packed; out / c: [M][ldc] of kind kout; bias of kind kin.
+// partial: fp32 [ks][M][N], slices `stride` elements apart; out / c: [M][ldc] of kind kout; bias of kind kin.
 struct ReduceParams {
   const float* partial;
   void* out;
   const void* c;
   const void* bias;
   int M, N, ks;
+  int64_t stride;  // a multiple of 4
   int64_t ldc;
   int kin, kout;
   float alpha, beta;
   int act;
 };
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(ReduceParams p) {
-  const int64_t idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;  // four consecutive columns; N % 4 == 0
+  const int64_t idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;  // four consecutive elements of the packed product
   const int64_t total = (int64_t)p.M * p.N;
   if (idx >= total) return;
-  const int m = (int)(idx / p.N), n = (int)(idx % p.N);
+  int m = (int)(idx / p.N), n = (int)(idx % p.N);
   floatx4 s = {0.f, 0.f, 0.f, 0.f};
-  for (int z = 0; z < p.ks; ++z) s += *reinterpret_cast<const floatx4*>(p.partial + (int64_t)z * total + idx);
-  const int64_t off = (int64_t)m * p.ldc + n;
+  for (int z = 0; z < p.ks; ++z) s += *reinterpret_cast<const floatx4*>(p.partial + z * p.stride + idx);
+  const int count = (int)min((int64_t)4, total - idx);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
+    if (j >= count) break;
+    const int64_t off = (int64_t)m * p.ldc + n;
     float v = p.alpha * s[j];
-    if (p.beta != 0.f && p.c) v += p.beta * load_as_f32(p.c, p.kout, off + j);
-    if (p.bias) v += load_as_f32(p.bias, p.kin, n + j);
+    if (p.beta != 0.f && p.c) v += p.beta * load_as_f32(p.c, p.kout, off);
+    if (p.bias) v += load_as_f32(p.bias, p.kin, n);
     v = apply_act(v, p.act);
     switch (p.kout) {
-      case G_BF16: reinterpret_cast<__bf16*>(p.out)[off + j] = (__bf16)v; break;
-      case G_F16: reinterpret_cast<_Float16*>(p.out)[off + j] = (_Float16)v; break;
-      default: reinterpret_cast<float*>(p.out)[off + j] = v; break;
+      case G_BF16: reinterpret_cast<__bf16*>(p.out)[off] = (__bf16)v; break;
+      case G_F16: reinterpret_cast<_Float16*>(p.out)[off] = (_Float16)v; break;
+      default: reinterpret_cast<float*>(p.out)[off] = v; break;
     }
+    if (++n == p.N) { n = 0; ++m; }
   }
 }
 
@@ -210,14 +216,19 @@ extern "C" const char* xmk_gemm_policy_name(int64_t m, int64_t n, int64_t k, int
 namespace {
 // out1 / out2: further outputs of the shared-lhs three-GEMM form, or null for a plain GEMM.
 // policy: tile policy to use instead of select_policy's choice (the K-split planner's), or -1.
-int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int policy = -1);
+// kslice: K slice of a batch member (the ragged kernel's K split; the operands are then those of the whole
+// product), or 0.
+int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int policy = -1, int kslice = 0);
 
-// The conditions of the direct (non-gathering) 16-bit kernels on the stored operands.
+// The conditions of the direct-to-LDS 16-bit kernels on the stored operands.
 bool direct_ok(const xmk_matrix& lhs, const xmk_matrix& rhs) {
   return xmk::aligned(lhs.data, 16) && xmk::aligned(rhs.data, 16) && lhs.leading_dim_stride % 8 == 0 &&
          rhs.leading_dim_stride % 8 == 0 && lhs.batch_stride % 8 == 0 && rhs.batch_stride % 8 == 0 &&
          lhs.num_cols % 8 == 0 && rhs.num_cols % 8 == 0;
 }
+
+// The condition of the ragged 16-bit kernel: the stored rows hold a whole 16-byte chunk.
+bool ragged_ok(const xmk_matrix& lhs, const xmk_matrix& rhs) { return lhs.num_cols >= 8 && rhs.num_cols >= 8; }
 
 // Which streaming kernel for a few rows (gemm_rows.hip) can run this descriptor's product, if any.
 int rows_kind_desc(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k) {
@@ -233,10 +244,22 @@ int rows_kind_desc(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k) {
 // K slices worth using for a plain 16-bit GEMM of this shape when scratch is available: few
 // output tiles (the device has 256 CUs) and a long reduction.  1: do not split.
 // *policy: the tile policy of the slices (-1: whatever select_policy picks for a slice).
-int plan_splitk(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k, int* policy) {
+// *kslice: K slice of the ragged kernel (a multiple of 64, the last slice takes the rest), 0 for the direct kernels.
+int plan_splitk(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k, int* policy, int* kslice) {
   *policy = -1;
-  if (d->batch_size != 1 || n % 4 != 0) return 1;
+  *kslice = 0;
+  if (d->batch_size != 1) return 1;
   if (d->dtype_in != XMK_BF16 && d->dtype_in != XMK_F16) return 1;
+  if (!direct_ok(d->lhs, d->rhs)) {
+    if (!ragged_ok(d->lhs, d->rhs)) return 1;
+    // Slices until the tiles are about two work-groups per CU, each slice keeping 256 k.
+    const int tile = ragged_tile(m, n, 1);
+    const int64_t tiles = xmk::ceil_div(m, tile) * xmk::ceil_div(n, tile);
+    const int64_t want = std::min<int64_t>({16, 512 / tiles, k / 256});
+    if (want < 2) return 1;
+    *kslice = (int)(xmk::ceil_div(xmk::ceil_div(k, want), 64) * 64);
+    return (int)xmk::ceil_div(k, *kslice);
+  }
   auto divides = [&](int ks) { return ks >= 1 && ks <= 16 && k % (ks * 8) == 0; };
   // XMK_GEMM_SPLITK=<slices> overrides the choice (read at every call; the autotuner's handle).
   const char* forced_env = getenv("XMK_GEMM_SPLITK");
@@ -268,6 +291,9 @@ int plan_splitk(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k, int* po
   return ks;
 }
 
+// Elements from one slice's partial sums to the next (16-byte aligned).
+int64_t slice_stride(int64_t m, int64_t n) { return (m * n + 3) / 4 * 4; }
+
 void gemm_dims(const xmk_gemm_desc* d, int64_t* m, int64_t* n, int64_t* k) {
   const bool t = d->out.transpose != 0;  // C^T = B^T A^T swaps the roles
   const xmk_matrix& lhs = t ? d->rhs : d->lhs;
@@ -286,9 +312,9 @@ extern "C" size_t xmk_gemm_workspace_bytes(const xmk_gemm_desc* d) {
   int64_t m, n, k;
   gemm_dims(d, &m, &n, &k);
   if (m <= 0 || n <= 0 || k <= 0) return 0;
-  int pol;
-  const int ks = plan_splitk(d, m, n, k, &pol);
-  return ks > 1 ? (size_t)ks * m * n * sizeof(float) : 0;
+  int pol, kslice;
+  const int ks = plan_splitk(d, m, n, k, &pol, &kslice);
+  return ks > 1 ? (size_t)ks * slice_stride(m, n) * sizeof(float) : 0;
 }
 
 extern "C" int xmk_gemm_ws(const xmk_gemm_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
@@ -298,17 +324,19 @@ extern "C" int xmk_gemm_ws(const xmk_gemm_desc* d, void* workspace, size_t works
     return run_gemm(d, nullptr, nullptr, stream);
   int64_t m, n, k;
   gemm_dims(d, &m, &n, &k);
-  int slice_policy;
-  const int ks = plan_splitk(d, m, n, k, &slice_policy);
+  int slice_policy, kslice;
+  const int ks = plan_splitk(d, m, n, k, &slice_policy, &kslice);
   // Pass 1: the K slices as a batched GEMM into fp32 partial sums (no epilogue); a slice is a
   // column range of lhs and a row (or column) range of rhs, so only the batch strides change.
   xmk_gemm_desc p = *d;
-  const int64_t kz = k / ks;
-  p.lhs.num_cols = kz;
-  p.lhs.batch_stride = kz;
-  if (p.rhs.transpose) { p.rhs.num_cols = kz; p.rhs.batch_stride = kz; }
-  else { p.rhs.num_rows = kz; p.rhs.batch_stride = kz * p.rhs.leading_dim_stride; }
-  p.out.data = workspace; p.out.leading_dim_stride = n; p.out.batch_stride = m * n;
+  if (!kslice) {
+    const int64_t kz = k / ks;
+    p.lhs.num_cols = kz;
+    p.lhs.batch_stride = kz;
+    if (p.rhs.transpose) { p.rhs.num_cols = kz; p.rhs.batch_stride = kz; }
+    else { p.rhs.num_rows = kz; p.rhs.batch_stride = kz * p.rhs.leading_dim_stride; }
+  }
+  p.out.data = workspace; p.out.leading_dim_stride = n; p.out.batch_stride = slice_stride(m, n);
   p.c = nullptr; p.bias = nullptr;
   p.dtype_out = XMK_F32;
   p.batch_size = ks; p.alpha = 1.0f; p.beta = 0.0f; p.epilogue = XMK_EPI_DEFAULT;
@@ -334,15 +362,15 @@ extern "C" int xmk_gemm_ws(const xmk_gemm_desc* d, void* workspace, size_t works
       (d->dtype_out != d->dtype_in && d->dtype_out != XMK_F32))
     return run_gemm(d, nullptr, nullptr, stream);  // reports the error
   xmk::trace("gemm m=%lld n=%lld k=%lld -> split K %d ways", (long long)m, (long long)n, (long long)k, ks);
-  int rc = run_gemm(&p, nullptr, nullptr, stream, slice_policy);
+  int rc = run_gemm(&p, nullptr, nullptr, stream, slice_policy, kslice);
   if (rc != XMK_OK) return rc;
   ReduceParams r;
   r.partial = (const float*)workspace; r.out = d->out.data; r.c = d->beta != 0.0f ? d->c : nullptr;
   r.bias = wants_bias ? d->bias : nullptr;
-  r.M = (int)m; r.N = (int)n; r.ks = ks; r.ldc = d->out.leading_dim_stride;
+  r.M = (int)m; r.N = (int)n; r.ks = ks; r.stride = slice_stride(m, n); r.ldc = d->out.leading_dim_stride;
   r.kin = generic_kind(d->dtype_in); r.kout = generic_kind(d->dtype_out);
   r.alpha = d->alpha; r.beta = d->beta; r.act = act;
-  hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((unsigned)xmk::ceil_div(m * n / 4, 256)), dim3(256), 0,
+  hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((unsigned)xmk::ceil_div(m * n, 4 * 256)), dim3(256), 0,
                      (hipStream_t)stream, r);
   return xmk::check_launch("gemm");
 }
@@ -358,7 +386,7 @@ extern "C" int xmk_gemm_qkv(const xmk_gemm_desc* d, void* out_k, void* out_v, vo
 }
 
 namespace {
-int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int policy) {
+int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int policy, int kslice) {
   if (!d) return xmk::fail(XMK_INVALID_ARGUMENT, "gemm: null descriptor");
   if (!d->lhs.data || !d->rhs.data || !d->out.data)
     return xmk::fail(XMK_INVALID_ARGUMENT, "gemm: null operand");
@@ -428,11 +456,11 @@ int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int p
   const bool sixteen = din == XMK_BF16 || din == XMK_F16;
   const bool fast = sixteen && direct_ok(lhs, rhs) && xmk::aligned(out.data, 16) && xmk::aligned(out1, 16) &&
                     xmk::aligned(out2, 16);
-  // 16-bit operands that miss those conditions still run on the matrix cores, with operands gathered
-  // element by element; the output pointers must allow the epilogue's vector stores.
-  const bool gather = !fast && sixteen && xmk::aligned(out.data, 16) && xmk::aligned(out1, 16) &&
-                      xmk::aligned(out2, 16) && xmk::aligned(d->c, 16);
-  if (fast || gather) {
+  // 16-bit operands that miss those conditions, and outputs of any alignment (fp32 outputs are stored in
+  // aligned quads): the ragged kernel.
+  const bool ragged = !fast && sixteen && ragged_ok(lhs, rhs) &&
+                      (dout != XMK_F32 || (xmk::aligned(out.data, 16) && xmk::aligned(out1, 16) && xmk::aligned(out2, 16)));
+  if (fast || ragged) {
     GemmParams p;
     p.a = lhs.data; p.b = rhs.data; p.out = out.data; p.c = d->beta != 0.0f ? d->c : nullptr;
     p.bias = wants_bias ? d->bias : nullptr;
@@ -442,16 +470,8 @@ int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int p
     p.alpha = d->alpha; p.beta = d->beta; p.act = act;
     p.out_alt[0] = out1; p.out_alt[1] = out2; p.sbias = 0;
     if (qkv) { p.sa = 0; p.sc = 0; p.sbias = n; }
-    // Widest load of the gathering kernel per operand: the pointer, the leading dimension, the batch
-    // stride and the stored row length must all be multiples of it.
-    auto widest = [](const xmk_matrix& x) {
-      int v = 8;
-      while (v > 1 && (!xmk::aligned(x.data, 2 * v) || x.leading_dim_stride % v || x.batch_stride % v || x.num_cols % v))
-        v /= 2;
-      return v;
-    };
-    p.vec_a = widest(lhs);
-    p.vec_b = widest(rhs);
+    p.kslice = kslice;
+    if (kslice) { p.sa = 0; p.sb = 0; }
     const bool a_mc = lhs.transpose != 0;   // stored [K, M]
     const bool b_mc = rhs.transpose == 0;   // stored [K, N]
     const int batch = qkv ? 3 : (int)d->batch_size;
@@ -460,16 +480,17 @@ int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int p
     const int pol = (forced_policy() < 0 && policy >= 0 && policy < kNumPolicies &&
                      (policy != kRowsPolicy || rows_kind != kRowsNone))
                         ? policy : select_policy(m, n, k, batch, rows_kind, b_mc);
+    const int tile = ragged_tile(m, n, kslice ? 1 : batch);
     xmk::trace("gemm m=%lld n=%lld k=%lld batch=%lld lhs_t=%d rhs_t=%d epilogue=%d beta=%g -> %s",
                (long long)m, (long long)n, (long long)k, (long long)d->batch_size, lhs.transpose,
-               rhs.transpose, d->epilogue, d->beta, gather ? kGatherPolicy.name : kPolicies[pol].name);
-    if (gather) {
+               rhs.transpose, d->epilogue, d->beta, !ragged ? kPolicies[pol].name : tile == 128 ? "ragged_128x128x64" : "ragged_64x64x64");
+    if (ragged) {
       if (din == XMK_BF16) {
-        if (dout == XMK_F32) launch_layout_gather<__bf16, true>(a_mc, b_mc, p, batch, st);
-        else launch_layout_gather<__bf16, false>(a_mc, b_mc, p, batch, st);
+        if (dout == XMK_F32) launch_ragged<__bf16, true>(a_mc, b_mc, p, batch, tile, st);
+        else launch_ragged<__bf16, false>(a_mc, b_mc, p, batch, tile, st);
       } else {
-        if (dout == XMK_F32) launch_layout_gather<_Float16, true>(a_mc, b_mc, p, batch, st);
-        else launch_layout_gather<_Float16, false>(a_mc, b_mc, p, batch, st);
+        if (dout == XMK_F32) launch_ragged<_Float16, true>(a_mc, b_mc, p, batch, tile, st);
+        else launch_ragged<_Float16, false>(a_mc, b_mc, p, batch, tile, st);
       }
       return xmk::check_launch("gemm");
     }

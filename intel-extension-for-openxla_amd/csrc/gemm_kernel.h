@@ -38,9 +38,11 @@ struct GemmParams {
   // out_alt[z - 1] instead of out + z * sc and reads bias + z * sbias.  Null when unused.
   void* out_alt[2];
   int64_t sbias;
-  // Gathering kernel only: elements per load (1, 2, 4 or 8) that the alignment of each operand's
-  // pointer, leading dimension, batch stride and row length allows.
+  // fp32 and int8 kernels only: elements per load that the alignment of each operand's pointer, leading
+  // dimension, batch stride and row length allows.
   int vec_a, vec_b;
+  // Ragged kernel only: K slice of one grid member (a multiple of its K step), 0 when K is not split.
+  int kslice;
 };
 
 __device__ __forceinline__ float gelu_tanh(float x) {
@@ -176,50 +178,6 @@ struct Loader {
 #pragma unroll
     for (int i = 0; i < NL; ++i) issue_one(i, rsrc, kleft, lds_tile, wave);
   }
-  // The same placement for operands the direct loads cannot take (rows that do not start on a
-  // 16-byte boundary, a row length that is not a multiple of 8): load i's chunk is gathered element
-  // by element, zero where the row, column or k does not exist, and written with one 16-byte LDS
-  // store.  Nothing outside the matrix is read.  base: tile origin for this K step; valid: rows
-  // (KC) or columns (MC) of the tile that exist; kleft as in issue_one; vec: elements per load
-  // (wave-uniform; every group of `vec` elements is aligned and lies inside the row or outside as a whole).
-  __device__ __forceinline__ void gather_one(int i, const uint16_t* base, int64_t ld, int valid, int kleft,
-                                             char* lds_tile, int wave, int lane, int vec) const {
-    scatter_one(i, gather_load(i, base, ld, valid, kleft, wave, lane, vec), lds_tile, wave, lane);
-  }
-  __device__ __forceinline__ void scatter_one(int i, u32x4 v, char* lds_tile, int wave, int lane) const {
-    *reinterpret_cast<u32x4*>(lds_tile + (i * NWAVES + wave) * 1024 + lane * 16) = v;
-  }
-  __device__ __forceinline__ u32x4 gather_load(int i, const uint16_t* base, int64_t ld, int valid, int kleft,
-                                               int wave, int lane, int vec) const {
-    const int lrow = wave * RPL + lane / CPR + i * LSTRIDE;                       // LSTRIDE % 8 == 0:
-    const int c0 = ((lane % CPR) ^ swz<MC, ROWS, BK, EB>(wave * RPL + lane / CPR)) * 8;  // same swizzle for every i
-    const int row = MC ? c0 : lrow;   // operand row / column of element 0
-    const int k = MC ? lrow : c0;     // k (inside the K step) of element 0
-    const uint16_t* src = MC ? base + (int64_t)k * ld + row : base + (int64_t)row * ld + k;
-    const bool line = MC ? k < kleft : row < valid;  // the stored row this chunk lies in exists
-    const int left = MC ? valid - row : kleft - k;    // elements of that row from element 0 on
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (vec == 8) {
-      if (line && left > 0) v = *reinterpret_cast<const u32x4*>(src);
-    } else if (vec == 4) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        if (line && 4 * j < left) {
-          const u32x2 w = *reinterpret_cast<const u32x2*>(src + 4 * j);
-          v[2 * j] = w[0];
-          v[2 * j + 1] = w[1];
-        }
-    } else if (vec == 2) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (line && 2 * j < left) v[j] = *reinterpret_cast<const uint32_t*>(src + 2 * j);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (line && j < left) v[j >> 1] |= (uint32_t)src[j] << (16 * (j & 1));
-    }
-    return v;
-  }
 };
 
 // Per-lane LDS byte offsets of an operand's fragments, computed once.  A fragment of the
@@ -340,86 +298,192 @@ __device__ __forceinline__ void store_quad(const GemmParams& p, floatx4 a, int m
   }
 }
 
-// The epilogue's arithmetic for four consecutive columns n..n+3 of row m that lie inside the matrix.
-// PLAIN: alpha == 1 and no addend, bias or activation.
-template <typename T, bool PLAIN>
-__device__ __forceinline__ floatx4 quad_values(const GemmParams& p, floatx4 a, int m, int n, int64_t coff) {
-  if constexpr (PLAIN) return a;
-  float v0 = p.alpha * a[0], v1 = p.alpha * a[1], v2 = p.alpha * a[2], v3 = p.alpha * a[3];
-  if (p.c) {
-    const u32x2 cw = *reinterpret_cast<const u32x2*>(reinterpret_cast<const T*>(p.c) + coff + (int64_t)m * p.ldc + n);
-    const T* cp = reinterpret_cast<const T*>(&cw);
-    v0 += p.beta * Elem<T>::to_f32(cp[0]); v1 += p.beta * Elem<T>::to_f32(cp[1]);
-    v2 += p.beta * Elem<T>::to_f32(cp[2]); v3 += p.beta * Elem<T>::to_f32(cp[3]);
+// What a tile's products become: out = act(alpha * acc + beta * c + bias) for eight consecutive columns of a row.
+// A lane's columns are the same for all its rows, so the bias is fetched once.
+template <typename T, bool OutF32>
+struct GemmEpilogue {
+  const void *c, *bias_vec;  // null when unused
+  int64_t ldc, coff;
+  float alpha, beta;
+  int act;
+  float bias[8];
+  // bz: batch member
+  __device__ __forceinline__ GemmEpilogue(const GemmParams& p, int64_t bz)
+      : c(p.c), bias_vec(p.bias ? reinterpret_cast<const T*>(p.bias) + bz * p.sbias : nullptr), ldc(p.ldc), coff(bz * p.sc),
+        alpha(p.alpha), beta(p.beta), act(p.act) {}
+  // Eight values at any alignment, of which `count` exist (the others repeat the last one: no branches, so that
+  // all loads are in flight together).
+  template <bool F32>
+  static __device__ __forceinline__ void fetch(const void* base, int64_t off, int count, float (&v)[8]) {
+    if constexpr (F32) {
+      const float* p = reinterpret_cast<const float*>(base) + off;
+      if (count >= 8) {
+        floatx4 lo, hi;
+        __builtin_memcpy(&lo, p, 16);
+        __builtin_memcpy(&hi, p + 4, 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = p[min(e, count - 1)];
+      }
+    } else {
+      const T* p = reinterpret_cast<const T*>(base) + off;
+      if (count >= 8) {
+        u32x4 w;
+        __builtin_memcpy(&w, p, 16);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = Elem<T>::to_f32(__builtin_bit_cast(T, (uint16_t)(w[e / 2] >> (16 * (e & 1)))));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = Elem<T>::to_f32(p[min(e, count - 1)]);
+      }
+    }
   }
-  if (p.bias) {
-    const T* bp = reinterpret_cast<const T*>(p.bias) + n;
-    v0 += Elem<T>::to_f32(bp[0]); v1 += Elem<T>::to_f32(bp[1]);
-    v2 += Elem<T>::to_f32(bp[2]); v3 += Elem<T>::to_f32(bp[3]);
+  // count: columns from n on that exist (8: all of the lane's).
+  __device__ __forceinline__ void columns(int n, int count) {
+    if (bias_vec && count > 0) fetch<sizeof(T) == 4>(bias_vec, n, count, bias);
   }
-  return floatx4{apply_act(v0, p.act), apply_act(v1, p.act), apply_act(v2, p.act), apply_act(v3, p.act)};
+  // U rows at once, rows[u] inside the matrix: every test below is uniform and is made once for them all.
+  template <int U>
+  __device__ __forceinline__ void apply(float (&v)[U][8], const int (&rows)[U], int n, int count) const {
+    if (alpha != 1.0f) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[u][e] *= alpha;
+    }
+    if (c) {  // non-null only when beta != 0
+      float cv[U][8];
+#pragma unroll
+      for (int u = 0; u < U; ++u) fetch<OutF32>(c, coff + (int64_t)rows[u] * ldc + n, count, cv[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[u][e] += beta * cv[u][e];
+    }
+    if (bias_vec) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[u][e] += bias[e];
+    }
+    if (act == ACT_RELU) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[u][e] = fmaxf(v[u][e], 0.f);
+    } else if (act == ACT_GELU) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[u][e] = gelu_tanh(v[u][e]);
+    }
+  }
+};
+
+// The output of batch member bz (offsets bz * p.sc are added by the caller).
+__device__ __forceinline__ void* member_out(const GemmParams& p, int64_t bz) {
+  return p.out_alt[0] && bz > 0 ? p.out_alt[bz - 1] : p.out;
 }
 
-// Epilogue of a tile that lies fully inside a 16-bit output matrix: each wave rounds its WTM x WTN
-// part, lays it out row-major in its own LDS region, and copies the region out with 16-byte stores
-// that cover whole row segments (the accumulator layout itself gives a lane 8 bytes in each of 32
-// different rows per store).  XOR on the 16-byte chunk index keeps both passes off the same banks.
-// vec: elements per global store (8, 4, 2 or 1) that the output's alignment allows; a lane always
-// owns 8 consecutive elements of a row.
-template <typename T, bool PLAIN, int WTM, int WTN, int TM, int TN>
-__device__ __forceinline__ void store_tile_via_lds(const GemmParams& q, const floatx16 (&acc)[TM][TN], char* region,
-                                                   int m_base, int n_base, int64_t coff, int lane, int vec = 8) {
-  constexpr int RBY = WTN * 2;       // bytes per row of the region
-  constexpr int CPRW = RBY / 16;     // 16-byte chunks per row (4, 8 or 16)
-  constexpr int RDIV = 16 / CPRW;    // rows that share one 256-byte bank sweep
-  static_assert(CPRW == 4 || CPRW == 8 || CPRW == 16, "unsupported wave tile width");
-  const int r1 = lane & 31;
-  const int s1 = (r1 / RDIV) & (CPRW - 1);
-  static_for<TM>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    static_for<TN>([&](auto J) {
-      constexpr int j = decltype(J)::value;
-      const floatx16 t = acc[i][j];
-      static_for<4>([&](auto Q) {
-        constexpr int qd = decltype(Q)::value;
-        const floatx4 v = quad_values<T, PLAIN>(q, floatx4{t[4 * qd], t[4 * qd + 1], t[4 * qd + 2], t[4 * qd + 3]},
-                                                m_base + i * 32 + r1, n_base + j * 32 + 8 * qd + 4 * (lane >> 5), coff);
-        u32x2 w;
-        w[0] = (uint32_t)Elem<T>::from_f32(v[0]) | ((uint32_t)Elem<T>::from_f32(v[1]) << 16);
-        w[1] = (uint32_t)Elem<T>::from_f32(v[2]) | ((uint32_t)Elem<T>::from_f32(v[3]) << 16);
-        *reinterpret_cast<u32x2*>(region + (i * 32 + r1) * RBY + (((4 * j + qd) ^ s1) << 4) + (lane >> 5) * 8) = w;
-      });
-    });
-  });
-  constexpr int RPI = 64 / CPRW;  // rows per copy instruction
-  uint16_t* out = reinterpret_cast<uint16_t*>(q.out) + coff + (int64_t)m_base * q.ldc + n_base + (lane % CPRW) * 8;
-#pragma unroll 4
-  for (int it = 0; it < WTM / RPI; ++it) {
-    const int row = it * RPI + lane / CPRW;
-    const int chunk = (lane % CPRW) ^ ((row / RDIV) & (CPRW - 1));
-    const u32x4 v = *reinterpret_cast<const u32x4*>(region + row * RBY + (chunk << 4));
-    uint16_t* dst = out + (int64_t)row * q.ldc;
-    if (vec == 8) {
-      *reinterpret_cast<u32x4*>(dst) = v;
-    } else if (vec == 4) {
-      *reinterpret_cast<u32x2*>(dst) = u32x2{v[0], v[1]};
-      *reinterpret_cast<u32x2*>(dst + 4) = u32x2{v[2], v[3]};
-    } else if (vec == 2) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) *reinterpret_cast<uint32_t*>(dst + 2 * j) = v[j];
+// Eight results of a row (count of them exist), rounded once, at any alignment: one 16-byte store per 16 bytes.
+template <typename T, bool OutF32>
+__device__ __forceinline__ void store8(void* out, int64_t off, const float (&v)[8], int count) {
+  if constexpr (OutF32) {
+    float* p = reinterpret_cast<float*>(out) + off;
+    if (count >= 8) {
+      __builtin_memcpy(p, v, 32);
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) dst[j] = (uint16_t)(v[j >> 1] >> (16 * (j & 1)));
+      for (int e = 0; e < 7; ++e)
+        if (e < count) p[e] = v[e];
+    }
+  } else {
+    uint16_t* p = reinterpret_cast<uint16_t*>(out) + off;
+    uint16_t h[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) h[e] = Elem<T>::from_f32(v[e]);
+    if (count >= 8) {
+      __builtin_memcpy(p, h, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 7; ++e)
+        if (e < count) p[e] = h[e];
     }
   }
 }
 
+// Epilogue of a wave's 32 TM x 32 TN part of a tile at (m_base, n_base), which may hang over the M x N matrix.
+// acc[i][j][e] is row 32 i + lane % 32, column 32 j + 8 (e / 4) + 4 (lane / 32) + e % 4.  The accumulators go
+// through the wave's LDS region (32 x 32 TN floats, 16-byte chunks XORed by the row so that both passes are free
+// of bank conflicts) one 32-row slab at a time and come back as eight consecutive columns per lane: the addend,
+// the bias and the result move in whole 16-byte pieces (in the accumulator layout a lane has 8 bytes in each of
+// 32 rows, and fetched the bias again for every one of them: 5120 x 2048 x 256 with a bias 28.2 us, without 14.5).
+template <typename T, bool OutF32, int TM, int TN, class Epilogue>
+__device__ __forceinline__ void store_tile(Epilogue& epi, const floatx16 (&acc)[TM][TN], char* region, void* out, int64_t ldc,
+                                           int64_t coff, int M, int N, int m_base, int n_base, int lane) {
+  constexpr int RBY = TN * 128;             // bytes of a row of the region
+  constexpr int XM = TN == 1 ? 7 : 15;      // 16-byte chunks that the XOR moves among
+  constexpr int LPR = TN * 4;               // lanes per row when copying out
+  constexpr int RPI = 64 / LPR;             // rows per copy step
+  const int r1 = lane & 31, h = lane >> 5;
+  const int c8 = lane % LPR;
+  const int n = n_base + c8 * 8;
+  const int count = N - n;
+  const bool whole = m_base + 32 * TM <= M && n_base + 32 * TN <= N;
+  epi.columns(n, count);
+  // The copy-out stays a loop: unrolled, the code outgrew the instruction cache and cost more than the stores
+  // (5120 x 2048 x 256 14.5 -> 26 us).
+  auto fetch_row = [&](int row, float (&v)[8]) {
+    *reinterpret_cast<floatx4*>(v) = *reinterpret_cast<const floatx4*>(region + row * RBY + (((2 * c8) ^ (row & XM)) << 4));
+    *reinterpret_cast<floatx4*>(v + 4) = *reinterpret_cast<const floatx4*>(region + row * RBY + (((2 * c8 + 1) ^ (row & XM)) << 4));
+  };
+  static_for<TM>([&](auto I) {
+    static_for<TN>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      const floatx16 t = acc[decltype(I)::value][j];
+      static_for<4>([&](auto Q) {
+        constexpr int qd = decltype(Q)::value;
+        *reinterpret_cast<floatx4*>(region + r1 * RBY + (((8 * j + 2 * qd + h) ^ (r1 & XM)) << 4)) =
+            floatx4{t[4 * qd], t[4 * qd + 1], t[4 * qd + 2], t[4 * qd + 3]};
+      });
+    });
+    const int m_slab = m_base + decltype(I)::value * 32;
+    if (whole) {  // uniform
+      constexpr int U = 32 / RPI < 4 ? 32 / RPI : 4;  // rows of a lane in flight together
+#pragma unroll 1
+      for (int it = 0; it < 32 / RPI; it += U) {
+        alignas(16) float v[U][8];
+        int rows[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int row = (it + u) * RPI + lane / LPR;
+          fetch_row(row, v[u]);
+          rows[u] = m_slab + row;
+        }
+        epi.template apply<U>(v, rows, n, 8);
+#pragma unroll
+        for (int u = 0; u < U; ++u) store8<T, OutF32>(out, coff + (int64_t)rows[u] * ldc + n, v[u], 8);
+      }
+    } else {
+#pragma unroll 1
+      for (int it = 0; it < 32 / RPI; ++it) {
+        const int row = it * RPI + lane / LPR;
+        if (count > 0 && m_slab + row < M) {
+          alignas(16) float v[1][8];
+          fetch_row(row, v[0]);
+          epi.template apply<1>(v, {m_slab + row}, n, count);
+          store8<T, OutF32>(out, coff + (int64_t)(m_slab + row) * ldc + n, v[0], count);
+        }
+      }
+    }
+  });
+}
+
 // T: element type; OutF32: fp32 output (else T); A_MC / B_MC: operand's free index is
 // contiguous; BM x BN tile; WGM x WGN waves; BK: K step (32 or 64); NSTAGE: LDS stages.
-// SLOW: operands are gathered element by element (Loader::gather_one) instead of loaded directly
-// into LDS; for leading dimensions and row lengths the direct loads cannot take.
-template <typename T, bool OutF32, bool A_MC, bool B_MC, int BM, int BN, int WGM, int WGN, int BK, int NSTAGE,
-          bool SLOW = false>
+template <typename T, bool OutF32, bool A_MC, bool B_MC, int BM, int BN, int WGM, int WGN, int BK, int NSTAGE>
 __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p) {
   constexpr int WTM = BM / WGM, WTN = BN / WGN;
   constexpr int TM = WTM / 32, TN = WTN / 32;
@@ -477,24 +541,12 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p)
   // vmcnt arithmetic below is uniform.
 #pragma unroll
   for (int st = 0; st < NSTAGE - 1; ++st) {
-    if constexpr (SLOW) {
-#pragma unroll
-      for (int i = 0; i < LoaderA::NL; ++i)
-        la.gather_one(i, reinterpret_cast<const uint16_t*>(a_tile), p.lda, p.M - m0, p.K - st * BK,
-                      lds + st * STAGE, wave, lane, p.vec_a);
-#pragma unroll
-      for (int i = 0; i < LoaderB::NL; ++i)
-        lb.gather_one(i, reinterpret_cast<const uint16_t*>(b_tile), p.ldb, p.N - n0, p.K - st * BK,
-                      lds + st * STAGE + A_BYTES, wave, lane, p.vec_b);
-    } else {
-      la.issue(a_tile, p.K - st * BK, lds + st * STAGE, wave);
-      lb.issue(b_tile, p.K - st * BK, lds + st * STAGE + A_BYTES, wave);
-    }
+    la.issue(a_tile, p.K - st * BK, lds + st * STAGE, wave);
+    lb.issue(b_tile, p.K - st * BK, lds + st * STAGE + A_BYTES, wave);
     a_tile += a_step;
     b_tile += b_step;
   }
-  if constexpr (SLOW) __builtin_amdgcn_s_waitcnt(0xc07f);                   // the gathers' LDS stores are done
-  else __builtin_amdgcn_s_waitcnt(vmcnt_imm((NSTAGE - 2) * LOADS));         // step 0 has landed (loads return in order)
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm((NSTAGE - 2) * LOADS));  // step 0 has landed (loads return in order)
   __builtin_amdgcn_s_barrier();
 
   FragAddr<A_MC, BM, BK, TM> faddr;
@@ -545,17 +597,6 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p)
     constexpr bool CHECK_K = decltype(CHECK)::value;
     const int kleft = p.K - (kt + NSTAGE - 1) * BK;
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(a_tile), rb = make_rsrc(b_tile);
-    // Gathering kernel: the whole K step's operand chunks are loaded into registers up front and go
-    // to LDS after the step's MFMAs, which cover most of the load latency.
-    u32x4 ga[SLOW ? LoaderA::NL : 1], gb[SLOW ? LoaderB::NL : 1];
-    if constexpr (SLOW) {
-#pragma unroll
-      for (int i = 0; i < LoaderA::NL; ++i)
-        ga[i] = la.gather_load(i, reinterpret_cast<const uint16_t*>(a_tile), p.lda, p.M - m0, kleft, wave, lane, p.vec_a);
-#pragma unroll
-      for (int i = 0; i < LoaderB::NL; ++i)
-        gb[i] = lb.gather_load(i, reinterpret_cast<const uint16_t*>(b_tile), p.ldb, p.N - n0, kleft, wave, lane, p.vec_b);
-    }
     static_for<KS>([&](auto KSI) {
       constexpr int ks = decltype(KSI)::value;
       // this k-step's share of the loads
@@ -566,24 +607,15 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p)
                                    ~(0xf << 8));  // and lgkmcnt(0)
         __builtin_amdgcn_s_barrier();
       }
-      if constexpr (!SLOW) {
 #pragma unroll
-        for (int i = la0; i < la1; ++i) la.template issue_one<CHECK_K>(i, ra, kleft, wr, wave);
+      for (int i = la0; i < la1; ++i) la.template issue_one<CHECK_K>(i, ra, kleft, wr, wave);
 #pragma unroll
-        for (int i = lb0; i < lb1; ++i) lb.template issue_one<CHECK_K>(i, rb, kleft, wr + A_BYTES, wave);
-      }
+      for (int i = lb0; i < lb1; ++i) lb.template issue_one<CHECK_K>(i, rb, kleft, wr + A_BYTES, wave);
       if constexpr (ks + 1 < KS) read_frags(cur, ks + 1, (ks + 1) & 1);
       else read_frags(nxt, 0, KS & 1);
       mma(ks & 1);
-      interleave(SLOW ? 0 : (la1 - la0) + (lb1 - lb0));
+      interleave((la1 - la0) + (lb1 - lb0));
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (SLOW && ks + 1 == KS) {
-#pragma unroll
-        for (int i = 0; i < LoaderA::NL; ++i) la.scatter_one(i, ga[i], wr, wave, lane);
-#pragma unroll
-        for (int i = 0; i < LoaderB::NL; ++i) lb.scatter_one(i, gb[i], wr + A_BYTES, wave, lane);
-        __builtin_amdgcn_sched_barrier(0);
-      }
     });
     a_tile += a_step;
     b_tile += b_step;
@@ -607,41 +639,11 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p)
 
   // Epilogue.  acc[i][j][e] is out[m][n] with m = m0 + wm WTM + 32 i + lane%32 and
   // n = n0 + wn WTN + 32 j + 8 (e/4) + 4 (lane/32) + e%4.
-  const int64_t coff = bz * p.sc;
-  GemmParams q = p;  // this batch member's view of the output and bias
-  if (p.out_alt[0] && bz > 0) q.out = p.out_alt[bz - 1];
-  if (p.bias) q.bias = reinterpret_cast<const T*>(p.bias) + bz * p.sbias;
-  if constexpr (!OutF32) {
-    static_assert(NSTAGE * STAGE >= BM * BN * 2, "the output tile is staged in the operand stages");
-    const bool inside = m0 + BM <= p.M && n0 + BN <= p.N &&
-                        (!p.c || (p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.c) + coff * 2) % 8 == 0));
-    if (inside) {                      // uniform over the work-group
-      __builtin_amdgcn_s_barrier();    // every wave has read its last fragments
-      char* region = lds + wave * (WTM * WTN * 2);
-      const int mb = m0 + wm * WTM, nb = n0 + wn * WTN;
-      int vec = 8;  // widest store that every row start of this batch member's output allows
-      while (vec > 1 && (p.ldc % vec != 0 || (reinterpret_cast<uintptr_t>(q.out) + coff * 2) % (2 * vec) != 0))
-        vec >>= 1;
-      if (p.alpha == 1.0f && !p.c && !p.bias && p.act == ACT_NONE)
-        store_tile_via_lds<T, true, WTM, WTN, TM, TN>(q, acc, region, mb, nb, coff, lane, vec);
-      else
-        store_tile_via_lds<T, false, WTM, WTN, TM, TN>(q, acc, region, mb, nb, coff, lane, vec);
-      return;
-    }
-  }
-  static_for<TM>([&](auto I) {
-    constexpr int i = decltype(I)::value;
-    const int m = m0 + wm * WTM + i * 32 + (lane & 31);
-    static_for<TN>([&](auto J) {
-      constexpr int j = decltype(J)::value;
-      const floatx16 t = acc[i][j];
-      const int nb = n0 + wn * WTN + j * 32 + (lane >> 5) * 4;
-      store_quad<T, OutF32>(q, floatx4{t[0], t[1], t[2], t[3]}, m, nb, coff);
-      store_quad<T, OutF32>(q, floatx4{t[4], t[5], t[6], t[7]}, m, nb + 8, coff);
-      store_quad<T, OutF32>(q, floatx4{t[8], t[9], t[10], t[11]}, m, nb + 16, coff);
-      store_quad<T, OutF32>(q, floatx4{t[12], t[13], t[14], t[15]}, m, nb + 24, coff);
-    });
-  });
+  static_assert(NSTAGE * STAGE >= NWAVES * TN * 4096, "a slab per wave is staged in the operand stages");
+  __builtin_amdgcn_s_barrier();  // every wave has read its last fragments
+  GemmEpilogue<T, OutF32> epi(p, bz);
+  store_tile<T, OutF32>(epi, acc, lds + wave * (TN * 4096), member_out(p, bz), p.ldc, bz * p.sc, p.M, p.N, m0 + wm * WTM, n0 + wn * WTN,
+                        lane);
 }
 
 // Tile policies, the counterpart of the reference's gemm_policy list
@@ -737,10 +739,9 @@ inline int select_policy(int64_t m, int64_t n, int64_t k, int64_t batch = 1, int
   return best;
 }
 
-template <typename T, bool OutF32, bool A_MC, bool B_MC, int BM, int BN, int WGM, int WGN, int BK, int NSTAGE,
-          bool SLOW = false>
+template <typename T, bool OutF32, bool A_MC, bool B_MC, int BM, int BN, int WGM, int WGN, int BK, int NSTAGE>
 void launch_mfma(const GemmParams& p, int batch, hipStream_t st) {
-  hipLaunchKernelGGL((gemm_mfma_kernel<T, OutF32, A_MC, B_MC, BM, BN, WGM, WGN, BK, NSTAGE, SLOW>),
+  hipLaunchKernelGGL((gemm_mfma_kernel<T, OutF32, A_MC, B_MC, BM, BN, WGM, WGN, BK, NSTAGE>),
                      dim3(p.tiles_m * p.tiles_n, 1, batch), dim3(WGM * WGN * 64), 0, st, p);
 }
 
@@ -765,30 +766,8 @@ void launch_layout_impl(bool a_mc, bool b_mc, int pol, GemmParams& p, int batch,
   else launch_policy<T, OutF32, true, true>(pol, p, batch, st);
 }
 
-
-// The gathering variant (operands the direct loads cannot take) has one tile, 128x128x32 in 3
-// stages: its loads go through registers and are waited for inside the K step, so what hides their
-// latency is occupancy -- 48 KB of LDS and about 150 registers let three work-groups share a CU.
-constexpr Policy kGatherPolicy = {"mfma_128x128x32_w2x2_s3_gather", 128, 128, 2, 2, 32, 3};
-template <typename T, bool OutF32, bool A_MC, bool B_MC>
-void launch_policy_gather(GemmParams& p, int batch, hipStream_t st) {
-  p.tiles_m = (int)xmk::ceil_div(p.M, kGatherPolicy.bm);
-  p.tiles_n = (int)xmk::ceil_div(p.N, kGatherPolicy.bn);
-  launch_mfma<T, OutF32, A_MC, B_MC, 128, 128, 2, 2, 32, 3, true>(p, batch, st);
-}
-
-template <typename T, bool OutF32>
-void launch_layout_gather_impl(bool a_mc, bool b_mc, GemmParams& p, int batch, hipStream_t st) {
-  if (!a_mc && !b_mc) launch_policy_gather<T, OutF32, false, false>(p, batch, st);
-  else if (!a_mc && b_mc) launch_policy_gather<T, OutF32, false, true>(p, batch, st);
-  else if (a_mc && !b_mc) launch_policy_gather<T, OutF32, true, false>(p, batch, st);
-  else launch_policy_gather<T, OutF32, true, true>(p, batch, st);
-}
-
 // Explicitly instantiated in gemm_inst_*.hip.
 template <typename T, bool OutF32>
 void launch_layout(bool a_mc, bool b_mc, int pol, GemmParams& p, int batch, hipStream_t st);
-template <typename T, bool OutF32>
-void launch_layout_gather(bool a_mc, bool b_mc, GemmParams& p, int batch, hipStream_t st);
 
 }  // namespace gemm_impl

@@ -478,3 +478,28 @@ def test_s8_gemm_batched(xmk):
     xmk.run_gemm(a.cuda(), b.cuda(), out)
     torch.cuda.synchronize()
     assert torch.equal(out.cpu(), torch.bmm(a.to(torch.int64), b.to(torch.int64)).to(torch.int32))
+
+
+@pytest.mark.parametrize("dt_name,out_f32", [("BF16", False), ("F16", False), ("BF16", True)])
+@pytest.mark.parametrize("lhs_t,rhs_t", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k", [(8, 9, 9), (9, 8, 15), (65, 129, 65), (127, 63, 8), (64, 64, 63), (130, 515, 1027),
+                                   (1300, 1290, 77)])
+def test_ragged_operands(xmk, oracle, dt_name, out_f32, lhs_t, rhs_t, m, n, k):
+    """Rows that start on any 2-byte boundary and hold no whole number of 16-byte chunks: tiles of 64 and 128, K tails,
+    rows of a single chunk, the K split over caller scratch, outputs of odd row length."""
+    dt = getattr(oracle, dt_name)
+    kind = _kind(dt, oracle)
+    a = oracle.from_f32(oracle.normal((k, m) if lhs_t else (m, k), 90, 0.3), dt)
+    b = oracle.from_f32(oracle.normal((n, k) if rhs_t else (k, n), 91, 0.3), dt)
+    bias = oracle.from_f32(oracle.normal((n,), 92, 0.5), dt)
+    _, ref = oracle.gemm(a, b, dt, oracle.F32 if out_f32 else dt, lhs_t=lhs_t, rhs_t=rhs_t, bias=bias, epilogue=oracle.EPI_BIAS_GELU)
+    da, db = to_dev(a, kind), to_dev(b, kind)
+    tdt = torch.float32 if out_f32 else torch.bfloat16 if kind == "bf16" else torch.float16
+    out = torch.empty((m, n), dtype=tdt, device="cuda")
+    nbytes = xmk.gemm_workspace_bytes(da, db, out, lhs_transpose=lhs_t, rhs_transpose=rhs_t)
+    for ws in (None, torch.empty((nbytes,), dtype=torch.uint8, device="cuda")) if nbytes else (None,):
+        out.fill_(float("nan"))
+        xmk.run_gemm(da, db, out, lhs_transpose=lhs_t, rhs_transpose=rhs_t, bias=to_dev(bias, kind), epilogue=xmk.EPI_BIAS_GELU,
+                     workspace=ws)
+        torch.cuda.synchronize()
+        _check(oracle, out.float().cpu().numpy(), ref[0])
