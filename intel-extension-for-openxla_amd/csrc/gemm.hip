@@ -22,11 +22,11 @@
 // the reference falls back to oneDNN (onednn_matmul_utils.cc:394-491).
 #include <algorithm>
 
-#include "gemm_f32.h"
 #include "gemm_kernel.h"
 #include "gemm_ragged.h"
 #include "gemm_rows.h"
 #include "gemm_s8.h"
+#include "gemm_slices.h"
 
 namespace {
 
@@ -204,13 +204,14 @@ extern "C" const char* xmk_gemm_policy_name(int64_t m, int64_t n, int64_t k, int
   if (dtype_in == XMK_F32 && dtype_out == XMK_F32) return "mfma_f32_128x128x16";
   if (dtype_in == XMK_S8 && dtype_out == XMK_S32) return "mfma_s8_128x128x64";
   if (!sixteen || !(dtype_out == dtype_in || dtype_out == XMK_F32)) return "generic_64x64";
-  // (packed, aligned operands assumed, as everywhere in this query)
+  // (packed operands at aligned addresses assumed, as everywhere in this query)
+  const int packed_class = k % 8 != 0 || (!rhs_transpose && n % 8 != 0) ? kClassRagged : rhs_transpose ? kClassNK : kClassKN;
   int rows_kind = kRowsNone;
   if (m >= 1 && m <= kRowsMaxM && k % 8 == 0) {
     if (!rhs_transpose && n % 8 == 0) rows_kind = kRowsMC;
     if (rhs_transpose && k <= kColsMaxK) rows_kind = kRowsKC;
   }
-  return kPolicies[select_policy(m, n, k, 1, rows_kind, !rhs_transpose)].name;
+  return kPolicies[select_policy(m, n, k, 1, rows_kind, packed_class)].name;
 }
 
 namespace {
@@ -227,8 +228,11 @@ bool direct_ok(const xmk_matrix& lhs, const xmk_matrix& rhs) {
          lhs.num_cols % 8 == 0 && rhs.num_cols % 8 == 0;
 }
 
-// The condition of the ragged 16-bit kernel: the stored rows hold a whole 16-byte chunk.
-bool ragged_ok(const xmk_matrix& lhs, const xmk_matrix& rhs) { return lhs.num_cols >= 8 && rhs.num_cols >= 8; }
+// The condition of the kernels that take any alignment (gemm_loader.h): the stored rows hold a whole 16-byte chunk.
+bool ragged_ok(const xmk_matrix& lhs, const xmk_matrix& rhs, int dtype) {
+  const int chunk = dtype == XMK_F32 ? 4 : 8;
+  return lhs.num_cols >= chunk && rhs.num_cols >= chunk;
+}
 
 // Which streaming kernel for a few rows (gemm_rows.hip) can run this descriptor's product, if any.
 int rows_kind_desc(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k) {
@@ -249,21 +253,21 @@ int plan_splitk(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k, int* po
   *policy = -1;
   *kslice = 0;
   if (d->batch_size != 1) return 1;
-  if (d->dtype_in != XMK_BF16 && d->dtype_in != XMK_F16) return 1;
-  if (!direct_ok(d->lhs, d->rhs)) {
-    if (!ragged_ok(d->lhs, d->rhs)) return 1;
-    // Slices until the tiles are about two work-groups per CU, each slice keeping 256 k.
-    const int tile = ragged_tile(m, n, 1);
-    const int64_t tiles = xmk::ceil_div(m, tile) * xmk::ceil_div(n, tile);
-    const int64_t want = std::min<int64_t>({16, 512 / tiles, k / 256});
-    if (want < 2) return 1;
-    *kslice = (int)(xmk::ceil_div(xmk::ceil_div(k, want), 64) * 64);
-    return (int)xmk::ceil_div(k, *kslice);
-  }
-  auto divides = [&](int ks) { return ks >= 1 && ks <= 16 && k % (ks * 8) == 0; };
+  if (d->dtype_in != XMK_BF16 && d->dtype_in != XMK_F16 && d->dtype_in != XMK_F32) return 1;
   // XMK_GEMM_SPLITK=<slices> overrides the choice (read at every call; the autotuner's handle).
   const char* forced_env = getenv("XMK_GEMM_SPLITK");
   const int forced = forced_env ? atoi(forced_env) : 0;
+  if (d->dtype_in == XMK_F32 || !direct_ok(d->lhs, d->rhs)) {
+    if (!ragged_ok(d->lhs, d->rhs, d->dtype_in)) return 1;
+    Choice c = cheapest(m, n, k, 1, d->dtype_in == XMK_F32 ? kClassF32 : kClassRagged, true);
+    if (forced >= 1) c.slices = forced;
+    if (forced_policy() >= 0) c.policy = forced_policy();
+    if (c.slices < 2) return 1;
+    *policy = c.policy;
+    *kslice = (int)(xmk::ceil_div(xmk::ceil_div(k, c.slices), 64) * 64);
+    return (int)xmk::ceil_div(k, *kslice);
+  }
+  auto divides = [&](int ks) { return ks >= 1 && ks <= 16 && k % (ks * 8) == 0; };
   if (forced >= 1) return divides(forced) ? forced : 1;
   const int rows_kind = (forced_policy() < 0 || forced_policy() == kRowsPolicy) ? rows_kind_desc(d, m, n, k) : kRowsNone;
   const bool rows_ok = rows_kind != kRowsNone;
@@ -284,11 +288,9 @@ int plan_splitk(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k, int* po
     if (ks > 1) *policy = kRowsPolicy;
     return ks;
   }
-  const Policy& pol = kPolicies[select_policy(m, n, k, 1, kRowsNone, !d->rhs.transpose)];
-  const int64_t tiles = xmk::ceil_div(m, pol.bm) * xmk::ceil_div(n, pol.bn);
-  int ks = 1;
-  while (ks < 8 && tiles * ks * 2 <= 256 && k % (ks * 2 * 8) == 0 && k / (ks * 2) >= 512) ks *= 2;
-  return ks;
+  const Choice c = cheapest(m, n, k, 1, d->rhs.transpose ? kClassNK : kClassKN, true);
+  if (c.slices > 1) *policy = c.policy;
+  return c.slices;
 }
 
 // Elements from one slice's partial sums to the next (16-byte aligned).
@@ -313,19 +315,26 @@ extern "C" size_t xmk_gemm_workspace_bytes(const xmk_gemm_desc* d) {
   gemm_dims(d, &m, &n, &k);
   if (m <= 0 || n <= 0 || k <= 0) return 0;
   int pol, kslice;
-  const int ks = plan_splitk(d, m, n, k, &pol, &kslice);
+  int ks = plan_splitk(d, m, n, k, &pol, &kslice);
+  // A long reduction into few tiles keeps asking for scratch where the planner does without a split at present.
+  if (d->batch_size == 1 && n % 4 == 0 && direct_ok(d->lhs, d->rhs) && (d->dtype_in == XMK_BF16 || d->dtype_in == XMK_F16)) {
+    const int64_t tiles = xmk::ceil_div(m, 64) * xmk::ceil_div(n, 64);
+    int wide = 1;
+    while (wide < 8 && tiles * wide * 2 <= 256 && k % (wide * 2 * 8) == 0 && k / (wide * 2) >= 512) wide *= 2;
+    ks = std::max(ks, wide);
+  }
   return ks > 1 ? (size_t)ks * slice_stride(m, n) * sizeof(float) : 0;
 }
 
 extern "C" int xmk_gemm_ws(const xmk_gemm_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
   if (!d) return xmk::fail(XMK_INVALID_ARGUMENT, "gemm: null descriptor");
-  const size_t need = xmk_gemm_workspace_bytes(d);
-  if (need == 0 || !workspace || workspace_bytes < need || !xmk::aligned(workspace, 16) || d->lhs.transpose)
-    return run_gemm(d, nullptr, nullptr, stream);
+  if (!workspace || !xmk::aligned(workspace, 16) || d->lhs.transpose || d->out.transpose) return run_gemm(d, nullptr, nullptr, stream);
   int64_t m, n, k;
   gemm_dims(d, &m, &n, &k);
+  if (m <= 0 || n <= 0 || k <= 0) return run_gemm(d, nullptr, nullptr, stream);  // reports the error
   int slice_policy, kslice;
   const int ks = plan_splitk(d, m, n, k, &slice_policy, &kslice);
+  if (ks < 2 || workspace_bytes < (size_t)ks * slice_stride(m, n) * sizeof(float)) return run_gemm(d, nullptr, nullptr, stream);
   // Pass 1: the K slices as a batched GEMM into fp32 partial sums (no epilogue); a slice is a
   // column range of lhs and a row (or column) range of rhs, so only the batch strides change.
   xmk_gemm_desc p = *d;
@@ -456,10 +465,8 @@ int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int p
   const bool sixteen = din == XMK_BF16 || din == XMK_F16;
   const bool fast = sixteen && direct_ok(lhs, rhs) && xmk::aligned(out.data, 16) && xmk::aligned(out1, 16) &&
                     xmk::aligned(out2, 16);
-  // 16-bit operands that miss those conditions, and outputs of any alignment (fp32 outputs are stored in
-  // aligned quads): the ragged kernel.
-  const bool ragged = !fast && sixteen && ragged_ok(lhs, rhs) &&
-                      (dout != XMK_F32 || (xmk::aligned(out.data, 16) && xmk::aligned(out1, 16) && xmk::aligned(out2, 16)));
+  // 16-bit operands that miss those conditions and fp32 operands: the kernels that take any alignment.
+  const bool ragged = !fast && (sixteen || din == XMK_F32) && ragged_ok(lhs, rhs, din);
   if (fast || ragged) {
     GemmParams p;
     p.a = lhs.data; p.b = rhs.data; p.out = out.data; p.c = d->beta != 0.0f ? d->c : nullptr;
@@ -476,22 +483,29 @@ int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int p
     const bool b_mc = rhs.transpose == 0;   // stored [K, N]
     const int batch = qkv ? 3 : (int)d->batch_size;
     const int rows_kind = fast ? gemm_rows_applicable(p, a_mc, b_mc) : kRowsNone;
-    // the forced policy first, then the K-split planner's, then the table and the rules
+    // the forced policy first, then the K-split planner's, then the table and the rules (three products that share
+    // an operand take the tile one of them would: the results are then the same bits)
     const int pol = (forced_policy() < 0 && policy >= 0 && policy < kNumPolicies &&
                      (policy != kRowsPolicy || rows_kind != kRowsNone))
-                        ? policy : select_policy(m, n, k, batch, rows_kind, b_mc);
-    const int tile = ragged_tile(m, n, kslice ? 1 : batch);
+                        ? policy : select_policy(m, n, k, qkv ? 1 : batch, qkv ? kRowsNone : rows_kind, din == XMK_F32 ? kClassF32 : ragged ? kClassRagged : b_mc ? kClassKN : kClassNK);
     xmk::trace("gemm m=%lld n=%lld k=%lld batch=%lld lhs_t=%d rhs_t=%d epilogue=%d beta=%g -> %s",
                (long long)m, (long long)n, (long long)k, (long long)d->batch_size, lhs.transpose,
-               rhs.transpose, d->epilogue, d->beta, !ragged ? kPolicies[pol].name : tile == 128 ? "ragged_128x128x64" : "ragged_64x64x64");
+               rhs.transpose, d->epilogue, d->beta,
+               !ragged || pol >= kSlicesPolicy ? kPolicies[pol].name : kPolicies[pol].bm == 128 ? "ragged_128x128" : "ragged_64x64");
+    // f(element type, fp32 output)
+    auto typed = [&](auto&& f) {
+      if (din == XMK_F32) f(float{}, std::true_type{});
+      else if (din == XMK_BF16 && dout == XMK_F32) f(__bf16{}, std::true_type{});
+      else if (din == XMK_BF16) f(__bf16{}, std::false_type{});
+      else if (dout == XMK_F32) f(_Float16{}, std::true_type{});
+      else f(_Float16{}, std::false_type{});
+    };
+    if (pol >= kSlicesPolicy) {
+      typed([&](auto t, auto o) { launch_slices<decltype(t), decltype(o)::value>(a_mc, b_mc, pol - kSlicesPolicy, p, batch, st); });
+      return xmk::check_launch("gemm");
+    }
     if (ragged) {
-      if (din == XMK_BF16) {
-        if (dout == XMK_F32) launch_ragged<__bf16, true>(a_mc, b_mc, p, batch, tile, st);
-        else launch_ragged<__bf16, false>(a_mc, b_mc, p, batch, tile, st);
-      } else {
-        if (dout == XMK_F32) launch_ragged<_Float16, true>(a_mc, b_mc, p, batch, tile, st);
-        else launch_ragged<_Float16, false>(a_mc, b_mc, p, batch, tile, st);
-      }
+      typed([&](auto t, auto o) { launch_ragged<decltype(t), decltype(o)::value>(a_mc, b_mc, p, batch, kPolicies[pol].bm, st); });
       return xmk::check_launch("gemm");
     }
     if (pol == kRowsPolicy) {
@@ -508,27 +522,6 @@ int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int p
     return xmk::check_launch("gemm");
   }
 
-  if (din == XMK_F32 && dout == XMK_F32 && xmk::aligned(out.data, 16) && xmk::aligned(out1, 16) &&
-      xmk::aligned(out2, 16) && xmk::aligned(d->c, 16) && xmk::aligned(lhs.data, 4) && xmk::aligned(rhs.data, 4)) {
-    GemmParams p;
-    p.a = lhs.data; p.b = rhs.data; p.out = out.data; p.c = d->beta != 0.0f ? d->c : nullptr;
-    p.bias = wants_bias ? d->bias : nullptr;
-    p.M = (int)m; p.N = (int)n; p.K = (int)k;
-    p.lda = lhs.leading_dim_stride; p.ldb = rhs.leading_dim_stride; p.ldc = out.leading_dim_stride;
-    p.sa = lhs.batch_stride; p.sb = rhs.batch_stride; p.sc = out.batch_stride;
-    p.alpha = d->alpha; p.beta = d->beta; p.act = act;
-    p.out_alt[0] = out1; p.out_alt[1] = out2; p.sbias = 0;
-    if (qkv) { p.sa = 0; p.sc = 0; p.sbias = n; }
-    auto vec4 = [](const xmk_matrix& x) {
-      return (xmk::aligned(x.data, 16) && x.leading_dim_stride % 4 == 0 && x.batch_stride % 4 == 0 && x.num_cols % 4 == 0) ? 4 : 1;
-    };
-    p.vec_a = vec4(lhs);
-    p.vec_b = vec4(rhs);
-    xmk::trace("gemm m=%lld n=%lld k=%lld batch=%lld lhs_t=%d rhs_t=%d -> mfma_f32_128x128x16", (long long)m,
-               (long long)n, (long long)k, (long long)d->batch_size, lhs.transpose, rhs.transpose);
-    launch_gemm_f32(p, lhs.transpose != 0, rhs.transpose == 0, qkv ? 3 : (int)d->batch_size, st);
-    return xmk::check_launch("gemm");
-  }
   if (din == XMK_S8 && (d->alpha != 1.0f || d->beta != 0.0f || d->epilogue != XMK_EPI_DEFAULT))
     return xmk::fail(XMK_UNIMPLEMENTED, "gemm: s8 x s8 -> s32 supports alpha=1, beta=0, no epilogue");
   if (din == XMK_S8 && dout == XMK_S32 && xmk::aligned(out.data, 16) && xmk::aligned(out1, 16) && xmk::aligned(out2, 16)) {

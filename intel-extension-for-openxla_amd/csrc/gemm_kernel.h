@@ -4,6 +4,8 @@
 #pragma once
 #include <hip/hip_bf16.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <utility>
 
@@ -38,8 +40,8 @@ struct GemmParams {
   // out_alt[z - 1] instead of out + z * sc and reads bias + z * sbias.  Null when unused.
   void* out_alt[2];
   int64_t sbias;
-  // fp32 and int8 kernels only: elements per load that the alignment of each operand's pointer, leading
-  // dimension, batch stride and row length allows.
+  // int8 kernel only: elements per load that the alignment of each operand's pointer, leading dimension, batch
+  // stride and row length allows.
   int vec_a, vec_b;
   // Ragged kernel only: K slice of one grid member (a multiple of its K step), 0 when K is not split.
   int kslice;
@@ -119,6 +121,7 @@ typedef __attribute__((address_space(3))) void* lds_void_ptr;
 template <bool MC, int ROWS, int BK, int EB = 2>
 __device__ __forceinline__ int swz(int row_or_k) {
   if constexpr (!MC) return BK == 64 ? ((row_or_k >> 1) & 7) : ((row_or_k >> 2) & 3);
+  else if constexpr (ROWS < 64) return 0;  // four rows of 64 bytes are one sweep of the banks
   else if constexpr (ROWS < 128) return (row_or_k & 3) << 1;  // 8 chunks per row: the XOR stays below 8
   else if constexpr (EB == 1) return (row_or_k & 7) << 1;
   else return (row_or_k & 3) << 2;
@@ -651,19 +654,29 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p)
 struct Policy {
   const char* name;
   int bm, bn, wgm, wgn, bk, stages;
+  bool alone;          // one work-group fills a CU (LDS)
+  bool any_alignment;  // also a tile of the kernels that take any alignment (gemm_ragged.h, gemm_slices.h)
 };
 constexpr Policy kPolicies[] = {
-    {"mfma_256x256x32_w2x2_s4", 256, 256, 2, 2, 32, 4},
-    {"mfma_128x128x64_w2x2_s3", 128, 128, 2, 2, 64, 3},
-    {"mfma_128x64x64_w2x2_s4", 128, 64, 2, 2, 64, 4},
-    {"mfma_64x64x64_w2x2_s4", 64, 64, 2, 2, 64, 4},
-    {"mfma_256x128x64_w2x2_s3", 256, 128, 2, 2, 64, 3},
+    {"mfma_256x256x32_w2x2_s4", 256, 256, 2, 2, 32, 4, true, false},
+    {"mfma_128x128x64_w2x2_s3", 128, 128, 2, 2, 64, 3, true, true},
+    {"mfma_128x64x64_w2x2_s4", 128, 64, 2, 2, 64, 4, true, false},
+    {"mfma_64x64x64_w2x2_s4", 64, 64, 2, 2, 64, 4, false, true},
+    {"mfma_256x128x64_w2x2_s3", 256, 128, 2, 2, 64, 3, true, false},
     // not a matrix-core tile: the streaming kernel for up to eight rows (gemm_rows.hip), eight waves
     // that split the reduction of a 512-column block
-    {"stream_rows_8x512_w8", 8, 512, 8, 1, 8, 2},
+    {"stream_rows_8x512_w8", 8, 512, 8, 1, 8, 2, true, false},
+    // small tiles whose reduction is split over the waves of a work-group (gemm_slices.h)
+    {"slices_32x32_w4", 32, 32, 4, 1, 64, 2, false, true},
+    {"slices_32x32_w8", 32, 32, 8, 1, 64, 2, true, true},
+    {"slices_32x32_w16", 32, 32, 16, 1, 64, 2, true, true},
+    {"slices_32x64_w8", 32, 64, 8, 1, 64, 2, true, true},
+    {"slices_64x64_w4", 64, 64, 4, 1, 64, 2, false, true},
+    {"slices_64x64_w8", 64, 64, 8, 1, 64, 2, true, true},
 };
 constexpr int kNumPolicies = sizeof(kPolicies) / sizeof(kPolicies[0]);
-constexpr int kRowsPolicy = kNumPolicies - 1;
+constexpr int kRowsPolicy = 5;
+constexpr int kSlicesPolicy = 6;        // first of the slices variants
 constexpr int kRowsMaxM = 8;            // rows the streaming kernel takes
 constexpr int kRowsMinBN = 64;          // its output columns per work-group: 64, 128, 256 or 512
 constexpr int kRowsEnoughBlocks = 192;  // work-groups from which on a launch pulls the memory system's rate
@@ -708,35 +721,133 @@ inline int forced_policy() {
   }
   return -1;
 }
+// Which kernels a product's operands allow, and which cost table below applies.
+enum : int { kClassKN = 0, kClassNK = 1, kClassRagged = 2, kClassF32 = 3 };
+
+// Estimated microseconds of a launch: with KT K steps of 128 bytes, KTw = ceil(KT / waves that split K) of them per
+// wave, and L output tiles per CU (the mean of the tiles / 256 and, for kernels of which one work-group fills a CU,
+// that rounded up; at least 1),
+//     start + step * KTw + fill * KT * min(tiles / 256, 1) / 8 + (L - 1) * (more_step * KT + more).
+// Least-squares fits (non-negative, relative error) to 380 shapes per class, m 1 .. 8192, n and k 64 .. 16384 at
+// random, every policy: mean error 5 - 12 %; the policy that this picks is on average 2 % (fp32: 4 %) slower than the
+// best of all measured, where tile rate x occupancy x inside area, the rule before, lost 7 - 26 %.
+struct TileCost {
+  float start, step, more_step, more, fill;
+};
+constexpr TileCost kTileCost[4][kNumPolicies] = {
+    {  // 16-bit direct, B stored [K, N]
+     {8.373f, 0.954f, 1.661f, 15.214f, 4.693f},
+     {4.788f, 0.378f, 0.591f, 4.147f, 1.594f},
+     {3.925f, 0.223f, 0.354f, 2.871f, 1.259f},
+     {3.315f, 0.176f, 0.248f, 0.898f, 0.942f},
+     {6.316f, 0.534f, 0.953f, 7.21f, 2.587f},
+     {},
+     {3.273f, 0.446f, 0.13f, 0.989f, 0.957f},
+     {2.886f, 0.741f, 0.146f, 1.178f, 1.332f},
+     {2.15f, 1.583f, 0.154f, 1.989f, 1.236f},
+     {2.848f, 1.134f, 0.18f, 2.468f, 1.249f},
+     {4.155f, 0.935f, 0.288f, 4.668f, 1.363f},
+     {3.083f, 1.668f, 0.28f, 3.357f, 1.473f},
+    },
+    {  // 16-bit direct, B stored [N, K]
+     {8.285f, 0.961f, 1.792f, 14.552f, 5.814f},
+     {4.513f, 0.321f, 0.584f, 3.969f, 2.095f},
+     {3.939f, 0.228f, 0.359f, 2.89f, 1.152f},
+     {3.306f, 0.181f, 0.249f, 0.916f, 0.777f},
+     {6.152f, 0.49f, 0.956f, 6.848f, 2.857f},
+     {},
+     {3.226f, 0.389f, 0.115f, 0.532f, 0.575f},
+     {3.015f, 0.611f, 0.129f, 1.129f, 0.808f},
+     {2.413f, 1.299f, 0.135f, 2.04f, 0.789f},
+     {2.88f, 1.036f, 0.177f, 2.48f, 1.265f},
+     {4.164f, 0.838f, 0.286f, 4.583f, 1.295f},
+     {3.141f, 1.517f, 0.272f, 3.334f, 1.384f},
+    },
+    {  // 16-bit, any alignment
+     {},
+     {5.132f, 0.864f, 0.735f, 2.1f, 1.177f},
+     {},
+     {3.342f, 0.416f, 0.347f, 0.429f, 1.271f},
+     {},
+     {},
+     {3.537f, 0.554f, 0.16f, 0.842f, 1.054f},
+     {2.936f, 1.095f, 0.178f, 1.369f, 1.239f},
+     {1.897f, 2.27f, 0.184f, 2.157f, 1.15f},
+     {2.919f, 1.783f, 0.249f, 2.844f, 0.952f},
+     {4.859f, 1.118f, 0.353f, 5.027f, 1.788f},
+     {3.277f, 2.307f, 0.379f, 3.525f, 1.647f},
+    },
+    {  // fp32
+     {},
+     {4.318f, 2.272f, 2.212f, 5.565f, 2.005f},
+     {},
+     {3.0f, 0.69f, 0.54f, 0.959f, 1.348f},
+     {},
+     {},
+     {3.369f, 0.742f, 0.179f, 1.072f, 0.546f},
+     {3.031f, 1.28f, 0.193f, 1.82f, 0.775f},
+     {1.889f, 3.022f, 0.214f, 2.796f, 0.817f},
+     {2.62f, 2.464f, 0.321f, 3.37f, 0.993f},
+     {4.534f, 2.268f, 0.601f, 5.912f, 2.133f},
+     {2.298f, 4.447f, 0.57f, 5.419f, 2.004f},
+    },
+};
+// What a K split adds for its second launch, and the least it takes end to end when launched from a host program.
+constexpr float kSplitCost = 4.0f, kSplitFloor = 8.0f;
+
+inline float tile_cost(int pol, uint32_t m, uint32_t n, uint32_t k, uint32_t batch, int cls) {
+  const Policy& P = kPolicies[pol];
+  const TileCost& c = kTileCost[cls][pol];
+  auto blocks = [](uint32_t v, int b) { return (v + b - 1) >> __builtin_ctz((unsigned)b); };  // b: a power of two
+  const uint64_t tiles = (uint64_t)blocks(m, P.bm) * blocks(n, P.bn) * batch;
+  const float load = (float)tiles * (1.0f / 256);
+  const uint32_t kt = blocks(k, cls == kClassF32 ? 32 : 64);
+  const uint32_t ktw = pol >= kSlicesPolicy ? blocks(kt, P.wgm) : kt;
+  const float l = P.alone ? 0.5f * (load + (float)((tiles + 255) >> 8)) : load;
+  return c.start + c.step * (float)ktw + c.fill * (float)kt * (load < 1.0f ? load : 1.0f) * 0.125f +
+         (l > 1.0f ? l - 1.0f : 0.0f) * (c.more_step * (float)kt + c.more);
+}
+
+struct Choice {
+  int policy, slices;
+};
+// The cheapest policy and number of K slices (1 unless may_split; direct kernels: only slices of whole chunks).
+inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, bool may_split) {
+  Choice best{3, 1};
+  float best_cost = 1e30f;
+  const bool direct = cls == kClassKN || cls == kClassNK;
+  auto each = [&](int s, float extra, float least) {
+    for (int pol = 0; pol < kNumPolicies; ++pol) {
+      if (pol == kRowsPolicy || (!direct && !kPolicies[pol].any_alignment)) continue;
+      const float cost = std::max(tile_cost(pol, (uint32_t)m, (uint32_t)n, (uint32_t)((k + s - 1) / s), (uint32_t)(batch * s), cls) + extra, least);
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = {pol, s};
+      }
+    }
+  };
+  each(1, 0.0f, 0.0f);
+  for (int s = 2; may_split && s <= 16 && best_cost > kSplitFloor; s *= 2) {
+    if (k / s < 128 || (direct && k % (8 * s) != 0) || (float)m * (float)n * (float)s > 6.4e7f) break;
+    each(s, kSplitCost + (float)m * (float)n * (float)s * (8.0f / 3e6f), kSplitFloor);
+  }
+  return best;
+}
+
 // rows_kind: which streaming kernel the operands allow (gemm_rows_applicable); it is never chosen otherwise.
-// tuned_ok: the operands have the layout the tuned table was measured with (B stored [K, N]).
-inline int select_policy(int64_t m, int64_t n, int64_t k, int64_t batch = 1, int rows_kind = kRowsNone,
-                         bool tuned_ok = true) {
+// The tuned table applies to the layout it was measured with (direct operands, B stored [K, N]).
+inline int select_policy(int64_t m, int64_t n, int64_t k, int64_t batch, int rows_kind, int cls) {
   const bool rows_ok = rows_kind != kRowsNone;
-  auto usable = [&](int v) { return v >= 0 && v < kNumPolicies && (v != kRowsPolicy || rows_ok); };
+  const bool direct = cls == kClassKN || cls == kClassNK;
+  auto usable = [&](int v) {
+    return v >= 0 && v < kNumPolicies && (v != kRowsPolicy || rows_ok) && (direct || kPolicies[v].any_alignment);
+  };
   if (const int v = forced_policy(); usable(v)) return v;
-  if (batch == 1 && tuned_ok)
+  if (batch == 1 && cls == kClassKN)
     if (const TunedShape* t = tuned_shape(m, n, k); t && t->ksplit <= 1 && usable(t->policy)) return t->policy;
   // A few rows against a very wide matrix: stream it.
   if (batch == 1 && rows_streams_by_default(rows_kind, m, n)) return kRowsPolicy;
-  // Heuristic: the policy with the best estimated throughput = (what the tile sustains when the
-  // device is full) x (share of the 256 CUs busy over the tile waves) x (share of the tiles' area
-  // inside the matrix).  The per-tile figures are measured large-shape rates relative to 256x256.
-  static constexpr float kTileRate[kRowsPolicy] = {1.0f, 0.75f, 0.60f, 0.55f, 0.90f};
-  int best = kRowsPolicy - 1;
-  float best_score = -1.0f;
-  for (int i = 0; i < kRowsPolicy; ++i) {
-    const int64_t tiles = xmk::ceil_div(m, kPolicies[i].bm) * xmk::ceil_div(n, kPolicies[i].bn) * batch;
-    const int64_t waves = xmk::ceil_div(tiles, 256);
-    const float busy = (float)tiles / (float)(waves * 256);
-    const float inside = (float)((double)m * (double)n / ((double)tiles * kPolicies[i].bm * kPolicies[i].bn));
-    const float score = kTileRate[i] * busy * inside;
-    if (score > best_score) {
-      best = i;
-      best_score = score;
-    }
-  }
-  return best;
+  return cheapest(m, n, k, batch, cls, false).policy;
 }
 
 template <typename T, bool OutF32, bool A_MC, bool B_MC, int BM, int BN, int WGM, int WGN, int BK, int NSTAGE>

@@ -1,0 +1,165 @@
+// MFMA GEMM for products with too few output tiles to fill the device: a small tile per work-group, the reduction
+// split over the work-group's waves.
+//
+// What bounds these products is latency, not a rate: with one 64 x 64 tile per CU the tile kernels spend 0.3 us per
+// 64 k waiting for the three K steps they keep in flight.  Here each of the NW waves owns the whole 32 TM x 32 TN
+// tile for every NW-th K step, keeps two of its K steps in flight in registers (NW times the bytes in flight per
+// CU), passes them through an LDS region of its own (no barrier in the loop: the LDS serves a wave in order), and
+// the waves' partial sums meet in LDS once at the end, added in wave order.  Small tiles also make more
+// work-groups out of a small output.  Operands of any alignment, 16-bit and fp32 (gemm_loader.h).
+#pragma once
+#include "gemm_loader.h"
+
+namespace gemm_impl {
+
+template <typename T, bool OutF32, bool A_MC, bool B_MC, int TM, int TN, int NW>
+__global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(GemmParams p) {
+  constexpr int BK = 128 / sizeof(T), KS = 4;
+  constexpr int STAGE = (TM + TN) * 4096;                 // LDS per wave
+  constexpr int RBY = TN * 128, XM = TN == 1 ? 7 : 15;    // partial sums: as in store_tile
+  static_assert(STAGE >= TM * TN * 4096, "a wave's partial sums replace its operands");
+  typedef AnyLoader<T, A_MC, 32 * TM, 64> LoaderA;
+  typedef AnyLoader<T, B_MC, 32 * TN, 64> LoaderB;
+  typedef typename Elem<T>::vec8 V8;
+  __shared__ __attribute__((aligned(1024))) char lds[NW * STAGE];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int pid = blockIdx.x;  // consecutive blocks go to different XCDs: each gets a contiguous run of tiles
+  const int ntiles = p.tiles_m * p.tiles_n;
+  if (ntiles % 8 == 0) pid = (pid % 8) * (ntiles / 8) + pid / 8;
+  const int m0 = pid % p.tiles_m * (32 * TM), n0 = pid / p.tiles_m * (32 * TN);
+
+  const int64_t bz = blockIdx.z;
+  const int64_t k0 = bz * p.kslice;  // as in gemm_ragged_kernel
+  const int K = p.kslice ? min(p.K - (int)k0, p.kslice) : p.K;
+  const char* a_base = (const char*)(reinterpret_cast<const T*>(p.a) + bz * p.sa + (A_MC ? k0 * p.lda : (int64_t)m0 * p.lda + k0));
+  const char* b_base = (const char*)(reinterpret_cast<const T*>(p.b) + bz * p.sb + (B_MC ? k0 * p.ldb : (int64_t)n0 * p.ldb + k0));
+  const int64_t a_step = (A_MC ? BK * p.lda : BK) * (int64_t)sizeof(T), b_step = (B_MC ? BK * p.ldb : BK) * (int64_t)sizeof(T);
+  const bool a_edge = A_MC && m0 + 32 * TM > p.M, b_edge = B_MC && n0 + 32 * TN > p.N;
+  LoaderA la;
+  LoaderB lb;
+  la.init(p.lda, m0, p.M, lane);
+  lb.init(p.ldb, n0, p.N, lane);
+  AnyFrag<T, A_MC, 32 * TM, TM> faddr;
+  AnyFrag<T, B_MC, 32 * TN, TN> fbddr;
+  faddr.init(0, lane);
+  fbddr.init(0, lane);
+
+  floatx16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = zero16();
+
+  const int KT = (K + BK - 1) / BK;
+  char* region = lds + wave * STAGE;
+  u32x4 ga[2][LoaderA::NL], gb[2][LoaderB::NL];
+  auto load = [&](int kt, u32x4 (&a)[LoaderA::NL], u32x4 (&b)[LoaderB::NL]) {
+    const char *ap = a_base + kt * a_step, *bp = b_base + kt * b_step;
+    const int kleft = K - kt * BK;
+    if (kleft >= BK) {
+      la.load(ap, a);
+      lb.load(bp, b);
+    } else {
+      la.load_tail(ap, p.lda, kleft, a);
+      lb.load_tail(bp, p.ldb, kleft, b);
+    }
+  };
+  // Multiplies K step kt, which is in the registers a and b, and sends K step kt + 2 NW into them.
+  auto step = [&](int kt, u32x4 (&a)[LoaderA::NL], u32x4 (&b)[LoaderB::NL]) {
+    const int kleft = K - kt * BK;
+    if (kleft < BK) {
+      la.fix_tail(kleft, a);
+      lb.fix_tail(kleft, b);
+    }
+    la.store(region, lane, a_edge, a);
+    lb.store(region + TM * 4096, lane, b_edge, b);
+    if (kt + 2 * NW < KT) load(kt + 2 * NW, a, b);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      V8 fa[TM], fb[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fa[i] = faddr.read(region, i, ks);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) fb[j] = fbddr.read(region + TM * 4096, j, ks);
+      mma_block<T, TM, TN>(acc, fa, fb);
+    }
+  };
+  if (wave < KT) load(wave, ga[0], gb[0]);
+  if (wave + NW < KT) load(wave + NW, ga[1], gb[1]);
+  for (int kt = wave; kt < KT; kt += 2 * NW) {
+    step(kt, ga[0], gb[0]);
+    if (kt + NW < KT) step(kt + NW, ga[1], gb[1]);
+  }
+
+  // The waves' partial sums, in store_tile's layout (slab i of 32 rows after the other).
+  const int r1 = lane & 31, h = lane >> 5;
+  static_for<TM>([&](auto I) {
+    constexpr int i = decltype(I)::value;
+    static_for<TN>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      const floatx16 t = acc[i][j];
+      static_for<4>([&](auto Q) {
+        constexpr int qd = decltype(Q)::value;
+        *reinterpret_cast<floatx4*>(region + (i * 32 + r1) * RBY + (((8 * j + 2 * qd + h) ^ (r1 & XM)) << 4)) =
+            floatx4{t[4 * qd], t[4 * qd + 1], t[4 * qd + 2], t[4 * qd + 3]};
+      });
+    });
+  });
+  // Eight columns of a row per thread.
+  constexpr int GROUPS = 128 * TM * TN, GPT = (GROUPS + NW * 64 - 1) / (NW * 64);
+  const int waves = min(NW, KT);  // waves that had a K step
+  GemmEpilogue<T, OutF32> epi(p, bz);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < GPT; ++u) {
+    const int gidx = u * NW * 64 + tid;
+    const int row = gidx / (4 * TN), c8 = gidx % (4 * TN);
+    const int m = m0 + row, n = n0 + c8 * 8, count = p.N - n;
+    if ((GROUPS % (NW * 64) == 0 || gidx < GROUPS) && m < p.M && count > 0) {
+      epi.columns(n, count);
+      const char* src = lds + row * RBY;
+      const int lo = ((2 * c8) ^ (row & XM)) << 4, hi = ((2 * c8 + 1) ^ (row & XM)) << 4;
+      floatx4 s0 = *reinterpret_cast<const floatx4*>(src + lo), s1 = *reinterpret_cast<const floatx4*>(src + hi);
+      for (int w = 1; w < waves; ++w) {
+        s0 += *reinterpret_cast<const floatx4*>(src + w * STAGE + lo);
+        s1 += *reinterpret_cast<const floatx4*>(src + w * STAGE + hi);
+      }
+      float v[1][8] = {{s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]}};
+      epi.template apply<1>(v, {m}, n, count);
+      store8<T, OutF32>(member_out(p, bz), bz * p.sc + (int64_t)m * p.ldc + n, v[0], count);
+    }
+  }
+}
+
+// The kernel's variants, by index from kSlicesPolicy on in kPolicies.
+template <typename T, bool OutF32, bool A_MC, bool B_MC>
+void launch_slices_variant(int v, GemmParams& p, int batch, hipStream_t st) {
+  const Policy& pol = kPolicies[kSlicesPolicy + v];
+  p.tiles_m = (int)xmk::ceil_div(p.M, pol.bm);
+  p.tiles_n = (int)xmk::ceil_div(p.N, pol.bn);
+  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)batch), block((unsigned)(pol.wgm * 64));
+  switch (v) {
+    case 0: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 1, 4>), grid, block, 0, st, p); break;
+    case 1: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 1, 8>), grid, block, 0, st, p); break;
+    case 2: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 1, 16>), grid, block, 0, st, p); break;
+    case 3: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 2, 8>), grid, block, 0, st, p); break;
+    case 4: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 2, 2, 4>), grid, block, 0, st, p); break;
+    default: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 2, 2, 8>), grid, block, 0, st, p); break;
+  }
+}
+
+template <typename T, bool OutF32>
+void launch_slices_impl(bool a_mc, bool b_mc, int v, GemmParams& p, int batch, hipStream_t st) {
+  if (!a_mc && !b_mc) launch_slices_variant<T, OutF32, false, false>(v, p, batch, st);
+  else if (!a_mc && b_mc) launch_slices_variant<T, OutF32, false, true>(v, p, batch, st);
+  else if (a_mc && !b_mc) launch_slices_variant<T, OutF32, true, false>(v, p, batch, st);
+  else launch_slices_variant<T, OutF32, true, true>(v, p, batch, st);
+}
+
+// Explicitly instantiated in gemm_inst_slices_*.hip.
+template <typename T, bool OutF32>
+void launch_slices(bool a_mc, bool b_mc, int v, GemmParams& p, int batch, hipStream_t st);
+
+}  // namespace gemm_impl

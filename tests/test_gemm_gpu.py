@@ -503,3 +503,30 @@ def test_ragged_operands(xmk, oracle, dt_name, out_f32, lhs_t, rhs_t, m, n, k):
                      workspace=ws)
         torch.cuda.synchronize()
         _check(oracle, out.float().cpu().numpy(), ref[0])
+
+
+@pytest.mark.parametrize("policy", [1, 3, 6, 7, 8, 9, 10, 11])
+@pytest.mark.parametrize("dt_name", ["BF16", "F16", "F32"])
+@pytest.mark.parametrize("lhs_t,rhs_t", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k", [(8, 8, 8), (9, 11, 13), (33, 40, 72), (64, 65, 1100), (100, 136, 200)])
+def test_small_products(xmk, oracle, monkeypatch, policy, dt_name, lhs_t, rhs_t, m, n, k):
+    """Every tile of the kernels that split K over a work-group's waves, and fp32 on both tile edges: aligned and ragged
+    operands, fewer K steps than waves and more, K tails, tiles that hang over; unsplit and K-split into scratch."""
+    monkeypatch.setenv("XMK_GEMM_POLICY", str(policy))
+    dt = getattr(oracle, dt_name)
+    kind = "f32" if dt_name == "F32" else _kind(dt, oracle)
+    a = oracle.from_f32(oracle.normal((k, m) if lhs_t else (m, k), 95, 0.3), dt)
+    b = oracle.from_f32(oracle.normal((n, k) if rhs_t else (k, n), 96, 0.3), dt)
+    c = oracle.from_f32(oracle.normal((m, n), 97, 1.0), dt)
+    bias = oracle.from_f32(oracle.normal((n,), 98, 0.5), dt)
+    _, ref = oracle.gemm(a, b, dt, dt, lhs_t=lhs_t, rhs_t=rhs_t, c=c, bias=bias, beta=0.5, epilogue=oracle.EPI_BIAS_RELU)
+    da, db = to_dev(a, kind), to_dev(b, kind)
+    for split in ("1", "3"):
+        monkeypatch.setenv("XMK_GEMM_SPLITK", split)
+        out = to_dev(c, kind)
+        nbytes = xmk.gemm_workspace_bytes(da, db, out, lhs_transpose=lhs_t, rhs_transpose=rhs_t)
+        ws = torch.empty((nbytes,), dtype=torch.uint8, device="cuda") if nbytes else None
+        xmk.run_gemm(da, db, out, lhs_transpose=lhs_t, rhs_transpose=rhs_t, c=out, beta=0.5, bias=to_dev(bias, kind),
+                     epilogue=xmk.EPI_BIAS_RELU, workspace=ws)
+        torch.cuda.synchronize()
+        _check(oracle, out.float().cpu().numpy(), ref[0], tol=1e-5 if dt_name == "F32" else TOL)
