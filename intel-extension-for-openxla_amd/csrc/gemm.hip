@@ -228,12 +228,6 @@ bool direct_ok(const xmk_matrix& lhs, const xmk_matrix& rhs) {
          lhs.num_cols % 8 == 0 && rhs.num_cols % 8 == 0;
 }
 
-// The condition of the kernels that take any alignment (gemm_loader.h): the stored rows hold a whole 16-byte chunk.
-bool ragged_ok(const xmk_matrix& lhs, const xmk_matrix& rhs, int dtype) {
-  const int chunk = dtype == XMK_F32 ? 4 : 8;
-  return lhs.num_cols >= chunk && rhs.num_cols >= chunk;
-}
-
 // Which streaming kernel for a few rows (gemm_rows.hip) can run this descriptor's product, if any.
 int rows_kind_desc(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k) {
   if (d->out.transpose || d->lhs.transpose || !direct_ok(d->lhs, d->rhs) || !xmk::aligned(d->out.data, 16))
@@ -258,7 +252,6 @@ int plan_splitk(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k, int* po
   const char* forced_env = getenv("XMK_GEMM_SPLITK");
   const int forced = forced_env ? atoi(forced_env) : 0;
   if (d->dtype_in == XMK_F32 || !direct_ok(d->lhs, d->rhs)) {
-    if (!ragged_ok(d->lhs, d->rhs, d->dtype_in)) return 1;
     Choice c = cheapest(m, n, k, 1, d->dtype_in == XMK_F32 ? kClassF32 : kClassRagged, true);
     if (forced >= 1) c.slices = forced;
     if (forced_policy() >= 0) c.policy = forced_policy();
@@ -465,8 +458,10 @@ int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int p
   const bool sixteen = din == XMK_BF16 || din == XMK_F16;
   const bool fast = sixteen && direct_ok(lhs, rhs) && xmk::aligned(out.data, 16) && xmk::aligned(out1, 16) &&
                     xmk::aligned(out2, 16);
-  // 16-bit operands that miss those conditions and fp32 operands: the kernels that take any alignment.
-  const bool ragged = !fast && (sixteen || din == XMK_F32) && ragged_ok(lhs, rhs, din);
+  // 16-bit operands that miss those conditions and fp32 operands: the kernels that take any alignment (they read
+  // 16 bytes at a time, wherever an operand has that many).
+  auto spans = [&](const xmk_matrix& x) { return ((x.num_rows - 1) * x.leading_dim_stride + x.num_cols) * elem_size(din) >= 16; };
+  const bool ragged = !fast && (sixteen || din == XMK_F32) && spans(lhs) && spans(rhs);
   if (fast || ragged) {
     GemmParams p;
     p.a = lhs.data; p.b = rhs.data; p.out = out.data; p.c = d->beta != 0.0f ? d->c : nullptr;
@@ -478,6 +473,11 @@ int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int p
     p.out_alt[0] = out1; p.out_alt[1] = out2; p.sbias = 0;
     if (qkv) { p.sa = 0; p.sc = 0; p.sbias = n; }
     p.kslice = kslice;
+    auto misaligned = [&](const xmk_matrix& x) {
+      const int64_t size = elem_size(din);
+      return !xmk::aligned(x.data, 16) || x.leading_dim_stride * size % 16 || x.batch_stride * size % 16;
+    };
+    p.misaligned = misaligned(lhs) || misaligned(rhs);
     if (kslice) { p.sa = 0; p.sb = 0; }
     const bool a_mc = lhs.transpose != 0;   // stored [K, M]
     const bool b_mc = rhs.transpose == 0;   // stored [K, N]

@@ -43,8 +43,10 @@ struct GemmParams {
   // int8 kernel only: elements per load that the alignment of each operand's pointer, leading dimension, batch
   // stride and row length allows.
   int vec_a, vec_b;
-  // Ragged kernel only: K slice of one grid member (a multiple of its K step), 0 when K is not split.
+  // Kernels that take any alignment only: K slice of one grid member (a multiple of the K step), 0 when K is not
+  // split; some row of an operand does not start on a 16-byte boundary.
   int kslice;
+  bool misaligned;
 };
 
 __device__ __forceinline__ float gelu_tanh(float x) {
@@ -736,60 +738,60 @@ struct TileCost {
 };
 constexpr TileCost kTileCost[4][kNumPolicies] = {
     {  // 16-bit direct, B stored [K, N]
-     {8.373f, 0.954f, 1.661f, 15.214f, 4.693f},
-     {4.788f, 0.378f, 0.591f, 4.147f, 1.594f},
-     {3.925f, 0.223f, 0.354f, 2.871f, 1.259f},
-     {3.315f, 0.176f, 0.248f, 0.898f, 0.942f},
-     {6.316f, 0.534f, 0.953f, 7.21f, 2.587f},
+     {8.351f, 0.951f, 1.639f, 13.748f, 4.611f},
+     {4.75f, 0.383f, 0.581f, 4.353f, 1.658f},
+     {3.917f, 0.227f, 0.359f, 2.594f, 1.268f},
+     {3.311f, 0.176f, 0.264f, 0.864f, 1.132f},
+     {6.284f, 0.544f, 0.927f, 7.589f, 2.347f},
      {},
-     {3.273f, 0.446f, 0.13f, 0.989f, 0.957f},
-     {2.886f, 0.741f, 0.146f, 1.178f, 1.332f},
-     {2.15f, 1.583f, 0.154f, 1.989f, 1.236f},
-     {2.848f, 1.134f, 0.18f, 2.468f, 1.249f},
-     {4.155f, 0.935f, 0.288f, 4.668f, 1.363f},
-     {3.083f, 1.668f, 0.28f, 3.357f, 1.473f},
+     {3.046f, 0.4f, 0.134f, 0.51f, 0.997f},
+     {2.739f, 0.775f, 0.133f, 0.904f, 1.128f},
+     {2.414f, 1.588f, 0.142f, 2.431f, 1.071f},
+     {2.953f, 1.099f, 0.213f, 2.398f, 1.076f},
+     {3.747f, 0.862f, 0.313f, 3.855f, 1.603f},
+     {3.11f, 1.488f, 0.285f, 3.156f, 1.679f},
     },
     {  // 16-bit direct, B stored [N, K]
-     {8.285f, 0.961f, 1.792f, 14.552f, 5.814f},
-     {4.513f, 0.321f, 0.584f, 3.969f, 2.095f},
-     {3.939f, 0.228f, 0.359f, 2.89f, 1.152f},
-     {3.306f, 0.181f, 0.249f, 0.916f, 0.777f},
-     {6.152f, 0.49f, 0.956f, 6.848f, 2.857f},
+     {8.272f, 0.959f, 1.836f, 11.842f, 5.729f},
+     {4.462f, 0.33f, 0.572f, 4.093f, 2.144f},
+     {3.935f, 0.233f, 0.359f, 2.565f, 1.197f},
+     {3.294f, 0.181f, 0.264f, 0.822f, 1.065f},
+     {6.1f, 0.504f, 0.92f, 7.263f, 2.622f},
      {},
-     {3.226f, 0.389f, 0.115f, 0.532f, 0.575f},
-     {3.015f, 0.611f, 0.129f, 1.129f, 0.808f},
-     {2.413f, 1.299f, 0.135f, 2.04f, 0.789f},
-     {2.88f, 1.036f, 0.177f, 2.48f, 1.265f},
-     {4.164f, 0.838f, 0.286f, 4.583f, 1.295f},
-     {3.141f, 1.517f, 0.272f, 3.334f, 1.384f},
+     {3.126f, 0.344f, 0.115f, 0.396f, 0.677f},
+     {2.961f, 0.618f, 0.116f, 0.923f, 0.773f},
+     {2.642f, 1.273f, 0.127f, 2.333f, 0.754f},
+     {2.982f, 1.019f, 0.208f, 2.326f, 1.129f},
+     {3.735f, 0.806f, 0.31f, 3.754f, 1.666f},
+     {2.945f, 1.596f, 0.302f, 3.078f, 2.018f},
     },
     {  // 16-bit, any alignment
      {},
-     {5.132f, 0.864f, 0.735f, 2.1f, 1.177f},
+     {5.669f, 0.788f, 0.716f, 2.853f, 1.6f},
      {},
-     {3.342f, 0.416f, 0.347f, 0.429f, 1.271f},
+     {3.676f, 0.372f, 0.345f, 0.464f, 1.275f},
      {},
      {},
-     {3.537f, 0.554f, 0.16f, 0.842f, 1.054f},
-     {2.936f, 1.095f, 0.178f, 1.369f, 1.239f},
-     {1.897f, 2.27f, 0.184f, 2.157f, 1.15f},
-     {2.919f, 1.783f, 0.249f, 2.844f, 0.952f},
-     {4.859f, 1.118f, 0.353f, 5.027f, 1.788f},
-     {3.277f, 2.307f, 0.379f, 3.525f, 1.647f},
+     {3.458f, 0.555f, 0.191f, 0.405f, 0.898f},
+     {3.075f, 1.115f, 0.217f, 1.339f, 1.047f},
+     {2.134f, 2.386f, 0.219f, 2.215f, 0.885f},
+     {3.127f, 1.701f, 0.27f, 2.754f, 1.078f},
+     {4.579f, 1.086f, 0.361f, 4.139f, 1.668f},
+     {3.475f, 2.21f, 0.388f, 3.206f, 1.537f},
     },
     {  // fp32
      {},
-     {4.318f, 2.272f, 2.212f, 5.565f, 2.005f},
+     {4.281f, 1.894f, 1.858f, 5.761f, 3.191f},
      {},
-     {3.0f, 0.69f, 0.54f, 0.959f, 1.348f},
+     {3.391f, 0.597f, 0.512f, 1.128f, 0.934f},
      {},
      {},
-     {3.369f, 0.742f, 0.179f, 1.072f, 0.546f},
-     {3.031f, 1.28f, 0.193f, 1.82f, 0.775f},
-     {1.889f, 3.022f, 0.214f, 2.796f, 0.817f},
-     {2.62f, 2.464f, 0.321f, 3.37f, 0.993f},
-     {4.534f, 2.268f, 0.601f, 5.912f, 2.133f},
-     {2.298f, 4.447f, 0.57f, 5.419f, 2.004f},
+     {3.307f, 0.657f, 0.155f, 0.72f, 0.466f},
+     {3.068f, 1.181f, 0.16f, 1.243f, 0.639f},
+     {2.366f, 2.376f, 0.17f, 2.807f, 0.659f},
+     {3.185f, 2.181f, 0.291f, 3.548f, 0.841f},
+     {4.218f, 2.231f, 0.586f, 5.833f, 1.448f},
+     {2.873f, 4.47f, 0.562f, 5.601f, 1.5f},
     },
 };
 // What a K split adds for its second launch, and the least it takes end to end when launched from a host program.

@@ -5,9 +5,15 @@
 //   KC operand (reduction index contiguous): LDS [row][128 bytes], chunks XORed by pairs of rows.
 //   MC operand (free index contiguous): LDS [k][rows], 16-bit elements read with the transpose loads, fp32 ones
 //       as scalars.
-// Every lane fetches whole chunks (the hardware takes global loads at any byte address), never element by
-// element: a chunk that would reach past the end of its row is read from 16 bytes before that end and shifted
-// into place, so nothing outside the matrix is touched and no lane branches.
+// Rows may start on any element: every lane fetches whole chunks, at whatever byte address they lie (the hardware
+// takes global loads at any), never element by element.  Nothing branches and nothing outside the operand is read:
+// a chunk that would reach past the operand's end is read from 16 bytes before it and shifted into place, and what
+// lies past the end of K is masked in the last step's fragments.
+// At an unaligned address the address unit takes the 64 lanes of a load one by one (64 cycles of the CU's load path
+// instead of 16; by the cache-access counter 59 accesses per load), which bounds the large products.  Loading the
+// aligned chunks around it instead and picking each lane's piece out of its own and its neighbour's (24 vector
+// instructions per chunk) was level on 1023 x 5003 x 2047 (51 us) and slower on 4001^3 (191 -> 224 us) and on the
+// slices kernel: the vector issue port then is what the address unit was.
 #pragma once
 #include "gemm_kernel.h"
 
@@ -20,99 +26,92 @@ template <> struct Elem<float> {
 };
 
 // v moved down by `bytes` (>= 0), zeros behind.
-__device__ __forceinline__ u32x4 shift_bytes(u32x4 v, int bytes) {
-  const int d = bytes >> 2;
+__device__ __forceinline__ u32x4 shift_bytes(u32x4 v, uint32_t bytes) {
+  const uint32_t d = bytes >> 2;
   if (d & 1) v = u32x4{v[1], v[2], v[3], 0u};
   if (d & 2) v = u32x4{v[2], v[3], 0u, 0u};
-  if (d & ~3) v = u32x4{0u, 0u, 0u, 0u};
+  if (d & ~3u) v = u32x4{0u, 0u, 0u, 0u};
   const uint32_t b = bytes & 3;
   return u32x4{__builtin_amdgcn_alignbyte(v[1], v[0], b), __builtin_amdgcn_alignbyte(v[2], v[1], b),
                __builtin_amdgcn_alignbyte(v[3], v[2], b), __builtin_amdgcn_alignbyte(0u, v[3], b)};
 }
 
-__device__ __forceinline__ u32x4 load16_any(const char* base, uint32_t off) {
-  u32x4 v;
-  __builtin_memcpy(&v, base + off, 16);  // one global_load_dwordx4 at any alignment
-  return v;
-}
-
 // One operand tile of ROWS rows (or columns) x one K step, fetched by NT threads as NL chunks of 16 bytes each.
-// Chunk i of thread t goes to LDS bytes [16 (i NT + t), +16).
-template <typename T, bool MC, int ROWS, int NT>
+// Thread t takes chunk t % CPR of the LDS rows t / CPR + i RPL.
+// MIS: rows may start anywhere; otherwise every row starts on a 16-byte boundary (its length may be anything; the
+// chunk with an operand's last bytes then ends inside the 16-byte granule that holds them).
+template <typename T, bool MC, int ROWS, int NT, bool MIS>
 struct AnyLoader {
-  static constexpr int EB = sizeof(T), CE = 16 / EB, BK = 128 / EB;
-  static constexpr int CPR = MC ? ROWS * EB / 16 : 8;  // chunks per LDS row
-  static constexpr int RPL = NT / CPR;                 // LDS rows per load
+  static constexpr int EB = sizeof(T), BK = 128 / EB;
+  static constexpr int RB = MC ? ROWS * EB : 128;  // bytes of an LDS row
+  static constexpr int CPR = RB / 16;              // chunks per LDS row
+  static constexpr int RPL = NT / CPR;             // LDS rows per load
   static constexpr int NL = ROWS * 8 / NT;
-  static_assert(NL >= 1 && RPL % 4 == 0 && (MC || RPL % 8 == 0), "the swizzle repeats, or changes by element()'s term");
-  uint32_t off[NL];  // byte offset of chunk i from the operand's K step origin
-  int lrow, c0;      // LDS row and first element within that row of chunk 0
-  int shift;         // MC: bytes by which the chunks were moved back to stay inside their rows
+  static_assert(NL >= 1 && RPL % 4 == 0 && (MC || RPL % 8 == 0), "the swizzle repeats, or changes by store()'s term");
+  struct Regs {
+    u32x4 g[NL];
+    int32_t limit;  // (uniform) the largest offset that could be loaded from
+  };
+  const char* base;    // the next K step's origin
+  int64_t left, step;  // from there to the last place a chunk can be loaded from; to the next K step
+  uint32_t off[NL];    // byte offsets of the lane's chunks
+  int32_t reach;       // (uniform) no lane's offset is larger
+  int lds0;            // LDS byte offset of chunk 0
 
   static __device__ __forceinline__ int swizzle(int row_or_k) {
     if constexpr (MC && EB == 4) return 0;
     else return swz<MC, ROWS, 64>(row_or_k);
   }
-  // First element of chunk i within its LDS row.  (KC: the XOR counts pairs of rows modulo 16 rows.)
-  __device__ __forceinline__ int element(int i) const { return !MC && RPL % 16 != 0 && (i & 1) ? c0 ^ (4 * CE) : c0; }
-  // row0: first row (KC) or column (MC) of the tile; rows: how many the matrix has (MC: at least CE).
-  __device__ __forceinline__ void init(int64_t ld, int row0, int rows, int tid) {
-    lrow = tid / CPR;
-    c0 = ((tid % CPR) ^ swizzle(lrow)) * CE;
-    shift = 0;
-    if constexpr (MC) {
-      const int col = row0 + c0, at = min(col, rows - CE);
-      shift = (col - at) * EB;
-#pragma unroll
-      for (int i = 0; i < NL; ++i) off[i] = (uint32_t)(((int64_t)(lrow + i * RPL) * ld + at) * EB);
-    } else {
-#pragma unroll
-      for (int i = 0; i < NL; ++i) {  // rows past the end repeat the last one: their products are not stored
-        const int r = min(row0 + lrow + i * RPL, rows - 1) - row0;
-        off[i] = (uint32_t)(((int64_t)r * ld + element(i)) * EB);
-      }
-    }
-  }
-  // base: the operand at this K step's first k (KC: of the tile's first row; MC: of column 0).
-  __device__ __forceinline__ void load(const char* base, u32x4 (&g)[NL]) const {
-#pragma unroll
-    for (int i = 0; i < NL; ++i) g[i] = load16_any(base, off[i]);
-  }
-  // The same for a K step of which only the first kleft k exist (1 <= kleft < BK; KC: the row has at least CE
-  // elements up to its end): chunks are moved back to end with the row (KC), rows of k past the end repeat the
-  // last (MC).
-  __device__ __forceinline__ void load_tail(const char* base, int64_t ld, int kleft, u32x4 (&g)[NL]) const {
+  // op: the operand (of this batch member), rows x depth elements (stored depth x rows when MC), ld elements from one
+  // stored row to the next; at least 16 bytes in all.  The tile starts at row (column) row0 and at reduction index k0.
+  __device__ __forceinline__ void init(const T* op, int64_t ld, int row0, int rows, int64_t k0, int depth, int tid) {
+    const T* origin = op + (MC ? k0 * ld + row0 : (int64_t)row0 * ld + k0);
+    const T* past = op + (MC ? (int64_t)(depth - 1) * ld + rows : (int64_t)(rows - 1) * ld + depth);
+    base = reinterpret_cast<const char*>(origin);
+    left = (reinterpret_cast<const char*>(past) - base) - 16;
+    if constexpr (!MIS) left = (left + 15) & ~(int64_t)15;
+    step = MC ? BK * ld * EB : 128;
+    const int lrow = tid / CPR, c = tid % CPR;
+    lds0 = lrow * RB + ((c ^ swizzle(lrow)) << 4);
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-      if constexpr (MC) {
-        const int over = max(lrow + i * RPL - (kleft - 1), 0);
-        g[i] = load16_any(base - (int64_t)over * ld * EB, off[i]);
-      } else {
-        const int over = max(element(i) + CE - kleft, 0);
-        g[i] = load16_any(base - over * EB, off[i]);
-      }
+      int r = lrow + i * RPL;
+      if constexpr (!MC) r = min(r, rows - 1 - row0);  // rows past the end repeat the last one: their products are not stored
+      off[i] = (uint32_t)((int64_t)r * ld * EB) + c * 16;
     }
+    const int r = MC ? BK - 1 : min(ROWS, rows - row0) - 1;
+    reach = (int32_t)((int64_t)r * ld * EB) + RB - 16;
   }
-  __device__ __forceinline__ void fix_tail(int kleft, u32x4 (&g)[NL]) const {
+  __device__ __forceinline__ void advance(int steps) {
+    base += steps * step;
+    left -= steps * step;
+  }
+  // Sends for the next K step.
+  __device__ __forceinline__ void load(Regs& r) {
+    r.limit = (int32_t)min(left, (int64_t)0x7ffffff0);
+    const char* from = r.limit < 0 ? base + r.limit : base;
+    const uint32_t cap = (uint32_t)max(r.limit, 0);
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-      if constexpr (MC) {
-        if (lrow + i * RPL >= kleft) g[i] = u32x4{0u, 0u, 0u, 0u};
-      } else {
-        g[i] = shift_bytes(g[i], max(element(i) + CE - kleft, 0) * EB);
-      }
+      const uint32_t at = min(off[i], cap);
+      if constexpr (MIS) __builtin_memcpy(&r.g[i], from + at, 16);
+      else r.g[i] = *reinterpret_cast<const u32x4*>(from + at);
     }
+    advance(1);
   }
-  // edge: some column of the tile does not exist (uniform).
-  __device__ __forceinline__ void store(char* tile, int tid, bool edge, u32x4 (&g)[NL]) const {
-    if constexpr (MC) {
-      if (edge) {
+  __device__ __forceinline__ void store(char* tile, Regs& r) const {
+    if constexpr (MIS) {
+      if (reach > r.limit) {  // only at the operand's end
 #pragma unroll
-        for (int i = 0; i < NL; ++i) g[i] = shift_bytes(g[i], shift);
+        for (int i = 0; i < NL; ++i) r.g[i] = shift_bytes(r.g[i], (uint32_t)max((int32_t)off[i] - r.limit, 0));
       }
     }
 #pragma unroll
-    for (int i = 0; i < NL; ++i) *reinterpret_cast<u32x4*>(tile + (i * NT + tid) * 16) = g[i];
+    for (int i = 0; i < NL; ++i) {
+      // (KC: the XOR counts pairs of rows modulo 16 rows)
+      const int at = (!MC && RPL % 16 != 0 && (i & 1)) ? lds0 ^ 64 : lds0;
+      *reinterpret_cast<u32x4*>(tile + at + i * RPL * RB) = r.g[i];
+    }
   }
 };
 
@@ -151,6 +150,20 @@ struct AnyFrag<float, MC, ROWS, TT> {
     }
   }
 };
+
+// Zeroes the elements of a fragment (quarter ks of a K step) from k = kleft on.
+template <typename T, typename V>
+__device__ __forceinline__ void mask_fragment(V& v, int ks, int lane, int kleft) {
+  constexpr int E = sizeof(T) == 4 ? 4 : 8;  // consecutive k of a lane
+  const int n = kleft - (2 * ks + (lane >> 5)) * E;
+  u32x4 w = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if constexpr (E == 4) w[q] = n > q ? w[q] : 0u;
+    else w[q] &= n >= 2 * q + 2 ? 0xffffffffu : n == 2 * q + 1 ? 0xffffu : 0u;
+  }
+  v = __builtin_bit_cast(V, w);
+}
 
 // acc[i][j] += the products of fragments fb[j] and fa[i] (operands swapped: gemm_kernel.h).
 template <typename T, int TM, int TN, typename V>

@@ -3,7 +3,7 @@
 //
 // What bounds these products is latency, not a rate: with one 64 x 64 tile per CU the tile kernels spend 0.3 us per
 // 64 k waiting for the three K steps they keep in flight.  Here each of the NW waves owns the whole 32 TM x 32 TN
-// tile for every NW-th K step, keeps two of its K steps in flight in registers (NW times the bytes in flight per
+// tile for every NW-th K step, keeps one or two of its K steps in flight in registers (NW times the bytes in flight per
 // CU), passes them through an LDS region of its own (no barrier in the loop: the LDS serves a wave in order), and
 // the waves' partial sums meet in LDS once at the end, added in wave order.  Small tiles also make more
 // work-groups out of a small output.  Operands of any alignment, 16-bit and fp32 (gemm_loader.h).
@@ -12,14 +12,14 @@
 
 namespace gemm_impl {
 
-template <typename T, bool OutF32, bool A_MC, bool B_MC, int TM, int TN, int NW>
+template <typename T, bool OutF32, bool A_MC, bool B_MC, int TM, int TN, int NW, bool MIS>
 __global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(GemmParams p) {
   constexpr int BK = 128 / sizeof(T), KS = 4;
   constexpr int STAGE = (TM + TN) * 4096;                 // LDS per wave
   constexpr int RBY = TN * 128, XM = TN == 1 ? 7 : 15;    // partial sums: as in store_tile
   static_assert(STAGE >= TM * TN * 4096, "a wave's partial sums replace its operands");
-  typedef AnyLoader<T, A_MC, 32 * TM, 64> LoaderA;
-  typedef AnyLoader<T, B_MC, 32 * TN, 64> LoaderB;
+  typedef AnyLoader<T, A_MC, 32 * TM, 64, MIS> LoaderA;
+  typedef AnyLoader<T, B_MC, 32 * TN, 64, MIS> LoaderB;
   typedef typename Elem<T>::vec8 V8;
   __shared__ __attribute__((aligned(1024))) char lds[NW * STAGE];
 
@@ -33,14 +33,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(GemmParams p) {
   const int64_t bz = blockIdx.z;
   const int64_t k0 = bz * p.kslice;  // as in gemm_ragged_kernel
   const int K = p.kslice ? min(p.K - (int)k0, p.kslice) : p.K;
-  const char* a_base = (const char*)(reinterpret_cast<const T*>(p.a) + bz * p.sa + (A_MC ? k0 * p.lda : (int64_t)m0 * p.lda + k0));
-  const char* b_base = (const char*)(reinterpret_cast<const T*>(p.b) + bz * p.sb + (B_MC ? k0 * p.ldb : (int64_t)n0 * p.ldb + k0));
-  const int64_t a_step = (A_MC ? BK * p.lda : BK) * (int64_t)sizeof(T), b_step = (B_MC ? BK * p.ldb : BK) * (int64_t)sizeof(T);
-  const bool a_edge = A_MC && m0 + 32 * TM > p.M, b_edge = B_MC && n0 + 32 * TN > p.N;
   LoaderA la;
   LoaderB lb;
-  la.init(p.lda, m0, p.M, lane);
-  lb.init(p.ldb, n0, p.N, lane);
+  la.init(reinterpret_cast<const T*>(p.a) + bz * p.sa, p.lda, m0, p.M, k0, p.K, lane);
+  lb.init(reinterpret_cast<const T*>(p.b) + bz * p.sb, p.ldb, n0, p.N, k0, p.K, lane);
+  la.advance(wave);  // K step `wave`, and every NW-th from there
+  lb.advance(wave);
+  la.step *= NW;
+  lb.step *= NW;
   AnyFrag<T, A_MC, 32 * TM, TM> faddr;
   AnyFrag<T, B_MC, 32 * TN, TN> fbddr;
   faddr.init(0, lane);
@@ -54,28 +54,25 @@ __global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(GemmParams p) {
 
   const int KT = (K + BK - 1) / BK;
   char* region = lds + wave * STAGE;
-  u32x4 ga[2][LoaderA::NL], gb[2][LoaderB::NL];
-  auto load = [&](int kt, u32x4 (&a)[LoaderA::NL], u32x4 (&b)[LoaderB::NL]) {
-    const char *ap = a_base + kt * a_step, *bp = b_base + kt * b_step;
-    const int kleft = K - kt * BK;
-    if (kleft >= BK) {
-      la.load(ap, a);
-      lb.load(bp, b);
-    } else {
-      la.load_tail(ap, p.lda, kleft, a);
-      lb.load_tail(bp, p.ldb, kleft, b);
-    }
+  struct Regs {
+    typename LoaderA::Regs a;
+    typename LoaderB::Regs b;
   };
-  // Multiplies K step kt, which is in the registers a and b, and sends K step kt + 2 NW into them.
-  auto step = [&](int kt, u32x4 (&a)[LoaderA::NL], u32x4 (&b)[LoaderB::NL]) {
-    const int kleft = K - kt * BK;
-    if (kleft < BK) {
-      la.fix_tail(kleft, a);
-      lb.fix_tail(kleft, b);
+  constexpr bool TWO = TM * TN < 4;  // K steps in flight per wave: two, or one where the registers allow no more
+  Regs r0, r1;
+  auto load = [&](Regs& r) {
+    la.load(r.a);
+    lb.load(r.b);
+  };
+  // Multiplies K step kt, which is in the registers r, and sends the next but one (or the next) of this wave into
+  // them.  LAST: the wave's last step, of which only some k may exist.
+  auto step = [&](auto LAST, int kt, Regs& r) {
+    la.store(region, r.a);
+    lb.store(region + TM * 4096, r.b);
+    if constexpr (!decltype(LAST)::value) {
+      if (!TWO || kt + 2 * NW < KT) load(r);
+      __builtin_amdgcn_sched_barrier(0);  // (the loads would sink behind the matrix instructions)
     }
-    la.store(region, lane, a_edge, a);
-    lb.store(region + TM * 4096, lane, b_edge, b);
-    if (kt + 2 * NW < KT) load(kt + 2 * NW, a, b);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       V8 fa[TM], fb[TN];
@@ -83,18 +80,33 @@ __global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(GemmParams p) {
       for (int i = 0; i < TM; ++i) fa[i] = faddr.read(region, i, ks);
 #pragma unroll
       for (int j = 0; j < TN; ++j) fb[j] = fbddr.read(region + TM * 4096, j, ks);
+      if constexpr (decltype(LAST)::value) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) mask_fragment<T>(fa[i], ks, lane, K - kt * BK);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) mask_fragment<T>(fb[j], ks, lane, K - kt * BK);
+      }
       mma_block<T, TM, TN>(acc, fa, fb);
     }
   };
-  if (wave < KT) load(wave, ga[0], gb[0]);
-  if (wave + NW < KT) load(wave + NW, ga[1], gb[1]);
-  for (int kt = wave; kt < KT; kt += 2 * NW) {
-    step(kt, ga[0], gb[0]);
-    if (kt + NW < KT) step(kt + NW, ga[1], gb[1]);
+  constexpr std::false_type inner;
+  constexpr std::true_type last;
+  int kt = wave;
+  if (kt < KT) load(r0);
+  if (TWO && kt + NW < KT) load(r1);
+  for (; kt + 2 * NW < KT; kt += 2 * NW) {
+    step(inner, kt, r0);
+    step(inner, kt + NW, TWO ? r1 : r0);
+  }
+  if (kt + NW < KT) {
+    step(inner, kt, r0);
+    step(last, kt + NW, TWO ? r1 : r0);
+  } else if (kt < KT) {
+    step(last, kt, r0);
   }
 
   // The waves' partial sums, in store_tile's layout (slab i of 32 rows after the other).
-  const int r1 = lane & 31, h = lane >> 5;
+  const int row32 = lane & 31, h = lane >> 5;
   static_for<TM>([&](auto I) {
     constexpr int i = decltype(I)::value;
     static_for<TN>([&](auto J) {
@@ -102,7 +114,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(GemmParams p) {
       const floatx16 t = acc[i][j];
       static_for<4>([&](auto Q) {
         constexpr int qd = decltype(Q)::value;
-        *reinterpret_cast<floatx4*>(region + (i * 32 + r1) * RBY + (((8 * j + 2 * qd + h) ^ (r1 & XM)) << 4)) =
+        *reinterpret_cast<floatx4*>(region + (i * 32 + row32) * RBY + (((8 * j + 2 * qd + h) ^ (row32 & XM)) << 4)) =
             floatx4{t[4 * qd], t[4 * qd + 1], t[4 * qd + 2], t[4 * qd + 3]};
       });
     });
@@ -134,28 +146,34 @@ __global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(GemmParams p) {
 }
 
 // The kernel's variants, by index from kSlicesPolicy on in kPolicies.
-template <typename T, bool OutF32, bool A_MC, bool B_MC>
+template <typename T, bool OutF32, bool A_MC, bool B_MC, bool MIS>
 void launch_slices_variant(int v, GemmParams& p, int batch, hipStream_t st) {
   const Policy& pol = kPolicies[kSlicesPolicy + v];
   p.tiles_m = (int)xmk::ceil_div(p.M, pol.bm);
   p.tiles_n = (int)xmk::ceil_div(p.N, pol.bn);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)batch), block((unsigned)(pol.wgm * 64));
   switch (v) {
-    case 0: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 1, 4>), grid, block, 0, st, p); break;
-    case 1: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 1, 8>), grid, block, 0, st, p); break;
-    case 2: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 1, 16>), grid, block, 0, st, p); break;
-    case 3: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 2, 8>), grid, block, 0, st, p); break;
-    case 4: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 2, 2, 4>), grid, block, 0, st, p); break;
-    default: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 2, 2, 8>), grid, block, 0, st, p); break;
+    case 0: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 1, 4, MIS>), grid, block, 0, st, p); break;
+    case 1: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 1, 8, MIS>), grid, block, 0, st, p); break;
+    case 2: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 1, 16, MIS>), grid, block, 0, st, p); break;
+    case 3: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 2, 8, MIS>), grid, block, 0, st, p); break;
+    case 4: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 2, 2, 4, MIS>), grid, block, 0, st, p); break;
+    default: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 2, 2, 8, MIS>), grid, block, 0, st, p); break;
   }
+}
+
+template <typename T, bool OutF32, bool A_MC, bool B_MC>
+void launch_slices_rows(int v, GemmParams& p, int batch, hipStream_t st) {
+  if (p.misaligned) launch_slices_variant<T, OutF32, A_MC, B_MC, true>(v, p, batch, st);
+  else launch_slices_variant<T, OutF32, A_MC, B_MC, false>(v, p, batch, st);
 }
 
 template <typename T, bool OutF32>
 void launch_slices_impl(bool a_mc, bool b_mc, int v, GemmParams& p, int batch, hipStream_t st) {
-  if (!a_mc && !b_mc) launch_slices_variant<T, OutF32, false, false>(v, p, batch, st);
-  else if (!a_mc && b_mc) launch_slices_variant<T, OutF32, false, true>(v, p, batch, st);
-  else if (a_mc && !b_mc) launch_slices_variant<T, OutF32, true, false>(v, p, batch, st);
-  else launch_slices_variant<T, OutF32, true, true>(v, p, batch, st);
+  if (!a_mc && !b_mc) launch_slices_rows<T, OutF32, false, false>(v, p, batch, st);
+  else if (!a_mc && b_mc) launch_slices_rows<T, OutF32, false, true>(v, p, batch, st);
+  else if (a_mc && !b_mc) launch_slices_rows<T, OutF32, true, false>(v, p, batch, st);
+  else launch_slices_rows<T, OutF32, true, true>(v, p, batch, st);
 }
 
 // Explicitly instantiated in gemm_inst_slices_*.hip.
