@@ -12,62 +12,36 @@
 // B stored [K,N] (rhs_transpose == 0) takes the same kernel: its 64 k x BN tile goes into LDS as it
 // lies in memory (n contiguous, the 16-bit GEMM's loader for that layout) and the fragments are read
 // with ds_read_b64_tr_b8, which hands a lane 8 consecutive k of one column.
+// Operands that the direct loads cannot take, and products with few output tiles, run the kernels that take any
+// alignment (gemm_fp8.h).
 #include <utility>
 
-#include "gemm_gather8.h"
-#include "gemm_kernel.h"
+#include "gemm_fp8.h"
+
+namespace gemm_impl {
+// (gemm_inst_fp8_nk.hip / gemm_inst_fp8_kn.hip)
+void launch_fp8_any_nk(int policy, Fp8Params& p, hipStream_t st);
+void launch_fp8_any_kn(int policy, Fp8Params& p, hipStream_t st);
+void launch_fp8_any(int policy, bool b_mc, Fp8Params& p, hipStream_t st) {
+  if (b_mc) launch_fp8_any_kn(policy, p, st);
+  else launch_fp8_any_nk(policy, p, st);
+}
+}  // namespace gemm_impl
 
 namespace {
 
 using gemm_impl::floatx16;
+using gemm_impl::Fp8Epilogue;
+using gemm_impl::Fp8Params;
+using gemm_impl::intx8;
+using gemm_impl::mfma_fp8;
 using gemm_impl::static_for;
 using gemm_impl::u32x2;
 using gemm_impl::u32x4;
 using gemm_impl::zero16;
-typedef int intx8 __attribute__((ext_vector_type(8)));
 
 constexpr int BKB = 64;  // K step in bytes (= fp8 elements)
 constexpr uint32_t kOob = gemm_impl::kOob;
-
-struct Fp8Params {
-  const uint8_t* a;
-  const uint8_t* b;
-  const float* a_scale;
-  const float* b_scale;
-  const float* d_scale;  // optional: multiplies the result after the bias
-  const __bf16* bias;    // optional: [N], added to a_scale * b_scale * A B
-  __bf16* out;
-  int M, N, K;
-  int tiles_m, tiles_n;
-};
-
-// out element = bf16(d_scale * (a_scale * b_scale * acc + bias[n])); `scale` = a_scale * b_scale.
-struct Fp8Epilogue {
-  float scale, post;
-  const __bf16* bias;
-  float b[8];  // the bias of the lane's columns (gemm_impl::store_tile)
-  __device__ __forceinline__ explicit Fp8Epilogue(const Fp8Params& p)
-      : scale(p.a_scale[0] * p.b_scale[0]), post(p.d_scale ? p.d_scale[0] : 1.0f), bias(p.bias) {}
-  __device__ __forceinline__ __bf16 operator()(float acc, int n) const {
-    float v = acc * scale;
-    if (bias) v += (float)bias[n];
-    return (__bf16)(v * post);
-  }
-  __device__ __forceinline__ void columns(int n, int count) {
-    if (bias && count > 0) gemm_impl::GemmEpilogue<__bf16, false>::fetch<false>(bias, n, count, b);
-  }
-  template <int U>
-  __device__ __forceinline__ void apply(float (&v)[U][8], const int (&)[U], int, int) const {
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        v[u][e] *= scale;
-        if (bias) v[u][e] += b[e];
-        v[u][e] *= post;
-      }
-  }
-};
 
 // Per-lane LDS byte offsets of an operand's fragments: lane l of the 32-row slab t gets row
 // 32 t + l%32, bytes 32 (l/32) .. +31 of the 64-byte row, i.e. the two 16-byte chunks 2 (l/32)
@@ -124,11 +98,6 @@ struct Fp8FragKN {
   }
 };
 
-__device__ __forceinline__ floatx16 mfma_fp8(intx8 a, intx8 b, floatx16 c) {
-  // cbsz = blgp = 0: both operands e4m3; block scales 127 = 2^0 (E8M0).
-  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 127, 0, 127);
-}
-
 template <int BM, int BN, int WGM, int WGN, int NSTAGE, bool BKN = false>
 __global__ __launch_bounds__(WGM * WGN * 64) void fp8_gemm_kernel(Fp8Params p) {
   constexpr int NWAVES = WGM * WGN;
@@ -170,8 +139,8 @@ __global__ __launch_bounds__(WGM * WGN * 64) void fp8_gemm_kernel(Fp8Params p) {
   la.init(p.K / 2, p.M - m0, wave, lane);
   if constexpr (BKN) lb.init(p.N / 2, (p.N - n0) / 2, wave, lane);
   else lb.init(p.K / 2, p.N - n0, wave, lane);
-  const uint8_t* a_tile = p.a + (int64_t)m0 * p.K;
-  const uint8_t* b_tile = BKN ? p.b + n0 : p.b + (int64_t)n0 * p.K;
+  const uint8_t* a_tile = reinterpret_cast<const uint8_t*>(p.a) + (int64_t)m0 * p.K;
+  const uint8_t* b_tile = reinterpret_cast<const uint8_t*>(p.b) + (BKN ? n0 : (int64_t)n0 * p.K);
   const int64_t b_step = BKN ? (int64_t)BKB * p.N : BKB;  // bytes from one K step's B tile to the next
   // k of a K step that exist, in the unit the loader compares with: two-byte units along a
   // k-contiguous row, rows of the [k,n] tile.
@@ -260,121 +229,7 @@ __global__ __launch_bounds__(WGM * WGN * 64) void fp8_gemm_kernel(Fp8Params p) {
   gemm_impl::store_tile<__bf16, false>(epi, acc, lds + wave * (TN * 4096), p.out, p.N, 0, p.M, p.N, m0 + wm * WTM, n0 + wn * WTN, lane);
 }
 
-// Any layout, size and alignment on the matrix cores: the operands are gathered (gemm_gather8.h) into
-// the k-contiguous LDS layout, 16-byte chunks of 16 k; a lane's two neighbouring chunks are one operand
-// of v_mfma_scale_f32_32x32x64_f8f6f4 (row l % 32, k = 32 (l / 32) .. +31).  256 threads = 4 waves in
-// 2 x 2, tile 64 TW x 64 TW x 64, 4 LDS stages; the structure of the int8 kernel (gemm_s8.hip).
-template <int TW, int NSTAGE, int AMODE, int BMODE>
-__global__ __launch_bounds__(256) void fp8_gemm_gather_kernel(Fp8Params p) {
-  using namespace gather8;
-  constexpr bool b_kc = BMODE != MC;
-  constexpr int BM = 64 * TW, BN = 64 * TW;
-  constexpr int OP_BYTES = BM * BKB;
-  constexpr int STAGE = 2 * OP_BYTES;
-  constexpr int NLD = OP_BYTES / (256 * 16);
-  __shared__ __attribute__((aligned(1024))) char lds[NSTAGE * STAGE];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
-  const int l32 = lane & 31, g = lane >> 5;
-  const int tile_m = blockIdx.x / p.tiles_n, tile_n = blockIdx.x % p.tiles_n;
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
-  const int8_t* A = reinterpret_cast<const int8_t*>(p.a);
-  const int8_t* B = reinterpret_cast<const int8_t*>(p.b);
-  const int8_t* a_tile = A + (int64_t)m0 * p.K;                       // A is [M, K]
-  const int8_t* b_tile = b_kc ? B + (int64_t)n0 * p.K : B + n0;       // B is [N, K] or [K, N]
-  const int64_t ldb = b_kc ? p.K : p.N;
-  const int64_t b_step = b_kc ? BKB : (int64_t)BKB * p.N;
-
-  floatx16 acc[TW][TW];
-#pragma unroll
-  for (int i = 0; i < TW; ++i)
-#pragma unroll
-    for (int j = 0; j < TW; ++j) acc[i][j] = zero16();
-
-  const int KT = (p.K + BKB - 1) / BKB;
-  auto load_step = [&](int kt, intx4 (&ga)[NLD], intx4 (&gb)[NLD]) {
-    const int kleft = p.K - kt * BKB;  // <= 0 past the end: zeros (fp8 zero is the zero byte)
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      ga[i] = gather<AMODE>(a_tile, A, p.K, p.M - m0, kleft, i, tid);
-      gb[i] = gather<BMODE>(b_tile, B, ldb, p.N - n0, kleft, i, tid);
-    }
-    a_tile += BKB;
-    b_tile += b_step;
-  };
-  auto store_step = [&](char* stage, const intx4 (&ga)[NLD], const intx4 (&gb)[NLD]) {
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      *reinterpret_cast<intx4*>(stage + i * 4096 + tid * 16) = ga[i];
-      *reinterpret_cast<intx4*>(stage + OP_BYTES + i * 4096 + tid * 16) = gb[i];
-    }
-  };
-  Fp8Frag fa_addr, fb_addr;
-  fa_addr.init(wm * 32 * TW, lane);
-  fb_addr.init(wn * 32 * TW, lane);
-
-  {
-    intx4 ga[NLD], gb[NLD];
-    for (int st = 0; st < NSTAGE - 1; ++st) {
-      load_step(st, ga, gb);
-      store_step(lds + st * STAGE, ga, gb);
-    }
-  }
-  __syncthreads();
-  for (int kt = 0; kt < KT; ++kt) {
-    const char* cur = lds + (kt % NSTAGE) * STAGE;
-    char* wr = lds + ((kt + NSTAGE - 1) % NSTAGE) * STAGE;  // read during step kt - 1
-    intx4 ga[NLD], gb[NLD];
-    load_step(kt + NSTAGE - 1, ga, gb);
-    intx8 fa[TW], fb[TW];
-#pragma unroll
-    for (int t = 0; t < TW; ++t) {
-      fa[t] = fa_addr.read(cur, t);
-      fb[t] = fb_addr.read(cur + OP_BYTES, t);
-    }
-#pragma unroll
-    for (int ti = 0; ti < TW; ++ti)
-#pragma unroll
-      for (int tj = 0; tj < TW; ++tj) acc[ti][tj] = mfma_fp8(fb[tj], fa[ti], acc[ti][tj]);
-    store_step(wr, ga, gb);
-    __syncthreads();  // step kt + NSTAGE - 1 is in LDS for every wave; every wave is done with `cur`
-  }
-
-  // acc[i][j][e] is out[m][n], m = m0 + 32 TW wm + 32 i + lane % 32, n = n0 + 32 TW wn + 32 j + 8 (e/4) + 4 (lane/32) + e%4.
-  Fp8Epilogue epi(p);
-  static_assert(NSTAGE * STAGE >= 4 * TW * 4096, "a slab per wave is staged in the operand stages");
-  gemm_impl::store_tile<__bf16, false>(epi, acc, lds + wave * (TW * 4096), p.out, p.N, 0, p.M, p.N, m0 + wm * 32 * TW,
-                                       n0 + wn * 32 * TW, lane);
-}
-
-template <int TW, int AMODE>
-void launch_gather_b(const Fp8Params& p, int bmode, dim3 grid, hipStream_t st) {
-  using namespace gather8;
-  if (bmode == KC_VEC) hipLaunchKernelGGL((fp8_gemm_gather_kernel<TW, 4, AMODE, KC_VEC>), grid, dim3(256), 0, st, p);
-  else if (bmode == KC_SCALAR) hipLaunchKernelGGL((fp8_gemm_gather_kernel<TW, 4, AMODE, KC_SCALAR>), grid, dim3(256), 0, st, p);
-  else hipLaunchKernelGGL((fp8_gemm_gather_kernel<TW, 4, AMODE, MC>), grid, dim3(256), 0, st, p);
-}
-
-// a_vec / b_vec: 16-byte aligned pointer and K % 16 == 0 (the k-contiguous operand can be read 16 bytes at a time).
-void launch_gather(Fp8Params& p, bool rhs_is_nk, bool a_vec, bool b_vec, hipStream_t st) {
-  using namespace gather8;
-  const bool large = xmk::ceil_div(p.M, 128) * xmk::ceil_div(p.N, 128) >= 256;
-  const int edge = large ? 128 : 64;
-  p.tiles_m = (int)xmk::ceil_div(p.M, edge);
-  p.tiles_n = (int)xmk::ceil_div(p.N, edge);
-  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n));
-  const int bmode = !rhs_is_nk ? MC : (b_vec ? KC_VEC : KC_SCALAR);
-  if (large) {
-    if (a_vec) launch_gather_b<2, KC_VEC>(p, bmode, grid, st);
-    else launch_gather_b<2, KC_SCALAR>(p, bmode, grid, st);
-  } else {
-    if (a_vec) launch_gather_b<1, KC_VEC>(p, bmode, grid, st);
-    else launch_gather_b<1, KC_SCALAR>(p, bmode, grid, st);
-  }
-}
-
-// Plain tiled kernel for outputs that are not 8-byte aligned: 64x64 tile, fp8 decoded with the hardware
+// Plain tiled kernel for operands of less than 16 bytes: 64x64 tile, fp8 decoded with the hardware
 // conversion while staging, fp32 FMA.
 __global__ __launch_bounds__(256) void fp8_gemm_generic_kernel(Fp8Params p, int rhs_transpose) {
   __shared__ float As[16][65];
@@ -387,10 +242,10 @@ __global__ __launch_bounds__(256) void fp8_gemm_generic_kernel(Fp8Params p, int 
       const int kk = e / 64, r = e % 64, k = k0 + kk;
       float av = 0.f, bv = 0.f;
       if (k < p.K && m0 + r < p.M)
-        av = __builtin_amdgcn_cvt_f32_fp8((int)p.a[(int64_t)(m0 + r) * p.K + k], 0);
+        av = __builtin_amdgcn_cvt_f32_fp8((int)reinterpret_cast<const uint8_t*>(p.a)[(int64_t)(m0 + r) * p.K + k], 0);
       if (k < p.K && n0 + r < p.N) {
         const int64_t i = rhs_transpose ? (int64_t)(n0 + r) * p.K + k : (int64_t)k * p.N + (n0 + r);
-        bv = __builtin_amdgcn_cvt_f32_fp8((int)p.b[i], 0);
+        bv = __builtin_amdgcn_cvt_f32_fp8((int)reinterpret_cast<const uint8_t*>(p.b)[i], 0);
       }
       As[kk][r] = av;
       Bs[kk][r] = bv;
@@ -414,8 +269,28 @@ __global__ __launch_bounds__(256) void fp8_gemm_generic_kernel(Fp8Params p, int 
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int m = m0 + ty * 4 + i, n = n0 + tx * 4 + j;
-      if (m < p.M && n < p.N) p.out[(int64_t)m * p.N + n] = epi(acc[i][j], n);
+      if (m < p.M && n < p.N) reinterpret_cast<__bf16*>(p.out)[(int64_t)m * p.N + n] = epi(acc[i][j], n);
     }
+}
+
+// XMK_FP8_POLICY=<index into kFp8Policies> forces a tile where the operands allow it (read at every call).
+int choose_fp8(int64_t m, int64_t n, int64_t k, bool direct, bool any, bool rhs_t) {
+  using namespace gemm_impl;
+  auto usable = [&](int v) { return v >= 0 && v < kFp8Policies_n && (v < kFp8Direct ? direct : any); };
+  if (const char* e = getenv("XMK_FP8_POLICY"))
+    if (*e && usable(atoi(e))) return atoi(e);
+  int best = -1;
+  float best_cost = 1e30f;
+  const uint32_t kt = (uint32_t)((k + 127) / 128);
+  for (int pol = direct ? 0 : kFp8Direct; pol < kFp8Policies_n; ++pol) {
+    if (!usable(pol)) continue;
+    const float cost = launch_cost(kFp8Policies[pol], kFp8Cost[!direct ? 2 : rhs_t ? 1 : 0][pol], pol >= kFp8Slices, (uint32_t)m, (uint32_t)n, kt, 1);
+    if (cost < best_cost) {
+      best = pol;
+      best_cost = cost;
+    }
+  }
+  return best;
 }
 
 }  // namespace
@@ -433,44 +308,43 @@ extern "C" int xmk_fp8_gemm_ex(const void* a, const void* b, const float* a_scal
   if (m <= 0 || n <= 0 || k <= 0) return xmk::fail(XMK_INVALID_ARGUMENT, "fp8_gemm: empty dimension");
   if (m > (1 << 30) || n > (1 << 30) || k > (1 << 30))
     return xmk::fail(XMK_INVALID_ARGUMENT, "fp8_gemm: dimension too large");
-  Fp8Params p;
-  p.a = (const uint8_t*)a; p.b = (const uint8_t*)b; p.a_scale = a_scale; p.b_scale = b_scale;
-  p.d_scale = d_scale; p.bias = (const __bf16*)bias;
-  p.out = (__bf16*)out; p.M = (int)m; p.N = (int)n; p.K = (int)k;
+  Fp8Params p{};
+  p.a = a; p.b = b; p.out = out; p.bias = bias;
+  p.a_scale = a_scale; p.b_scale = b_scale; p.d_scale = d_scale;
+  p.M = (int)m; p.N = (int)n; p.K = (int)k;
+  p.lda = k; p.ldb = rhs_transpose ? k : n; p.ldc = n;
+  p.alpha = 1.0f;
   hipStream_t st = (hipStream_t)stream;
+  const bool aligned = xmk::aligned(a, 16) && xmk::aligned(b, 16) && k % 16 == 0 && p.ldb % 16 == 0;
+  p.misaligned = !aligned;
   // The direct-to-LDS kernel: A rows and the stored rows of B start on 16-byte boundaries and hold whole
   // 16-byte chunks; one K step's tile of either operand lies within the 2 GiB a buffer descriptor spans.
-  const bool fast_nk = rhs_transpose != 0 && k % 16 == 0 && n % 4 == 0 && 256 * k < (int64_t)kOob;
-  const bool fast_kn = rhs_transpose == 0 && k % 16 == 0 && n % 16 == 0 && 256 * k < (int64_t)kOob &&
-                       64 * n < (int64_t)kOob;
-  if ((fast_nk || fast_kn) && xmk::aligned(a, 16) && xmk::aligned(b, 16) && xmk::aligned(out, 8)) {
-    const bool big = xmk::ceil_div(m, 256) * xmk::ceil_div(n, 256) >= 256;
-    // Between the two: about one 256 x 128 tile per CU (the 16-bit GEMM's third tile, for the same shapes).
-    static const char* tile_env = getenv("XMK_FP8_TILE");
-    const int64_t mid_tiles = xmk::ceil_div(m, 256) * xmk::ceil_div(n, 128);
-    const bool mid = tile_env ? atoi(tile_env) == 1 : (!big && mid_tiles >= 192 && mid_tiles <= 256);
-    xmk::trace("fp8_gemm m=%lld n=%lld k=%lld rhs_t=%d -> %s", (long long)m, (long long)n, (long long)k, rhs_transpose,
-               mid ? "mfma_256x128" : big ? "mfma_256x256" : "mfma_128x128");
-    if (mid) {
-      p.tiles_m = (int)xmk::ceil_div(m, 256); p.tiles_n = (int)xmk::ceil_div(n, 128);
-      if (fast_kn) hipLaunchKernelGGL((fp8_gemm_kernel<256, 128, 2, 2, 4, true>), dim3(p.tiles_m * p.tiles_n), dim3(256), 0, st, p);
-      else hipLaunchKernelGGL((fp8_gemm_kernel<256, 128, 2, 2, 4>), dim3(p.tiles_m * p.tiles_n), dim3(256), 0, st, p);
-    } else if (tile_env ? atoi(tile_env) == 2 : big) {
-      p.tiles_m = (int)xmk::ceil_div(m, 256); p.tiles_n = (int)xmk::ceil_div(n, 256);
-      if (fast_kn) hipLaunchKernelGGL((fp8_gemm_kernel<256, 256, 2, 4, 4, true>), dim3(p.tiles_m * p.tiles_n), dim3(512), 0, st, p);
-      else hipLaunchKernelGGL((fp8_gemm_kernel<256, 256, 2, 4, 4>), dim3(p.tiles_m * p.tiles_n), dim3(512), 0, st, p);
+  const bool direct = aligned && 256 * k < (int64_t)kOob && (rhs_transpose || 64 * n < (int64_t)kOob);
+  // The tile loaders of the other kernels form byte offsets of up to 128 rows in 31 bits, from operands of 16 bytes
+  // or more.
+  const bool any = m * k >= 16 && n * k >= 16 && p.lda < (1 << 24) && p.ldb < (1 << 24);
+  const int pol = choose_fp8(m, n, k, direct, any, rhs_transpose != 0);
+  xmk::trace("fp8_gemm m=%lld n=%lld k=%lld rhs_t=%d -> %s", (long long)m, (long long)n, (long long)k, rhs_transpose,
+             pol < 0 ? "generic_64x64" : gemm_impl::kFp8Policies[pol].name);
+  if (pol >= gemm_impl::kFp8Direct) {
+    gemm_impl::launch_fp8_any(pol, rhs_transpose == 0, p, st);
+  } else if (pol >= 0) {
+    const gemm_impl::Policy& P = gemm_impl::kFp8Policies[pol];
+    p.tiles_m = (int)xmk::ceil_div(m, P.bm);
+    p.tiles_n = (int)xmk::ceil_div(n, P.bn);
+    const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block((unsigned)(P.wgm * P.wgn * 64));
+    const bool kn = rhs_transpose == 0;
+    if (pol == 0) {
+      if (kn) hipLaunchKernelGGL((fp8_gemm_kernel<256, 256, 2, 4, 4, true>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((fp8_gemm_kernel<256, 256, 2, 4, 4>), grid, block, 0, st, p);
+    } else if (pol == 1) {
+      if (kn) hipLaunchKernelGGL((fp8_gemm_kernel<256, 128, 2, 2, 4, true>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((fp8_gemm_kernel<256, 128, 2, 2, 4>), grid, block, 0, st, p);
     } else {
-      p.tiles_m = (int)xmk::ceil_div(m, 128); p.tiles_n = (int)xmk::ceil_div(n, 128);
-      if (fast_kn) hipLaunchKernelGGL((fp8_gemm_kernel<128, 128, 2, 2, 4, true>), dim3(p.tiles_m * p.tiles_n), dim3(256), 0, st, p);
-      else hipLaunchKernelGGL((fp8_gemm_kernel<128, 128, 2, 2, 4>), dim3(p.tiles_m * p.tiles_n), dim3(256), 0, st, p);
+      if (kn) hipLaunchKernelGGL((fp8_gemm_kernel<128, 128, 2, 2, 4, true>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((fp8_gemm_kernel<128, 128, 2, 2, 4>), grid, block, 0, st, p);
     }
-  } else if (xmk::aligned(out, 8) && (int64_t)m * k < (int64_t)1 << 40) {
-    xmk::trace("fp8_gemm m=%lld n=%lld k=%lld rhs_t=%d -> mfma_gather", (long long)m, (long long)n, (long long)k,
-               rhs_transpose);
-    launch_gather(p, rhs_transpose != 0, k % 16 == 0 && xmk::aligned(a, 16), k % 16 == 0 && xmk::aligned(b, 16), st);
   } else {
-    xmk::trace("fp8_gemm m=%lld n=%lld k=%lld rhs_t=%d -> generic_64x64", (long long)m, (long long)n,
-               (long long)k, rhs_transpose);
     hipLaunchKernelGGL(fp8_gemm_generic_kernel, dim3((unsigned)xmk::ceil_div(n, 64), (unsigned)xmk::ceil_div(m, 64)),
                        dim3(256), 0, st, p, (int)rhs_transpose);
   }

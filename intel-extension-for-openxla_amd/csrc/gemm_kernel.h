@@ -797,14 +797,12 @@ constexpr TileCost kTileCost[4][kNumPolicies] = {
 // What a K split adds for its second launch, and the least it takes end to end when launched from a host program.
 constexpr float kSplitCost = 4.0f, kSplitFloor = 8.0f;
 
-inline float tile_cost(int pol, uint32_t m, uint32_t n, uint32_t k, uint32_t batch, int cls) {
-  const Policy& P = kPolicies[pol];
-  const TileCost& c = kTileCost[cls][pol];
+// kt: K steps of 128 bytes.
+inline float launch_cost(const Policy& P, const TileCost& c, bool slices, uint32_t m, uint32_t n, uint32_t kt, uint32_t batch) {
   auto blocks = [](uint32_t v, int b) { return (v + b - 1) >> __builtin_ctz((unsigned)b); };  // b: a power of two
   const uint64_t tiles = (uint64_t)blocks(m, P.bm) * blocks(n, P.bn) * batch;
   const float load = (float)tiles * (1.0f / 256);
-  const uint32_t kt = blocks(k, cls == kClassF32 ? 32 : 64);
-  const uint32_t ktw = pol >= kSlicesPolicy ? blocks(kt, P.wgm) : kt;
+  const uint32_t ktw = slices ? blocks(kt, P.wgm) : kt;
   const float l = P.alone ? 0.5f * (load + (float)((tiles + 255) >> 8)) : load;
   return c.start + c.step * (float)ktw + c.fill * (float)kt * (load < 1.0f ? load : 1.0f) * 0.125f +
          (l > 1.0f ? l - 1.0f : 0.0f) * (c.more_step * (float)kt + c.more);
@@ -818,10 +816,13 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
   Choice best{3, 1};
   float best_cost = 1e30f;
   const bool direct = cls == kClassKN || cls == kClassNK;
+  const int kstep = cls == kClassF32 ? 32 : 64;
   auto each = [&](int s, float extra, float least) {
     for (int pol = 0; pol < kNumPolicies; ++pol) {
       if (pol == kRowsPolicy || (!direct && !kPolicies[pol].any_alignment)) continue;
-      const float cost = std::max(tile_cost(pol, (uint32_t)m, (uint32_t)n, (uint32_t)((k + s - 1) / s), (uint32_t)(batch * s), cls) + extra, least);
+      const uint32_t kt = (uint32_t)(((k + s - 1) / s + kstep - 1) / kstep);
+      const float cost = std::max(launch_cost(kPolicies[pol], kTileCost[cls][pol], pol >= kSlicesPolicy, (uint32_t)m, (uint32_t)n, kt,
+                                              (uint32_t)(batch * s)) + extra, least);
       if (cost < best_cost) {
         best_cost = cost;
         best = {pol, s};

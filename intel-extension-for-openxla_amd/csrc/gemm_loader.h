@@ -1,10 +1,10 @@
 // Operand tiles for the kernels that take any alignment (gemm_ragged.h, gemm_slices.h): global memory -> registers
 // -> LDS in 16-byte chunks, and the matrix-core fragments read back from LDS.
 //
-// A K step is 128 bytes of a reduction-contiguous row: 64 elements of 16 bits, 32 of fp32.
+// A K step is 128 bytes of a reduction-contiguous row: 64 elements of 16 bits, 32 of fp32, 128 of fp8.
 //   KC operand (reduction index contiguous): LDS [row][128 bytes], chunks XORed by pairs of rows.
-//   MC operand (free index contiguous): LDS [k][rows], 16-bit elements read with the transpose loads, fp32 ones
-//       as scalars.
+//   MC operand (free index contiguous): LDS [k][rows], 8- and 16-bit elements read with the transpose loads, fp32
+//       ones as scalars.
 // Rows may start on any element: every lane fetches whole chunks, at whatever byte address they lie (the hardware
 // takes global loads at any), never element by element.  Nothing branches and nothing outside the operand is read:
 // a chunk that would reach past the operand's end is read from 16 bytes before it and shifted into place, and what
@@ -18,6 +18,15 @@
 #include "gemm_kernel.h"
 
 namespace gemm_impl {
+
+// What the kernels need to know of an element type beyond Elem: the kernel's parameters, the type of 16-bit results,
+// the fragments of a K step, and the epilogue.
+template <typename T> struct AnyType {
+  typedef GemmParams Params;
+  typedef T Out;
+  static constexpr int KS = 4;
+  template <bool OutF32> using Epilogue = GemmEpilogue<T, OutF32>;
+};
 
 template <> struct Elem<float> {
   typedef floatx4 vec8;  // four consecutive k: operands of four matrix instructions
@@ -47,7 +56,7 @@ struct AnyLoader {
   static constexpr int CPR = RB / 16;              // chunks per LDS row
   static constexpr int RPL = NT / CPR;             // LDS rows per load
   static constexpr int NL = ROWS * 8 / NT;
-  static_assert(NL >= 1 && RPL % 4 == 0 && (MC || RPL % 8 == 0), "the swizzle repeats, or changes by store()'s term");
+  static_assert(NL >= 1 && RPL % (EB == 1 ? 8 : 4) == 0 && (MC || RPL % 8 == 0), "the swizzle repeats, or changes by store()'s term");
   struct Regs {
     u32x4 g[NL];
     int32_t limit;  // (uniform) the largest offset that could be loaded from
@@ -60,6 +69,8 @@ struct AnyLoader {
 
   static __device__ __forceinline__ int swizzle(int row_or_k) {
     if constexpr (MC && EB == 4) return 0;
+    // 8-bit transpose reads: 32 lanes take 32 bytes of each of 8 consecutive k
+    else if constexpr (MC && EB == 1) return ROWS < 64 ? 0 : ROWS < 128 ? ((row_or_k >> 2) & 1) << 1 : ((row_or_k >> 1) & 3) << 1;
     else return swz<MC, ROWS, 64>(row_or_k);
   }
   // op: the operand (of this batch member), rows x depth elements (stored depth x rows when MC), ld elements from one
@@ -154,6 +165,15 @@ struct AnyFrag<float, MC, ROWS, TT> {
 // Zeroes the elements of a fragment (quarter ks of a K step) from k = kleft on.
 template <typename T, typename V>
 __device__ __forceinline__ void mask_fragment(V& v, int ks, int lane, int kleft) {
+  if constexpr (sizeof(T) == 1) {
+    const int n = kleft - (2 * ks + (lane >> 5)) * 32;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int b = min(max(n - 4 * q, 0), 4);  // bytes of the word that exist
+      v[q] &= b == 4 ? -1 : (1 << (8 * b)) - 1;
+    }
+    return;
+  } else {
   constexpr int E = sizeof(T) == 4 ? 4 : 8;  // consecutive k of a lane
   const int n = kleft - (2 * ks + (lane >> 5)) * E;
   u32x4 w = __builtin_bit_cast(u32x4, v);
@@ -163,6 +183,7 @@ __device__ __forceinline__ void mask_fragment(V& v, int ks, int lane, int kleft)
     else w[q] &= n >= 2 * q + 2 ? 0xffffffffu : n == 2 * q + 1 ? 0xffffu : 0u;
   }
   v = __builtin_bit_cast(V, w);
+  }
 }
 
 // acc[i][j] += the products of fragments fb[j] and fa[i] (operands swapped: gemm_kernel.h).

@@ -16,8 +16,8 @@ namespace gemm_impl {
 
 // BT x BT tile, 2 x WGN waves, K step of 128 bytes, two LDS stages.
 template <typename T, bool OutF32, bool A_MC, bool B_MC, int BT, int WGN, bool MIS>
-__global__ __launch_bounds__(2 * WGN * 64) void gemm_ragged_kernel(GemmParams p) {
-  constexpr int BK = 128 / sizeof(T), KS = 4;
+__global__ __launch_bounds__(2 * WGN * 64) void gemm_ragged_kernel(typename AnyType<T>::Params p) {
+  constexpr int BK = 128 / sizeof(T), KS = AnyType<T>::KS;
   constexpr int NT = 2 * WGN * 64, TM = BT / 64, TN = BT / WGN / 32;
   constexpr int OP_BYTES = BT * 128, STAGE = 2 * OP_BYTES;
   typedef typename Elem<T>::vec8 V8;
@@ -131,18 +131,18 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_ragged_kernel(GemmParams p)
 
   // acc[i][j][e] is out[m][n], m = m0 + 32 TM wm + 32 i + lane % 32, n = n0 + 32 TN wn + 32 j + 8 (e / 4) + 4 (lane / 32) + e % 4.
   barrier();  // every wave has read its last fragments
-  GemmEpilogue<T, OutF32> epi(p, bz);
-  store_tile<T, OutF32>(epi, acc, lds + wave * (TN * 4096), member_out(p, bz), p.ldc, bz * p.sc, p.M, p.N, m0 + wm * 32 * TM,
+  typename AnyType<T>::template Epilogue<OutF32> epi(p, bz);
+  store_tile<typename AnyType<T>::Out, OutF32>(epi, acc, lds + wave * (TN * 4096), member_out(p, bz), p.ldc, bz * p.sc, p.M, p.N, m0 + wm * 32 * TM,
                         n0 + wn * 32 * TN, lane);
 }
 
 template <typename T, bool OutF32, bool A_MC, bool B_MC>
-void launch_ragged_tile(GemmParams& p, int batch, int tile, hipStream_t st) {
+void launch_ragged_tile(typename AnyType<T>::Params& p, int batch, int tile, hipStream_t st) {
   p.tiles_m = (int)xmk::ceil_div(p.M, tile);
   p.tiles_n = (int)xmk::ceil_div(p.N, tile);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)batch);
   constexpr int WGN = sizeof(T) == 4 ? 4 : 2;
-  if constexpr (sizeof(T) == 4) {  // (16-bit operands without misaligned rows take the direct kernels)
+  if constexpr (sizeof(T) != 2) {  // (16-bit operands without misaligned rows take the direct kernels)
     if (!p.misaligned) {
       if (tile == 128) hipLaunchKernelGGL((gemm_ragged_kernel<T, OutF32, A_MC, B_MC, 128, WGN, false>), grid, dim3(WGN * 128), 0, st, p);
       else hipLaunchKernelGGL((gemm_ragged_kernel<T, OutF32, A_MC, B_MC, 64, 2, false>), grid, dim3(256), 0, st, p);
@@ -154,7 +154,7 @@ void launch_ragged_tile(GemmParams& p, int batch, int tile, hipStream_t st) {
 }
 
 template <typename T, bool OutF32>
-void launch_ragged_impl(bool a_mc, bool b_mc, GemmParams& p, int batch, int tile, hipStream_t st) {
+void launch_ragged_impl(bool a_mc, bool b_mc, typename AnyType<T>::Params& p, int batch, int tile, hipStream_t st) {
   if (!a_mc && !b_mc) launch_ragged_tile<T, OutF32, false, false>(p, batch, tile, st);
   else if (!a_mc && b_mc) launch_ragged_tile<T, OutF32, false, true>(p, batch, tile, st);
   else if (a_mc && !b_mc) launch_ragged_tile<T, OutF32, true, false>(p, batch, tile, st);
@@ -163,6 +163,6 @@ void launch_ragged_impl(bool a_mc, bool b_mc, GemmParams& p, int batch, int tile
 
 // Explicitly instantiated in gemm_inst_ragged_*.hip.
 template <typename T, bool OutF32>
-void launch_ragged(bool a_mc, bool b_mc, GemmParams& p, int batch, int tile, hipStream_t st);
+void launch_ragged(bool a_mc, bool b_mc, typename AnyType<T>::Params& p, int batch, int tile, hipStream_t st);
 
 }  // namespace gemm_impl

@@ -13,8 +13,8 @@
 namespace gemm_impl {
 
 template <typename T, bool OutF32, bool A_MC, bool B_MC, int TM, int TN, int NW, bool MIS>
-__global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(GemmParams p) {
-  constexpr int BK = 128 / sizeof(T), KS = 4;
+__global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(typename AnyType<T>::Params p) {
+  constexpr int BK = 128 / sizeof(T), KS = AnyType<T>::KS;
   constexpr int STAGE = (TM + TN) * 4096;                 // LDS per wave
   constexpr int RBY = TN * 128, XM = TN == 1 ? 7 : 15;    // partial sums: as in store_tile
   static_assert(STAGE >= TM * TN * 4096, "a wave's partial sums replace its operands");
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(GemmParams p) {
   // Eight columns of a row per thread.
   constexpr int GROUPS = 128 * TM * TN, GPT = (GROUPS + NW * 64 - 1) / (NW * 64);
   const int waves = min(NW, KT);  // waves that had a K step
-  GemmEpilogue<T, OutF32> epi(p, bz);
+  typename AnyType<T>::template Epilogue<OutF32> epi(p, bz);
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < GPT; ++u) {
@@ -140,15 +140,15 @@ __global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(GemmParams p) {
       }
       float v[1][8] = {{s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]}};
       epi.template apply<1>(v, {m}, n, count);
-      store8<T, OutF32>(member_out(p, bz), bz * p.sc + (int64_t)m * p.ldc + n, v[0], count);
+      store8<typename AnyType<T>::Out, OutF32>(member_out(p, bz), bz * p.sc + (int64_t)m * p.ldc + n, v[0], count);
     }
   }
 }
 
 // The kernel's variants, by index from kSlicesPolicy on in kPolicies.
 template <typename T, bool OutF32, bool A_MC, bool B_MC, bool MIS>
-void launch_slices_variant(int v, GemmParams& p, int batch, hipStream_t st) {
-  const Policy& pol = kPolicies[kSlicesPolicy + v];
+void launch_slices_variant(int v, typename AnyType<T>::Params& p, int batch, hipStream_t st) {
+  const Policy& pol = kPolicies[kSlicesPolicy + v];  // (fp8 has the same tiles under its own numbers)
   p.tiles_m = (int)xmk::ceil_div(p.M, pol.bm);
   p.tiles_n = (int)xmk::ceil_div(p.N, pol.bn);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)batch), block((unsigned)(pol.wgm * 64));
@@ -163,13 +163,13 @@ void launch_slices_variant(int v, GemmParams& p, int batch, hipStream_t st) {
 }
 
 template <typename T, bool OutF32, bool A_MC, bool B_MC>
-void launch_slices_rows(int v, GemmParams& p, int batch, hipStream_t st) {
+void launch_slices_rows(int v, typename AnyType<T>::Params& p, int batch, hipStream_t st) {
   if (p.misaligned) launch_slices_variant<T, OutF32, A_MC, B_MC, true>(v, p, batch, st);
   else launch_slices_variant<T, OutF32, A_MC, B_MC, false>(v, p, batch, st);
 }
 
 template <typename T, bool OutF32>
-void launch_slices_impl(bool a_mc, bool b_mc, int v, GemmParams& p, int batch, hipStream_t st) {
+void launch_slices_impl(bool a_mc, bool b_mc, int v, typename AnyType<T>::Params& p, int batch, hipStream_t st) {
   if (!a_mc && !b_mc) launch_slices_rows<T, OutF32, false, false>(v, p, batch, st);
   else if (!a_mc && b_mc) launch_slices_rows<T, OutF32, false, true>(v, p, batch, st);
   else if (a_mc && !b_mc) launch_slices_rows<T, OutF32, true, false>(v, p, batch, st);
@@ -178,6 +178,6 @@ void launch_slices_impl(bool a_mc, bool b_mc, int v, GemmParams& p, int batch, h
 
 // Explicitly instantiated in gemm_inst_slices_*.hip.
 template <typename T, bool OutF32>
-void launch_slices(bool a_mc, bool b_mc, int v, GemmParams& p, int batch, hipStream_t st);
+void launch_slices(bool a_mc, bool b_mc, int v, typename AnyType<T>::Params& p, int batch, hipStream_t st);
 
 }  // namespace gemm_impl

@@ -88,3 +88,25 @@ def test_config4_fp8_8192_sampled_rows(xmk, oracle, rhs_t):
     got = out.double().sum(dim=1).cpu().numpy()
     # a row sum adds 8192 bf16 roundings of elements near 90: about 10 in all, against sums of 1e4
     assert np.abs(got - expect).max() <= 2e-3 * np.abs(expect).max() + 1.0
+
+
+@pytest.mark.parametrize("policy", [3, 4, 5, 6, 7, 8, 9, 10])
+@pytest.mark.parametrize("rhs_t", [True, False])
+@pytest.mark.parametrize("m,n,k", [(1, 16, 16), (16, 16, 128), (17, 33, 65), (65, 127, 129), (100, 272, 208), (129, 130, 2300)])
+def test_fp8_any_alignment(xmk, oracle, monkeypatch, policy, rhs_t, m, n, k):
+    """Every tile of the kernels that take any alignment and split K over waves: rows on any byte, K tails, fewer K steps than
+    waves and more, tiles that hang over; with and without bias and output scale."""
+    monkeypatch.setenv("XMK_FP8_POLICY", str(policy))
+    a, sa = _quant(oracle, (m, k), 15)
+    b, sb = _quant(oracle, (n, k) if rhs_t else (k, n), 16)
+    bias = oracle.from_f32(oracle.normal((n,), 17, 8.0), oracle.BF16)
+    _, prod = oracle.fp8_gemm(a, b, sa, sb, rhs_t=rhs_t)
+    s = lambda v: torch.tensor([v], device="cuda")
+    for with_bias in (False, True):
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        xmk.fp8_gemm(to_dev(a, "f8"), to_dev(b, "f8"), s(sa), s(sb), out, rhs_transpose=rhs_t, d_scale=s(0.5) if with_bias else None,
+                     bias=to_dev(bias, "bf16") if with_bias else None)
+        torch.cuda.synchronize()
+        ref = 0.5 * (prod + oracle.to_f32(bias, oracle.BF16)[None, :]) if with_bias else prod
+        g, e = oracle.rel_err(out.float().cpu().numpy(), ref)
+        assert g <= 1e-2 and e <= 1e-2, (g, e)
