@@ -26,9 +26,9 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-I", INCLUDE, "
          "-Wall", "-Wno-unused-function", "-Wno-unknown-attributes"] + os.environ.get("XMK_CXXFLAGS", "").split()
 
 
-# Per-file flags.  fmha_fwd.hip: matrix instructions write VGPRs, so that the softmax reads the
+# Per-file flags.  Attention forward: matrix instructions write VGPRs, so that the softmax reads the
 # scores where they were produced (the whole register budget is then one file of 256 per wave).
-EXTRA = {"fmha_fwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("fmha_fwd.hip", "fmha_short.hip")}
 
 
 def sources():

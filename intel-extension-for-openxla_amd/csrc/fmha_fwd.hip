@@ -57,6 +57,10 @@ extern "C" int xmk_fmha_fwd(const void* query, const void* key, const void* valu
   xmk::trace("fmha_fwd B=%u N=%u F=%u T=%u H=%u causal=%d bias=%d lse=%d", num_batches, num_heads,
              num_queries, num_keys, head_size, causal, bias != nullptr, lse != nullptr);
   hipStream_t st = (hipStream_t)stream;
+  if (short_keys(num_keys, head_size, units, num_queries)) {
+    launch_short(p, dtype, units, num_queries, causal != 0, st);
+    return xmk::check_launch("fmha_fwd");
+  }
   // The staged bias path needs whole 16-byte chunks per row and offsets inside one query block
   // that fit the 31-bit buffer offset.
   const int bias_mode = !bias ? 0

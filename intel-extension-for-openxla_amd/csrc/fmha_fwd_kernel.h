@@ -768,4 +768,14 @@ void launch_cfg(FmhaParams p, uint64_t units, uint32_t F, bool causal, int bias,
 void launch_h256(const FmhaParams& p, int32_t dtype, uint64_t units, uint32_t F, bool causal, int bias,
                  hipStream_t st);
 
+// At most 128 keys, all in LDS at once (fmha_short.hip).  With four 32-key tiles and heads above 96 the keys, values and
+// queries take more than half a CU's LDS, so that one work-group per CU runs load, compute and store one after the
+// other: level with the pipelined kernel while the launch is a single round of the chip ([8,32,128,128] x 128: 9.8
+// against 10.2 us) and behind it in more ([8,32,2048,128] x 128: 104 against 76 us).  With three tiles it is ahead at
+// any size ([8,32,2048,256] x 96: 175 against 207 us), as the pipelined kernel's tiles round the keys up to 128.
+inline bool short_keys(uint32_t keys, uint32_t head, uint64_t units, uint32_t queries) {
+  return keys <= 96 || (keys <= 128 && (head <= 96 || units * ((queries + 127) / 128) <= 256));
+}
+void launch_short(const FmhaParams& p, int32_t dtype, uint64_t units, uint32_t F, bool causal, hipStream_t st);
+
 }  // namespace fmha_fwd_impl

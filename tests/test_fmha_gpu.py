@@ -126,6 +126,20 @@ def test_masks_bias_lse(xmk, oracle, name, causal, use_bias, F, T, H):
     _run(xmk, oracle, name, 2, 3, F, T, H, causal=causal, use_bias=use_bias, lse=True, seed=F * 7 + T)
 
 
+@pytest.mark.parametrize("F,T,H", [(1, 1, 8), (33, 31, 64), (129, 32, 72), (128, 33, 96), (31, 64, 104), (160, 65, 128),
+                                   (97, 96, 136), (257, 97, 96), (64, 128, 160), (130, 128, 168), (40, 90, 256),
+                                   (65, 125, 256)])
+@pytest.mark.parametrize("causal,use_bias", [(False, False), (True, True)])
+def test_short_keys(xmk, oracle, F, T, H, causal, use_bias):
+    """At most 128 keys: the edges of the 32-key and 32-row tiles and of the head-size classes."""
+    _run(xmk, oracle, "fp16", 2, 3, F, T, H, causal=causal, use_bias=use_bias, lse=True, seed=F + T + H)
+
+
+def test_short_keys_many_groups(xmk, oracle):
+    """128 keys, heads above 96, more work-groups than one per CU: the pipelined kernel serves these."""
+    _run(xmk, oracle, "bf16", 4, 33, 300, 128, 128, units=[0, 131], seed=5)
+
+
 def test_bias_paths_agree(xmk):
     """The same bias through the LDS-staged path (16-byte aligned) and, from a copy that starts 2 bytes
     later, through the element-wise path: identical scores, so identical outputs."""
