@@ -18,6 +18,7 @@
 
 #include "common.h"
 #include "int4_gemm.h"
+#include "int4_tile.h"
 
 namespace {
 
@@ -803,16 +804,55 @@ int xmk::int4_gemm_launch(const void* act, const void* qweight, const void* scal
   return int4_gemm_launch2(c, nullptr, m, group, st);
 }
 
+namespace {
+
+// Rows from which on the row tiles take a product.  Up to 40, int4_gemm_kernel's second pass carries at most eight rows and
+// is the cheap one that decode steps use (k 6656, n 2608: 33 rows 14.2 us against 17.6; k 3584, n 14000: 37 rows 18.3
+// against 20.2; level at k = n = 4096), and up to 48 where a long reduction meets few column blocks, on whose work-groups
+// that kernel's narrower blocks are spread wider (42 rows, k 12928, n 1120: 23.0 against 30.0; 48 rows, k = n = 4096: 12.4
+// against 11.4).
+bool tile_rows(int64_t m, int64_t k, int64_t n) { return m > 48 || (m > 40 && (k <= 8192 || n > 8192)); }
+
+bool run_tiles(const void* act, const void* qweight, const void* scales, const void* zeros, const void* bias, void* out,
+               int64_t m, int64_t k, int64_t n, int64_t group, hipStream_t st) {
+  constexpr int64_t kMax = 1 << 24;
+  if (!tile_rows(m, k, n) || m > kMax || k > kMax || n > kMax || group > kMax) return false;
+  const xmk::Int4TileArgs t{(const _Float16*)act, (const uint32_t*)qweight, (const _Float16*)scales, (const _Float16*)zeros,
+                            (const _Float16*)bias, (_Float16*)out, (int)m, (int)k, (int)n, (int)group, 0, 0};
+  if (!xmk::int4_tile_applicable(t)) return false;
+  xmk::trace("int4_gemm m=%lld k=%lld n=%lld group=%lld row tiles", (long long)m, (long long)k, (long long)n, (long long)group);
+  xmk::int4_tile_launch(t, st);
+  return true;
+}
+
+// What writing the fp16 weights out and the dense fp16 product on them take, in microseconds: two launches, 2.5 bytes per
+// weight at 5.5 TB/s, and a product that is bound by its flops or, with few rows, by the latency of its K steps.
+// (k 4096, n 16384: 128 rows 58.6 measured, 55 from this; 512 93 / 95; 1024 142 / 150; k = n = 4096: 256 rows 32.8 / 32.6.)
+double dense_cost(int64_t m, int64_t k, int64_t n) {
+  const double kn = (double)k * (double)n;
+  const double by_flops = 2.0 * kn * (double)m / 1.25e9, by_steps = 0.0036 * (double)k;
+  return 10.0 + kn * 2.5 / 5.5e6 + (by_flops > by_steps ? by_flops : by_steps);
+}
+
+}  // namespace
+
 extern "C" int xmk_int4_gemm(const void* act, const void* qweight, const void* scales,
                              const void* zeros, const void* bias, void* out, int64_t m, int64_t k,
                              int64_t n, int64_t group, void* stream) {
+  if (tile_rows(m, k, n)) {
+    xmk::Int4Call c;
+    c.act = act; c.qweight = qweight; c.scales = scales; c.zeros = zeros; c.out = out;
+    c.k = k; c.n = n;
+    Config cfg;
+    const int rc = prepare(c, m, group, &cfg);
+    if (rc != XMK_OK) return rc;
+    if (run_tiles(act, qweight, scales, zeros, bias, out, m, k, n, group, (hipStream_t)stream)) return xmk::check_launch("int4_gemm");
+  }
   return xmk::int4_gemm_launch(act, qweight, scales, zeros, bias, out, m, k, n, group,
                                xmk::Int4Epilogue{}, (hipStream_t)stream);
 }
 
-// From this many rows on, writing the fp16 weight matrix out once and running the dense fp16 GEMM on it is
-// faster than streaming the packed weights once per 32 rows (measured at 128 rows: 54 against 68 us for
-// k 4096, n 16384; 82 against 131 us for k 16384, n 4096; at 96 rows the first shape is a tie).
+// From this many rows on scratch for the fp16 weights is asked for: the dense product on them can be the faster way.
 constexpr int64_t kInt4DenseRows = 96;
 
 extern "C" size_t xmk_int4_gemm_workspace_bytes(int64_t m, int64_t k, int64_t n) {
@@ -829,6 +869,10 @@ extern "C" int xmk_int4_gemm_ws(const void* act, const void* qweight, const void
     return xmk_int4_gemm(act, qweight, scales, zeros, bias, out, m, k, n, group, stream);
   if (group <= 0 || group % 32 != 0 || group > 256)  // the same contract whatever the path
     return xmk::fail(XMK_UNIMPLEMENTED, "int4_gemm: group must be 32, 64, 128 or 256");
+  // (Both sides from the fitted costs; they meet at 500 to 800 rows where n is large.)
+  if (xmk::int4_tile_cost(m, k, n, group) < dense_cost(m, k, n) &&
+      run_tiles(act, qweight, scales, zeros, bias, out, m, k, n, group, (hipStream_t)stream))
+    return xmk::check_launch("int4_gemm");
   xmk::trace("int4_gemm m=%lld k=%lld n=%lld group=%d dense: dequantise + fp16 GEMM", (long long)m, (long long)k,
              (long long)n, (int)group);
   const int rc = xmk_int4_dequant(qweight, scales, zeros, workspace, k, n, group, stream);

@@ -133,6 +133,54 @@ def test_int4_gemm_many_rows_with_scratch(xmk, oracle, m, k, n, group, with_bias
     assert (outs[0] - outs[1]).abs().max().item() <= 1e-2 * outs[1].abs().max().item()
 
 
+@pytest.mark.parametrize("m,k,n,group", [
+    # 32-row tiles, eight waves on one reduction: one row past a tile, one column block, odd step count, every group size
+    (41, 1056, 72, 32), (64, 3136, 136, 64), (65, 4096, 1000, 128), (96, 2304, 64, 256),
+    # the same with four waves: a single step (and less than one), more than one round of work-groups
+    (41, 32, 8, 32), (49, 512, 200, 64), (70, 1024, 8200, 128), (67, 768, 6152, 256),
+    # 64 rows x 128 columns on eight and on four waves
+    (128, 640, 16328, 128), (97, 768, 16264, 256), (128, 1056, 16328, 32), (100, 1088, 16384, 64),
+    (255, 512, 16392, 256), (200, 384, 4000, 128), (250, 480, 8000, 32), (130, 320, 9000, 64),
+    # 64 rows x 256 columns
+    (310, 128, 16400, 128), (300, 256, 16400, 256), (257, 224, 16400, 32), (383, 192, 16328, 64),
+])
+def test_int4_gemm_row_tiles(xmk, oracle, m, k, n, group):
+    """Products of more than 32 rows, without scratch: every tile shape at the edges of its rows, columns and steps.
+    The error is the output's rounding, 2^-11 of a value, plus that of the fp32 sums: a group's sum of a (1024 + q)
+    stays below 1039 * 4 sqrt(group), is rounded eight times per 128 k and scaled by up to 0.02, and the K / group
+    groups' errors add like noise."""
+    act, qw, s, z = _case(oracle, m, k, n, group, 3000 + m + n)
+    bias = oracle.from_f32(oracle.normal((n,), 57), oracle.F16) if m % 2 else None
+    _, ref = oracle.int4_gemm(act, qw, s, z, group, bias=bias)
+    guard = 64  # rows before and behind the result stay as they were
+    out = torch.full((m + 2 * guard, n), 7.0, dtype=torch.float16, device="cuda")
+    xmk.int4_gemm(to_dev(act, "f16"), to_dev(qw, "u32"), to_dev(s, "f16"), to_dev(z, "f16"), out[guard:guard + m],
+                  group=group, bias=None if bias is None else to_dev(bias, "f16"))
+    torch.cuda.synchronize()
+    got = out[guard:guard + m].float().cpu().numpy()
+    ref = np.asarray(ref, np.float32).reshape(m, n)
+    assert np.all(np.abs(got - ref) <= np.abs(ref) * 2.0 ** -11 + 2.0 ** -24 * 1039 * 4 * k ** 0.5 * 8 * 0.02)
+    assert bool((out[:guard] == 7).all()) and bool((out[guard + m:] == 7).all())
+
+
+def test_int4_gemm_row_tiles_keep_rows_apart(xmk, oracle):
+    """An infinity in one row of the activations reaches no other row, also where a step reaches past the end of K."""
+    m, k, n, group = 70, 160, 200, 32
+    act, qw, s, z = _case(oracle, m, k, n, group, 77)
+    a = to_dev(act, "f16")
+    outs = []
+    for bad in (False, True):
+        b = a.clone()
+        if bad:
+            b[41, 0] = float("inf")
+        out = torch.empty((m, n), dtype=torch.float16, device="cuda")
+        xmk.int4_gemm(b, to_dev(qw, "u32"), to_dev(s, "f16"), to_dev(z, "f16"), out, group=group)
+        torch.cuda.synchronize()
+        outs.append(out)
+    keep = [i for i in range(m) if i != 41]
+    assert torch.equal(outs[0][keep], outs[1][keep])
+
+
 def test_int4_errors(xmk):
     a = torch.zeros((1, 256), dtype=torch.float16, device="cuda")
     qw = torch.zeros((32, 64), dtype=torch.int32, device="cuda")
