@@ -23,10 +23,13 @@ struct Args {
   int H, F, T;
   float scale;
   bool causal;
+  bool stats_ready;      // lse and dsum have been formed; required where one_grid() says so
 };
 
 // Head sizes up to 256 (multiples of 8); a bias of at most 2 GiB per unit.
 bool eligible(const Args& a, uint64_t units);
+// Whether all passes should run as one grid, on statistics that are formed before it.
+bool one_grid(const Args& a, uint64_t units);
 // Queries own (dQ; it also forms the two per-row statistics), then keys own (dK, dV).
 void launch(const Args& a, uint64_t units, bool bf16, hipStream_t stream);
 

@@ -8,6 +8,7 @@
 // with  P = exp(scale S - LSE),  dS = P o (dP - D),  S = Q K^T,  dP = dO V^T,  D = rowsum(dO o O).
 // S (and dP) are recomputed in every pass (8 matrix products instead of 5) so that no gradient needs
 // atomics or a second pass over partial sums: every output element is written once, in a fixed order.
+// Problems of few work-groups run all passes as one grid (one_grid() below).
 //
 // As in the forward kernel, every product is issued so that a lane owns ONE owner row:
 //   scores  = Stream_tile . Owner^T : A operand = fragment of the streamed tile (LDS), B operand =
@@ -81,8 +82,8 @@ struct KParams {
   const void* strm2;  // streamed operand of the dP product:    dO (owner = keys) or V
   const void* bias;   // [units, F, T] additive bias of the scores, or null
   int bias_vec;       // queries-own pass: the bias may be read 4 keys (8 bytes) at a time
-  float* lse;         // [units, F] LSE of the forward pass times log2(e)    } the queries-own launch writes them,
-  float* dsum;        // [units, F] D = rowsum(dO o O)                       } the keys-own launches read them
+  float* lse;         // [units, F] LSE of the forward pass times log2(e)    } the queries-own launch writes them and
+  float* dsum;        // [units, F] D = rowsum(dO o O)                       } the keys-own ones read them; in one grid, all read
   const void* o;      // [units, F, H] forward output and
   const float* lse_fwd;  // [units, F] its LSE (queries-own launch)
   void* out1;         // scale * dS^T Q (dK)  or  scale * dS K (dQ)
@@ -101,8 +102,11 @@ struct KParams {
 // BIAS: S + bias enters the softmax; the bias is read from global memory at the start of each block
 // (keys-own pass: 2-byte loads that are contiguous across the lanes of a wave; queries-own pass: each
 // lane reads its own row, 8 bytes at a time where the alignment allows).
-template <typename T, int HP, bool OWNER_K, bool CAUSAL, bool DS, bool PV, bool BIAS>
-__global__ __launch_bounds__(256, (HP <= 128 && !BIAS && !(DS && PV && HP > 64)) ? 2 : 1) void fmha_bwd_kernel(KParams p) {
+// STATS_IN: the row statistics are there (the queries-own pass reads them as the keys-own passes do, and writes none).
+// lds: bwd_lds_bytes(HP) bytes; block: the work-group's number among the pass's.
+constexpr int bwd_lds_bytes(int HP) { return 4 * BS * HP * 2 + 2 * (2 * BS * 4); }
+template <typename T, int HP, bool OWNER_K, bool CAUSAL, bool DS, bool PV, bool BIAS, bool STATS_IN>
+__device__ __forceinline__ void bwd_pass(const KParams& p, char* lds, int block_id) {
   static_assert(DS || PV, "nothing to compute");
   static_assert(!PV || OWNER_K, "P^T dO belongs to the keys-own pass");
   typedef typename Elem<T>::vec8 V8;
@@ -119,7 +123,7 @@ __global__ __launch_bounds__(256, (HP <= 128 && !BIAS && !(DS && PV && HP > 64))
   constexpr int HT = HP / 32;                // 32-wide h tiles of the gradients
   constexpr int STATS = 2 * BS * 4;          // LSE and D of one block's 64 query rows (owner = keys)
   static_assert(NL >= 1 && LROWS % 8 == 0 && (2 * LROWS) % (KMASK + 1) == 0, "tile / wave split");
-  __shared__ __attribute__((aligned(1024))) char lds[4 * TILE + 2 * STATS];
+  static_assert(bwd_lds_bytes(HP) == 4 * TILE + 2 * STATS, "what the kernels below reserve");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -136,8 +140,8 @@ __global__ __launch_bounds__(256, (HP <= 128 && !BIAS && !(DS && PV && HP > 64))
   };
   // Each XCD (own L2) gets a contiguous range of (unit, owner block) pairs: the owner blocks of a
   // unit stream the same tiles.
-  const int wg = (int)(blockIdx.x % 8) * p.per_xcd + (int)(blockIdx.x / 8);
-  if (wg >= p.total) return;
+  const int wg = (block_id % 8) * p.per_xcd + block_id / 8;
+  if (wg >= p.total || block_id >= 8 * p.per_xcd) return;
   // Inside the range, units go four at a time, owner blocks outermost and (causal) heaviest first, so that an
   // XCD's slots run dry at about the same time.
   const int UG = p.ug;
@@ -337,7 +341,12 @@ __global__ __launch_bounds__(256, (HP <= 128 && !BIAS && !(DS && PV && HP > 64))
   // the wave holds anyway and the same pieces of O, and written out for the keys-own launches that follow: a
   // separate pass over O and dO for them was 45 us at [8,32,2048,128].
   float own_lse2 = 0.f, own_d = 0.f;
-  if constexpr (!OWNER_K) {
+  if constexpr (!OWNER_K && STATS_IN) {
+    if (orow < p.F) {
+      own_lse2 = lse[orow];
+      own_d = dsum[orow];
+    }
+  } else if constexpr (!OWNER_K) {
     static_assert(DS, "the queries-own launch holds dO");
     const T* Oo = reinterpret_cast<const T*>(p.o) + (int64_t)unit * n_own * H;
     issue_rows(Oo, o0, s1, n_own);
@@ -498,13 +507,35 @@ __global__ __launch_bounds__(256, (HP <= 128 && !BIAS && !(DS && PV && HP > 64))
   }
 }
 
-template <typename T, int HP, bool OWNER_K, bool DS, bool PV>
-void launch_pass(KParams p, uint64_t units, bool causal, hipStream_t st) {
-  const int n_own = OWNER_K ? p.T : p.F;
+template <typename T, int HP, bool OWNER_K, bool CAUSAL, bool DS, bool PV, bool BIAS>
+__global__ __launch_bounds__(256, (HP <= 128 && !BIAS && !(DS && PV && HP > 64)) ? 2 : 1) void fmha_bwd_kernel(KParams p) {
+  __shared__ __attribute__((aligned(1024))) char lds[bwd_lds_bytes(HP)];
+  bwd_pass<T, HP, OWNER_K, CAUSAL, DS, PV, BIAS, false>(p, lds, (int)blockIdx.x);
+}
+
+// All passes in one grid, a row of it each, on statistics formed before: for problems of which a single pass leaves the
+// device idle.  What bounds those is the walk of one work-group over the streamed rows (2 us per 64 rows, one wave per
+// SIMD), once per launch: [2,7,463,128] causal took three of them.
+template <typename T, int HP, bool CAUSAL>
+__global__ __launch_bounds__(256, HP <= 128 ? 2 : 1) void fmha_bwd_small_kernel(KParams dq, KParams dk, KParams dv) {
+  __shared__ __attribute__((aligned(1024))) char lds[bwd_lds_bytes(HP)];
+  const int block = (int)blockIdx.x;
+  if (blockIdx.y == 0) bwd_pass<T, HP, false, CAUSAL, true, false, false, true>(dq, lds, block);
+  else if constexpr (HP <= 64) bwd_pass<T, HP, true, CAUSAL, true, true, false, true>(dk, lds, block);
+  else if (blockIdx.y == 1) bwd_pass<T, HP, true, CAUSAL, true, false, false, true>(dk, lds, block);
+  else bwd_pass<T, HP, true, CAUSAL, false, true, false, true>(dv, lds, block);
+}
+
+void split(KParams& p, int n_own, uint64_t units) {
   p.nob = (n_own + BO - 1) / BO;
   p.total = (int)(units * p.nob);
   p.per_xcd = (p.total + 7) / 8;
   p.ug = std::max(4, (64 + p.nob - 1) / p.nob);  // enough units to fill an XCD's slots with one round
+}
+
+template <typename T, int HP, bool OWNER_K, bool DS, bool PV>
+void launch_pass(KParams p, uint64_t units, bool causal, hipStream_t st) {
+  split(p, OWNER_K ? p.T : p.F, units);
   const dim3 grid((unsigned)(p.per_xcd * 8)), block(256);
   if (p.bias) {
     if (causal) hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, true, DS, PV, true>), grid, block, 0, st, p);
@@ -522,8 +553,18 @@ void launch_both(const fmha_bwd_fused::Args& a, uint64_t units, hipStream_t st) 
   p.bias = a.bias;
   p.bias_vec = a.bias && a.T % 4 == 0 && xmk::aligned(a.bias, 8);
   p.nob = p.total = p.per_xcd = 0;
-  // owner = queries first: dQ, and the per-row statistics the other launches read
   p.own1 = a.q; p.own2 = a.d_o; p.strm1 = a.k; p.strm2 = a.v; p.out1 = a.dq; p.out2 = nullptr;
+  if (a.stats_ready) {
+    KParams k = p;
+    k.own1 = a.k; k.own2 = a.v; k.strm1 = a.q; k.strm2 = a.d_o; k.out1 = a.dk; k.out2 = a.dv;
+    split(p, a.F, units);
+    split(k, a.T, units);
+    const dim3 grid((unsigned)(std::max(p.per_xcd, k.per_xcd) * 8), HP <= 64 ? 2 : 3), block(256);
+    if (a.causal) hipLaunchKernelGGL((fmha_bwd_small_kernel<T, HP, true>), grid, block, 0, st, p, k, k);
+    else hipLaunchKernelGGL((fmha_bwd_small_kernel<T, HP, false>), grid, block, 0, st, p, k, k);
+    return;
+  }
+  // owner = queries first: dQ, and the per-row statistics the other launches read
   launch_pass<T, HP, false, true, false>(p, units, a.causal, st);
   // owner = keys: dK, then dV
   p.own1 = a.k; p.own2 = a.v; p.strm1 = a.q; p.strm2 = a.d_o; p.out1 = a.dk; p.out2 = a.dv;
@@ -547,6 +588,17 @@ bool eligible(const Args& a, uint64_t units) {
   return a.H <= 256 && a.H % 8 == 0 && units * ((uint64_t)((a.F > a.T ? a.F : a.T) + BO - 1) / BO) < 0x7fffffffull &&
          (uint64_t)a.F * a.H * 2 < kOob && (uint64_t)a.T * a.H * 2 < kOob &&
          (!a.bias || (uint64_t)a.F * a.T * 2 < kOob);
+}
+
+// One grid (plus a launch for the statistics) against a launch per pass, causal bf16: 14 units of 463 rows, heads of 128,
+// 56 -> 26 us; 4 x 4096 336 -> 155; 16 x 2048 183 -> 116; heads of 64, 32 x 1024 51 -> 39; heads of 256, 14 x 463
+// 121 -> 48.  Up to 384 work-groups per pass all that was timed gained 10 % or more, 512 still 2 - 18 % on 512 rows and
+// more; 512 of 64 or 128 rows lost 5 % (23 -> 24 us), 256 x 128 with heads of 256 2 %.  Kernels with a bias run one
+// wave per SIMD and hold other accumulators; they keep their launches.
+bool one_grid(const Args& a, uint64_t units) {
+  const uint64_t rows = (uint64_t)std::max(a.F, a.T), groups = units * ((rows + BO - 1) / BO);
+  const uint64_t most = rows >= 512 ? 512 : (a.H > 128 && rows <= 128) ? 128 : 384;
+  return !a.bias && groups <= most;
 }
 
 void launch(const Args& a, uint64_t units, bool bf16, hipStream_t st) {

@@ -59,6 +59,18 @@ def test_backward_shapes(xmk, oracle, name, causal, use_bias, F, T, H):
     _run(xmk, oracle, name, 2, 3, F, T, H, causal, use_bias)
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("B,N,F,T,H", [
+    # (not a single key: its softmax is constant, dQ and dK are exactly zero and an error relative to them has no bound)
+    (1, 1, 2, 3, 128), (1, 3, 129, 513, 64), (1, 2, 640, 127, 80), (1, 3, 385, 129, 256),  # one grid: passes of different widths
+    (96, 4, 64, 65, 64), (96, 4, 33, 128, 128),                                         # the most work-groups it takes
+    (97, 4, 65, 64, 64), (97, 4, 128, 40, 128), (43, 3, 32, 64, 256),                   # one more: a launch per pass
+])
+def test_backward_one_grid_or_three_launches(xmk, oracle, causal, B, N, F, T, H):
+    """fp16: few work-groups run all passes as one grid, on statistics formed before; more, a launch per pass."""
+    _run(xmk, oracle, "fp16", B, N, F, T, H, causal, False, seed=F + T)
+
+
 def test_backward_large(xmk, oracle):
     """Many blocks with a bias and a causal mask; the elementwise bound of the large shapes."""
     errs = _run(xmk, oracle, "bf16", 1, 12, 2048, 2048, 64, True, True, seed=9, tol_elem=TOL_ELEM_LARGE["bf16"])
