@@ -43,8 +43,8 @@ struct GemmParams {
   // int8 kernel only: elements per load that the alignment of each operand's pointer, leading dimension, batch
   // stride and row length allows.
   int vec_a, vec_b;
-  // Kernels that take any alignment only: K slice of one grid member (a multiple of the K step), 0 when K is not
-  // split; some row of an operand does not start on a 16-byte boundary.
+  // K slice of one grid member (a multiple of the K step), 0 when K is not
+  // split.  Kernels that take any alignment: some row of an operand does not start on a 16-byte boundary.
   int kslice;
   bool misaligned;
 };
@@ -520,8 +520,10 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p)
   const int m0 = tile_m * BM, n0 = tile_n * BN;
 
   const int64_t bz = blockIdx.z;
-  const T* A = reinterpret_cast<const T*>(p.a) + bz * p.sa;
-  const T* B = reinterpret_cast<const T*>(p.b) + bz * p.sb;
+  const int64_t k0 = bz * p.kslice;  // K slices (kslice > 0): grid member z takes k0 .. k0 + kslice - 1
+  const int K = p.kslice ? min(p.K - (int)k0, p.kslice) : p.K;
+  const T* A = reinterpret_cast<const T*>(p.a) + bz * p.sa + (A_MC ? k0 * p.lda : k0);
+  const T* B = reinterpret_cast<const T*>(p.b) + bz * p.sb + (B_MC ? k0 * p.ldb : k0);
 
   floatx16 acc[TM][TN];
 #pragma unroll
@@ -531,7 +533,7 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p)
 
   LoaderA la;
   LoaderB lb;
-  const int KT = (p.K + BK - 1) / BK;
+  const int KT = (K + BK - 1) / BK;
   la.init(p.lda, p.M - m0, wave, lane);
   lb.init(p.ldb, p.N - n0, wave, lane);
   // Tile origins; one K step further is +BK elements (KC) or +BK rows (MC).
@@ -546,8 +548,8 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p)
   // vmcnt arithmetic below is uniform.
 #pragma unroll
   for (int st = 0; st < NSTAGE - 1; ++st) {
-    la.issue(a_tile, p.K - st * BK, lds + st * STAGE, wave);
-    lb.issue(b_tile, p.K - st * BK, lds + st * STAGE + A_BYTES, wave);
+    la.issue(a_tile, K - st * BK, lds + st * STAGE, wave);
+    lb.issue(b_tile, K - st * BK, lds + st * STAGE + A_BYTES, wave);
     a_tile += a_step;
     b_tile += b_step;
   }
@@ -600,7 +602,7 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p)
   auto k_step = [&](auto CHECK, const char* __restrict__ cur, const char* __restrict__ nxt, char* __restrict__ wr,
                     int kt) {
     constexpr bool CHECK_K = decltype(CHECK)::value;
-    const int kleft = p.K - (kt + NSTAGE - 1) * BK;
+    const int kleft = K - (kt + NSTAGE - 1) * BK;
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(a_tile), rb = make_rsrc(b_tile);
     static_for<KS>([&](auto KSI) {
       constexpr int ks = decltype(KSI)::value;
@@ -632,7 +634,7 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p)
   // Step kt loads K step kt + NSTAGE - 1: all of it exists until that index reaches the last
   // (possibly partial) step, so only the final NSTAGE - 1 iterations (and a partial last K step)
   // need the per-lane K test.
-  const int kt_full = min(KT, p.K / BK - (NSTAGE - 1));
+  const int kt_full = min(KT, K / BK - (NSTAGE - 1));
   int kt = 0;
   for (; kt < kt_full; ++kt)
     k_step(std::false_type{}, lds + (kt % NSTAGE) * STAGE, lds + ((kt + 1) % NSTAGE) * STAGE,
@@ -811,7 +813,7 @@ inline float launch_cost(const Policy& P, const TileCost& c, bool slices, uint32
 struct Choice {
   int policy, slices;
 };
-// The cheapest policy and number of K slices (1 unless may_split; direct kernels: only slices of whole chunks).
+// The cheapest policy and number of K slices (1 unless may_split).
 inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, bool may_split) {
   Choice best{3, 1};
   float best_cost = 1e30f;
@@ -831,7 +833,7 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
   };
   each(1, 0.0f, 0.0f);
   for (int s = 2; may_split && s <= 16 && best_cost > kSplitFloor; s *= 2) {
-    if (k / s < 128 || (direct && k % (8 * s) != 0) || (float)m * (float)n * (float)s > 6.4e7f) break;
+    if (k / s < 128 || (float)m * (float)n * (float)s > 6.4e7f) break;
     each(s, kSplitCost + (float)m * (float)n * (float)s * (8.0f / 3e6f), kSplitFloor);
   }
   return best;

@@ -279,6 +279,28 @@ def test_split_k_with_workspace(xmk, oracle, dt_name, m, n, k, rhs_t, epi):
     assert xmk.gemm_workspace_bytes(big, w, big) == 0
 
 
+@pytest.mark.parametrize("dt_name", ["BF16", "F16"])
+@pytest.mark.parametrize("m,n,k,rhs_t", [(128, 1024, 8200, True), (100, 264, 5128, False), (16, 1032, 4104, False),
+                                         (70, 512, 12296, True), (65, 520, 9736, False), (33, 256, 16376, False),
+                                         (3, 520, 5000, False), (130, 200, 16376, True)])
+def test_split_k_unequal_slices(xmk, oracle, dt_name, m, n, k, rhs_t):
+    """A reduction that does not divide into equal 16-byte aligned slices: slices of whole K steps, a shorter last one."""
+    dt = getattr(oracle, dt_name)
+    kind = _kind(dt, oracle)
+    a = oracle.from_f32(oracle.normal((m, k), 84, k ** -0.5), dt)
+    b = oracle.from_f32(oracle.normal((n, k) if rhs_t else (k, n), 85, 1.0), dt)
+    bias = oracle.from_f32(oracle.normal((n,), 86, 0.5), dt)
+    _, ref = oracle.gemm(a, b, dt, dt, rhs_t=rhs_t, bias=bias, epilogue=oracle.EPI_BIAS)
+    da, db = to_dev(a, kind), to_dev(b, kind)
+    out = torch.full((m, n), float("nan"), dtype=da.dtype, device="cuda")
+    nbytes = xmk.gemm_workspace_bytes(da, db, out, rhs_transpose=rhs_t)
+    assert nbytes > 0, "these shapes are meant to split"
+    ws = torch.full((nbytes,), 0xff, dtype=torch.uint8, device="cuda")
+    xmk.run_gemm(da, db, out, rhs_transpose=rhs_t, bias=to_dev(bias, kind), epilogue=xmk.EPI_BIAS, workspace=ws)
+    torch.cuda.synchronize()
+    _check(oracle, out.float().cpu().numpy(), ref[0])
+
+
 @pytest.mark.parametrize("m,rhs_t", [(1, False), (4, False), (4, True), (32, False)])
 def test_vocabulary_projection_n50400(xmk, oracle, m, rhs_t):
     """The decode rows of the reference's tile table against a vocabulary of 50400 columns
