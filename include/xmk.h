@@ -228,6 +228,9 @@ int xmk_fmha_decode_static(const void* query, const void* key, const void* value
  *   W[k, n] = fp16(w[k, n]), rounded to nearest even, is what xmk_int4_dequant writes;
  *   out[m, n] = fp16( sum_k float(act[m, k]) * w[k, n] + float(bias[n]) ),
  *     fp32 accumulation, no intermediate rounding of w to fp16; bias fp16 [N] or NULL.
+ *     The sums of act q and of act are formed apart and combined per group, so a row of act that holds an
+ *     infinity comes out as NaN (on the dense path of xmk_int4_gemm_ws as infinities or NaN); other rows are
+ *     not touched by it.
  * act fp16 [M, K] packed, out fp16 [M, N] packed.  K % group == 0, N % 8 == 0;
  * group is 32, 64, 128 or 256 for xmk_int4_gemm and any multiple of 8 for
  * xmk_int4_dequant. */
