@@ -167,6 +167,12 @@ int xmk_fmha_fwd(const void* query, const void* key, const void* value, const vo
 size_t xmk_fmha_bwd_workspace_bytes(uint32_t num_batches, uint32_t num_heads, uint32_t head_size,
                                     uint32_t num_queries, uint32_t num_keys);
 
+/* Bytes of workspace with which xmk_fmha_bwd (without a bias) runs fastest: given more than
+ * xmk_fmha_bwd_workspace_bytes(), it keeps the score gradients there, of all (batch, head) units or some at a time,
+ * instead of forming them twice.  At most 2 GiB more. */
+size_t xmk_fmha_bwd_best_workspace_bytes(uint32_t num_batches, uint32_t num_heads, uint32_t head_size,
+                                         uint32_t num_queries, uint32_t num_keys, int32_t causal);
+
 /* Fused multi-head-attention backward.  Replaces fmha_backward_kernel_fp16 / _bf16
  * (xetla/sdp/sdp_backward.h:22-36; same tensors, with the reference's two scratch arguments
  * dp_sum and grad_query_accum folded into one workspace, the dtype and `causal` as arguments).

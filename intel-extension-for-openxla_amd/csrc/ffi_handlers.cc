@@ -334,13 +334,19 @@ XLA_FFI_Error* fmha_bwd_common(XLA_FFI_CallFrame* f, bool with_bias) {
   void* stream = fr.stream();
   if (fr.code != XMK_OK) return finish(fr, XMK_OK);
   // dp_sum / grad_query_accum of the reference (:392-399) are one workspace here, from the
-  // executor's scratch allocator.
-  const size_t need = xmk_fmha_bwd_workspace_bytes((uint32_t)B, (uint32_t)N, (uint32_t)H, (uint32_t)F, (uint32_t)T);
-  return finish(fr, with_scratch(f, need, [&](void* ws) {
+  // executor's scratch allocator; where it does not give the most the kernels use, the least they take.
+  const uint32_t b = (uint32_t)B, n = (uint32_t)N, h = (uint32_t)H, nq = (uint32_t)F, nk = (uint32_t)T;
+  const size_t least = xmk_fmha_bwd_workspace_bytes(b, n, h, nq, nk);
+  const size_t best = bias ? least : xmk_fmha_bwd_best_workspace_bytes(b, n, h, nq, nk, causal);
+  auto run = [&](void* ws, size_t bytes) {
     if (!ws) return xmk::fail(XMK_INTERNAL, "fmha backward: the host's API table has no scratch allocator");
     return xmk_fmha_bwd(q->data, k->data, v->data, bias ? bias->data : nullptr, fwd_out->data, d_out->data,
                         static_cast<const float*>(act->data), dq->data, dk->data, dv->data, (int32_t)q->dtype,
-                        (uint32_t)B, (uint32_t)N, (uint32_t)H, (uint32_t)F, (uint32_t)T, scale, causal, ws, need, stream);
+                        b, n, h, nq, nk, scale, causal, ws, bytes, stream);
+  };
+  return finish(fr, with_scratch(f, best, [&](void* ws) {
+    if (ws || best == least) return run(ws, best);
+    return with_scratch(f, least, [&](void* ws2) { return run(ws2, least); });
   }));
 }
 

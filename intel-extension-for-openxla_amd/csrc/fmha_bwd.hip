@@ -12,6 +12,7 @@
 // also takes its scratch, dp_sum and grad_query_accum, from the caller:
 // xetla_gpu_fused_mha_runner.cc:331-339); the chunk size bounds them.  No gradient is produced
 // for the bias, as in the reference (xetla_gpu_fused_mha_runner.cc:383-385).
+#include <algorithm>
 #include <cstdlib>
 
 #include "common.h"
@@ -149,7 +150,7 @@ size_t fused_bytes(uint64_t units, uint64_t F) { return 2 * dsum_bytes(units, F)
 template <typename T>
 int run(const void* q, const void* k, const void* v, const void* bias, const void* o, const void* d_o,
         const float* lse, void* dq, void* dk, void* dv, int dtype, int64_t units, int64_t H, int64_t F, int64_t Tk,
-        float scale, int causal, char* ws, const Plan& pl, void* stream) {
+        float scale, int causal, char* ws, size_t ws_bytes, const Plan& pl, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   float* dsum = reinterpret_cast<float*>(ws);
   float* s32 = reinterpret_cast<float*>(ws + pl.off_s);
@@ -173,8 +174,12 @@ int run(const void* q, const void* k, const void* v, const void* bias, const voi
                          rows, (int)H, lse_in, lse2_out);
   };
   if (fused) {
-    fmha_bwd_fused::Args a{q, k, v, d_o, o, bias, lse, lse2, dsum, dq, dk, dv, (int)H, (int)F, (int)Tk, scale, causal != 0, false};
-    if (fmha_bwd_fused::one_grid(a, (uint64_t)units)) {
+    fmha_bwd_fused::Args a{q, k, v, d_o, o, bias, lse, lse2, dsum, dq, dk, dv, (int)H, (int)F, (int)Tk, scale, causal != 0, false, nullptr, 0};
+    const size_t stats = fused_bytes((uint64_t)units, (uint64_t)F);
+    a.ds_units = fmha_bwd_fused::saved_units(a, (uint64_t)units, ws_bytes - stats);
+    if (a.ds_units) {
+      a.ds = ws + stats;
+    } else if (fmha_bwd_fused::one_grid(a, (uint64_t)units)) {
       row_stats(lse, lse2);
       a.stats_ready = true;
     }
@@ -231,6 +236,18 @@ extern "C" size_t xmk_fmha_bwd_workspace_bytes(uint32_t num_batches, uint32_t nu
   return make_plan(units, num_queries, num_keys).total;
 }
 
+extern "C" size_t xmk_fmha_bwd_best_workspace_bytes(uint32_t num_batches, uint32_t num_heads, uint32_t head_size,
+                                                    uint32_t num_queries, uint32_t num_keys, int32_t causal) {
+  const size_t least = xmk_fmha_bwd_workspace_bytes(num_batches, num_heads, head_size, num_queries, num_keys);
+  if (least == 0) return 0;
+  const uint64_t units = (uint64_t)num_batches * num_heads;
+  if (!fused_path(units, head_size, num_queries, num_keys, false)) return least;
+  fmha_bwd_fused::Args a{};
+  a.H = (int)head_size; a.F = (int)num_queries; a.T = (int)num_keys; a.causal = causal != 0;
+  const uint64_t kept = fmha_bwd_fused::saved_units(a, units, UINT64_MAX);
+  return std::max(least, kept ? fused_bytes(units, num_queries) + fmha_bwd_fused::saved_bytes(a, kept) : 0);
+}
+
 extern "C" int xmk_fmha_bwd(const void* query, const void* key, const void* value, const void* bias,
                             const void* out, const void* grad_out, const float* lse, void* grad_query,
                             void* grad_key, void* grad_value, int32_t dtype, uint32_t num_batches,
@@ -260,9 +277,9 @@ extern "C" int xmk_fmha_bwd(const void* query, const void* key, const void* valu
              num_keys, head_size, causal, bias != nullptr, (long long)pl.chunk);
   if (dtype == XMK_BF16)
     return run<__bf16>(query, key, value, bias, out, grad_out, lse, grad_query, grad_key, grad_value, dtype,
-                       (int64_t)units, head_size, num_queries, num_keys, head_scale, causal != 0, (char*)workspace, pl,
-                       stream);
+                       (int64_t)units, head_size, num_queries, num_keys, head_scale, causal != 0, (char*)workspace, workspace_bytes,
+                       pl, stream);
   return run<_Float16>(query, key, value, bias, out, grad_out, lse, grad_query, grad_key, grad_value, dtype,
-                       (int64_t)units, head_size, num_queries, num_keys, head_scale, causal != 0, (char*)workspace, pl,
-                       stream);
+                       (int64_t)units, head_size, num_queries, num_keys, head_scale, causal != 0, (char*)workspace, workspace_bytes,
+                       pl, stream);
 }

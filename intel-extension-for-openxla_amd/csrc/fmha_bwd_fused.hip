@@ -8,7 +8,8 @@
 // with  P = exp(scale S - LSE),  dS = P o (dP - D),  S = Q K^T,  dP = dO V^T,  D = rowsum(dO o O).
 // S (and dP) are recomputed in every pass (8 matrix products instead of 5) so that no gradient needs
 // atomics or a second pass over partial sums: every output element is written once, in a fixed order.
-// Problems of few work-groups run all passes as one grid (one_grid() below).
+// With scratch for it, and heads of more than 64, the owner = queries pass keeps dS, and dK takes it from there (6
+// products; bwd_saved_pass).  Problems of few work-groups run all passes as one grid (one_grid() below).
 //
 // As in the forward kernel, every product is issued so that a lane owns ONE owner row:
 //   scores  = Stream_tile . Owner^T : A operand = fragment of the streamed tile (LDS), B operand =
@@ -38,6 +39,7 @@ typedef __attribute__((address_space(3))) void* lds_void_ptr;
 constexpr int BS = 64;   // streamed rows per block
 constexpr int BO = 128;  // owner rows per work-group
 constexpr uint32_t kOob = 0x80000000u;
+constexpr int kNonTemporal = 2;  // cache policy of dS, written once and read once: 1079 -> 1034 us against the default ([8,32,2048,128] causal)
 constexpr float kLog2e = 1.4426950408889634f;
 
 template <typename F, int... I>
@@ -88,6 +90,7 @@ struct KParams {
   const float* lse_fwd;  // [units, F] its LSE (queries-own launch)
   void* out1;         // scale * dS^T Q (dK)  or  scale * dS K (dQ)
   void* out2;         // P^T dO (dV), owner = keys only
+  char* ds;           // dS of the launch's units (layout: ds_* below): the queries-own pass writes it, the saved-dS one reads it
   int H, F, T;
   int nob;            // owner blocks per unit
   int total, per_xcd, ug;
@@ -103,11 +106,36 @@ struct KParams {
 // (keys-own pass: 2-byte loads that are contiguous across the lanes of a wave; queries-own pass: each
 // lane reads its own row, 8 bytes at a time where the alignment allows).
 // STATS_IN: the row statistics are there (the queries-own pass reads them as the keys-own passes do, and writes none).
+// SAVE_DS: the queries-own pass also writes dS, rounded as its own products take it, for bwd_saved_pass below.
 // lds: bwd_lds_bytes(HP) bytes; block: the work-group's number among the pass's.
+
+// Saved dS: tiles of 32 queries x 64 keys (4 KiB), a unit's tiles by blocks of 128 queries, in a block by 32 queries, then
+// by keys; causal units hold no tiles past the diagonal block.  In a tile, the 16 bytes that a lane of the queries-own pass
+// holds (query q, keys 16 u + 4 g + {0..3, 8..11}) are chunk (u / 2) 128 + (q / 4) 16 + (u % 2) 8 + 4 g + q % 4: a wave's
+// store covers whole 128-byte lines, and the transpose reads of the saved-dS pass, which take 4 queries x 32 keys at a
+// time, fall on 16 different chunks modulo the 256 bytes of the LDS banks.
+constexpr int DS_TILE = 32 * BS * 2;
+__host__ __device__ inline int ds_key_blocks(int T) { return (T + BO - 1) / BO * (BO / BS); }  // an even number
+// Key blocks that the tiles of query block r cover, and how many tiles come before that block's.
+__host__ __device__ inline int ds_width(int r, int nkb, bool causal) {
+  const int w = (r + 1) * (BO / BS);
+  return causal && w < nkb ? w : nkb;
+}
+__host__ __device__ inline int64_t ds_before(int r, int nkb, bool causal) {
+  const int full = causal ? nkb / (BO / BS) : 0;  // blocks from here on are nkb wide
+  const int64_t lo = r < full ? r : full;
+  return (BO / 32) * (lo * (lo + 1) + (int64_t)(r - lo) * nkb);
+}
+// Bytes per unit.
+inline size_t ds_unit_bytes(int F, int T, bool causal) {
+  return (size_t)ds_before((F + BO - 1) / BO, ds_key_blocks(T), causal) * DS_TILE;
+}
+
 constexpr int bwd_lds_bytes(int HP) { return 4 * BS * HP * 2 + 2 * (2 * BS * 4); }
-template <typename T, int HP, bool OWNER_K, bool CAUSAL, bool DS, bool PV, bool BIAS, bool STATS_IN>
+template <typename T, int HP, bool OWNER_K, bool CAUSAL, bool DS, bool PV, bool BIAS, bool STATS_IN, bool SAVE_DS>
 __device__ __forceinline__ void bwd_pass(const KParams& p, char* lds, int block_id) {
   static_assert(DS || PV, "nothing to compute");
+  static_assert(!SAVE_DS || !OWNER_K, "the queries-own pass saves dS");
   static_assert(!PV || OWNER_K, "P^T dO belongs to the keys-own pass");
   typedef typename Elem<T>::vec8 V8;
   constexpr int NW = 4;
@@ -375,6 +403,15 @@ __device__ __forceinline__ void bwd_pass(const KParams& p, char* lds, int block_
   }
 
 
+  // This wave's tiles of dS, and the lane's chunk in each.
+  [[maybe_unused]] __amdgpu_buffer_rsrc_t ds_rsrc;
+  [[maybe_unused]] const uint32_t ds_lane = (l32 >> 2) * 256 + g * 64 + (l32 & 3) * 16;
+  if constexpr (SAVE_DS) {
+    const int nkb = ds_key_blocks(p.T), w = ds_width(ob, nkb, CAUSAL);
+    ds_rsrc = make_rsrc(p.ds + (int64_t)DS_TILE * (unit * ds_before(p.nob, nkb, CAUSAL) + ds_before(ob, nkb, CAUSAL) + (int64_t)wave * w),
+                        (uint32_t)w * DS_TILE);
+  }
+
   // One block: its tiles are in `c1`, `c2`, `cst`; the next block's go to `n1`, `n2`, `nst`.
   auto block = [&](int it, const char* __restrict__ c1, const char* __restrict__ c2, const char* __restrict__ cst,
                    char* __restrict__ n1, char* __restrict__ n2, char* __restrict__ nst) {
@@ -450,11 +487,18 @@ __device__ __forceinline__ void bwd_pass(const KParams& p, char* lds, int block_
       if (masked) elementwise(std::true_type{}, i0{}, i2{});
       else elementwise(std::false_type{}, i0{}, i2{});
     }
+    if constexpr (SAVE_DS) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, df[u]), ds_rsrc, ds_lane,
+                                               it * DS_TILE + (u >> 1) * 2048 + (u & 1) * 128, kNonTemporal);
+    }
     if constexpr (DS) accumulate(c1, df, acc1);
     if constexpr (PV) accumulate(c2, pf, acc2);
     // The next block's tiles have landed (this wave's loads; every wave's after the barrier), and
-    // this wave is done reading the tiles that the loads after the next block overwrite.
-    __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(0));
+    // this wave is done reading the tiles that the loads after the next block overwrite.  The stores of dS, issued
+    // after those loads, are left in flight.
+    __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(SAVE_DS ? 4 : 0));
     __builtin_amdgcn_s_barrier();
   };
 
@@ -507,10 +551,245 @@ __device__ __forceinline__ void bwd_pass(const KParams& p, char* lds, int block_
   }
 }
 
-template <typename T, int HP, bool OWNER_K, bool CAUSAL, bool DS, bool PV, bool BIAS>
+// Keys own, dS from memory: dK = scale dS^T Q, and with PV also dV = P^T dO, whose P it forms again from S.
+// What bounds the keys-own passes is the matrix pipe under the package's power limit: forming dS here takes two products
+// (S and dP) for the one that uses it, and the registers of a second owner operand, without which both accumulators fit at
+// two waves per SIMD.  The queries-own pass has dS at hand; it costs a write and a read of 2 bytes per score, hidden behind
+// the products: [8,32,2048,128] causal bf16 1255 -> 1034 us (dQ 482 -> 540, dK and dV 488 + 354 -> 490), without a mask
+// 2145 -> 1775; 600 x 300 causal heads of 128 95 -> 72; 64 x 2048 heads of 256 953 -> 703.  At heads of 64 the traffic
+// weighs twice as much and dK and dV share their products anyway: 180 -> 194 us, not used.  A work-group owns 128 keys and walks the queries in blocks of 32 through three LDS stages (two blocks
+// ahead, 75 KiB, two work-groups per CU).
+constexpr int SBS = 32;
+template <int HP, bool PV> struct SavedLds {
+  static constexpr int TILE = SBS * HP * 2, DSB = BO * SBS * 2, STAT = PV ? 4 * 256 : 0;
+  static constexpr int STAGE = (PV ? 2 : 1) * TILE + DSB + STAT, ALL = 3 * STAGE;
+};
+template <typename T, int HP, bool CAUSAL, bool PV>
+__device__ __forceinline__ void bwd_saved_pass(const KParams& p, char* lds, int block_id) {
+  typedef typename Elem<T>::vec8 V8;
+  typedef SavedLds<HP, PV> L;
+  constexpr int NW = 4;
+  constexpr int ROWB = HP * 2, CPR = ROWB / 16, RPL = 1024 / ROWB, LROWS = NW * RPL;
+  constexpr int NL = L::TILE / 1024 / NW;  // loads per wave per tile
+  constexpr int KV = (LROWS % 16 == 0) ? 1 : 2;
+  constexpr int KS = HP / 16, HT = HP / 32;
+  constexpr int LOADS = NL * (PV ? 2 : 1) + 2 + (PV ? 1 : 0);  // loads per wave per block
+  static_assert(NL >= 1 && L::DSB == NW * 2 * 1024, "tile / wave split");
+  static_assert(!PV || BO * ROWB <= L::ALL, "the owner rows are staged in the stages");
+  static_assert(NW * 32 * ROWB <= L::ALL, "and so are the output rows");
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 5, l32 = lane & 31;
+  auto swz = [](int row) {
+    return CPR >= 16 ? (((row & 3) << 2) | ((row >> 2) & 3)) : ((((row >> 1) & 1) << 2) | ((row >> 2) & 3));
+  };
+  const int wg = (block_id % 8) * p.per_xcd + block_id / 8;
+  if (wg >= p.total || block_id >= 8 * p.per_xcd) return;
+  const int UG = p.ug;
+  const int ublk = wg / (UG * p.nob), r = wg % (UG * p.nob);
+  const int gb = min(UG, p.total / p.nob - ublk * UG);
+  const int unit = ublk * UG + r % gb;
+  const int ob = r / gb;
+  const int o0 = ob * BO;
+  const int H = p.H;
+  const int wo0 = o0 + wave * 32, orow = wo0 + l32;
+  const T* Q = reinterpret_cast<const T*>(p.strm1) + (int64_t)unit * p.F * H;
+  const T* dO = reinterpret_cast<const T*>(p.strm2) + (int64_t)unit * p.F * H;
+  const T* K = reinterpret_cast<const T*>(p.own1) + (int64_t)unit * p.T * H;
+  const float* lse = p.lse + (int64_t)unit * p.F;
+  const int nkb = ds_key_blocks(p.T);
+  const char* const ds_unit = p.ds + (int64_t)DS_TILE * unit * ds_before((p.F + BO - 1) / BO, nkb, CAUSAL);
+
+  const int lrow = wave * RPL + lane / CPR;
+  uint32_t koff[KV];
+#pragma unroll
+  for (int v = 0; v < KV; ++v) {
+    const int chunk = (lane % CPR) ^ swz(lrow + v * LROWS);
+    koff[v] = chunk * 8 < H ? (uint32_t)((lrow * H + chunk * 8) * 2) : kOob;
+  }
+  const uint32_t lstride = (uint32_t)(LROWS * H * 2);
+  // 32 rows from t0 on; rows past n_rows come as zeros.
+  auto issue_rows = [&](const T* base, int t0, char* __restrict__ tile, int n_rows) {
+    const int rows_left = n_rows - t0;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(base + (int64_t)t0 * H, 0x7fffffffu);
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const uint32_t off = lrow + i * LROWS < rows_left ? koff[i % KV] : kOob;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_ptr)(tile + (i * NW + wave) * 1024), 16, off, i * lstride, 0, 0);
+    }
+  };
+  const int b0 = CAUSAL ? o0 / SBS : 0, b1 = (p.F + SBS - 1) / SBS;
+  // Everything of query block it; past the last block nothing is read, and the number of loads is the same.
+  auto issue_block = [&](int it, char* __restrict__ st) {
+    issue_rows(Q, it * SBS, st, p.F);
+    if constexpr (PV) issue_rows(dO, it * SBS, st + L::TILE, p.F);
+    char* const d = st + (PV ? 2 : 1) * L::TILE;
+    const int rb = it / (BO / SBS);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(
+        ds_unit + (int64_t)DS_TILE * (ds_before(rb, nkb, CAUSAL) + (int64_t)(it % (BO / SBS)) * ds_width(rb, nkb, CAUSAL) + ob * (BO / BS)),
+        it < b1 ? (uint32_t)L::DSB : 0u);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_ptr)(d + (i * NW + wave) * 1024), 16, (uint32_t)(lane * 16),
+                                               (i * NW + wave) * 1024, 0, kNonTemporal);
+    if constexpr (PV) {  // each wave its own copy: 32 floats (the other lanes' 32 are not used)
+      const __amdgpu_buffer_rsrc_t rl = make_rsrc(lse, (uint32_t)p.F * 4);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rl, (lds_void_ptr)(d + L::DSB + wave * 256), 4, (uint32_t)((it * SBS + lane) * 4), 0, 0, 0);
+    }
+  };
+
+  int kbase[KS];  // row fragment s: tile row l%32, logical chunk 2 s + g
+#pragma unroll
+  for (int s = 0; s < KS; ++s) kbase[s] = l32 * ROWB + (((2 * s + g) ^ swz(l32)) << 4);
+  int tbase[HT][2];  // transposed fragments, as in bwd_pass
+  const int pl = lane & 15;
+#pragma unroll
+  for (int ht = 0; ht < HT; ++ht) {
+    const int col = 32 * ht + ((lane >> 4) & 1) * 16 + 4 * (pl & 3);
+#pragma unroll
+    for (int h2 = 0; h2 < 2; ++h2) {
+      const int row = 4 * g + (pl >> 2) + 8 * h2;
+      tbase[ht][h2] = row * ROWB + (((col >> 3) ^ swz(row)) << 4) + (col & 7) * 2;
+    }
+  }
+  // dS fragment (16 queries u, this wave's 32 keys): 4 queries x 16 keys per 16 lanes; + u * 1024, + 512 for the second read.
+  const int dbase = (wave >> 1) * DS_TILE + (wave & 1) * 2048 + g * 256 + ((lane >> 4) & 1) * 128 + (pl & 1) * 64 +
+                    (pl >> 2) * 16 + ((pl >> 1) & 1) * 8;
+  auto tr_read = [](const char* __restrict__ lo_at, const char* __restrict__ hi_at) -> V8 {
+    typedef short4v __attribute__((address_space(3))) * lds_ptr;
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)lo_at));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)hi_at));
+    return __builtin_bit_cast(V8, u32x4{lo[0], lo[1], hi[0], hi[1]});
+  };
+
+  V8 of[PV ? KS : 1];
+  if constexpr (PV) {
+#pragma unroll
+    for (int i = 0; i < BO / SBS; ++i) issue_rows(K, o0 + i * SBS, lds + i * L::TILE, p.T);
+    __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(0));
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int s = 0; s < KS; ++s) of[s] = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(lds + wave * L::TILE + kbase[s]));
+    __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(0));
+    __builtin_amdgcn_s_barrier();
+  }
+
+  floatx16 acc1[HT], acc2[PV ? HT : 1];
+#pragma unroll
+  for (int i = 0; i < HT; ++i) acc1[i] = zero16();
+#pragma unroll
+  for (int i = 0; i < (PV ? HT : 1); ++i) acc2[i] = zero16();
+  const float scale2 = p.scale * kLog2e;
+
+  auto block = [&](int it, const char* __restrict__ st, char* __restrict__ next) {
+    const int t0 = it * SBS;
+    issue_block(it + 2, next);
+    const char* const qt = st;
+    const char* const ot = st + L::TILE;
+    const char* const dt = st + (PV ? 2 : 1) * L::TILE;
+    if (!CAUSAL || t0 + SBS - 1 >= wo0) {  // (all of a wave's keys lie past these queries: nothing to add)
+      floatx16 sc;
+      if constexpr (PV) {
+        sc = zero16();
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+          sc = Elem<T>::mfma(__builtin_bit_cast(V8, *reinterpret_cast<const u32x4*>(qt + kbase[s])), of[s], sc);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const V8 df = tr_read(dt + dbase + u * 1024, dt + dbase + u * 1024 + 512);
+#pragma unroll
+        for (int ht = 0; ht < HT; ++ht)
+          acc1[ht] = Elem<T>::mfma(tr_read(qt + u * 16 * ROWB + tbase[ht][0], qt + u * 16 * ROWB + tbase[ht][1]), df, acc1[ht]);
+      }
+      if constexpr (PV) {
+        V8 pf[2];
+        auto probs = [&](auto MASKED_T) {
+#pragma unroll
+          for (int qd = 0; qd < 4; ++qd) {
+            const floatx4 l2 = *reinterpret_cast<const floatx4*>(dt + L::DSB + wave * 256 + (8 * qd + 4 * g) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              float arg = __builtin_fmaf(sc[4 * qd + e], scale2, -l2[e]);
+              if constexpr (decltype(MASKED_T)::value) {
+                const int q = t0 + 8 * qd + 4 * g + e;
+                arg = (q >= p.F || (CAUSAL && orow > q)) ? -INFINITY : arg;
+              }
+              pf[qd >> 1][4 * (qd & 1) + e] = (T)__builtin_amdgcn_exp2f(arg);
+            }
+          }
+        };
+        if (t0 + SBS > p.F || (CAUSAL && wo0 + 31 > t0)) probs(std::true_type{});
+        else probs(std::false_type{});
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int ht = 0; ht < HT; ++ht)
+            acc2[ht] = Elem<T>::mfma(tr_read(ot + u * 16 * ROWB + tbase[ht][0], ot + u * 16 * ROWB + tbase[ht][1]), pf[u], acc2[ht]);
+      }
+    }
+    // The next block's loads have landed; those of the one after it may be in flight.
+    __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(LOADS));
+    __builtin_amdgcn_s_barrier();
+  };
+
+  if (b0 < b1) {
+    char* const st0 = lds;
+    char* const st1 = lds + L::STAGE;
+    char* const st2 = lds + 2 * L::STAGE;
+    issue_block(b0, st0);
+    issue_block(b0 + 1, st1);
+    __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(LOADS));
+    __builtin_amdgcn_s_barrier();
+    for (int it = b0; it < b1; it += 3) {
+      block(it, st0, st2);
+      if (it + 1 < b1) block(it + 1, st1, st0);
+      if (it + 2 < b1) block(it + 2, st2, st1);
+    }
+    __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(0));  // (the loads past the end: zeros for the stages)
+    __builtin_amdgcn_s_barrier();
+  }
+
+  // ---- store, as in bwd_pass
+  constexpr int OCPR = HP / 8;
+  char* const region = lds + wave * (32 * ROWB);
+  auto store = [&](void* out, const floatx16 (&acc)[HT], float mul) {
+    static_for<HT>([&](auto HTI) {
+      constexpr int ht = decltype(HTI)::value;
+      const floatx16 o = acc[ht];
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd) {
+        union { T e[4]; u32x2 w; } v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v.e[e] = (T)(o[4 * qd + e] * mul);
+        *reinterpret_cast<u32x2*>(region + l32 * ROWB + (((4 * ht + qd) ^ (l32 & (OCPR - 1))) << 4) + g * 8) = v.w;
+      }
+    });
+    constexpr int RPI = 64 / OCPR;
+    const int c = lane % OCPR;
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; ++i) {
+      const int row = i * RPI + lane / OCPR;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(region + row * ROWB + ((c ^ (row & (OCPR - 1))) << 4));
+      if (wo0 + row < p.T && c * 8 < H)
+        *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(out) + ((int64_t)unit * p.T + wo0 + row) * H + c * 8) = v;
+    }
+  };
+  store(p.out1, acc1, p.scale);
+  if constexpr (PV) store(p.out2, acc2, 1.0f);
+}
+
+template <typename T, int HP, bool CAUSAL, bool PV>
+__global__ __launch_bounds__(256, 2) void fmha_bwd_saved_kernel(KParams p) {
+  __shared__ __attribute__((aligned(1024))) char lds[SavedLds<HP, PV>::ALL];
+  bwd_saved_pass<T, HP, CAUSAL, PV>(p, lds, (int)blockIdx.x);
+}
+
+template <typename T, int HP, bool OWNER_K, bool CAUSAL, bool DS, bool PV, bool BIAS, bool SAVE_DS>
 __global__ __launch_bounds__(256, (HP <= 128 && !BIAS && !(DS && PV && HP > 64)) ? 2 : 1) void fmha_bwd_kernel(KParams p) {
   __shared__ __attribute__((aligned(1024))) char lds[bwd_lds_bytes(HP)];
-  bwd_pass<T, HP, OWNER_K, CAUSAL, DS, PV, BIAS, false>(p, lds, (int)blockIdx.x);
+  bwd_pass<T, HP, OWNER_K, CAUSAL, DS, PV, BIAS, false, SAVE_DS>(p, lds, (int)blockIdx.x);
 }
 
 // All passes in one grid, a row of it each, on statistics formed before: for problems of which a single pass leaves the
@@ -520,10 +799,10 @@ template <typename T, int HP, bool CAUSAL>
 __global__ __launch_bounds__(256, HP <= 128 ? 2 : 1) void fmha_bwd_small_kernel(KParams dq, KParams dk, KParams dv) {
   __shared__ __attribute__((aligned(1024))) char lds[bwd_lds_bytes(HP)];
   const int block = (int)blockIdx.x;
-  if (blockIdx.y == 0) bwd_pass<T, HP, false, CAUSAL, true, false, false, true>(dq, lds, block);
-  else if constexpr (HP <= 64) bwd_pass<T, HP, true, CAUSAL, true, true, false, true>(dk, lds, block);
-  else if (blockIdx.y == 1) bwd_pass<T, HP, true, CAUSAL, true, false, false, true>(dk, lds, block);
-  else bwd_pass<T, HP, true, CAUSAL, false, true, false, true>(dv, lds, block);
+  if (blockIdx.y == 0) bwd_pass<T, HP, false, CAUSAL, true, false, false, true, false>(dq, lds, block);
+  else if constexpr (HP <= 64) bwd_pass<T, HP, true, CAUSAL, true, true, false, true, false>(dk, lds, block);
+  else if (blockIdx.y == 1) bwd_pass<T, HP, true, CAUSAL, true, false, false, true, false>(dk, lds, block);
+  else bwd_pass<T, HP, true, CAUSAL, false, true, false, true, false>(dv, lds, block);
 }
 
 void split(KParams& p, int n_own, uint64_t units) {
@@ -538,12 +817,35 @@ void launch_pass(KParams p, uint64_t units, bool causal, hipStream_t st) {
   split(p, OWNER_K ? p.T : p.F, units);
   const dim3 grid((unsigned)(p.per_xcd * 8)), block(256);
   if (p.bias) {
-    if (causal) hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, true, DS, PV, true>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, false, DS, PV, true>), grid, block, 0, st, p);
+    if (causal) hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, true, DS, PV, true, false>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, false, DS, PV, true, false>), grid, block, 0, st, p);
   } else {
-    if (causal) hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, true, DS, PV, false>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, false, DS, PV, false>), grid, block, 0, st, p);
+    if (causal) hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, true, DS, PV, false, false>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, false, DS, PV, false, false>), grid, block, 0, st, p);
   }
+}
+
+// The same pass from unit u0 on (no bias); `owner_k` says which of q / o / dO and k / v are the owners.
+KParams at_unit(KParams p, uint64_t u0, bool owner_k) {
+  const uint64_t rows_q = u0 * p.F, q = rows_q * p.H * 2, k = u0 * p.T * p.H * 2;
+  auto at = [](const void* v, uint64_t bytes) { return static_cast<const void*>(static_cast<const char*>(v) + bytes); };
+  auto to = [](void* v, uint64_t bytes) { return v ? static_cast<void*>(static_cast<char*>(v) + bytes) : nullptr; };
+  const uint64_t own = owner_k ? k : q, strm = owner_k ? q : k;
+  p.own1 = at(p.own1, own); p.own2 = at(p.own2, own); p.strm1 = at(p.strm1, strm); p.strm2 = at(p.strm2, strm);
+  p.o = at(p.o, q); p.lse += rows_q; p.dsum += rows_q; p.lse_fwd += rows_q;
+  p.out1 = to(p.out1, own); p.out2 = to(p.out2, own);
+  return p;
+}
+
+// dQ and dS (kept), then dK and dV from it; with heads of more than 128 dV has its own pass, as its accumulators need.
+template <typename T, int HP, bool CAUSAL>
+void launch_saved(KParams p, KParams kv, uint64_t units, hipStream_t st) {
+  split(p, p.F, units);
+  split(kv, kv.T, units);
+  const dim3 block(256);
+  hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, false, CAUSAL, true, false, false, true>), dim3((unsigned)(p.per_xcd * 8)), block, 0, st, p);
+  hipLaunchKernelGGL((fmha_bwd_saved_kernel<T, HP, CAUSAL, (HP <= 128)>), dim3((unsigned)(kv.per_xcd * 8)), block, 0, st, kv);
+  if constexpr (HP > 128) launch_pass<T, HP, true, false, true>(kv, units, CAUSAL, st);
 }
 
 template <typename T, int HP>
@@ -553,10 +855,19 @@ void launch_both(const fmha_bwd_fused::Args& a, uint64_t units, hipStream_t st) 
   p.bias = a.bias;
   p.bias_vec = a.bias && a.T % 4 == 0 && xmk::aligned(a.bias, 8);
   p.nob = p.total = p.per_xcd = 0;
+  p.ds = static_cast<char*>(a.ds);
   p.own1 = a.q; p.own2 = a.d_o; p.strm1 = a.k; p.strm2 = a.v; p.out1 = a.dq; p.out2 = nullptr;
+  KParams k = p;
+  k.own1 = a.k; k.own2 = a.v; k.strm1 = a.q; k.strm2 = a.d_o; k.out1 = a.dk; k.out2 = a.dv;
+  if constexpr (HP > 64) if (a.ds) {
+    for (uint64_t u0 = 0; u0 < units; u0 += a.ds_units) {
+      const uint64_t n = std::min<uint64_t>(a.ds_units, units - u0);
+      if (a.causal) launch_saved<T, HP, true>(at_unit(p, u0, false), at_unit(k, u0, true), n, st);
+      else launch_saved<T, HP, false>(at_unit(p, u0, false), at_unit(k, u0, true), n, st);
+    }
+    return;
+  }
   if (a.stats_ready) {
-    KParams k = p;
-    k.own1 = a.k; k.own2 = a.v; k.strm1 = a.q; k.strm2 = a.d_o; k.out1 = a.dk; k.out2 = a.dv;
     split(p, a.F, units);
     split(k, a.T, units);
     const dim3 grid((unsigned)(std::max(p.per_xcd, k.per_xcd) * 8), HP <= 64 ? 2 : 3), block(256);
@@ -567,16 +878,15 @@ void launch_both(const fmha_bwd_fused::Args& a, uint64_t units, hipStream_t st) 
   // owner = queries first: dQ, and the per-row statistics the other launches read
   launch_pass<T, HP, false, true, false>(p, units, a.causal, st);
   // owner = keys: dK, then dV
-  p.own1 = a.k; p.own2 = a.v; p.strm1 = a.q; p.strm2 = a.d_o; p.out1 = a.dk; p.out2 = a.dv;
   // One pass for both where the two accumulators fit beside everything else (S is then computed once for the
   // two): head size <= 64 (S = 4096, H = 64 causal: 0.69 -> 0.57 ms), and head size <= 128 with a bias, whose
   // kernels run one wave per SIMD anyway (6.2 -> 5.3 ms).  Without a bias the merged H = 128 pass would have to
   // give up the second wave per SIMD and comes out 2-4 % slower; at H = 256 it spills.
   if (HP <= 64 || (HP <= 128 && a.bias)) {
-    launch_pass<T, HP, true, true, true>(p, units, a.causal, st);
+    launch_pass<T, HP, true, true, true>(k, units, a.causal, st);
   } else {
-    launch_pass<T, HP, true, true, false>(p, units, a.causal, st);
-    launch_pass<T, HP, true, false, true>(p, units, a.causal, st);
+    launch_pass<T, HP, true, true, false>(k, units, a.causal, st);
+    launch_pass<T, HP, true, false, true>(k, units, a.causal, st);
   }
 }
 
@@ -600,6 +910,25 @@ bool one_grid(const Args& a, uint64_t units) {
   const uint64_t most = rows >= 512 ? 512 : (a.H > 128 && rows <= 128) ? 128 : 384;
   return !a.bias && groups <= most;
 }
+
+// All units in one part run with fewer launches than without dS; what a part of them loses is its last, partly empty
+// rounds of 512 work-groups: 896 per part (32 x 16384, 7 units at a time) 8.2 -> 10.9 ms, 1408 (64 x 8192) 4.19 -> 4.02.
+// Against the one grid of a small problem (us, one grid / dS kept; causal first): 512 groups, 32 x 2048, 195 / 179 and
+// 291 / 236; 384, 24 x 2048, 145 / 150 and 235 / 197, 192 x 256 50 / 43; 320, 10 x 4096, 278 / 264; 256, 16 x 2048, 123 / 130;
+// 96, 96 x 128, 14 / 20.  Heads of 256: 256 groups, 16 x 2048, 341 / 305 and 406 / 323; 56 groups 48 / 90.
+uint64_t saved_units(const Args& a, uint64_t units, uint64_t bytes) {
+  constexpr uint64_t kMost = (uint64_t)2 << 30, kPartGroups = 1280;
+  const uint64_t rows = (uint64_t)std::max(a.F, a.T), per_unit = (rows + BO - 1) / BO;
+  if (a.bias || a.H <= 64) return 0;
+  if (units * per_unit < (a.H > 128 ? 256u : a.causal && rows > 1024 ? 385u : 257u)) return 0;
+  const uint64_t fit = std::min(bytes, kMost) / saved_bytes(a, 1);
+  if (fit >= units) return units;
+  if (fit == 0) return 0;
+  const uint64_t parts = (units + fit - 1) / fit, each = (units + parts - 1) / parts;
+  return each * per_unit >= kPartGroups ? each : 0;
+}
+
+size_t saved_bytes(const Args& a, uint64_t units) { return units * ds_unit_bytes(a.F, a.T, a.causal); }
 
 void launch(const Args& a, uint64_t units, bool bf16, hipStream_t st) {
   if (bf16) {

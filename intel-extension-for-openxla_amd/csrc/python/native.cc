@@ -27,7 +27,7 @@ namespace {
 struct Api {
 #define XMK_FUNCTIONS(F)                                                                                   \
   F(xmk_gemm) F(xmk_gemm_ws) F(xmk_gemm_qkv) F(xmk_fmha_fwd) F(xmk_fmha_bwd)   \
-  F(xmk_fmha_bwd_workspace_bytes) F(xmk_fmha_decode) F(xmk_fmha_decode_static) F(xmk_int4_gemm)            \
+  F(xmk_fmha_bwd_workspace_bytes) F(xmk_fmha_bwd_best_workspace_bytes) F(xmk_fmha_decode) F(xmk_fmha_decode_static) F(xmk_int4_gemm)            \
   F(xmk_int4_gemm_ws) F(xmk_fp8_gemm_ex) F(xmk_gptj_decode_step)
 #define XMK_DECLARE(name) decltype(&::name) name = nullptr;
   XMK_FUNCTIONS(XMK_DECLARE)
@@ -242,8 +242,18 @@ XMK_PY(fmha_backward) {
     void *o = data(tensor(a[3])), *d_o = data(tensor(a[4])), *lse = data(tensor(a[5])), *bias = data_or_null(a[6]);
     const int32_t dt = dtype_code(q), causal = truth(a[8]);
     void* st = stream(a[9]);
-    const size_t bytes = api.xmk_fmha_bwd_workspace_bytes(s.b, s.n, s.h, s.f, s.t);
-    const at::Tensor ws = at::empty({(int64_t)(bytes > 256 ? bytes : 256)}, q.options().dtype(at::kByte));
+    // Where memory is short, the least that the call takes.
+    const size_t least = api.xmk_fmha_bwd_workspace_bytes(s.b, s.n, s.h, s.f, s.t);
+    size_t bytes = bias ? least : api.xmk_fmha_bwd_best_workspace_bytes(s.b, s.n, s.h, s.f, s.t, causal);
+    auto scratch = [&] { return at::empty({(int64_t)(bytes > 256 ? bytes : 256)}, q.options().dtype(at::kByte)); };
+    at::Tensor ws;
+    try {
+      ws = scratch();
+    } catch (const c10::OutOfMemoryError&) {
+      if (bytes == least) throw;
+      bytes = least;
+      ws = scratch();
+    }
     const at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     const int rc = unlocked([&] {
       return api.xmk_fmha_bwd(data(q), data(k), data(v), bias, o, d_o, (const float*)lse, data(dq), data(dk), data(dv), dt, s.b,

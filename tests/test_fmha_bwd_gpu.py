@@ -145,3 +145,42 @@ def test_backward_on_a_side_stream(xmk):
     junk = [torch.full((n,), 0xff, dtype=torch.uint8, device="cuda") for n in (1 << 12, 1 << 16, 1 << 18, 1 << 20, 1 << 22, 1 << 24) for _ in range(4)]
     torch.cuda.synchronize()
     assert len(junk) == 24 and all(torch.equal(x, y) for x, y in zip(got, ref))
+
+
+@pytest.mark.parametrize("name,causal", [("bf16", True), ("fp16", True), ("fp16", False)])
+@pytest.mark.parametrize("B,N,F,T,H,parts", [
+    (10, 16, 130, 257, 128, 1), (13, 16, 257, 130, 80, 1), (29, 9, 33, 65, 256, 1), (12, 11, 129, 1, 200, 1), (130, 4, 1, 64, 72, 1),
+    (57, 47, 100, 96, 128, 2),
+])
+def test_backward_with_kept_score_gradients(xmk, name, causal, B, N, F, T, H, parts):
+    """dS kept in the workspace (all units at once, or as many as a smaller workspace holds) against a call with the least
+    workspace, which forms it twice: the same products of factors that are rounded alike, so that results differ by their last bit
+    (a single key's dQ and dK are zero but for rounding: those are held to 1e-5)."""
+    import ctypes as C
+    L, tdt = xmk.lib(), torch.bfloat16 if name == "bf16" else torch.float16
+    L.xmk_fmha_bwd_best_workspace_bytes.restype = C.c_size_t
+    u = [C.c_uint32(x) for x in (B, N, H, F, T)]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(F * T + H)
+    q, d_o = (torch.randn((B, N, F, H), generator=g, device="cuda", dtype=tdt) for _ in range(2))
+    k, v = (torch.randn((B, N, T, H), generator=g, device="cuda", dtype=tdt) for _ in range(2))
+    out, lse = torch.empty_like(q), torch.empty((B * N, F), device="cuda")
+    xmk.fmha_forward(q, k, v, out, lse=lse, causal=causal)
+    least = L.xmk_fmha_bwd_workspace_bytes(*u)
+    best = L.xmk_fmha_bwd_best_workspace_bytes(*u, C.c_int32(causal))
+    assert best > least and (best - least) % (B * N) == 0
+    results = []
+    for size in (least, least + (best - least) // (B * N) * -(-B * N // parts)):
+        ws = torch.full((size,), 0xff, dtype=torch.uint8, device="cuda")
+        grads = [torch.full_like(x, float("nan")) for x in (q, k, v)]
+        p = [C.c_void_p(x.data_ptr()) for x in (q, k, v, out, d_o, lse, *grads, ws)]
+        rc = L.xmk_fmha_bwd(*p[:3], None, *p[3:9], C.c_int32(xmk.BF16 if name == "bf16" else xmk.F16), *u, C.c_float(H ** -0.5),
+                            C.c_int32(causal), p[9], C.c_size_t(size), C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        assert rc == 0
+        results.append(grads)
+    ulp = 2.0 ** (-7 if name == "bf16" else -10)  # relative spacing of the results, and of the dS that enter them, at most
+    for nm, a, b in zip(("dq", "dk", "dv"), *results):
+        a, b = a.float(), b.float()
+        diff, size = (a - b).norm().item(), a.norm().item()
+        assert torch.isfinite(b).all() and (diff <= ulp * size or diff <= 1e-5 * a.numel() ** 0.5), (nm, diff, size)
