@@ -117,16 +117,8 @@ __global__ __launch_bounds__(WGM * WGN * 64) void fp8_gemm_kernel(Fp8Params p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
 
-  int pid = blockIdx.x;
-  const int ntiles = p.tiles_m * p.tiles_n;
-  if (ntiles % 8 == 0) pid = (pid % 8) * (ntiles / 8) + pid / 8;  // one contiguous run of tiles per XCD
-  constexpr int GM = 8;
-  const int group = pid / (GM * p.tiles_n);
-  const int first_m = group * GM;
-  const int gsize = min(p.tiles_m - first_m, GM);
-  const int tile_m = first_m + (pid % (GM * p.tiles_n)) % gsize;
-  const int tile_n = (pid % (GM * p.tiles_n)) / gsize;
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  const gemm_impl::TileAt tile = gemm_impl::tile_at(blockIdx.x, p.tiles_m, p.tiles_n, p.K);
+  const int m0 = tile.m * BM, n0 = tile.n * BN;
 
   floatx16 acc[TM][TN];
 #pragma unroll

@@ -29,15 +29,8 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_ragged_kernel(typename AnyT
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
 
-  int pid = blockIdx.x;  // tile order: as in gemm_mfma_kernel
-  const int ntiles = p.tiles_m * p.tiles_n;
-  if (ntiles % 8 == 0) pid = (pid % 8) * (ntiles / 8) + pid / 8;
-  constexpr int GM = 8;
-  const int group = pid / (GM * p.tiles_n);
-  const int first_m = group * GM;
-  const int gsize = min(p.tiles_m - first_m, GM);
-  const int m0 = (first_m + (pid % (GM * p.tiles_n)) % gsize) * BT;
-  const int n0 = (pid % (GM * p.tiles_n)) / gsize * BT;
+  const TileAt tile = tile_at(blockIdx.x, p.tiles_m, p.tiles_n, p.K);
+  const int m0 = tile.m * BT, n0 = tile.n * BT;
 
   const int64_t bz = blockIdx.z;
   const int64_t k0 = bz * p.kslice;  // K slices (kslice > 0): grid member z takes k0 .. k0 + kslice - 1

@@ -29,10 +29,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(typename AnyType<T
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int pid = blockIdx.x;  // consecutive blocks go to different XCDs: each gets a contiguous run of tiles
-  const int ntiles = p.tiles_m * p.tiles_n;
-  if (ntiles % 8 == 0) pid = (pid % 8) * (ntiles / 8) + pid / 8;
-  const int m0 = pid % p.tiles_m * (32 * TM), n0 = pid / p.tiles_m * (32 * TN);
+  // (along the shorter side: a run then covers few rows and columns of tiles)
+  const int pid = (int)xcd_run(blockIdx.x, (uint32_t)(p.tiles_m * p.tiles_n), p.K);
+  const bool down = p.tiles_m <= p.tiles_n;
+  const int side = down ? p.tiles_m : p.tiles_n, major = pid / side, minor = pid - major * side;
+  const int m0 = (down ? minor : major) * (32 * TM), n0 = (down ? major : minor) * (32 * TN);
 
   const int64_t bz = blockIdx.z;
   const int64_t k0 = bz * p.kslice;  // as in gemm_ragged_kernel
