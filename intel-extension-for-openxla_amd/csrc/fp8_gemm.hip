@@ -40,24 +40,24 @@ using gemm_impl::u32x2;
 using gemm_impl::u32x4;
 using gemm_impl::zero16;
 
-constexpr int BKB = 64;  // K step in bytes (= fp8 elements)
 constexpr uint32_t kOob = gemm_impl::kOob;
 
 // Per-lane LDS byte offsets of an operand's fragments: lane l of the 32-row slab t gets row
-// 32 t + l%32, bytes 32 (l/32) .. +31 of the 64-byte row, i.e. the two 16-byte chunks 2 (l/32)
-// and 2 (l/32) + 1, each XOR-swizzled like the loader placed them.  Adding 32 t rows does not
+// 32 t + l%32, bytes 64 ks + 32 (l/32) .. +31 of the row of BKB bytes, i.e. the two 16-byte chunks
+// 4 ks + 2 (l/32) and + 1, each XOR-swizzled like the loader placed them.  Adding 32 t rows does not
 // change the swizzle.
+template <int BKB>
 struct Fp8Frag {
-  int base[2];
+  int base[BKB / 32];
   __device__ __forceinline__ void init(int row0, int lane) {
     const int row = row0 + (lane & 31);
-    const int s = gemm_impl::swz<false, 0, 32>(row);
+    const int s = gemm_impl::swz<false, 0, BKB / 2>(row);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) base[h] = row * BKB + ((((lane >> 5) * 2 + h) ^ s) << 4);
+    for (int c = 0; c < BKB / 32; ++c) base[c] = row * BKB + (((c / 2 * 4 + (lane >> 5) * 2 + c % 2) ^ s) << 4);
   }
-  __device__ __forceinline__ intx8 read(const char* __restrict__ tile, int t) const {
-    const u32x4 lo = *reinterpret_cast<const u32x4*>(tile + base[0] + t * 32 * BKB);
-    const u32x4 hi = *reinterpret_cast<const u32x4*>(tile + base[1] + t * 32 * BKB);
+  __device__ __forceinline__ intx8 read(const char* __restrict__ tile, int t, int ks) const {
+    const u32x4 lo = *reinterpret_cast<const u32x4*>(tile + base[2 * ks] + t * 32 * BKB);
+    const u32x4 hi = *reinterpret_cast<const u32x4*>(tile + base[2 * ks + 1] + t * 32 * BKB);
     intx8 v;
     v[0] = (int)lo[0]; v[1] = (int)lo[1]; v[2] = (int)lo[2]; v[3] = (int)lo[3];
     v[4] = (int)hi[0]; v[5] = (int)hi[1]; v[6] = (int)hi[2]; v[7] = (int)hi[3];
@@ -65,7 +65,7 @@ struct Fp8Frag {
   }
 };
 
-// The same fragments from a tile stored [64 k][BN columns] (row = BN bytes, 16-byte chunks XOR-swizzled
+// The same fragments from a tile stored [BKB k][BN columns] (row = BN bytes, 16-byte chunks XOR-swizzled
 // by the loader with swz<true, BN / 2, 64, 1>(k)).  ds_read_b64_tr_b8 works on blocks of 16 lanes: lane p
 // of a block addresses row kb + p / 2, bytes cb + 8 (p % 2) .. +7 and receives column cb + p, rows
 // kb .. kb + 7.  Blocks 0 and 1 of the wave cover columns 0..15 and 16..31 of the slab for k half 0,
@@ -84,13 +84,13 @@ struct Fp8FragKN {
     }
   }
   // t counts 32-column slabs from col0; only slabs this wave owns are read.
-  __device__ __forceinline__ intx8 read(const char* __restrict__ tile, int t) const {
+  __device__ __forceinline__ intx8 read(const char* __restrict__ tile, int t, int ks) const {
     typedef int int2v __attribute__((ext_vector_type(2)));
     typedef int2v __attribute__((address_space(3))) * lds_ptr;
     intx8 v;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int2v r = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_ptr)(tile + base[t] + q * 8 * BN));
+      const int2v r = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_ptr)(tile + base[t] + (ks * 64 + q * 8) * BN));
       v[2 * q] = r[0];
       v[2 * q + 1] = r[1];
     }
@@ -98,16 +98,18 @@ struct Fp8FragKN {
   }
 };
 
-template <int BM, int BN, int WGM, int WGN, int NSTAGE, bool BKN = false>
+// BKB: bytes (k) of a K step, 64 or 128.
+template <int BM, int BN, int WGM, int WGN, int NSTAGE, int BKB, bool BKN>
 __global__ __launch_bounds__(WGM * WGN * 64) void fp8_gemm_kernel(Fp8Params p) {
   constexpr int NWAVES = WGM * WGN;
   constexpr int WTM = BM / WGM, WTN = BN / WGN;
   constexpr int TM = WTM / 32, TN = WTN / 32;
   constexpr int A_BYTES = BM * BKB, B_BYTES = BN * BKB, STAGE = A_BYTES + B_BYTES;
-  // The loader works in 2-byte units: BK = 32 units = 64 bytes.
-  typedef gemm_impl::Loader<false, BM, 32, NWAVES> LoaderA;
-  // B [n,k]: BN rows of 64 bytes; B [k,n]: 64 rows of BN bytes (BN / 2 two-byte units).
-  typedef std::conditional_t<BKN, gemm_impl::Loader<true, BN / 2, 64, NWAVES, 1>, gemm_impl::Loader<false, BN, 32, NWAVES>>
+  constexpr int KS = BKB / 64;  // matrix instructions' k steps per K step
+  // The loader works in 2-byte units.
+  typedef gemm_impl::Loader<false, BM, BKB / 2, NWAVES> LoaderA;
+  // B [n,k]: BN rows of BKB bytes; B [k,n]: BKB rows of BN bytes (BN / 2 two-byte units).
+  typedef std::conditional_t<BKN, gemm_impl::Loader<true, BN / 2, BKB, NWAVES, 1>, gemm_impl::Loader<false, BN, BKB / 2, NWAVES>>
       LoaderB;
   constexpr int LOADS = LoaderA::NL + LoaderB::NL;  // per wave per K step
   static_assert(NSTAGE >= 3, "the barrier leaves the running step's loads in flight");
@@ -151,8 +153,8 @@ __global__ __launch_bounds__(WGM * WGN * 64) void fp8_gemm_kernel(Fp8Params p) {
   __builtin_amdgcn_s_waitcnt(gemm_impl::vmcnt_imm((NSTAGE - 2) * LOADS));  // step 0 has landed
   __builtin_amdgcn_s_barrier();
 
-  Fp8Frag fa_addr;
-  std::conditional_t<BKN, Fp8FragKN<BN, TN>, Fp8Frag> fb_addr;
+  Fp8Frag<BKB> fa_addr;
+  std::conditional_t<BKN, Fp8FragKN<BN, TN>, Fp8Frag<BKB>> fb_addr;
   fa_addr.init(wm * WTM, lane);
   fb_addr.init(wn * WTN, lane);
   // Fragment registers: the B fragments of a step are double-buffered (those of step kt + 1 are
@@ -178,24 +180,30 @@ __global__ __launch_bounds__(WGM * WGN * 64) void fp8_gemm_kernel(Fp8Params p) {
     for (int i = 0; i < LoaderA::NL; ++i) la.issue_one(i, ra, kleft, wr, wave);
 #pragma unroll
     for (int i = 0; i < LoaderB::NL; ++i) lb.issue_one(i, rb, kleft_b(kt + NSTAGE - 1), wr + A_BYTES, wave);
-    static_for<TM>([&](auto I) {
-      constexpr int i = decltype(I)::value;
-      if constexpr (i + 1 < TM) fa[(i + 1) & 1] = fa_addr.read(cur, i + 1);
-      else fa[0] = fa_addr.read(nxt, 0);
-      if constexpr (i < TN) fb[par ^ 1][i] = fb_addr.read(nxt + A_BYTES, i);
+    static_for<KS>([&](auto KSI) {
+      constexpr int ks = decltype(KSI)::value, b = (par + ks) & 1;
+      const char* const ahead = ks + 1 < KS ? cur : nxt;  // where the next k step's fragments are
+      constexpr int nks = (ks + 1) % KS;
+      static_for<TM>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        if constexpr (i + 1 < TM) fa[(i + 1) & 1] = fa_addr.read(cur, i + 1, ks);
+        else fa[0] = fa_addr.read(ahead, 0, nks);
+        if constexpr (i < TN) fb[b ^ 1][i] = fb_addr.read(ahead + A_BYTES, i, nks);
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int jj = (i & 1) ? TN - 1 - j : j;  // boustrophedon: consecutive MFMAs share one operand
-        acc[i][jj] = mfma_fp8(fb[par][jj], fa[i & 1], acc[i][jj]);
-      }
+        for (int j = 0; j < TN; ++j) {
+          const int jj = (i & 1) ? TN - 1 - j : j;  // boustrophedon: consecutive MFMAs share one operand
+          acc[i][jj] = mfma_fp8(fb[b][jj], fa[i & 1], acc[i][jj]);
+        }
+      });
     });
     // Issue order: each row of MFMAs starts with its LDS reads (4 x 16 bytes), the global loads
     // are spread evenly.
-    static_for<NMFMA>([&](auto R) {
+    static_for<KS * NMFMA>([&](auto R) {
       constexpr int r = decltype(R)::value;
-      if constexpr (r % TN == 0) __builtin_amdgcn_sched_group_barrier(0x100, (r / TN < TN) ? (BKN ? 6 : 4) : 2, 0);
+      if constexpr (r % TN == 0) __builtin_amdgcn_sched_group_barrier(0x100, (r / TN % TM < TN) ? (BKN ? 6 : 4) : 2, 0);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if constexpr ((r + 1) * LOADS / NMFMA > r * LOADS / NMFMA) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      if constexpr ((r + 1) * LOADS / (KS * NMFMA) > r * LOADS / (KS * NMFMA))
+        __builtin_amdgcn_sched_group_barrier(0x020, (r + 1) * LOADS / (KS * NMFMA) - r * LOADS / (KS * NMFMA), 0);
     });
     __builtin_amdgcn_sched_barrier(0);
     a_tile += BKB;
@@ -203,13 +211,13 @@ __global__ __launch_bounds__(WGM * WGN * 64) void fp8_gemm_kernel(Fp8Params p) {
   };
 
 #pragma unroll
-  for (int j = 0; j < TN; ++j) fb[0][j] = fb_addr.read(lds + A_BYTES, j);
-  fa[0] = fa_addr.read(lds, 0);
+  for (int j = 0; j < TN; ++j) fb[0][j] = fb_addr.read(lds + A_BYTES, j, 0);
+  fa[0] = fa_addr.read(lds, 0, 0);
   for (int kt = 0; kt < KT; kt += 2) {
     k_step(std::integral_constant<int, 0>{}, lds + (kt % NSTAGE) * STAGE, lds + ((kt + 1) % NSTAGE) * STAGE,
            lds + ((kt + NSTAGE - 1) % NSTAGE) * STAGE, kt);
     if (kt + 1 < KT)
-      k_step(std::integral_constant<int, 1>{}, lds + ((kt + 1) % NSTAGE) * STAGE,
+      k_step(std::integral_constant<int, KS & 1>{}, lds + ((kt + 1) % NSTAGE) * STAGE,
              lds + ((kt + 2) % NSTAGE) * STAGE, lds + ((kt + NSTAGE) % NSTAGE) * STAGE, kt + 1);
   }
   __builtin_amdgcn_s_waitcnt(gemm_impl::vmcnt_imm(0));  // drain the zero-fill loads before LDS is released
@@ -265,6 +273,14 @@ __global__ __launch_bounds__(256) void fp8_gemm_generic_kernel(Fp8Params p, int 
     }
 }
 
+// Up to 256 tiles of 128 x 128 a CU has one work-group, which may then fill its LDS: K steps of 128 bytes in four stages
+// instead of 64.  Half the barriers, and whole cache lines from rows of k (268 instead of 366 MB at 256 x 16384 x 4096, B
+// [n,k]).  Microseconds: there 22.6 -> 20.6, B [k,n] 23.5 -> 20.4; 512 x 4096 x 4096 19.3 -> 15.0, 128 x 16384 x 4096 20.2 ->
+// 16.4.  (Three stages 25.2, five 20.9: neither the depth nor the barriers alone.)  With more tiles two work-groups share a CU,
+// which the small stages allow: 700 x 6000 x 2048 18.3 against 19.9.  The 256 x 128 tile on steps of 128 bytes, three stages:
+// 2048 x 4096 x 4096 37.9 -> 36.4 with B [n,k], 35.8 -> 36.8 with [k,n], 1024 x 8192 x 8192 74.9 -> 76.6: left alone.
+bool one_per_cu(int64_t m, int64_t n) { return xmk::ceil_div(m, 128) * xmk::ceil_div(n, 128) <= 256; }
+
 // XMK_FP8_POLICY=<index into kFp8Policies> forces a tile where the operands allow it (read at every call).
 int choose_fp8(int64_t m, int64_t n, int64_t k, bool direct, bool any, bool rhs_t) {
   using namespace gemm_impl;
@@ -276,7 +292,8 @@ int choose_fp8(int64_t m, int64_t n, int64_t k, bool direct, bool any, bool rhs_
   const uint32_t kt = (uint32_t)((k + 127) / 128);
   for (int pol = direct ? 0 : kFp8Direct; pol < kFp8Policies_n; ++pol) {
     if (!usable(pol)) continue;
-    const float cost = launch_cost(kFp8Policies[pol], kFp8Cost[!direct ? 2 : rhs_t ? 1 : 0][pol], pol >= kFp8Slices, (uint32_t)m, (uint32_t)n, kt, 1);
+    const TileCost& c = pol == 2 && one_per_cu(m, n) ? kFp8OnePerCu[rhs_t] : kFp8Cost[!direct ? 2 : rhs_t ? 1 : 0][pol];
+    const float cost = launch_cost(kFp8Policies[pol], c, pol >= kFp8Slices, (uint32_t)m, (uint32_t)n, kt, 1);
     if (cost < best_cost) {
       best = pol;
       best_cost = cost;
@@ -327,14 +344,17 @@ extern "C" int xmk_fp8_gemm_ex(const void* a, const void* b, const float* a_scal
     const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block((unsigned)(P.wgm * P.wgn * 64));
     const bool kn = rhs_transpose == 0;
     if (pol == 0) {
-      if (kn) hipLaunchKernelGGL((fp8_gemm_kernel<256, 256, 2, 4, 4, true>), grid, block, 0, st, p);
-      else hipLaunchKernelGGL((fp8_gemm_kernel<256, 256, 2, 4, 4>), grid, block, 0, st, p);
+      if (kn) hipLaunchKernelGGL((fp8_gemm_kernel<256, 256, 2, 4, 4, 64, true>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((fp8_gemm_kernel<256, 256, 2, 4, 4, 64, false>), grid, block, 0, st, p);
     } else if (pol == 1) {
-      if (kn) hipLaunchKernelGGL((fp8_gemm_kernel<256, 128, 2, 2, 4, true>), grid, block, 0, st, p);
-      else hipLaunchKernelGGL((fp8_gemm_kernel<256, 128, 2, 2, 4>), grid, block, 0, st, p);
+      if (kn) hipLaunchKernelGGL((fp8_gemm_kernel<256, 128, 2, 2, 4, 64, true>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((fp8_gemm_kernel<256, 128, 2, 2, 4, 64, false>), grid, block, 0, st, p);
+    } else if (one_per_cu(m, n)) {
+      if (kn) hipLaunchKernelGGL((fp8_gemm_kernel<128, 128, 2, 2, 4, 128, true>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((fp8_gemm_kernel<128, 128, 2, 2, 4, 128, false>), grid, block, 0, st, p);
     } else {
-      if (kn) hipLaunchKernelGGL((fp8_gemm_kernel<128, 128, 2, 2, 4, true>), grid, block, 0, st, p);
-      else hipLaunchKernelGGL((fp8_gemm_kernel<128, 128, 2, 2, 4>), grid, block, 0, st, p);
+      if (kn) hipLaunchKernelGGL((fp8_gemm_kernel<128, 128, 2, 2, 4, 64, true>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((fp8_gemm_kernel<128, 128, 2, 2, 4, 64, false>), grid, block, 0, st, p);
     }
   } else {
     hipLaunchKernelGGL(fp8_gemm_generic_kernel, dim3((unsigned)xmk::ceil_div(n, 64), (unsigned)xmk::ceil_div(m, 64)),

@@ -124,36 +124,36 @@ constexpr Policy kFp8Policies[] = {
 constexpr int kFp8Policies_n = sizeof(kFp8Policies) / sizeof(kFp8Policies[0]);
 constexpr int kFp8Direct = 3, kFp8Slices = 5;
 
-// Estimated microseconds (launch_cost in gemm_kernel.h), fitted to 240 shapes per class, m 1 .. 8192, n and k
-// 64 .. 16384 at random: on those on average 2 % from the best policy of all measured, on 60 other shapes per class with
-// weights from memory 3 to 4 % (one in ten more than 6 to 9 %, the worst 44 %).  The rule before (256 x 256 tiles from 256
-// of them on, 256 x 128 for about one per CU, else 128 x 128; gathered where not aligned) lost 37 / 49 / 21 %.
+// Estimated microseconds (launch_cost in gemm_kernel.h).  The direct classes are fitted to 350 shapes each, m 2 .. 8192, n 64 ..
+// 16384, k 256 .. 16384, weights from memory: on 115 others per class 3 % from the best policy of all measured, one in ten
+// more than 10 %, the worst 34 % (the table before the tiles' present order: [k,n] 7 %, 23 %, 64 %).  The any-alignment class:
+// 240 shapes, m 1 .. 8192, 2 % on those, 3 to 4 % on others.
 constexpr TileCost kFp8Cost[3][kFp8Policies_n] = {
     {  // direct loads possible, B stored [K, N]
-     {5.158f, 0.998f, 1.528f, 12.703f, 4.362f},
-     {4.603f, 0.609f, 0.997f, 6.658f, 3.077f},
-     {3.475f, 0.425f, 0.606f, 2.401f, 2.979f},
-     {3.921f, 0.674f, 0.588f, 2.897f, 1.81f},
-     {2.915f, 0.333f, 0.306f, 0.581f, 1.482f},
-     {2.704f, 0.453f, 0.166f, 0.338f, 2.138f},
-     {2.325f, 0.949f, 0.176f, 1.086f, 2.102f},
-     {0.825f, 2.878f, 0.223f, 1.819f, 2.586f},
-     {2.395f, 1.25f, 0.211f, 2.128f, 2.406f},
-     {3.268f, 0.883f, 0.301f, 3.276f, 2.364f},
-     {2.39f, 2.187f, 0.391f, 3.225f, 3.577f},
+     {5.397f, 0.987f, 1.885f, 8.612f, 5.243f},
+     {4.759f, 0.596f, 1.095f, 6.471f, 3.21f},
+     {5.059f, 0.806f, 0.561f, 1.5f, 0.f},  // (more than 256 tiles)
+     {4.011f, 0.668f, 0.532f, 2.909f, 1.888f},
+     {3.027f, 0.32f, 0.225f, 0.672f, 1.311f},
+     {3.021f, 0.388f, 0.18f, 0.286f, 1.294f},
+     {2.704f, 0.875f, 0.194f, 0.936f, 1.195f},
+     {1.231f, 2.745f, 0.246f, 1.699f, 1.428f},
+     {2.836f, 1.194f, 0.219f, 1.978f, 1.25f},
+     {3.775f, 0.84f, 0.303f, 3.027f, 1.032f},
+     {3.356f, 1.986f, 0.388f, 3.034f, 2.102f},
     },
     {  // direct loads possible, B stored [N, K]
-     {5.013f, 1.017f, 1.565f, 13.717f, 5.199f},
-     {4.539f, 0.606f, 1.049f, 6.675f, 3.514f},
-     {3.383f, 0.396f, 0.681f, 2.154f, 3.096f},
-     {3.907f, 0.652f, 0.58f, 2.981f, 1.661f},
-     {2.962f, 0.303f, 0.255f, 0.702f, 0.91f},
-     {2.897f, 0.319f, 0.102f, 0.437f, 0.769f},
-     {2.693f, 0.636f, 0.115f, 1.196f, 0.785f},
-     {1.75f, 1.976f, 0.159f, 1.995f, 1.203f},
-     {2.594f, 1.028f, 0.188f, 2.155f, 1.471f},
-     {3.35f, 0.815f, 0.294f, 3.283f, 0.988f},
-     {2.768f, 1.517f, 0.294f, 2.985f, 1.483f},
+     {5.026f, 0.989f, 1.517f, 9.792f, 7.747f},
+     {4.458f, 0.597f, 1.115f, 4.438f, 5.174f},
+     {4.782f, 0.947f, 0.545f, 1.329f, 0.f},
+     {3.78f, 0.644f, 0.521f, 2.042f, 2.495f},
+     {3.042f, 0.276f, 0.186f, 0.633f, 1.407f},
+     {3.188f, 0.302f, 0.097f, 0.445f, 0.511f},
+     {3.186f, 0.579f, 0.122f, 1.073f, 0.565f},
+     {2.224f, 1.9f, 0.159f, 1.916f, 0.857f},
+     {3.155f, 0.942f, 0.179f, 2.022f, 1.003f},
+     {3.749f, 0.766f, 0.282f, 2.87f, 0.995f},
+     {3.497f, 1.359f, 0.296f, 2.632f, 1.294f},
     },
     {  // any alignment
      {},
@@ -169,6 +169,9 @@ constexpr TileCost kFp8Cost[3][kFp8Policies_n] = {
      {3.23f, 3.795f, 0.64f, 3.87f, 1.223f},
     },
 };
+
+// The 128 x 128 tile where every CU has one at most (K steps of 128 bytes), B stored [K, N] / [N, K]; fitted with them.
+constexpr TileCost kFp8OnePerCu[2] = {{3.919f, 0.324f, 0.f, 0.f, 2.146f}, {3.689f, 0.29f, 0.f, 0.f, 3.007f}};
 
 // Policies 3 and up; A is [M, K], b_mc: B stored [K, N].
 void launch_fp8_any(int policy, bool b_mc, Fp8Params& p, hipStream_t st);

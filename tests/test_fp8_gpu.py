@@ -110,3 +110,19 @@ def test_fp8_any_alignment(xmk, oracle, monkeypatch, policy, rhs_t, m, n, k):
         ref = 0.5 * (prod + oracle.to_f32(bias, oracle.BF16)[None, :]) if with_bias else prod
         g, e = oracle.rel_err(out.float().cpu().numpy(), ref)
         assert g <= 1e-2 and e <= 1e-2, (g, e)
+
+
+@pytest.mark.parametrize("rhs_t", [True, False])
+@pytest.mark.parametrize("m,n,k", [(16, 16, 16), (130, 272, 112), (128, 144, 128), (257, 128, 144), (2048, 2048, 272), (2049, 2048, 272), (300, 1040, 1040)])
+def test_fp8_long_and_short_steps(xmk, oracle, monkeypatch, rhs_t, m, n, k):
+    """128 x 128 tiles on either side of 256 of them: K steps of 128 bytes and of 64, K that ends in the first half of a step,
+    at its middle, in the second half; fewer steps than stages and more."""
+    monkeypatch.setenv("XMK_FP8_POLICY", "2")
+    a, sa = _quant(oracle, (m, k), 3)
+    b, sb = _quant(oracle, (n, k) if rhs_t else (k, n), 4)
+    _, ref = oracle.fp8_gemm(a, b, sa, sb, rhs_t=rhs_t)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    xmk.fp8_gemm(to_dev(a, "f8"), to_dev(b, "f8"), torch.tensor([sa], device="cuda"), torch.tensor([sb], device="cuda"), out, rhs_transpose=rhs_t)
+    torch.cuda.synchronize()
+    g, e = oracle.rel_err(out.float().cpu().numpy(), ref)
+    assert g <= 1e-2 and e <= 1e-2, (g, e)  # exact products, fp32 sums, one rounding to bf16
