@@ -119,8 +119,10 @@ int xmk_gemm(const xmk_gemm_desc* desc, void* stream);
  * is long (small-M decode shapes such as the 1_4096_4096 and 4_4096_16384 entries of the reference's
  * table, xetla/gemm/gemm.cc:32-37, which it runs with SLM_KS k-slicing), K is split over work-groups:
  * fp32 partial sums go to the workspace and a second kernel adds them in slice order and applies the
- * epilogue.  xmk_gemm_workspace_bytes returns the bytes that makes possible for this descriptor
- * (0: the call would not split).  With a NULL or too small workspace the call is xmk_gemm. */
+ * epilogue.  Large products of 16-bit operands whose rows do not hold whole, aligned 16-byte chunks have
+ * those operands copied into rows that do, in the workspace, first.  xmk_gemm_workspace_bytes returns the
+ * bytes that makes possible for this descriptor (0: the call would use none).  With a NULL or too small
+ * workspace the call is xmk_gemm. */
 size_t xmk_gemm_workspace_bytes(const xmk_gemm_desc* desc);
 int xmk_gemm_ws(const xmk_gemm_desc* desc, void* workspace, size_t workspace_bytes, void* stream);
 

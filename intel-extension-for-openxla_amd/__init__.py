@@ -72,6 +72,7 @@ def lib():
                               ("xmk_fmha_decode_cache_workspace_bytes", ctypes.c_size_t),
                               ("xmk_fmha_decode_static_max_bytes", ctypes.c_size_t),
                               ("xmk_fmha_bwd_workspace_bytes", ctypes.c_size_t),
+                              ("xmk_fmha_bwd_best_workspace_bytes", ctypes.c_size_t),
                               ("xmk_gemm_workspace_bytes", ctypes.c_size_t),
                               ("xmk_int4_gemm_workspace_bytes", ctypes.c_size_t)):
             if hasattr(L, name):

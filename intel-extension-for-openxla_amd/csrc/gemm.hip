@@ -175,6 +175,43 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(ReduceParams p)
   }
 }
 
+// Copies operands whose rows start anywhere into rows of whole, aligned 16-byte chunks, zeros behind a row's end.
+struct PackOperand {
+  const uint16_t* from;
+  uint16_t* to;
+  int64_t ld_from, ld_to;
+  int cols, row_chunks;  // chunks of eight elements
+  int chunks;            // in all
+};
+constexpr int kPackPerThread = 4;
+__global__ __launch_bounds__(256) void gemm_pack_kernel(PackOperand a, PackOperand b, int a_blocks) {
+  const bool second = (int)blockIdx.x >= a_blocks;
+  const PackOperand& p = second ? b : a;
+  const int first = ((int)blockIdx.x - (second ? a_blocks : 0)) * 256 * kPackPerThread + (int)threadIdx.x;
+  u32x4 v[kPackPerThread];
+  uint16_t* to[kPackPerThread];
+#pragma unroll
+  for (int i = 0; i < kPackPerThread; ++i) {
+    const int chunk = first + 256 * i;
+    to[i] = nullptr;
+    if (chunk >= p.chunks) continue;
+    const int row = (int)((uint32_t)chunk / (uint32_t)p.row_chunks), col = (chunk - row * p.row_chunks) * 8;
+    const uint16_t* from = p.from + row * p.ld_from + col;
+    to[i] = p.to + row * p.ld_to + col;
+    if (col + 8 <= p.cols) {
+      __builtin_memcpy(&v[i], from, 16);
+    } else {
+      uint16_t e[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) e[j] = col + j < p.cols ? from[j] : (uint16_t)0;
+      __builtin_memcpy(&v[i], e, 16);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kPackPerThread; ++i)
+    if (to[i]) *reinterpret_cast<u32x4*>(to[i]) = v[i];
+}
+
 // ------------------------------------------------------------------ host side
 
 int generic_kind(int dtype) {
@@ -229,13 +266,17 @@ namespace {
 // policy: tile policy to use instead of select_policy's choice (the K-split planner's), or -1.
 // kslice: K slice of a batch member (a K split into unequal slices; the operands are then those of the whole
 // product), or 0.
-int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int policy = -1, int kslice = 0);
+// padded: the operands' rows hold whole 16-byte chunks, whatever their lengths.
+int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int policy = -1, int kslice = 0, bool padded = false);
+
+// The tile loaders form byte offsets of up to 256 rows of an operand in 32 bits.
+constexpr int64_t kMaxLd = int64_t{1} << 22;
 
 // The conditions of the direct-to-LDS 16-bit kernels on the stored operands.
-bool direct_ok(const xmk_matrix& lhs, const xmk_matrix& rhs) {
+bool direct_ok(const xmk_matrix& lhs, const xmk_matrix& rhs, bool padded = false) {
   return xmk::aligned(lhs.data, 16) && xmk::aligned(rhs.data, 16) && lhs.leading_dim_stride % 8 == 0 &&
          rhs.leading_dim_stride % 8 == 0 && lhs.batch_stride % 8 == 0 && rhs.batch_stride % 8 == 0 &&
-         lhs.num_cols % 8 == 0 && rhs.num_cols % 8 == 0;
+         (padded || (lhs.num_cols % 8 == 0 && rhs.num_cols % 8 == 0));
 }
 
 // Which streaming kernel for a few rows (gemm_rows.hip) can run this descriptor's product, if any.
@@ -253,7 +294,7 @@ int rows_kind_desc(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k) {
 // output tiles (the device has 256 CUs) and a long reduction.  1: do not split.
 // *policy: the tile policy of the slices (-1: whatever select_policy picks for a slice).
 // *kslice: K slice (a multiple of 64, the last slice takes the rest) of operands passed whole, 0: equal slices as batch members.
-int plan_splitk(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k, int* policy, int* kslice) {
+int plan_splitk(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k, int* policy, int* kslice, bool padded = false) {
   *policy = -1;
   *kslice = 0;
   if (d->batch_size != 1) return 1;
@@ -261,7 +302,7 @@ int plan_splitk(const xmk_gemm_desc* d, int64_t m, int64_t n, int64_t k, int* po
   // XMK_GEMM_SPLITK=<slices> overrides the choice (read at every call; the autotuner's handle).
   const char* forced_env = getenv("XMK_GEMM_SPLITK");
   const int forced = forced_env ? atoi(forced_env) : 0;
-  if (d->dtype_in == XMK_F32 || !direct_ok(d->lhs, d->rhs)) {
+  if (d->dtype_in == XMK_F32 || !direct_ok(d->lhs, d->rhs, padded)) {
     Choice c = cheapest(m, n, k, 1, d->dtype_in == XMK_F32 ? kClassF32 : kClassRagged, true);
     if (forced >= 1) c.slices = forced;
     if (forced_policy() >= 0) c.policy = forced_policy();
@@ -319,12 +360,84 @@ extern "C" int xmk_gemm(const xmk_gemm_desc* d, void* stream) { return run_gemm(
 
 namespace {
 // The K slices that a call with scratch runs this descriptor's product in (see plan_splitk); 1: scratch is not used.
-int planned_slices(const xmk_gemm_desc* d, int64_t* m, int64_t* n, int64_t* k, int* policy, int* kslice) {
+int planned_slices(const xmk_gemm_desc* d, int64_t* m, int64_t* n, int64_t* k, int* policy, int* kslice, bool padded = false) {
   if (d->lhs.transpose || d->out.transpose) return 1;
   gemm_dims(d, m, n, k);
   if (*m <= 0 || *n <= 0 || *k <= 0) return 1;
-  return plan_splitk(d, *m, *n, *k, policy, kslice);
+  return plan_splitk(d, *m, *n, *k, policy, kslice, padded);
 }
+
+// Whether run_gemm would take the product (untransposed lhs and output): the scratch paths hand it other operands, and what it
+// would have rejected must still be rejected (a reduction size that differs between the operands, a leading dimension
+// shorter than the full row).
+bool valid_product(const xmk_gemm_desc* d, int* act, bool* wants_bias) {
+  *act = ACT_NONE;
+  *wants_bias = false;
+  switch (d->epilogue) {
+    case XMK_EPI_DEFAULT: break;
+    case XMK_EPI_RELU: *act = ACT_RELU; break;
+    case XMK_EPI_GELU: *act = ACT_GELU; break;
+    case XMK_EPI_BIAS: *wants_bias = true; break;
+    case XMK_EPI_BIAS_RELU: *wants_bias = true; *act = ACT_RELU; break;
+    case XMK_EPI_BIAS_GELU: *wants_bias = true; *act = ACT_GELU; break;
+    default: return false;
+  }
+  int64_t m, n, k;
+  gemm_dims(d, &m, &n, &k);
+  const int64_t k_rhs = d->rhs.transpose ? d->rhs.num_cols : d->rhs.num_rows;
+  if (k_rhs != k || d->lhs.leading_dim_stride < d->lhs.num_cols || d->rhs.leading_dim_stride < d->rhs.num_cols) return false;
+  return !((*wants_bias && !d->bias) || (d->beta != 0.0f && !d->c) || !d->out.data || d->out.num_rows != m || d->out.num_cols != n ||
+           d->out.leading_dim_stride < n || (d->dtype_out != d->dtype_in && d->dtype_out != XMK_F32));
+}
+
+// Copying operands with misaligned rows into scratch first, for the direct-to-LDS kernels: a load at an unaligned address
+// takes the CU's load path as long as four, and a large product makes every such load tens of times, the copy once.
+// Microseconds without / with the copy: 1023 x 5003 x 2047 55.7 / 43, 4001^3 197 / 142, 1418 x 8367 x 3357 176 / 114, 2047^3
+// 37 / 32; 64 x 5001 x 5001 23.5 / 34, 300 x 50257 x 769 65 / 101: chosen by the estimates of both ways.  The second one's: the
+// direct kernels' on aligned sizes, what the copy takes (fitted to 51 odd sizes: 5.2 us and 0.165 per MB) and what outputs of
+// odd row length cost beyond aligned ones (0.87 per million).  On those 51 it never chose the slower way.
+struct PackPlan {
+  bool a, b;             // which are copied
+  int64_t lda, ldb;      // leading dimensions of the copies
+  size_t b_at, total;    // bytes
+};
+bool plan_pack(const xmk_gemm_desc* d, PackPlan* p) {
+  if (d->lhs.transpose || d->out.transpose || d->batch_size != 1) return false;
+  if (d->dtype_in != XMK_BF16 && d->dtype_in != XMK_F16) return false;
+  if (direct_ok(d->lhs, d->rhs) || !xmk::aligned(d->out.data, 16)) return false;
+  auto ok = [](const xmk_matrix& x) { return xmk::aligned(x.data, 16) && x.leading_dim_stride % 8 == 0 && x.num_cols % 8 == 0; };
+  auto ld = [](const xmk_matrix& x) { return xmk::ceil_div(x.num_cols, 64) * 64; };
+  int64_t m, n, k;
+  gemm_dims(d, &m, &n, &k);
+  constexpr int64_t kMax = 1 << 29;
+  if (m <= 0 || n <= 0 || k <= 0 || m >= kMax || n >= kMax || k >= kMax || m * k >= kMax || n * k >= kMax) return false;
+  p->a = !ok(d->lhs);
+  p->b = !ok(d->rhs);
+  p->lda = ld(d->lhs);
+  p->ldb = ld(d->rhs);
+  p->b_at = p->a ? (size_t)m * p->lda * 2 : 0;
+  p->total = p->b_at + (p->b ? (size_t)d->rhs.num_rows * p->ldb * 2 : 0);
+  if (forced_policy() != kUnforced || getenv("XMK_GEMM_SPLITK")) return false;  // (they force what runs on the operands given)
+  if (!spans_a_load(m, d->lhs.leading_dim_stride, k, d->dtype_in) ||
+      !spans_a_load(d->rhs.num_rows, d->rhs.leading_dim_stride, d->rhs.num_cols, d->dtype_in)) return false;
+  const float copied = (float)((p->a ? m * k : 0) + (p->b ? n * k : 0)) * 2e-6f;
+  const float with = cheapest(m, n, k, 1, d->rhs.transpose ? kClassNK : kClassKN, true).us + 5.2f + 0.165f * copied + 0.87e-6f * (float)m * (float)n;
+  return cheapest(m, n, k, 1, kClassRagged, true).us > 1.03f * with;
+}
+// The descriptor with the copies at `ws` in place of the operands.
+xmk_gemm_desc packed_desc(const xmk_gemm_desc* d, const PackPlan& p, char* ws) {
+  xmk_gemm_desc q = *d;
+  if (p.a) { q.lhs.data = ws; q.lhs.leading_dim_stride = p.lda; q.lhs.batch_stride = 0; }
+  if (p.b) { q.rhs.data = ws + p.b_at; q.rhs.leading_dim_stride = p.ldb; q.rhs.batch_stride = 0; }
+  return q;
+}
+PackOperand pack_operand(const xmk_matrix& x, void* to, int64_t ld) {
+  PackOperand p{};
+  p.from = (const uint16_t*)x.data; p.to = (uint16_t*)to; p.ld_from = x.leading_dim_stride; p.ld_to = ld;
+  p.cols = (int)x.num_cols; p.row_chunks = (int)xmk::ceil_div(x.num_cols, 8); p.chunks = (int)(x.num_rows * p.row_chunks);
+  return p;
+}
+int gemm_ws(const xmk_gemm_desc* d, void* workspace, size_t workspace_bytes, void* stream, bool padded);
 }  // namespace
 
 extern "C" size_t xmk_gemm_workspace_bytes(const xmk_gemm_desc* d) {
@@ -332,16 +445,41 @@ extern "C" size_t xmk_gemm_workspace_bytes(const xmk_gemm_desc* d) {
   int64_t m, n, k;
   int policy, kslice;
   const int ks = planned_slices(d, &m, &n, &k, &policy, &kslice);
-  return ks > 1 ? (size_t)ks * slice_stride(m, n) * sizeof(float) : 0;
+  const size_t need = ks > 1 ? (size_t)ks * slice_stride(m, n) * sizeof(float) : 0;
+  PackPlan pk;
+  if (!plan_pack(d, &pk)) return need;
+  const xmk_gemm_desc q = packed_desc(d, pk, nullptr);
+  const int kp = planned_slices(&q, &m, &n, &k, &policy, &kslice, true);
+  return std::max(need, pk.total + (kp > 1 ? (size_t)kp * slice_stride(m, n) * sizeof(float) : 0));
 }
 
 extern "C" int xmk_gemm_ws(const xmk_gemm_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
   if (!d) return xmk::fail(XMK_INVALID_ARGUMENT, "gemm: null descriptor");
   if (!workspace || !xmk::aligned(workspace, 16)) return run_gemm(d, nullptr, nullptr, stream);
+  PackPlan pk;
+  int act;
+  bool wants_bias;
+  if (plan_pack(d, &pk) && pk.total <= workspace_bytes && d->lhs.data && d->rhs.data && d->lhs.leading_dim_stride < kMaxLd &&
+      d->rhs.leading_dim_stride < kMaxLd && d->out.leading_dim_stride < kMaxLd && valid_product(d, &act, &wants_bias)) {
+    const xmk_gemm_desc q = packed_desc(d, pk, (char*)workspace);
+    PackOperand a{}, b{};
+    if (pk.a) a = pack_operand(d->lhs, workspace, pk.lda);
+    if (pk.b) b = pack_operand(d->rhs, (char*)workspace + pk.b_at, pk.ldb);
+    auto blocks = [](const PackOperand& p) { return (int)xmk::ceil_div(p.chunks, 256 * kPackPerThread); };
+    xmk::trace("gemm: %s copied into aligned rows", pk.a && pk.b ? "both operands" : pk.a ? "lhs" : "rhs");
+    hipLaunchKernelGGL(gemm_pack_kernel, dim3((unsigned)(blocks(a) + blocks(b))), dim3(256), 0, (hipStream_t)stream, a, b, blocks(a));
+    return gemm_ws(&q, (char*)workspace + pk.total, workspace_bytes - pk.total, stream, true);
+  }
+  return gemm_ws(d, workspace, workspace_bytes, stream, false);
+}
+
+namespace {
+int gemm_ws(const xmk_gemm_desc* d, void* workspace, size_t workspace_bytes, void* stream, bool padded) {
   int64_t m, n, k;
   int slice_policy, kslice;
-  const int ks = planned_slices(d, &m, &n, &k, &slice_policy, &kslice);
-  if (ks < 2 || workspace_bytes < (size_t)ks * slice_stride(m, n) * sizeof(float)) return run_gemm(d, nullptr, nullptr, stream);
+  const int ks = planned_slices(d, &m, &n, &k, &slice_policy, &kslice, padded);
+  if (ks < 2 || workspace_bytes < (size_t)ks * slice_stride(m, n) * sizeof(float))
+    return run_gemm(d, nullptr, nullptr, stream, -1, 0, padded);
   // Pass 1: the K slices as a batched GEMM into fp32 partial sums (no epilogue); a slice is a
   // column range of lhs and a row (or column) range of rhs, so only the batch strides change.
   xmk_gemm_desc p = *d;
@@ -356,29 +494,11 @@ extern "C" int xmk_gemm_ws(const xmk_gemm_desc* d, void* workspace, size_t works
   p.c = nullptr; p.bias = nullptr;
   p.dtype_out = XMK_F32;
   p.batch_size = ks; p.alpha = 1.0f; p.beta = 0.0f; p.epilogue = XMK_EPI_DEFAULT;
-  // what the full call would have rejected must still be rejected: validate it first
-  int act = ACT_NONE;
-  bool wants_bias = false;
-  switch (d->epilogue) {
-    case XMK_EPI_DEFAULT: break;
-    case XMK_EPI_RELU: act = ACT_RELU; break;
-    case XMK_EPI_GELU: act = ACT_GELU; break;
-    case XMK_EPI_BIAS: wants_bias = true; break;
-    case XMK_EPI_BIAS_RELU: wants_bias = true; act = ACT_RELU; break;
-    case XMK_EPI_BIAS_GELU: wants_bias = true; act = ACT_GELU; break;
-    default: return run_gemm(d, nullptr, nullptr, stream);  // reports the error
-  }
-  // (the sliced copy would hide a reduction size that differs between the operands, or a leading
-  // dimension shorter than the full row)
-  const int64_t k_rhs = d->rhs.transpose ? d->rhs.num_cols : d->rhs.num_rows;
-  if (k_rhs != k || d->lhs.leading_dim_stride < d->lhs.num_cols || d->rhs.leading_dim_stride < d->rhs.num_cols)
-    return run_gemm(d, nullptr, nullptr, stream);  // reports the error
-  if ((wants_bias && !d->bias) || (d->beta != 0.0f && !d->c) || !d->out.data ||
-      d->out.num_rows != m || d->out.num_cols != n || d->out.leading_dim_stride < n ||
-      (d->dtype_out != d->dtype_in && d->dtype_out != XMK_F32))
-    return run_gemm(d, nullptr, nullptr, stream);  // reports the error
+  int act;
+  bool wants_bias;
+  if (!valid_product(d, &act, &wants_bias)) return run_gemm(d, nullptr, nullptr, stream);  // reports the error
   xmk::trace("gemm m=%lld n=%lld k=%lld -> split K %d ways", (long long)m, (long long)n, (long long)k, ks);
-  int rc = run_gemm(&p, nullptr, nullptr, stream, slice_policy, kslice);
+  int rc = run_gemm(&p, nullptr, nullptr, stream, slice_policy, kslice, padded);
   if (rc != XMK_OK) return rc;
   ReduceParams r;
   r.partial = (const float*)workspace; r.out = d->out.data; r.c = d->beta != 0.0f ? d->c : nullptr;
@@ -390,6 +510,7 @@ extern "C" int xmk_gemm_ws(const xmk_gemm_desc* d, void* workspace, size_t works
                      (hipStream_t)stream, r);
   return xmk::check_launch("gemm");
 }
+}  // namespace
 
 extern "C" int xmk_gemm_qkv(const xmk_gemm_desc* d, void* out_k, void* out_v, void* stream) {
   if (!d) return xmk::fail(XMK_INVALID_ARGUMENT, "gemm_qkv: null descriptor");
@@ -402,7 +523,7 @@ extern "C" int xmk_gemm_qkv(const xmk_gemm_desc* d, void* out_k, void* out_v, vo
 }
 
 namespace {
-int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int policy, int kslice) {
+int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int policy, int kslice, bool padded) {
   if (!d) return xmk::fail(XMK_INVALID_ARGUMENT, "gemm: null descriptor");
   if (!d->lhs.data || !d->rhs.data || !d->out.data)
     return xmk::fail(XMK_INVALID_ARGUMENT, "gemm: null operand");
@@ -462,15 +583,13 @@ int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int p
   if (m > INT32_MAX / 2 || n > INT32_MAX / 2 || k > INT32_MAX / 2 || d->batch_size > 65535)
     return xmk::fail(XMK_INVALID_ARGUMENT, "gemm: dimension too large");
   if (!d->bias && wants_bias) return xmk::fail(XMK_INVALID_ARGUMENT, "gemm: bias missing");
-  // The tile loaders form byte offsets of up to 256 rows of an operand in 32 bits.
-  constexpr int64_t kMaxLd = int64_t{1} << 22;
   if (lhs.leading_dim_stride >= kMaxLd || rhs.leading_dim_stride >= kMaxLd || out.leading_dim_stride >= kMaxLd)
     return xmk::fail(XMK_INVALID_ARGUMENT, "gemm: leading_dim_stride of 2^22 elements or more");
 
   hipStream_t st = (hipStream_t)stream;
   const bool qkv = out1 != nullptr;
   const bool sixteen = din == XMK_BF16 || din == XMK_F16;
-  const bool fast = sixteen && direct_ok(lhs, rhs) && xmk::aligned(out.data, 16) && xmk::aligned(out1, 16) &&
+  const bool fast = sixteen && direct_ok(lhs, rhs, padded) && xmk::aligned(out.data, 16) && xmk::aligned(out1, 16) &&
                     xmk::aligned(out2, 16);
   // 16-bit operands that miss those conditions and fp32 operands: the kernels that take any alignment (they read
   // 16 bytes at a time, wherever an operand has that many).

@@ -845,11 +845,11 @@ inline float launch_cost(const Policy& P, const TileCost& c, bool slices, uint32
 
 struct Choice {
   int policy, slices;
+  float us;
 };
 // The cheapest policy and number of K slices (1 unless may_split).
 inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, bool may_split) {
-  Choice best{3, 1};
-  float best_cost = 1e30f;
+  Choice best{3, 1, 1e30f};
   const bool direct = cls == kClassKN || cls == kClassNK;
   const int kstep = cls == kClassF32 ? 32 : 64;
   auto each = [&](int s, float extra, float least) {
@@ -858,14 +858,11 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
       const uint32_t kt = (uint32_t)(((k + s - 1) / s + kstep - 1) / kstep);
       const float cost = std::max(launch_cost(kPolicies[pol], kTileCost[cls][pol], pol >= kSlicesPolicy, (uint32_t)m, (uint32_t)n, kt,
                                               (uint32_t)(batch * s)) + extra, least);
-      if (cost < best_cost) {
-        best_cost = cost;
-        best = {pol, s};
-      }
+      if (cost < best.us) best = {pol, s, cost};
     }
   };
   each(1, 0.0f, 0.0f);
-  for (int s = 2; may_split && s <= 16 && best_cost > kSplitFloor; s *= 2) {
+  for (int s = 2; may_split && s <= 16 && best.us > kSplitFloor; s *= 2) {
     if (k / s < 128 || (float)m * (float)n * (float)s > 6.4e7f) break;
     each(s, kSplitCost + (float)m * (float)n * (float)s * (8.0f / 3e6f), kSplitFloor);
   }
