@@ -31,7 +31,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-I", INCLUDE, "
 
 # Per-file flags.  Attention forward: matrix instructions write VGPRs, so that the softmax reads the
 # scores where they were produced (the whole register budget is then one file of 256 per wave).
-EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("fmha_fwd.hip", "fmha_short.hip", "int4_tile.hip")}
+EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("fmha_fwd.hip", "fmha_fwd_h48.hip", "fmha_fwd_h80.hip", "fmha_fwd_h96.hip", "fmha_fwd_h160.hip", "fmha_short.hip", "int4_tile.hip")}
 
 
 def sources():

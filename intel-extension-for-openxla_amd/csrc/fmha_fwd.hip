@@ -17,8 +17,12 @@ void launch_t(const FmhaParams& p, int32_t dtype, uint64_t units, uint32_t F, bo
   // 32-row tile per wave (one wave per SIMD, O in AGPRs, every K / V fragment feeding two matrix
   // instructions) 1007 against 1033 without a mask and 789 against 872 with one, at a higher clock and
   // the same board power and energy per launch: the package power limit, not the schedule, sets the rate.
-  if (p.H <= 64) launch_cfg<T, 64, 4, 2>(p, units, F, causal, bias, st);
-  else if (p.H <= 128) launch_cfg<T, 128, 4, 2>(p, units, F, causal, bias, st);
+  if (p.H <= 48) launch_h48(p, dtype, units, F, causal, bias, st);
+  else if (p.H <= 64) launch_cfg<T, 64, 4, 2, 4, 2>(p, units, F, causal, bias, st);
+  else if (p.H <= 80) launch_h80(p, dtype, units, F, causal, bias, st);
+  else if (p.H <= 96) launch_h96(p, dtype, units, F, causal, bias, st);
+  else if (p.H <= 128) launch_cfg<T, 128, 8, 4, 4, 2>(p, units, F, causal, bias, st);
+  else if (p.H <= 160) launch_h160(p, dtype, units, F, causal, bias, st);
   else launch_h256(p, dtype, units, F, causal, bias, st);
 }
 

@@ -7,8 +7,8 @@ namespace fmha_fwd_impl {
 
 void launch_h256(const FmhaParams& p, int32_t dtype, uint64_t units, uint32_t F, bool causal, int bias,
                  hipStream_t st) {
-  if (dtype == XMK_BF16) launch_cfg<__bf16, 256, 4, 1>(p, units, F, causal, bias, st);
-  else launch_cfg<_Float16, 256, 4, 1>(p, units, F, causal, bias, st);
+  if (dtype == XMK_BF16) launch_cfg<__bf16, 256, 16, 8, 4, 1>(p, units, F, causal, bias, st);
+  else launch_cfg<_Float16, 256, 16, 8, 4, 1>(p, units, F, causal, bias, st);
 }
 
 }  // namespace fmha_fwd_impl

@@ -142,11 +142,12 @@ __host__ __device__ constexpr int wait_vm_lgkm0(int n) { return (n & 0xf) | ((n 
 #endif
 constexpr int kAhead = 3;  // matrix instructions by which the LDS fragment reads run ahead
 
-// T: element type; HP: head size padded to 64 / 128 / 256; NW: waves per work-group; WPS: waves
-// per SIMD the register budget is set for.
+// T: element type; HP: head size padded to 64 / 128 / 256, the length of an LDS row; KS, HT: steps of 16 and tiles of 32 that
+// cover the head size, which the products run over (the rest of a row is zeros that nothing reads); NW: waves per
+// work-group; WPS: waves per SIMD the register budget is set for.
 // BIAS: 0 none; 1 read from global memory element by element (any shape and alignment); 2 staged
 // through LDS one [rows x 64 keys] tile per key tile (T % 8 == 0, 16-byte aligned bias).
-template <typename T, int HP, int NW, int WPS, bool CAUSAL, int BIAS>
+template <typename T, int HP, int KS, int HT, int NW, int WPS, bool CAUSAL, int BIAS>
 __global__ __launch_bounds__(NW * 64, WPS) void fmha_fwd_kernel(FmhaParams p) {
   typedef typename Elem<T>::vec8 V8;
   constexpr int BR = NW * 32;                // query rows per work-group
@@ -159,8 +160,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fmha_fwd_kernel(FmhaParams p) {
   constexpr int NL = HALF / 1024 / NW;       // loads per wave per half tile
   constexpr int LROWS = NW * RPL;            // tile rows between consecutive loads of a wave
   constexpr int KV = (LROWS % (KMASK + 1) == 0) ? 1 : 2;  // distinct K swizzles among a wave's loads
-  constexpr int KS = HP / 16;                // k-steps of the S product
-  constexpr int HT = HP / 32;                // 32-wide h tiles of O
+  static_assert(16 * KS <= HP && 32 * HT <= HP && 16 * KS <= 32 * HT, "head size");
   static_assert(BR % BC == 0, "a query block spans whole key tiles");
   static_assert(NL >= 1 && NL * LROWS == 32 && LROWS % 8 == 0 && (2 * LROWS) % (KMASK + 1) == 0, "half tile / wave split");
   constexpr int BTILE = 32 * BC * 2;         // one wave's bias tile: its 32 query rows x 64 keys
@@ -743,7 +743,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fmha_fwd_kernel(FmhaParams p) {
   }
 }
 
-template <typename T, int HP, int NW, int WPS>
+template <typename T, int HP, int KS, int HT, int NW, int WPS>
 void launch_cfg(FmhaParams p, uint64_t units, uint32_t F, bool causal, int bias, hipStream_t st) {
   p.nqb = (int)((F + NW * 32 - 1) / (NW * 32));
   p.total = (int)(units * p.nqb);
@@ -754,17 +754,22 @@ void launch_cfg(FmhaParams p, uint64_t units, uint32_t F, bool causal, int bias,
   const dim3 grid((unsigned)(p.per_xcd * 8)), block(NW * 64);
   // bias: 0 none, 1 element-wise from global memory, 2 staged through LDS
   if (causal) {
-    if (bias == 2) hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, NW, WPS, true, 2>), grid, block, 0, st, p);
-    else if (bias == 1) hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, NW, WPS, true, 1>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, NW, WPS, true, 0>), grid, block, 0, st, p);
+    if (bias == 2) hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, KS, HT, NW, WPS, true, 2>), grid, block, 0, st, p);
+    else if (bias == 1) hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, KS, HT, NW, WPS, true, 1>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, KS, HT, NW, WPS, true, 0>), grid, block, 0, st, p);
   } else {
-    if (bias == 2) hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, NW, WPS, false, 2>), grid, block, 0, st, p);
-    else if (bias == 1) hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, NW, WPS, false, 1>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, NW, WPS, false, 0>), grid, block, 0, st, p);
+    if (bias == 2) hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, KS, HT, NW, WPS, false, 2>), grid, block, 0, st, p);
+    else if (bias == 1) hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, KS, HT, NW, WPS, false, 1>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, KS, HT, NW, WPS, false, 0>), grid, block, 0, st, p);
   }
 }
 
-// Head size above 128 (the accumulators of that class need both halves of the register file);
+// Head sizes up to 48, 65 to 80, 81 to 96, 129 to 160 (fmha_fwd_h*.hip).
+void launch_h48(const FmhaParams& p, int32_t dtype, uint64_t units, uint32_t F, bool causal, int bias, hipStream_t st);
+void launch_h80(const FmhaParams& p, int32_t dtype, uint64_t units, uint32_t F, bool causal, int bias, hipStream_t st);
+void launch_h96(const FmhaParams& p, int32_t dtype, uint64_t units, uint32_t F, bool causal, int bias, hipStream_t st);
+void launch_h160(const FmhaParams& p, int32_t dtype, uint64_t units, uint32_t F, bool causal, int bias, hipStream_t st);
+// Head size above 160 (the accumulators of that class need both halves of the register file);
 // defined in fmha_fwd_h256.hip.
 void launch_h256(const FmhaParams& p, int32_t dtype, uint64_t units, uint32_t F, bool causal, int bias,
                  hipStream_t st);
