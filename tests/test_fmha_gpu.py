@@ -260,6 +260,37 @@ def test_key_permutation_invariance(xmk):
     assert (o1.float() - o2.float()).abs().max().item() <= 2e-2
 
 
+@pytest.mark.parametrize("name", ["bf16", "fp16"])
+@pytest.mark.parametrize("causal,use_bias", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("F,T,H", [(257, 321, 40), (129, 264, 48), (300, 301, 56), (257, 323, 72), (130, 520, 80), (131, 257, 88),
+                                   (193, 328, 96), (161, 299, 136), (260, 256, 160), (129, 267, 168)])
+def test_head_size_classes(xmk, oracle, name, causal, use_bias, F, T, H):
+    """Each class of head sizes at its last size and just past the one below, with ragged rows and keys and both ways of
+    reading the bias (T a multiple of 8 or not).  Tolerances: the module's."""
+    _run(xmk, oracle, name, 1, 2, F, T, H, causal=causal, use_bias=use_bias, lse=True, seed=77, f_stride=7)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("F,T,H", [(5, 1, 64), (67, 37, 40), (131, 259, 64), (64, 333, 160), (33, 513, 256)])
+def test_bias_of_other_rows_stays_out(xmk, F, T, H, bad):
+    """A bias with T % 8 != 0 is read in pieces that may reach into the next row: whatever stands there, and past the whole
+    bias, must not be felt.  Same rounding steps on both sides, but the row maximum that the weights of a wave refer to may
+    move at another key: each weight and the output round to 8 bits on both sides, so 4 x 2^-8 of sum p |v| <= max |v|."""
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(2, 2, n, H, generator=g).bfloat16().cuda() for n in (F, T, T))
+    whole = torch.randn(4 * F * T + 64, generator=g).bfloat16().cuda()
+    whole[4 * F * T:] = bad
+    bias = whole[:4 * F * T].view(2, 2, F, T)
+    ref, got = torch.empty_like(q), torch.empty_like(q)
+    xmk.fmha_forward(q, k, v, ref, bias=bias, head_scale=H ** -0.5, causal=False)
+    bias[:, :, 1::2] = bad
+    xmk.fmha_forward(q, k, v, got, bias=bias, head_scale=H ** -0.5, causal=False)
+    torch.cuda.synchronize()
+    a, b = ref[:, :, ::2].float().cpu(), got[:, :, ::2].float().cpu()
+    assert torch.isfinite(a).all() and torch.isfinite(b).all()
+    assert (a - b).abs().max() <= 2.0 ** -6 * v.float().abs().max().cpu()
+
+
 def test_errors(xmk):
     q = torch.zeros((1, 1, 8, 12), dtype=torch.bfloat16, device="cuda")
     with pytest.raises(xmk.XmkError) as e:
