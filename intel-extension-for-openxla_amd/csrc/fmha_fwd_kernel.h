@@ -142,6 +142,51 @@ __host__ __device__ constexpr int wait_vm_lgkm0(int n) { return (n & 0xf) | ((n 
 #endif
 constexpr int kAhead = 3;  // matrix instructions by which the LDS fragment reads run ahead
 
+// Element e of four packed ones.
+template <typename T>
+__device__ __forceinline__ float bias_value(u32x2 w, int e) {
+  const uint32_t d = w[e >> 1];
+  if constexpr (sizeof(T) == 2 && __is_same(T, __bf16)) {
+    return __builtin_bit_cast(float, (e & 1) ? (d & 0xffff0000u) : (d << 16));
+  } else {
+    return (float)__builtin_bit_cast(_Float16, (uint16_t)((e & 1) ? (d >> 16) : (d & 0xffffu)));
+  }
+}
+
+// A bias of any row length and alignment: of 32 keys of a query row, lane g of the row fetches keys 16 g .. +15 (`at` is the
+// first) as two 16-byte pieces, wherever they lie (the hardware takes global loads at any address), and hands the eight keys
+// that are the other lane's to it when they are used.  Pieces may reach past the row, into the next one (the caller masks
+// those keys); where they would reach past the whole bias (`whole` false; uniform over the wave) keys are read one by one, the
+// row's last one, `keys` - 1 after `at` (also where that is before it), in place of those past it.  (With a load for each element, waited for where it is used, the wave stood still:
+// 4 x 15 heads of 1907 x 256 fp16 2011 us against 355 so, 5 of 5413 x 40 bf16 1095 against 146, 16 of 2876 x 160 causal 680
+// against 127.)
+template <typename T>
+__device__ __forceinline__ void fetch_bias_keys(const T* at, bool whole, int keys, u32x4 (&b)[2]) {
+  if (whole) {
+    __builtin_memcpy(&b[0], at, 16);
+    __builtin_memcpy(&b[1], at + 8, 16);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t lo = __builtin_bit_cast(uint16_t, at[min(2 * j, keys - 1)]);
+      const uint32_t hi = __builtin_bit_cast(uint16_t, at[min(2 * j + 1, keys - 1)]);
+      b[j / 4][j % 4] = lo | hi << 16;
+    }
+  }
+}
+// w[o]: the lane's keys 8 o + 4 g .. +3, o = 0 .. 3 (every lane of the wave takes part).
+__device__ __forceinline__ void exchange_bias_keys(const u32x4 (&b)[2], u32x2 (&w)[4]) {
+#pragma unroll
+  for (int o = 0; o < 2; ++o) {
+    uint32_t x0 = b[o][0], x1 = b[o][1], x2 = b[o][2], x3 = b[o][3];
+    // (upper half of the first operand <-> lower half of the second)
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3"
+                 : "+v"(x0), "+v"(x1), "+v"(x2), "+v"(x3));
+    w[o] = u32x2{x0, x1};
+    w[o + 2] = u32x2{x2, x3};
+  }
+}
+
 // T: element type; HP: head size padded to 64 / 128 / 256, the length of an LDS row; KS, HT: steps of 16 and tiles of 32 that
 // cover the head size, which the products run over (the rest of a row is zeros that nothing reads); NW: waves per
 // work-group; WPS: waves per SIMD the register budget is set for.
@@ -312,21 +357,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void fmha_fwd_kernel(FmhaParams p) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_ptr)(btile + i * 1024), 16, off, 0, 0, 0);
     }
   };
-  auto bias_value = [](u32x2 w, int e) -> float {
-    const uint32_t d = w[e >> 1];
-    if constexpr (sizeof(T) == 2 && __is_same(T, __bf16)) {
-      return __builtin_bit_cast(float, (e & 1) ? (d & 0xffff0000u) : (d << 16));
-    } else {
-      return (float)__builtin_bit_cast(_Float16, (uint16_t)((e & 1) ? (d >> 16) : (d & 0xffffu)));
-    }
-  };
 
-  // ---- bias, BIAS == 1: lane g of a row fetches keys 16 g .. +15 of a half tile as two 16-byte pieces, wherever they lie (the
-  // hardware takes global loads at any address), and hands the eight keys that are the other lane's to it when they are used.
-  // Pieces may reach past a row, into the next one (those keys are masked); where that would be past the whole bias, the
-  // wave goes element by element.  (With a load for each element, waited for where it is used, the wave stood still: 4 x 15
-  // heads of 1907 x 256 fp16 2011 us against 355 so, 5 of 5413 x 40 bf16 1095 against 146, 16 of 2876 x 160 causal 680
-  // against 127.)
+  // ---- bias, BIAS == 1, a half tile ahead of its use.
   u32x4 bnext[2];
   const T* bias_row = nullptr;
   int64_t bias_after = 0;  // (uniform) elements of the bias behind key 0 of this wave's last row
@@ -336,21 +368,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fmha_fwd_kernel(FmhaParams p) {
     bias_after = ((int64_t)(p.total / p.nqb) * F - first - min(wq0 + 31, F - 1)) * Tk;
   }
   auto fetch_bias = [&](int hh) {
-    if constexpr (BIAS == 1) {
-      const T* at = bias_row + 32 * hh;
-      if (32 * hh + 32 <= bias_after) {
-        __builtin_memcpy(&bnext[0], at, 16);
-        __builtin_memcpy(&bnext[1], at + 8, 16);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          uint32_t w = 0;
-          if (32 * hh + 16 * g + 2 * j < Tk) w = __builtin_bit_cast(uint16_t, at[2 * j]);
-          if (32 * hh + 16 * g + 2 * j + 1 < Tk) w |= (uint32_t)__builtin_bit_cast(uint16_t, at[2 * j + 1]) << 16;
-          bnext[j / 4][j % 4] = w;
-        }
-      }
-    }
+    if constexpr (BIAS == 1) fetch_bias_keys(bias_row + 32 * hh, 32 * hh + 32 <= bias_after, Tk - 32 * hh - 16 * g, bnext);
   };
 
   floatx16 ot[HT];
@@ -384,24 +402,13 @@ __global__ __launch_bounds__(NW * 64, WPS) void fmha_fwd_kernel(FmhaParams p) {
     const int k0 = 32 * h;
     if constexpr (BIAS == 2) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) st[i] += bias_value(bv[i / 4], i % 4) * inv_scale;
+      for (int i = 0; i < 16; ++i) st[i] += bias_value<T>(bv[i / 4], i % 4) * inv_scale;
     }
     if constexpr (BIAS == 1) {
-      // Lane g = 0 holds keys 0-15, g = 1 keys 16-31; of each eight it uses the first (second) four.
-      uint32_t w[2][4];
+      u32x2 w[4];
+      exchange_bias_keys(bnext, w);
 #pragma unroll
-      for (int o = 0; o < 2; ++o) {
-#pragma unroll
-        for (int d = 0; d < 4; ++d) w[o][d] = bnext[o][d];
-        // (upper half of the first operand <-> lower half of the second: see row_max_exceeds)
-        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3"
-                     : "+v"(w[o][0]), "+v"(w[o][1]), "+v"(w[o][2]), "+v"(w[o][3]));
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int o = i / 4;  // eight keys 8 o .. +7
-        st[i] += bias_value(u32x2{w[o % 2][o / 2 * 2], w[o % 2][o / 2 * 2 + 1]}, i % 4) * inv_scale;
-      }
+      for (int i = 0; i < 16; ++i) st[i] += bias_value<T>(w[i / 4], i % 4) * inv_scale;
     }
     if constexpr (decltype(MASKED)::value) {
       // Most masked steps of a wave have nothing to mask (the half tile lies below the wave's rows and inside

@@ -8,6 +8,8 @@
 // Layouts, fragments and the transposed products are those of fmha_fwd_kernel.h: a lane owns one query row.
 // Pipelined kernel -> this one, back to back in a graph, f16: [2,8,64,160] x 77 keys 10.2 -> 6.6 us, [2,8,1024,80] x 77
 // 7.1 -> 5.5, [4,20,4096,64] x 77 27.4 -> 22.4 (3.8 TB/s), [1,17,777,160] x 77 with a bias 21.0 -> 9.9.
+// With a bias in 16-byte pieces ahead of the values (element by element and behind them before): 4 x 4 heads of 6446 x 40 and
+// 77 keys 18.0 -> 12.4 us, 8 x 28 of 1118 x 40 31.1 -> 20.7, 2 x 26 of 614 x 160 18.4 -> 16.0.
 #include "fmha_fwd_kernel.h"
 
 namespace fmha_fwd_impl {
@@ -30,7 +32,7 @@ __device__ __forceinline__ void send(const void* base, int rows, int H, int j, c
 }
 
 // HP: head size padded to a multiple of 32; NKT: 32-key tiles; NW: waves, 32 query rows each.
-template <typename T, int HP, int NKT, int NW, bool CAUSAL>
+template <typename T, int HP, int NKT, int NW, bool CAUSAL, bool BIAS>
 __global__ __launch_bounds__(NW * 64) void fmha_short_kernel(FmhaParams p) {
   typedef typename Elem<T>::vec8 V8;
   constexpr int ROWB = HP * 2, CPR = HP / 8, KS = HP / 16, HT = HP / 32;
@@ -59,25 +61,31 @@ __global__ __launch_bounds__(NW * 64) void fmha_short_kernel(FmhaParams p) {
 #pragma unroll
   for (int i = 0; i < (NJ + NW - 1) / NW; ++i)
     if (i * NW + wave < NJ) send<CPR, false>(K, Tk, H, i * NW + wave, k_tile);
+  const bool active = wq0 < F;  // uniform over the wave
+  // The bias of the wave's rows, sent for ahead of the values.
+  u32x4 braw[BIAS ? NKT : 1][2];
+  if constexpr (BIAS) {
+    const int64_t first = (int64_t)unit * F;
+    const int row = min(qrow, F - 1), last_row = min(wq0 + 31, F - 1);
+    const T* bp = reinterpret_cast<const T*>(p.bias) + (first + row) * Tk + 16 * g;
+    const int64_t after = ((int64_t)(p.total / p.nqb) * F - first - last_row) * Tk;  // elements behind key 0 of the last row
+    if (active) {
+#pragma unroll
+      for (int t = 0; t < NKT; ++t) fetch_bias_keys(bp + 32 * t, 32 * t + 32 <= after, Tk - 32 * t - 16 * g, braw[t]);
+    }
+    asm volatile("" ::: "memory");
+  }
 #pragma unroll
   for (int i = 0; i < (NJ + NW - 1) / NW; ++i)
     if (i * NW + wave < NJ) send<CPR, true>(V, Tk, H, i * NW + wave, v_tile);
 
-  // Bias of the lane's 16 keys per tile: key 32 t + 8 (i / 4) + 4 g + i % 4.  (Keys past the end repeat the last one;
-  // they are masked.)
-  const bool active = wq0 < F;  // uniform over the wave
   floatx16 st[NKT];
-  const float inv_scale = kLog2e / p.scale2;  // the bias is added in score units: (s + b / scale) * scale
-  if (p.bias && active) {
-    const T* bp = reinterpret_cast<const T*>(p.bias) + ((int64_t)unit * F + min(qrow, F - 1)) * Tk;
 #pragma unroll
-    for (int t = 0; t < NKT; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) st[t][i] = (float)bp[min(32 * t + 8 * (i / 4) + 4 * g + i % 4, Tk - 1)] * inv_scale;
-  } else {
-#pragma unroll
-    for (int t = 0; t < NKT; ++t) st[t] = zero16();
-  }
+  for (int t = 0; t < NKT; ++t) st[t] = zero16();
+  // (Where a wave has one key tile the zeros are written here: behind the barrier they would be in the way, 8 x 25 heads of
+  // 183 x 128 and 25 keys 6.83 us against 6.72.  With more tiles they hide behind each other's products: 8 x 28 of 6498 x 160
+  // and 77 keys 266.8 us against 270.7 with the zeros here.)
+  if constexpr (!BIAS && NKT == 1) asm volatile("" : "+v"(st[0]));
 
   // (the empty asm statements keep the compiler from moving LDS reads across)
   __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(NJ / NW));  // queries and keys have landed (a wave sent at least NJ / NW loads of V)
@@ -86,6 +94,17 @@ __global__ __launch_bounds__(NW * 64) void fmha_short_kernel(FmhaParams p) {
   V8 pf[NKT][2];
   float l_run = 0.0f, mref = 0.0f;
   if (active) {
+    // Bias of the lane's 16 keys per tile: key 32 t + 8 (i / 4) + 4 g + i % 4.  (Keys past the end are masked below.)
+    const float inv_scale = kLog2e / p.scale2;  // the bias is added in score units: (s + b / scale) * scale
+    if constexpr (BIAS) {
+#pragma unroll
+      for (int t = 0; t < NKT; ++t) {
+        u32x2 w[4];
+        exchange_bias_keys(braw[t], w);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) st[t][i] = bias_value<T>(w[i / 4], i % 4) * inv_scale;
+      }
+    }
     int kbase[KS];
 #pragma unroll
     for (int s = 0; s < KS; ++s) kbase[s] = l32 * ROWB + (((2 * s + g) ^ key_swizzle<CPR>(l32)) << 4);
@@ -182,7 +201,7 @@ __global__ __launch_bounds__(NW * 64) void fmha_short_kernel(FmhaParams p) {
   }
 }
 
-template <typename T, int HP, bool CAUSAL>
+template <typename T, int HP, bool CAUSAL, bool BIAS>
 void launch_short_hp(FmhaParams p, uint64_t units, uint32_t F, hipStream_t st) {
   const int nkt = (p.T + 31) / 32;
   // (256 x 128 keys: K, V and four waves' queries would not fit the LDS)
@@ -192,26 +211,29 @@ void launch_short_hp(FmhaParams p, uint64_t units, uint32_t F, hipStream_t st) {
   p.per_xcd = (p.total + 7) / 8;
   const dim3 grid((unsigned)(p.per_xcd * 8)), block(nw * 64);
   switch (nkt) {
-    case 1: hipLaunchKernelGGL((fmha_short_kernel<T, HP, 1, 4, CAUSAL>), grid, block, 0, st, p); break;
-    case 2: hipLaunchKernelGGL((fmha_short_kernel<T, HP, 2, 4, CAUSAL>), grid, block, 0, st, p); break;
-    case 3: hipLaunchKernelGGL((fmha_short_kernel<T, HP, 3, 4, CAUSAL>), grid, block, 0, st, p); break;
-    default: hipLaunchKernelGGL((fmha_short_kernel<T, HP, 4, (HP == 256 ? 2 : 4), CAUSAL>), grid, block, 0, st, p); break;
+    case 1: hipLaunchKernelGGL((fmha_short_kernel<T, HP, 1, 4, CAUSAL, BIAS>), grid, block, 0, st, p); break;
+    case 2: hipLaunchKernelGGL((fmha_short_kernel<T, HP, 2, 4, CAUSAL, BIAS>), grid, block, 0, st, p); break;
+    case 3: hipLaunchKernelGGL((fmha_short_kernel<T, HP, 3, 4, CAUSAL, BIAS>), grid, block, 0, st, p); break;
+    default: hipLaunchKernelGGL((fmha_short_kernel<T, HP, 4, (HP == 256 ? 2 : 4), CAUSAL, BIAS>), grid, block, 0, st, p); break;
   }
 }
 
-template <typename T, bool CAUSAL>
+template <typename T, bool CAUSAL, bool BIAS>
 void launch_short_t(const FmhaParams& p, uint64_t units, uint32_t F, hipStream_t st) {
-  if (p.H <= 64) launch_short_hp<T, 64, CAUSAL>(p, units, F, st);
-  else if (p.H <= 96) launch_short_hp<T, 96, CAUSAL>(p, units, F, st);
-  else if (p.H <= 128) launch_short_hp<T, 128, CAUSAL>(p, units, F, st);
-  else if (p.H <= 160) launch_short_hp<T, 160, CAUSAL>(p, units, F, st);
-  else launch_short_hp<T, 256, CAUSAL>(p, units, F, st);
+  if (p.H <= 64) launch_short_hp<T, 64, CAUSAL, BIAS>(p, units, F, st);
+  else if (p.H <= 96) launch_short_hp<T, 96, CAUSAL, BIAS>(p, units, F, st);
+  else if (p.H <= 128) launch_short_hp<T, 128, CAUSAL, BIAS>(p, units, F, st);
+  else if (p.H <= 160) launch_short_hp<T, 160, CAUSAL, BIAS>(p, units, F, st);
+  else launch_short_hp<T, 256, CAUSAL, BIAS>(p, units, F, st);
 }
 
 template <typename T>
 void launch_short_t(const FmhaParams& p, uint64_t units, uint32_t F, bool causal, hipStream_t st) {
-  if (causal) launch_short_t<T, true>(p, units, F, st);
-  else launch_short_t<T, false>(p, units, F, st);
+  // (Forms of their own with and without a bias: one form with a branch took 1 to 3 % longer without.)
+  if (p.bias && causal) launch_short_t<T, true, true>(p, units, F, st);
+  else if (p.bias) launch_short_t<T, false, true>(p, units, F, st);
+  else if (causal) launch_short_t<T, true, false>(p, units, F, st);
+  else launch_short_t<T, false, false>(p, units, F, st);
 }
 
 }  // namespace
