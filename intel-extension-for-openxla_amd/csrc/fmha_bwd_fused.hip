@@ -97,7 +97,8 @@ struct KParams {
   float scale;
 };
 
-// T: element type; HP: head size padded to 64, 128 or 256 (one wave per SIMD at 256); OWNER_K: the work-group owns keys (else queries).
+// T: element type; HC: the head size that the products cover, 64, 96, 128, 160 or 256; HP: padded to 64, 128 or 256, the length
+// of an LDS row (one wave per SIMD at 256); OWNER_K: the work-group owns keys (else queries).
 // DS: accumulate out1 from dS (dK or dQ); PV: accumulate out2 from P (dV, owner = keys).  The
 // keys-own work is run as two launches, one per output: with both accumulator sets and both owner
 // operands a wave needs more than half the register file, and one wave per SIMD cannot overlap its
@@ -131,14 +132,16 @@ inline size_t ds_unit_bytes(int F, int T, bool causal) {
   return (size_t)ds_before((F + BO - 1) / BO, ds_key_blocks(T), causal) * DS_TILE;
 }
 
+constexpr int padded(int HC) { return HC <= 64 ? 64 : HC <= 128 ? 128 : 256; }
 constexpr int bwd_lds_bytes(int HP) { return 4 * BS * HP * 2 + 2 * (2 * BS * 4); }
-template <typename T, int HP, bool OWNER_K, bool CAUSAL, bool DS, bool PV, bool BIAS, bool STATS_IN, bool SAVE_DS>
+template <typename T, int HC, bool OWNER_K, bool CAUSAL, bool DS, bool PV, bool BIAS, bool STATS_IN, bool SAVE_DS>
 __device__ __forceinline__ void bwd_pass(const KParams& p, char* lds, int block_id) {
   static_assert(DS || PV, "nothing to compute");
   static_assert(!SAVE_DS || !OWNER_K, "the queries-own pass saves dS");
   static_assert(!PV || OWNER_K, "P^T dO belongs to the keys-own pass");
   typedef typename Elem<T>::vec8 V8;
   constexpr int NW = 4;
+  constexpr int HP = padded(HC);
   constexpr int ROWB = HP * 2;               // bytes of one tile row in LDS
   constexpr int CPR = ROWB / 16;             // 16-byte chunks per row
   constexpr int KMASK = 15;                  // the swizzle repeats every KMASK + 1 rows
@@ -147,8 +150,8 @@ __device__ __forceinline__ void bwd_pass(const KParams& p, char* lds, int block_
   constexpr int NL = TILE / 1024 / NW;       // loads per wave per tile
   constexpr int LROWS = NW * RPL;            // tile rows between consecutive loads of a wave
   constexpr int KV = (LROWS % (KMASK + 1) == 0) ? 1 : 2;  // distinct swizzles among a wave's loads
-  constexpr int KS = HP / 16;                // k-steps of the score products
-  constexpr int HT = HP / 32;                // 32-wide h tiles of the gradients
+  constexpr int KS = HC / 16;                // k-steps of the score products
+  constexpr int HT = HC / 32;                // 32-wide h tiles of the gradients
   constexpr int STATS = 2 * BS * 4;          // LSE and D of one block's 64 query rows (owner = keys)
   static_assert(NL >= 1 && LROWS % 8 == 0 && (2 * LROWS) % (KMASK + 1) == 0, "tile / wave split");
   static_assert(bwd_lds_bytes(HP) == 4 * TILE + 2 * STATS, "what the kernels below reserve");
@@ -564,15 +567,16 @@ template <int HP, bool PV> struct SavedLds {
   static constexpr int TILE = SBS * HP * 2, DSB = BO * SBS * 2, STAT = PV ? 4 * 256 : 0;
   static constexpr int STAGE = (PV ? 2 : 1) * TILE + DSB + STAT, ALL = 3 * STAGE;
 };
-template <typename T, int HP, bool CAUSAL, bool PV>
+template <typename T, int HC, bool CAUSAL, bool PV>
 __device__ __forceinline__ void bwd_saved_pass(const KParams& p, char* lds, int block_id) {
   typedef typename Elem<T>::vec8 V8;
+  constexpr int HP = padded(HC);
   typedef SavedLds<HP, PV> L;
   constexpr int NW = 4;
   constexpr int ROWB = HP * 2, CPR = ROWB / 16, RPL = 1024 / ROWB, LROWS = NW * RPL;
   constexpr int NL = L::TILE / 1024 / NW;  // loads per wave per tile
   constexpr int KV = (LROWS % 16 == 0) ? 1 : 2;
-  constexpr int KS = HP / 16, HT = HP / 32;
+  constexpr int KS = HC / 16, HT = HC / 32;
   constexpr int LOADS = NL * (PV ? 2 : 1) + 2 + (PV ? 1 : 0);  // loads per wave per block
   static_assert(NL >= 1 && L::DSB == NW * 2 * 1024, "tile / wave split");
   static_assert(!PV || BO * ROWB <= L::ALL, "the owner rows are staged in the stages");
@@ -780,29 +784,29 @@ __device__ __forceinline__ void bwd_saved_pass(const KParams& p, char* lds, int 
   if constexpr (PV) store(p.out2, acc2, 1.0f);
 }
 
-template <typename T, int HP, bool CAUSAL, bool PV>
+template <typename T, int HC, bool CAUSAL, bool PV>
 __global__ __launch_bounds__(256, 2) void fmha_bwd_saved_kernel(KParams p) {
-  __shared__ __attribute__((aligned(1024))) char lds[SavedLds<HP, PV>::ALL];
-  bwd_saved_pass<T, HP, CAUSAL, PV>(p, lds, (int)blockIdx.x);
+  __shared__ __attribute__((aligned(1024))) char lds[SavedLds<padded(HC), PV>::ALL];
+  bwd_saved_pass<T, HC, CAUSAL, PV>(p, lds, (int)blockIdx.x);
 }
 
-template <typename T, int HP, bool OWNER_K, bool CAUSAL, bool DS, bool PV, bool BIAS, bool SAVE_DS>
-__global__ __launch_bounds__(256, (HP <= 128 && !BIAS && !(DS && PV && HP > 64)) ? 2 : 1) void fmha_bwd_kernel(KParams p) {
-  __shared__ __attribute__((aligned(1024))) char lds[bwd_lds_bytes(HP)];
-  bwd_pass<T, HP, OWNER_K, CAUSAL, DS, PV, BIAS, false, SAVE_DS>(p, lds, (int)blockIdx.x);
+template <typename T, int HC, bool OWNER_K, bool CAUSAL, bool DS, bool PV, bool BIAS, bool SAVE_DS>
+__global__ __launch_bounds__(256, (HC <= 128 && !BIAS && !(DS && PV && HC > 64)) ? 2 : 1) void fmha_bwd_kernel(KParams p) {
+  __shared__ __attribute__((aligned(1024))) char lds[bwd_lds_bytes(padded(HC))];
+  bwd_pass<T, HC, OWNER_K, CAUSAL, DS, PV, BIAS, false, SAVE_DS>(p, lds, (int)blockIdx.x);
 }
 
 // All passes in one grid, a row of it each, on statistics formed before: for problems of which a single pass leaves the
 // device idle.  What bounds those is the walk of one work-group over the streamed rows (2 us per 64 rows, one wave per
 // SIMD), once per launch: [2,7,463,128] causal took three of them.
-template <typename T, int HP, bool CAUSAL>
-__global__ __launch_bounds__(256, HP <= 128 ? 2 : 1) void fmha_bwd_small_kernel(KParams dq, KParams dk, KParams dv) {
-  __shared__ __attribute__((aligned(1024))) char lds[bwd_lds_bytes(HP)];
+template <typename T, int HC, bool CAUSAL>
+__global__ __launch_bounds__(256, HC <= 128 ? 2 : 1) void fmha_bwd_small_kernel(KParams dq, KParams dk, KParams dv) {
+  __shared__ __attribute__((aligned(1024))) char lds[bwd_lds_bytes(padded(HC))];
   const int block = (int)blockIdx.x;
-  if (blockIdx.y == 0) bwd_pass<T, HP, false, CAUSAL, true, false, false, true, false>(dq, lds, block);
-  else if constexpr (HP <= 64) bwd_pass<T, HP, true, CAUSAL, true, true, false, true, false>(dk, lds, block);
-  else if (blockIdx.y == 1) bwd_pass<T, HP, true, CAUSAL, true, false, false, true, false>(dk, lds, block);
-  else bwd_pass<T, HP, true, CAUSAL, false, true, false, true, false>(dv, lds, block);
+  if (blockIdx.y == 0) bwd_pass<T, HC, false, CAUSAL, true, false, false, true, false>(dq, lds, block);
+  else if constexpr (HC <= 64) bwd_pass<T, HC, true, CAUSAL, true, true, false, true, false>(dk, lds, block);
+  else if (blockIdx.y == 1) bwd_pass<T, HC, true, CAUSAL, true, false, false, true, false>(dk, lds, block);
+  else bwd_pass<T, HC, true, CAUSAL, false, true, false, true, false>(dv, lds, block);
 }
 
 void split(KParams& p, int n_own, uint64_t units) {
@@ -812,16 +816,16 @@ void split(KParams& p, int n_own, uint64_t units) {
   p.ug = std::max(4, (64 + p.nob - 1) / p.nob);  // enough units to fill an XCD's slots with one round
 }
 
-template <typename T, int HP, bool OWNER_K, bool DS, bool PV>
+template <typename T, int HC, bool OWNER_K, bool DS, bool PV>
 void launch_pass(KParams p, uint64_t units, bool causal, hipStream_t st) {
   split(p, OWNER_K ? p.T : p.F, units);
   const dim3 grid((unsigned)(p.per_xcd * 8)), block(256);
   if (p.bias) {
-    if (causal) hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, true, DS, PV, true, false>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, false, DS, PV, true, false>), grid, block, 0, st, p);
+    if (causal) hipLaunchKernelGGL((fmha_bwd_kernel<T, HC, OWNER_K, true, DS, PV, true, false>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((fmha_bwd_kernel<T, HC, OWNER_K, false, DS, PV, true, false>), grid, block, 0, st, p);
   } else {
-    if (causal) hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, true, DS, PV, false, false>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, OWNER_K, false, DS, PV, false, false>), grid, block, 0, st, p);
+    if (causal) hipLaunchKernelGGL((fmha_bwd_kernel<T, HC, OWNER_K, true, DS, PV, false, false>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((fmha_bwd_kernel<T, HC, OWNER_K, false, DS, PV, false, false>), grid, block, 0, st, p);
   }
 }
 
@@ -838,17 +842,17 @@ KParams at_unit(KParams p, uint64_t u0, bool owner_k) {
 }
 
 // dQ and dS (kept), then dK and dV from it; with heads of more than 128 dV has its own pass, as its accumulators need.
-template <typename T, int HP, bool CAUSAL>
+template <typename T, int HC, bool CAUSAL>
 void launch_saved(KParams p, KParams kv, uint64_t units, hipStream_t st) {
   split(p, p.F, units);
   split(kv, kv.T, units);
   const dim3 block(256);
-  hipLaunchKernelGGL((fmha_bwd_kernel<T, HP, false, CAUSAL, true, false, false, true>), dim3((unsigned)(p.per_xcd * 8)), block, 0, st, p);
-  hipLaunchKernelGGL((fmha_bwd_saved_kernel<T, HP, CAUSAL, (HP <= 128)>), dim3((unsigned)(kv.per_xcd * 8)), block, 0, st, kv);
-  if constexpr (HP > 128) launch_pass<T, HP, true, false, true>(kv, units, CAUSAL, st);
+  hipLaunchKernelGGL((fmha_bwd_kernel<T, HC, false, CAUSAL, true, false, false, true>), dim3((unsigned)(p.per_xcd * 8)), block, 0, st, p);
+  hipLaunchKernelGGL((fmha_bwd_saved_kernel<T, HC, CAUSAL, (HC <= 128)>), dim3((unsigned)(kv.per_xcd * 8)), block, 0, st, kv);
+  if constexpr (HC > 128) launch_pass<T, HC, true, false, true>(kv, units, CAUSAL, st);
 }
 
-template <typename T, int HP>
+template <typename T, int HC>
 void launch_both(const fmha_bwd_fused::Args& a, uint64_t units, hipStream_t st) {
   KParams p;
   p.lse = a.lse; p.dsum = a.dsum; p.o = a.o; p.lse_fwd = a.lse_fwd; p.H = a.H; p.F = a.F; p.T = a.T; p.scale = a.scale;
@@ -859,34 +863,36 @@ void launch_both(const fmha_bwd_fused::Args& a, uint64_t units, hipStream_t st) 
   p.own1 = a.q; p.own2 = a.d_o; p.strm1 = a.k; p.strm2 = a.v; p.out1 = a.dq; p.out2 = nullptr;
   KParams k = p;
   k.own1 = a.k; k.own2 = a.v; k.strm1 = a.q; k.strm2 = a.d_o; k.out1 = a.dk; k.out2 = a.dv;
-  if constexpr (HP > 64) if (a.ds) {
+  if constexpr (HC > 64) if (a.ds) {
     for (uint64_t u0 = 0; u0 < units; u0 += a.ds_units) {
       const uint64_t n = std::min<uint64_t>(a.ds_units, units - u0);
-      if (a.causal) launch_saved<T, HP, true>(at_unit(p, u0, false), at_unit(k, u0, true), n, st);
-      else launch_saved<T, HP, false>(at_unit(p, u0, false), at_unit(k, u0, true), n, st);
+      if (a.causal) launch_saved<T, HC, true>(at_unit(p, u0, false), at_unit(k, u0, true), n, st);
+      else launch_saved<T, HC, false>(at_unit(p, u0, false), at_unit(k, u0, true), n, st);
     }
     return;
   }
   if (a.stats_ready) {
     split(p, a.F, units);
     split(k, a.T, units);
-    const dim3 grid((unsigned)(std::max(p.per_xcd, k.per_xcd) * 8), HP <= 64 ? 2 : 3), block(256);
-    if (a.causal) hipLaunchKernelGGL((fmha_bwd_small_kernel<T, HP, true>), grid, block, 0, st, p, k, k);
-    else hipLaunchKernelGGL((fmha_bwd_small_kernel<T, HP, false>), grid, block, 0, st, p, k, k);
+    const dim3 grid((unsigned)(std::max(p.per_xcd, k.per_xcd) * 8), HC <= 64 ? 2 : 3), block(256);
+    if (a.causal) hipLaunchKernelGGL((fmha_bwd_small_kernel<T, HC, true>), grid, block, 0, st, p, k, k);
+    else hipLaunchKernelGGL((fmha_bwd_small_kernel<T, HC, false>), grid, block, 0, st, p, k, k);
     return;
   }
   // owner = queries first: dQ, and the per-row statistics the other launches read
-  launch_pass<T, HP, false, true, false>(p, units, a.causal, st);
+  launch_pass<T, HC, false, true, false>(p, units, a.causal, st);
   // owner = keys: dK, then dV
   // One pass for both where the two accumulators fit beside everything else (S is then computed once for the
   // two): head size <= 64 (S = 4096, H = 64 causal: 0.69 -> 0.57 ms), and head size <= 128 with a bias, whose
   // kernels run one wave per SIMD anyway (6.2 -> 5.3 ms).  Without a bias the merged H = 128 pass would have to
   // give up the second wave per SIMD and comes out 2-4 % slower; at H = 256 it spills.
-  if (HP <= 64 || (HP <= 128 && a.bias)) {
-    launch_pass<T, HP, true, true, true>(k, units, a.causal, st);
-  } else {
-    launch_pass<T, HP, true, true, false>(k, units, a.causal, st);
-    launch_pass<T, HP, true, false, true>(k, units, a.causal, st);
+  if constexpr (HC <= 128) if (HC <= 64 || a.bias) {
+    launch_pass<T, HC, true, true, true>(k, units, a.causal, st);
+    return;
+  }
+  if constexpr (HC > 64) {
+    launch_pass<T, HC, true, true, false>(k, units, a.causal, st);
+    launch_pass<T, HC, true, false, true>(k, units, a.causal, st);
   }
 }
 
@@ -931,13 +937,19 @@ uint64_t saved_units(const Args& a, uint64_t units, uint64_t bytes) {
 size_t saved_bytes(const Args& a, uint64_t units) { return units * ds_unit_bytes(a.F, a.T, a.causal); }
 
 void launch(const Args& a, uint64_t units, bool bf16, hipStream_t st) {
+  // The products run over the head's own steps of 16 and tiles of 32; of 96 and 160 instead of 128 and 256 (us, both in one
+  // grid): 13 causal heads of 524 x 80 26.9 -> 23.0, 36 of 753 x 80 53.7 -> 42.1, 16 of 1024 x 160 127 -> 91, 8 of 256 x 160 26 -> 20.
   if (bf16) {
     if (a.H <= 64) launch_both<__bf16, 64>(a, units, st);
+    else if (a.H <= 96) launch_both<__bf16, 96>(a, units, st);
     else if (a.H <= 128) launch_both<__bf16, 128>(a, units, st);
+    else if (a.H <= 160) launch_both<__bf16, 160>(a, units, st);
     else launch_both<__bf16, 256>(a, units, st);
   } else {
     if (a.H <= 64) launch_both<_Float16, 64>(a, units, st);
+    else if (a.H <= 96) launch_both<_Float16, 96>(a, units, st);
     else if (a.H <= 128) launch_both<_Float16, 128>(a, units, st);
+    else if (a.H <= 160) launch_both<_Float16, 160>(a, units, st);
     else launch_both<_Float16, 256>(a, units, st);
   }
 }

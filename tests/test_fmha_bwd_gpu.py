@@ -184,3 +184,19 @@ def test_backward_with_kept_score_gradients(xmk, name, causal, B, N, F, T, H, pa
         a, b = a.float(), b.float()
         diff, size = (a - b).norm().item(), a.norm().item()
         assert torch.isfinite(b).all() and (diff <= ulp * size or diff <= 1e-5 * a.numel() ** 0.5), (nm, diff, size)
+
+
+@pytest.mark.parametrize("causal,use_bias", [(False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("name,B,N,F,T,H", [
+    ("bf16", 1, 3, 130, 203, 72), ("fp16", 1, 3, 203, 130, 96), ("fp16", 1, 3, 97, 257, 136), ("bf16", 1, 3, 257, 97, 160), ("fp16", 1, 2, 130, 131, 168),
+    ("bf16", 29, 9, 33, 65, 96), ("fp16", 29, 9, 65, 33, 160),  # dS kept
+])
+def test_backward_head_size_classes(xmk, oracle, name, causal, use_bias, B, N, F, T, H):
+    """Classes of head sizes at their last size and just past the one below, ragged in F and T, in one grid, with dS kept and
+    (with a bias) in launches of their own."""
+    _run(xmk, oracle, name, B, N, F, T, H, causal, use_bias, seed=9)
+
+
+@pytest.mark.parametrize("B,N,F,T,H", [(29, 9, 33, 65, 160), (9, 17, 257, 130, 136), (130, 4, 64, 33, 96)])
+def test_backward_with_kept_score_gradients_head_size_classes(xmk, B, N, F, T, H):
+    test_backward_with_kept_score_gradients(xmk, "bf16", True, B, N, F, T, H, 1)
