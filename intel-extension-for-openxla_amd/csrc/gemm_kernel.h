@@ -503,7 +503,10 @@ __device__ __forceinline__ uint32_t xcd_run(uint32_t block, uint32_t n, int K) {
 __device__ __forceinline__ TileAt tile_at(int block, int tiles_m, int tiles_n, int K) {
   const uint32_t n = (uint32_t)(tiles_m * tiles_n), pid = xcd_run((uint32_t)block, n, K), run = (n + 7) >> 3;
   int shift = run >= 24 ? 3 : run >= 6 ? 2 : run >= 2 ? 1 : 0;
-  if ((tiles_m & (tiles_m - 1)) == 0) shift = min(shift, __builtin_ctz(tiles_m));  // (all rows, without the division below)
+  if ((tiles_m & (tiles_m - 1)) == 0) {
+    shift = min(shift, __builtin_ctz(tiles_m));
+    if (tiles_m >> shift == 1) return {(int)pid & (tiles_m - 1), (int)(pid >> shift)};  // all rows at once: nothing to divide
+  }
   const int first_m = (int)(pid / (uint32_t)tiles_n) >> shift << shift, at = (int)pid - first_m * tiles_n;
   const int height = tiles_m - first_m;
   if (height >> shift) return {first_m + (at & ((1 << shift) - 1)), at >> shift};
