@@ -1,9 +1,9 @@
-// Host entry point of the fused multi-head attention forward and the head-size classes up to 128.
+// Host entry point of the fused multi-head attention forward and the head-size classes up to 64 and up to 128.
 // This translation unit is compiled with the matrix instructions in their VGPR form
 // (-mllvm -amdgpu-mfma-vgpr-form, set per file in build.py): the S accumulators are then read by the
 // softmax's vector instructions where the matrix cores wrote them, with no copies between register
-// files.  The class for head sizes above 128 needs both halves of the register file and lives in
-// fmha_fwd_h256.hip.
+// files.  The class for head sizes above 160 needs both halves of the register file and lives in
+// fmha_fwd_h256.hip; fmha_fwd_h48 / h80 / h96 / h160.hip hold the classes in between, compiled as this one.
 #include "fmha_fwd_kernel.h"
 
 namespace fmha_fwd_impl {
@@ -11,7 +11,11 @@ namespace {
 
 template <typename T>
 void launch_t(const FmhaParams& p, int32_t dtype, uint64_t units, uint32_t F, bool causal, int bias, hipStream_t st) {
-  // Head-size classes of the reference's policy choice (fmha_forward.h:622-646).  Four waves of 32
+  // Head-size classes of the reference's policy choice (fmha_forward.h:622-646), and between them 48, 80, 96 and 160: rows in
+  // LDS as in the next class, products over the steps of 16 and tiles of 32 that the head has.  What bounds the kernel is the
+  // products' rate, and heads of 40, 80 and 160 ran those of 64, 128 and 256: 15 heads of 6475 x 160 causal 460 -> 348 us, 16 of
+  // 2757 x 80 58 -> 49, 64 of 2750 x 40 141 -> 136; 50 drawn sizes with such heads 12 % on average, none slower.
+  // Four waves of 32
   // query rows, two work-groups per CU.  Measured against it on [8,32,2048,128] with the current step:
   // eight waves per work-group (half the K / V loads per row) 1020 against 1032 TFLOP/s; a second
   // 32-row tile per wave (one wave per SIMD, O in AGPRs, every K / V fragment feeding two matrix

@@ -490,7 +490,9 @@ __device__ __forceinline__ void store_tile(Epilogue& epi, const floatx16 (&acc)[
 // run of tiles, and a run walks the tiles in groups of some tile rows, so that it uses few rows of A and columns of B: about
 // as many of the one as of the other, up to eight rows.  Microseconds against runs only where the tiles divide by eight, always
 // in eight rows: 85 x 4001 x 2231 19.2 -> 12.5, 141 x 1280 x 7168 17.1 -> 13.6, 811 x 3488 x 4144 50 -> 40, 2244 x 9235 x 13131
-// 1077 -> 1017; 80 drawn sizes of 20 rows and more 4 % on average, the worst 4 % slower (short reductions).
+// 1077 -> 1017; 80 drawn sizes of 20 rows and more 4 % on average, 110 with k of 129 to 1300 3 %.  The worst are tall outputs
+// of few tile columns, where the plain order happened to give an XCD whole tile rows: 3148 x 352 x 888 8.3 -> 9.0, 3306 x 576 x 576
+// 7.3 -> 7.6.  (Row by row where a run spans two rows and more: those 4 % back, 7539 x 197 x 1649 22.4 -> 25.2.)
 // With k of 128 or less it is the output that takes the time, and neighbours on different XCDs write it faster (4305 x 12736 x 64
 // 46.0 against 44.5).
 struct TileAt {
