@@ -632,11 +632,14 @@ __device__ __forceinline__ void bwd_saved_pass(const KParams& p, char* lds, int 
     const int rb = it / (BO / SBS);
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(
         ds_unit + (int64_t)DS_TILE * (ds_before(rb, nkb, CAUSAL) + (int64_t)(it % (BO / SBS)) * ds_width(rb, nkb, CAUSAL) + ob * (BO / BS)),
-        it < b1 ? (uint32_t)L::DSB : 0u);
+        (uint32_t)L::DSB);
+    // (Past the end the lanes' offsets turn the loads off, not a buffer of no bytes: they are out of range whether the check adds
+    // the scalar offset, leaves it out or takes it from the buffer's size, which must then not be the smaller of the two.)
+    const uint32_t off = it < b1 ? (uint32_t)(lane * 16) : kOob;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_ptr)(d + (i * NW + wave) * 1024), 16, (uint32_t)(lane * 16),
-                                               (i * NW + wave) * 1024, 0, kNonTemporal);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_ptr)(d + (i * NW + wave) * 1024), 16, off, (i * NW + wave) * 1024, 0,
+                                               kNonTemporal);
     if constexpr (PV) {  // each wave its own copy: 32 floats (the other lanes' 32 are not used)
       const __amdgpu_buffer_rsrc_t rl = make_rsrc(lse, (uint32_t)p.F * 4);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rl, (lds_void_ptr)(d + L::DSB + wave * 256), 4, (uint32_t)((it * SBS + lane) * 4), 0, 0, 0);

@@ -151,6 +151,8 @@ def test_backward_on_a_side_stream(xmk):
 @pytest.mark.parametrize("B,N,F,T,H,parts", [
     (10, 16, 130, 257, 128, 1), (13, 16, 257, 130, 80, 1), (29, 9, 33, 65, 256, 1), (12, 11, 129, 1, 200, 1), (130, 4, 1, 64, 72, 1),
     (57, 47, 100, 96, 128, 2),
+    # whole query blocks: the loads past a unit's last one, and past the last unit's, start where the workspace ends
+    (10, 16, 256, 256, 128, 1), (17, 16, 128, 128, 96, 1), (29, 9, 128, 65, 256, 1), (57, 47, 128, 96, 128, 2),
 ])
 def test_backward_with_kept_score_gradients(xmk, name, causal, B, N, F, T, H, parts):
     """dS kept in the workspace (all units at once, or as many as a smaller workspace holds) against a call with the least
