@@ -491,6 +491,12 @@ __device__ __forceinline__ void bwd_pass(const KParams& p, char* lds, int block_
       else elementwise(std::false_type{}, i0{}, i2{});
     }
     if constexpr (SAVE_DS) {
+      // Rows past the last query hold what zeros make of the keys, which is NaN where a key holds an infinity or a NaN; the pass
+      // that reads dS adds it, times zero, to that key's gradient.
+      if (wo0 + 31 >= p.F) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) df[u] = orow < p.F ? df[u] : V8{};
+      }
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, df[u]), ds_rsrc, ds_lane,

@@ -188,6 +188,29 @@ def test_backward_with_kept_score_gradients(xmk, name, causal, B, N, F, T, H, pa
         assert torch.isfinite(b).all() and (diff <= ulp * size or diff <= 1e-5 * a.numel() ** 0.5), (nm, diff, size)
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,N,F,T,H", [(29, 9, 33, 65, 128), (29, 9, 100, 257, 80), (29, 9, 33, 65, 256)])
+def test_backward_infinite_key_without_weight(xmk, causal, B, N, F, T, H):
+    """A key with an infinity that no query gives any weight (behind the last query of a causal call, or a score of minus
+    infinity for every query) has gradients of zero, also where dS is kept and the last tile of queries is not full."""
+    import ctypes as C
+    L = xmk.lib()
+    u = [C.c_uint32(x) for x in (B, N, H, F, T)]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(7)
+    q, d_o = (torch.randn((B, N, F, H), generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    k, v = (torch.randn((B, N, T, H), generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    key = T - 3
+    q[..., 5] = q[..., 5].abs() + 0.5
+    k[:, :, key, 5] = float("inf") if causal else float("-inf")
+    out, lse = torch.empty_like(q), torch.empty((B * N, F), device="cuda")
+    xmk.fmha_forward(q, k, v, out, lse=lse, causal=causal)
+    assert L.xmk_fmha_bwd_best_workspace_bytes(*u, C.c_int32(causal)) > L.xmk_fmha_bwd_workspace_bytes(*u)
+    _, dk, dv = xmk.fmha_backward(q, k, v, out, d_o, lse, causal=causal)
+    assert torch.isfinite(out).all() and torch.isfinite(dk).all() and torch.isfinite(dv).all()
+    assert not dk[:, :, key].any() and not dv[:, :, key].any()
+
+
 @pytest.mark.parametrize("causal,use_bias", [(False, False), (True, False), (True, True)])
 @pytest.mark.parametrize("name,B,N,F,T,H", [
     ("bf16", 1, 3, 130, 203, 72), ("fp16", 1, 3, 203, 130, 96), ("fp16", 1, 3, 97, 257, 136), ("bf16", 1, 3, 257, 97, 160), ("fp16", 1, 2, 130, 131, 168),
