@@ -413,6 +413,7 @@ bool plan_pack(const xmk_gemm_desc* d, PackPlan* p) {
   if (m <= 0 || n <= 0 || k <= 0 || m >= kMax || n >= kMax || k >= kMax || m * k >= kMax || n * k >= kMax) return false;
   p->a = !ok(d->lhs);
   p->b = !ok(d->rhs);
+  if (!p->a && !p->b) return false;  // (only a batch stride, of a single member, is no multiple of eight)
   p->lda = ld(d->lhs);
   p->ldb = ld(d->rhs);
   p->b_at = p->a ? (size_t)m * p->lda * 2 : 0;
@@ -427,8 +428,9 @@ bool plan_pack(const xmk_gemm_desc* d, PackPlan* p) {
 // The descriptor with the copies at `ws` in place of the operands.
 xmk_gemm_desc packed_desc(const xmk_gemm_desc* d, const PackPlan& p, char* ws) {
   xmk_gemm_desc q = *d;
-  if (p.a) { q.lhs.data = ws; q.lhs.leading_dim_stride = p.lda; q.lhs.batch_stride = 0; }
-  if (p.b) { q.rhs.data = ws + p.b_at; q.rhs.leading_dim_stride = p.ldb; q.rhs.batch_stride = 0; }
+  q.lhs.batch_stride = q.rhs.batch_stride = 0;  // (one member: nothing is a stride away from it)
+  if (p.a) { q.lhs.data = ws; q.lhs.leading_dim_stride = p.lda; }
+  if (p.b) { q.rhs.data = ws + p.b_at; q.rhs.leading_dim_stride = p.ldb; }
   return q;
 }
 PackOperand pack_operand(const xmk_matrix& x, void* to, int64_t ld) {
