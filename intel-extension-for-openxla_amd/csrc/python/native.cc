@@ -12,6 +12,8 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 #include <torch/csrc/Dtype.h>
@@ -233,6 +235,31 @@ XMK_PY(fmha_forward) {
   });
 }
 
+// Whether `bytes` of scratch that a call can do without are to be asked for: the allocator holds that much in whole unused
+// segments, or the device has twice as much left.  A request that fails is no answer to that: torch then gives back every cached block and waits for the
+// device, in each such call of a program whose memory is nearly full.  Under stream capture nothing is queried (the memory is the
+// graph's, and asked for once).
+bool spare_memory(const at::Tensor& like, int64_t bytes, void* st) {
+  if (!like.is_cuda()) return false;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)st, &capture) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (capture != hipStreamCaptureStatusNone) return true;
+  try {
+    const auto stats = c10::hip::HIPCachingAllocator::getDeviceStats(like.get_device());
+    auto now = [](const c10::CachingDeviceAllocator::StatArray& of) { return of[0].current; };  // (0: all pools)
+    if (now(stats.reserved_bytes) - now(stats.active_bytes) - now(stats.inactive_split_bytes) >= bytes) return true;
+  } catch (const c10::Error&) {  // an allocator of the program's own, which keeps no such count
+  }
+  const c10::DeviceGuard on(like.device());
+  size_t left = 0, total = 0;
+  if (hipMemGetInfo(&left, &total) == hipSuccess) return left / 2 >= (size_t)bytes;
+  (void)hipGetLastError();
+  return false;
+}
+
 // (query, key, value, out, grad_out, lse, bias, head_scale, causal, stream) -> (dq, dk, dv), or the status code
 XMK_PY(fmha_backward) {
   return guarded([&]() -> PyObject* {
@@ -242,19 +269,20 @@ XMK_PY(fmha_backward) {
     void *o = data(tensor(a[3])), *d_o = data(tensor(a[4])), *lse = data(tensor(a[5])), *bias = data_or_null(a[6]);
     const int32_t dt = dtype_code(q), causal = truth(a[8]);
     void* st = stream(a[9]);
-    // Where memory is short, the least that the call takes.
-    const size_t least = api.xmk_fmha_bwd_workspace_bytes(s.b, s.n, s.h, s.f, s.t);
-    size_t bytes = bias ? least : api.xmk_fmha_bwd_best_workspace_bytes(s.b, s.n, s.h, s.f, s.t, causal);
-    auto scratch = [&] { return at::empty({(int64_t)(bytes > 256 ? bytes : 256)}, q.options().dtype(at::kByte)); };
-    at::Tensor ws;
-    try {
-      ws = scratch();
-    } catch (const c10::OutOfMemoryError&) {
-      if (bytes == least) throw;
-      bytes = least;
-      ws = scratch();
-    }
+    // The gradients first: what the call can do without must not take their memory.  Where memory is short, the least scratch.
     const at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+    size_t bytes = api.xmk_fmha_bwd_workspace_bytes(s.b, s.n, s.h, s.f, s.t);
+    const size_t best = bias ? bytes : api.xmk_fmha_bwd_best_workspace_bytes(s.b, s.n, s.h, s.f, s.t, causal);
+    auto scratch = [&](size_t size) { return at::empty({(int64_t)(size > 256 ? size : 256)}, q.options().dtype(at::kByte)); };
+    at::Tensor ws;
+    if (best > bytes && spare_memory(q, (int64_t)best, st)) {
+      try {
+        ws = scratch(best);
+        bytes = best;
+      } catch (const c10::OutOfMemoryError&) {
+      }
+    }
+    if (!ws.defined()) ws = scratch(bytes);
     const int rc = unlocked([&] {
       return api.xmk_fmha_bwd(data(q), data(k), data(v), bias, o, d_o, (const float*)lse, data(dq), data(dk), data(dv), dt, s.b,
                               s.n, s.h, s.f, s.t, s.scale, causal, data(ws), bytes, st);

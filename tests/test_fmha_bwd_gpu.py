@@ -188,6 +188,45 @@ def test_backward_with_kept_score_gradients(xmk, name, causal, B, N, F, T, H, pa
         assert torch.isfinite(b).all() and (diff <= ulp * size or diff <= 1e-5 * a.numel() ** 0.5), (nm, diff, size)
 
 
+def _rows_agree(nm, a, b, ulp):
+    """Two ways to the same sums of products of factors that are rounded alike.  Each result is rounded once (one spacing of it,
+    `ulp` of its size at most), and a few of the rounded factors may fall on the other side of a rounding boundary (less than as
+    much again); what remains of a row whose exact gradients cancel is the noise of 32-bit sums."""
+    a, b = a.float(), b.float()
+    diff, size = (a - b).norm(dim=-1), a.norm(dim=-1)
+    assert torch.isfinite(b).all(), nm
+    over = diff - 2 * ulp * size - 1e-5 * a.shape[-1] ** 0.5
+    at = int(over.argmax())
+    assert over.max().item() <= 0, (nm, at, diff.flatten()[at].item(), size.flatten()[at].item())
+
+
+def test_backward_where_memory_is_short(xmk):
+    """The scratch that keeps dS (80 MiB here) is one the call can do without: where there is room for it or for the gradients
+    (30 MiB) but not for both, the call runs with the least scratch."""
+    B, N, S, H = 1, 40, 1024, 128
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    q, k, v, d_o = (torch.randn((B, N, S, H), generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(4))
+    out, lse = torch.empty_like(q), torch.empty((B * N, S), device="cuda")
+    xmk.fmha_forward(q, k, v, out, lse=lse)
+    want = xmk.fmha_backward(q, k, v, out, d_o, lse)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    room = (S * S * 2 * N) + (8 << 20)
+    before = torch.cuda.memory_reserved()
+    torch.cuda.set_per_process_memory_fraction((before + room) / torch.cuda.mem_get_info()[1])
+    try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            torch.empty((room + (16 << 20),), dtype=torch.uint8, device="cuda")
+        got = xmk.fmha_backward(q, k, v, out, d_o, lse)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    torch.cuda.synchronize()
+    assert torch.cuda.memory_reserved() <= before + room
+    for nm, a, b in zip(("dq", "dk", "dv"), want, got):
+        _rows_agree(nm, a, b, 2.0 ** -7)
+
+
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("B,N,F,T,H", [(29, 9, 33, 65, 128), (29, 9, 100, 257, 80), (29, 9, 33, 65, 256)])
 def test_backward_infinite_key_without_weight(xmk, causal, B, N, F, T, H):
