@@ -147,6 +147,18 @@ def test_backward_on_a_side_stream(xmk):
     assert len(junk) == 24 and all(torch.equal(x, y) for x, y in zip(got, ref))
 
 
+def _rows_agree(nm, a, b, ulp):
+    """Two ways to the same sums of products of factors that are rounded alike.  Each result is rounded once (one spacing of it,
+    `ulp` of its size at most), and a few of the rounded factors may fall on the other side of a rounding boundary (less than as
+    much again); what remains of a row whose exact gradients cancel is the noise of 32-bit sums."""
+    a, b = a.float(), b.float()
+    diff, size = (a - b).norm(dim=-1), a.norm(dim=-1)
+    assert torch.isfinite(b).all(), nm
+    over = diff - 2 * ulp * size - 1e-5 * a.shape[-1] ** 0.5
+    at = int(over.argmax())
+    assert over.max().item() <= 0, (nm, at, diff.flatten()[at].item(), size.flatten()[at].item())
+
+
 @pytest.mark.parametrize("name,causal", [("bf16", True), ("fp16", True), ("fp16", False)])
 @pytest.mark.parametrize("B,N,F,T,H,parts", [
     (10, 16, 130, 257, 128, 1), (13, 16, 257, 130, 80, 1), (29, 9, 33, 65, 256, 1), (12, 11, 129, 1, 200, 1), (130, 4, 1, 64, 72, 1),
@@ -156,8 +168,7 @@ def test_backward_on_a_side_stream(xmk):
 ])
 def test_backward_with_kept_score_gradients(xmk, name, causal, B, N, F, T, H, parts):
     """dS kept in the workspace (all units at once, or as many as a smaller workspace holds) against a call with the least
-    workspace, which forms it twice: the same products of factors that are rounded alike, so that results differ by their last bit
-    (a single key's dQ and dK are zero but for rounding: those are held to 1e-5)."""
+    workspace, which forms it twice, row by row; and the units at the ends of the parts against float64."""
     import ctypes as C
     L, tdt = xmk.lib(), torch.bfloat16 if name == "bf16" else torch.float16
     L.xmk_fmha_bwd_best_workspace_bytes.restype = C.c_size_t
@@ -183,21 +194,18 @@ def test_backward_with_kept_score_gradients(xmk, name, causal, B, N, F, T, H, pa
         results.append(grads)
     ulp = 2.0 ** (-7 if name == "bf16" else -10)  # relative spacing of the results, and of the dS that enter them, at most
     for nm, a, b in zip(("dq", "dk", "dv"), *results):
-        a, b = a.float(), b.float()
-        diff, size = (a - b).norm().item(), a.norm().item()
-        assert torch.isfinite(b).all() and (diff <= ulp * size or diff <= 1e-5 * a.numel() ** 0.5), (nm, diff, size)
-
-
-def _rows_agree(nm, a, b, ulp):
-    """Two ways to the same sums of products of factors that are rounded alike.  Each result is rounded once (one spacing of it,
-    `ulp` of its size at most), and a few of the rounded factors may fall on the other side of a rounding boundary (less than as
-    much again); what remains of a row whose exact gradients cancel is the noise of 32-bit sums."""
-    a, b = a.float(), b.float()
-    diff, size = (a - b).norm(dim=-1), a.norm(dim=-1)
-    assert torch.isfinite(b).all(), nm
-    over = diff - 2 * ulp * size - 1e-5 * a.shape[-1] ** 0.5
-    at = int(over.argmax())
-    assert over.max().item() <= 0, (nm, at, diff.flatten()[at].item(), size.flatten()[at].item())
+        _rows_agree(nm, a, b, ulp)
+    each = -(-B * N // parts)
+    for unit in {0, each - 1, each % (B * N), B * N - 1}:
+        Q, K, V, O, G = (x.flatten(0, 1)[unit].double() for x in (q, k, v, out, d_o))
+        S = Q @ K.T * H ** -0.5
+        if causal:
+            S.masked_fill_(torch.ones_like(S).triu(1).bool(), float("-inf"))
+        P = torch.exp(S - lse[unit].double()[:, None])
+        dS = P * (G @ V.T - (G * O).sum(1, keepdim=True)) * H ** -0.5
+        for nm, got, ref in zip(("dq", "dk", "dv"), results[1], (dS @ K, dS.T @ Q, P.T @ G)):
+            err = (got.flatten(0, 1)[unit].double() - ref).abs().max().item()
+            assert err <= TOL * max(ref.abs().max().item(), 1e-2), (nm, unit, err)
 
 
 def test_backward_where_memory_is_short(xmk):
