@@ -171,7 +171,8 @@ size_t xmk_fmha_bwd_workspace_bytes(uint32_t num_batches, uint32_t num_heads, ui
 
 /* Bytes of workspace with which xmk_fmha_bwd (without a bias) runs fastest: given more than
  * xmk_fmha_bwd_workspace_bytes(), it keeps the score gradients there, of all (batch, head) units or some at a time,
- * instead of forming them twice.  At most 2 GiB more. */
+ * instead of forming them twice.  At most 2 GiB more.  The gradients' last bits may depend on which of the two the
+ * workspace allows. */
 size_t xmk_fmha_bwd_best_workspace_bytes(uint32_t num_batches, uint32_t num_heads, uint32_t head_size,
                                          uint32_t num_queries, uint32_t num_keys, int32_t causal);
 

@@ -169,6 +169,44 @@ def test_fmha_backward_handlers(ffi, oracle, with_bias):
     assert handler(C.byref(f)) is not None and "scratch allocator" in host.errors[-1][1]
 
 
+@pytest.mark.parametrize("granted", [True, False])
+def test_fmha_backward_handler_keeps_score_gradients(ffi, oracle, granted):
+    """Enough units for dS to be kept: the handler asks for the scratch that holds it, and where the host refuses that, for the
+    least that the call takes."""
+    B, N, Fq, T, H = 29, 9, 33, 65, 128
+    dt, scale = oracle.BF16, H ** -0.5
+    q, g = (oracle.from_f32(oracle.normal((B, N, Fq, H), s), dt) for s in (40, 41))
+    k, v = (oracle.from_f32(oracle.normal((B, N, T, H), s), dt) for s in (42, 43))
+    refs = oracle.fmha_bwd(q, k, v, g, dt, scale, causal=True)
+    tq, tk, tv, tg = (to_dev(x, "bf16") for x in (q, k, v, g))
+    out, act = torch.empty_like(tq), torch.empty((B, N, Fq), dtype=torch.float32, device="cuda")
+    scratch = torch.empty((16,), dtype=torch.uint8, device="cuda")
+    attrs = {"fmha_scale": (F.F64, scale), "dropout_rate": (F.F64, 0.0), "is_causal_mask": (F.S32, 1)}
+    host = _host()
+    f = host.frame([_buf(tq, F.BF16), _buf(tk, F.BF16), _buf(tv, F.BF16)], [_buf(out, F.BF16), _buf(scratch, 6), _buf(act, F.F32)], attrs)
+    _ok(host, ffi.xmk_ffi_fmha_softmax(C.byref(f)))
+    ffi.xmk_fmha_bwd_workspace_bytes.restype = ffi.xmk_fmha_bwd_best_workspace_bytes.restype = C.c_size_t
+    sizes = [C.c_uint32(x) for x in (B, N, H, Fq, T)]
+    least, best = ffi.xmk_fmha_bwd_workspace_bytes(*sizes), ffi.xmk_fmha_bwd_best_workspace_bytes(*sizes, C.c_int32(1))
+    assert best > least
+
+    def allocator(size, alignment):
+        if size == best and not granted:
+            return None, None
+        t = torch.empty((size + alignment,), dtype=torch.uint8, device="cuda")
+        return (t.data_ptr() + alignment - 1) // alignment * alignment, t
+    grads = [torch.full_like(x, float("nan")) for x in (tq, tk, tv)]
+    host = F.FakeHost(stream=torch.cuda.current_stream().cuda_stream, allocator=allocator)
+    f = host.frame([_buf(x, F.F32 if x is act else F.BF16) for x in (tq, tk, act, tv, tg, out)],
+                   [_buf(x, F.BF16) for x in grads] + [_buf(scratch, 6)], attrs)
+    _ok(host, ffi.xmk_ffi_fmha_softmax_backward(C.byref(f)))
+    assert [size for size, _ in host.allocations] == ([best] if granted else [best, least])
+    assert host.freed == [best if granted else least]
+    for name, got, ref in zip(("dq", "dk", "dv"), grads, refs):
+        ge, ee = oracle.rel_err(got.float().cpu().numpy(), ref.astype(np.float32))
+        assert ge <= 1e-2 and ee <= 1.5e-1, (name, ge, ee)
+
+
 def test_fmha_scale_above_one_is_recomputed(ffi, oracle):
     """The reference replaces a scale attribute above 1 by 1/sqrt(H) (xetla_gpu_fused_mha_runner.cc:129)."""
     B, N, Fq, T, H = 1, 2, 64, 64, 64
