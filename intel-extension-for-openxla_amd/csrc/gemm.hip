@@ -416,6 +416,7 @@ bool plan_pack(const xmk_gemm_desc* d, PackPlan* p) {
   if (!p->a && !p->b) return false;  // (only a batch stride, of a single member, is no multiple of eight)
   p->lda = ld(d->lhs);
   p->ldb = ld(d->rhs);
+  if ((p->a && p->lda >= kMaxLd) || (p->b && p->ldb >= kMaxLd)) return false;  // (rows of just under 2^22 are taken as they are)
   p->b_at = p->a ? (size_t)m * p->lda * 2 : 0;
   p->total = p->b_at + (p->b ? (size_t)d->rhs.num_rows * p->ldb * 2 : 0);
   if (forced_policy() != kUnforced || getenv("XMK_GEMM_SPLITK")) return false;  // (they force what runs on the operands given)
