@@ -119,7 +119,8 @@ __global__ __launch_bounds__(WGM * WGN * 64) void fp8_gemm_kernel(Fp8Params p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
 
-  const gemm_impl::TileAt tile = gemm_impl::tile_at(blockIdx.x, p.tiles_m, p.tiles_n, p.K);
+  gemm_impl::request_first_args(p);
+  const gemm_impl::TileAt tile = gemm_impl::tile_at(blockIdx.x, p.order);
   const int m0 = tile.m * BM, n0 = tile.n * BN;
 
   floatx16 acc[TM][TN];
@@ -341,6 +342,7 @@ extern "C" int xmk_fp8_gemm_ex(const void* a, const void* b, const float* a_scal
     const gemm_impl::Policy& P = gemm_impl::kFp8Policies[pol];
     p.tiles_m = (int)xmk::ceil_div(m, P.bm);
     p.tiles_n = (int)xmk::ceil_div(n, P.bn);
+    p.order = gemm_impl::tile_order((uint32_t)p.tiles_m, (uint32_t)p.tiles_n, p.K);
     const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block((unsigned)(P.wgm * P.wgn * 64));
     const bool kn = rhs_transpose == 0;
     if (pol == 0) {

@@ -10,6 +10,7 @@
 #include <utility>
 
 #include "common.h"
+#include "tile_order.h"
 
 namespace gemm_impl {
 
@@ -25,17 +26,22 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 enum : int { ACT_NONE = 0, ACT_RELU = 1, ACT_GELU = 2 };
 
 struct GemmParams {
+  // What a work-group needs for its first loads (request_first_args).
   const void* a;
   const void* b;
+  int64_t lda, ldb;             // elements between stored rows
+  int64_t sa, sb;               // batch strides, elements
+  int M, N, K;
+  int kslice;                   // K slice of one grid member (a multiple of the K step), 0 when K is not split
+  TileOrder order;
+  // The rest.
+  int tiles_m, tiles_n;
   void* out;
   const void* c;
   const void* bias;
-  int M, N, K;
-  int64_t lda, ldb, ldc;        // elements between stored rows
-  int64_t sa, sb, sc;           // batch strides, elements
+  int64_t ldc, sc;
   float alpha, beta;
   int act;
-  int tiles_m, tiles_n;
   // Shared-lhs multi-output form (three GEMMs with one A): batch member z > 0 writes to
   // out_alt[z - 1] instead of out + z * sc and reads bias + z * sbias.  Null when unused.
   void* out_alt[2];
@@ -43,11 +49,18 @@ struct GemmParams {
   // int8 kernel only: elements per load that the alignment of each operand's pointer, leading dimension, batch
   // stride and row length allows.
   int vec_a, vec_b;
-  // K slice of one grid member (a multiple of the K step), 0 when K is not
-  // split.  Kernels that take any alignment: some row of an operand does not start on a 16-byte boundary.
-  int kslice;
+  // Kernels that take any alignment: some row of an operand does not start on a 16-byte boundary.
   bool misaligned;
 };
+
+// Asks for the arguments in front of the first loads at once: where their uses are spread over the prologue, the compiler asks
+// for them there, and every cache line of them is a round trip to memory of its own (the smallest launches 0.1 to 0.3 us).
+__device__ __forceinline__ void request_first_args(const GemmParams& p) {
+  const TileOrder& o = p.order;
+  asm volatile("" ::"s"(p.a), "s"(p.b), "s"(p.lda), "s"(p.ldb), "s"(p.sa), "s"(p.sb), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.kslice),
+               "s"(o.xcd_step), "s"(o.rest), "s"(o.round_step), "s"(o.group), "s"(o.inv_group), "s"(o.last_group), "s"(o.last_rows),
+               "s"(o.inv_last), "s"(o.shift));
+}
 
 __device__ __forceinline__ float gelu_tanh(float x) {
   // 0.5 x (1 + tanh(u)) = x * sigmoid(2u) = x / (1 + exp(-2u)), u = sqrt(2/pi)(x + 0.044715 x^3)
@@ -486,35 +499,6 @@ __device__ __forceinline__ void store_tile(Epilogue& epi, const floatx16 (&acc)[
   });
 }
 
-// Tile order.  Consecutive blocks land on different XCDs (eight of them, each with its own L2), so each XCD gets a contiguous
-// run of tiles, and a run walks the tiles in groups of some tile rows, so that it uses few rows of A and columns of B: about
-// as many of the one as of the other, up to eight rows.  Microseconds against runs only where the tiles divide by eight, always
-// in eight rows: 85 x 4001 x 2231 19.2 -> 12.5, 141 x 1280 x 7168 17.1 -> 13.6, 811 x 3488 x 4144 50 -> 40, 2244 x 9235 x 13131
-// 1077 -> 1017; 80 drawn sizes of 20 rows and more 4 % on average, 110 with k of 129 to 1300 3 %.  The worst are tall outputs
-// of few tile columns, where the plain order happened to give an XCD whole tile rows: 3148 x 352 x 888 8.3 -> 9.0, 3306 x 576 x 576
-// 7.3 -> 7.6.  (Row by row where a run spans two rows and more: those 4 % back, 7539 x 197 x 1649 22.4 -> 25.2.)
-// With k of 128 or less it is the output that takes the time, and neighbours on different XCDs write it faster (4305 x 12736 x 64
-// 46.0 against 44.5).
-struct TileAt {
-  int m, n;
-};
-__device__ __forceinline__ uint32_t xcd_run(uint32_t block, uint32_t n, int K) {
-  const uint32_t x = block & 7, rest = n & 7;
-  return rest && K <= 128 ? block : x * (n >> 3) + min(x, rest) + (block >> 3);
-}
-__device__ __forceinline__ TileAt tile_at(int block, int tiles_m, int tiles_n, int K) {
-  const uint32_t n = (uint32_t)(tiles_m * tiles_n), pid = xcd_run((uint32_t)block, n, K), run = (n + 7) >> 3;
-  int shift = run >= 24 ? 3 : run >= 6 ? 2 : run >= 2 ? 1 : 0;
-  if ((tiles_m & (tiles_m - 1)) == 0) {
-    shift = min(shift, __builtin_ctz(tiles_m));
-    if (tiles_m >> shift == 1) return {(int)pid & (tiles_m - 1), (int)(pid >> shift)};  // all rows at once: nothing to divide
-  }
-  const int first_m = (int)(pid / (uint32_t)tiles_n) >> shift << shift, at = (int)pid - first_m * tiles_n;
-  const int height = tiles_m - first_m;
-  if (height >> shift) return {first_m + (at & ((1 << shift) - 1)), at >> shift};
-  return {first_m + at % height, at / height};  // the last rows
-}
-
 // T: element type; OutF32: fp32 output (else T); A_MC / B_MC: operand's free index is
 // contiguous; BM x BN tile; WGM x WGN waves; BK: K step (32 or 64); NSTAGE: LDS stages.
 template <typename T, bool OutF32, bool A_MC, bool B_MC, int BM, int BN, int WGM, int WGN, int BK, int NSTAGE>
@@ -534,7 +518,8 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_mfma_kernel(GemmParams p)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
 
-  const TileAt tile = tile_at(blockIdx.x, p.tiles_m, p.tiles_n, p.K);
+  request_first_args(p);
+  const TileAt tile = tile_at(blockIdx.x, p.order);
   const int m0 = tile.m * BM, n0 = tile.n * BN;
 
   const int64_t bz = blockIdx.z;
@@ -902,6 +887,7 @@ template <typename T, bool OutF32, bool A_MC, bool B_MC>
 void launch_policy(int pol, GemmParams& p, int batch, hipStream_t st) {
   p.tiles_m = (int)xmk::ceil_div(p.M, kPolicies[pol].bm);
   p.tiles_n = (int)xmk::ceil_div(p.N, kPolicies[pol].bn);
+  p.order = tile_order((uint32_t)p.tiles_m, (uint32_t)p.tiles_n, p.K);
   switch (pol) {
     case 0: launch_mfma<T, OutF32, A_MC, B_MC, 256, 256, 2, 2, 32, 4>(p, batch, st); break;
     case 1: launch_mfma<T, OutF32, A_MC, B_MC, 128, 128, 2, 2, 64, 4>(p, batch, st); break;

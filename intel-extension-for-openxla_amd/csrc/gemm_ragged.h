@@ -29,7 +29,8 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_ragged_kernel(typename AnyT
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
 
-  const TileAt tile = tile_at(blockIdx.x, p.tiles_m, p.tiles_n, p.K);
+  request_first_args(p);
+  const TileAt tile = tile_at(blockIdx.x, p.order);
   const int m0 = tile.m * BT, n0 = tile.n * BT;
 
   const int64_t bz = blockIdx.z;
@@ -133,6 +134,7 @@ template <typename T, bool OutF32, bool A_MC, bool B_MC>
 void launch_ragged_tile(typename AnyType<T>::Params& p, int batch, int tile, hipStream_t st) {
   p.tiles_m = (int)xmk::ceil_div(p.M, tile);
   p.tiles_n = (int)xmk::ceil_div(p.N, tile);
+  p.order = tile_order((uint32_t)p.tiles_m, (uint32_t)p.tiles_n, p.K);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)batch);
   constexpr int WGN = sizeof(T) == 4 ? 4 : 2;
   if constexpr (sizeof(T) != 2) {  // (16-bit operands without misaligned rows take the direct kernels)

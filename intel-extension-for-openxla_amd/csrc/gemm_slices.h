@@ -29,11 +29,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_slices_kernel(typename AnyType<T
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // (along the shorter side: a run then covers few rows and columns of tiles)
-  const int pid = (int)xcd_run(blockIdx.x, (uint32_t)(p.tiles_m * p.tiles_n), p.K);
-  const bool down = p.tiles_m <= p.tiles_n;
-  const int side = down ? p.tiles_m : p.tiles_n, major = pid / side, minor = pid - major * side;
-  const int m0 = (down ? minor : major) * (32 * TM), n0 = (down ? major : minor) * (32 * TN);
+  request_first_args(p);
+  const TileAt tile = tile_at(blockIdx.x, p.order);
+  const int m0 = tile.m * (32 * TM), n0 = tile.n * (32 * TN);
 
   const int64_t bz = blockIdx.z;
   const int64_t k0 = bz * p.kslice;  // as in gemm_ragged_kernel
@@ -156,6 +154,7 @@ void launch_slices_variant(int v, typename AnyType<T>::Params& p, int batch, hip
   const Policy& pol = kPolicies[kSlicesPolicy + v];  // (fp8 has the same tiles under its own numbers)
   p.tiles_m = (int)xmk::ceil_div(p.M, pol.bm);
   p.tiles_n = (int)xmk::ceil_div(p.N, pol.bn);
+  p.order = tile_order_slices((uint32_t)p.tiles_m, (uint32_t)p.tiles_n, p.K);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)batch), block((unsigned)(pol.wgm * 64));
   switch (v) {
     case 0: hipLaunchKernelGGL((gemm_slices_kernel<T, OutF32, A_MC, B_MC, 1, 1, 4, MIS>), grid, block, 0, st, p); break;
