@@ -70,12 +70,17 @@ inline TileOrder tile_order(uint32_t tiles_m, uint32_t tiles_n, int K) {
   return o;
 }
 // Tiles of a kernel that splits K over a work-group's waves: along the shorter side, so that a run covers few rows and
-// columns of tiles.
+// columns of tiles.  But where a few tile columns and a long K come to a second round of up to 128 work-groups, column by
+// column over all XCDs: the second round is then of rows that the first has brought into a cache.  2274 x 112 x 5128 28.2 ->
+// 21.6 us, 4598 x 64 x 2752 16.0 -> 13.5, 4938 x 64 x 5568 29.3 -> 25.3; of 60 sizes with k of 2100 to 8900 the worst 16.7 -> 17.4
+// (the tile rows no multiple of eight, so that a row's tiles are on two XCDs).  With a shorter K it is the other way round:
+// 3032 x 80 x 1088 7.0 against 8.5; with two tile columns the two are level at about 1300, with four at 2100.
 inline TileOrder tile_order_slices(uint32_t tiles_m, uint32_t tiles_n, int K) {
   const uint32_t tiles = tiles_m * tiles_n;
-  TileOrder o = tile_numbers(tiles, tiles % 8 == 0 || K > 128);
+  const bool again = tiles_m > tiles_n && tiles_n <= 4 && tiles > 256 && tiles <= 384 && K > 512 * ((int)tiles_n + 1);
+  TileOrder o = tile_numbers(tiles, !again && (tiles % 8 == 0 || K > 128));
   tile_groups(o, tiles_m, tiles_n, 0);
-  if (tiles_m <= tiles_n) {  // column by column: one group of all rows
+  if (again || tiles_m <= tiles_n) {  // column by column: one group of all rows
     o.group = tiles;
     o.last_group = 0;
     o.last_rows = tiles_m;

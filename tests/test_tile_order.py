@@ -81,3 +81,11 @@ def test_first_loads_follow_one_round_of_arguments(tmp_path, header, kernel):
     first = next(i for i, l in enumerate(lines) if "buffer_load" in l or "global_load" in l)
     waits = [l for l in lines[:first] if "s_waitcnt" in l and "lgkmcnt" in l]
     assert len(waits) == 1 and not any("v_rcp" in l for l in lines[:first]), waits
+
+
+@pytest.mark.parametrize("tiles_m,tiles_n", [(129, 2), (155, 2), (192, 2), (95, 3), (128, 3), (72, 4), (96, 4)])
+def test_second_round_of_tall_outputs_rereads_rows(order, tiles_m, tiles_n):
+    """A few tile columns and a long K, K split over the waves: what does not fit the first 256 work-groups takes rows of A that
+    the first ones have read."""
+    t = order[1](tiles_m, tiles_n, 4096, 1)
+    assert set(t[256:, 0]) <= set(t[:256, 0])
