@@ -928,14 +928,22 @@ bool one_grid(const Args& a, uint64_t units) {
 
 // All units in one part run with fewer launches than without dS; what a part of them loses is its last, partly empty
 // rounds of 512 work-groups: 896 per part (32 x 16384, 7 units at a time) 8.2 -> 10.9 ms, 1408 (64 x 8192) 4.19 -> 4.02.
-// Against the one grid of a small problem (us, one grid / dS kept; causal first): 512 groups, 32 x 2048, 195 / 179 and
-// 291 / 236; 384, 24 x 2048, 145 / 150 and 235 / 197, 192 x 256 50 / 43; 320, 10 x 4096, 278 / 264; 256, 16 x 2048, 123 / 130;
-// 96, 96 x 128, 14 / 20.  Heads of 256: 256 groups, 16 x 2048, 341 / 305 and 406 / 323; 56 groups 48 / 90.
+// The one grid of a small problem fills the device with the work-groups of all passes; with dS kept each pass has to by itself.
+// One grid / dS kept, us, two work-groups per CU: 512 groups, 32 x 2048, causal 195 / 179, no mask 291 / 236; 384, 24 x 2048, 145 /
+// 150 and 235 / 197; 352, 352 x 180 34.6 / 32.3; 320, 10 x 4096, 278 / 264, but 269 x 61 causal 21.4 / 23.9, 277 x 46 20.2 / 22.1,
+// 280 groups of 1014 79 / 87.  Heads of more than 128: no mask 272 groups of 2154 353 / 418, 302 of 225 111 / 118, 348 of 471
+// 0.95; causal level at 256.  And where queries or keys are few, so is the work of one pass: 86 x 302 queries and 77 keys 26.0 /
+// 30.9, 48 x 54 and 884 29.9 / 39.2, 69 x 125 and 583, heads of 256, 72 / 98 (up to 160 rows of such heads: level).  Of 858 drawn sizes 4 lose more than 2 % by this
+// rule, the worst 3 %; with 256 work-groups of the longer side as the rule 49 did, up to 48 %.
 uint64_t saved_units(const Args& a, uint64_t units, uint64_t bytes) {
   constexpr uint64_t kMost = (uint64_t)2 << 30, kPartGroups = 1280;
+  auto groups = [&](uint64_t rows) { return units * ((rows + BO - 1) / BO); };
   const uint64_t rows = (uint64_t)std::max(a.F, a.T), per_unit = (rows + BO - 1) / BO;
-  if (a.bias || a.H <= 64) return 0;
-  if (units * per_unit < (a.H > 128 ? 256u : a.causal && rows > 1024 ? 385u : 257u)) return 0;
+  if (a.bias || a.H <= 64 || groups(rows) < 256) return 0;
+  if (one_grid(a, units) && (a.H <= 128 || rows > 160)) {
+    if (groups(rows) < (a.H > 128 ? a.causal ? 256u : 336u : a.causal && rows > 1024 ? 385u : 352u)) return 0;
+    if (groups((uint64_t)std::min(a.F, a.T)) < 128) return 0;
+  }
   const uint64_t fit = std::min(bytes, kMost) / saved_bytes(a, 1);
   if (fit >= units) return units;
   if (fit == 0) return 0;

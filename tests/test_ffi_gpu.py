@@ -173,7 +173,7 @@ def test_fmha_backward_handlers(ffi, oracle, with_bias):
 def test_fmha_backward_handler_keeps_score_gradients(ffi, oracle, granted):
     """Enough units for dS to be kept: the handler asks for the scratch that holds it, and where the host refuses that, for the
     least that the call takes."""
-    B, N, Fq, T, H = 29, 9, 33, 65, 128
+    B, N, Fq, T, H = 40, 9, 33, 65, 128
     dt, scale = oracle.BF16, H ** -0.5
     q, g = (oracle.from_f32(oracle.normal((B, N, Fq, H), s), dt) for s in (40, 41))
     k, v = (oracle.from_f32(oracle.normal((B, N, T, H), s), dt) for s in (42, 43))
