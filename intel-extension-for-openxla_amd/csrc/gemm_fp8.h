@@ -108,70 +108,72 @@ struct AnyFrag<Fp8, MC, ROWS, TT> {
 };
 
 // The fp8 product's tiles.  0 .. 2: the direct-to-LDS kernel of fp8_gemm.hip; the others take any alignment.
+// ("alone" where the estimates fit better so, also of tiles of which two share a CU.)
 constexpr Policy kFp8Policies[] = {
     {"mfma_256x256", 256, 256, 2, 4, 64, 4, true, false},
     {"mfma_256x128", 256, 128, 2, 2, 64, 4, true, false},
-    {"mfma_128x128", 128, 128, 2, 2, 64, 4, false, false},
-    {"any_128x128", 128, 128, 2, 2, 128, 2, false, true},
+    {"mfma_128x128", 128, 128, 2, 2, 64, 4, true, false},
+    {"any_128x128", 128, 128, 2, 2, 128, 2, true, true},
     {"any_64x64", 64, 64, 2, 2, 128, 2, false, true},
-    {"slices_32x32_w4", 32, 32, 4, 1, 128, 2, false, true},
+    {"slices_32x32_w4", 32, 32, 4, 1, 128, 2, true, true},
     {"slices_32x32_w8", 32, 32, 8, 1, 128, 2, true, true},
     {"slices_32x32_w16", 32, 32, 16, 1, 128, 2, true, true},
     {"slices_32x64_w8", 32, 64, 8, 1, 128, 2, true, true},
-    {"slices_64x64_w4", 64, 64, 4, 1, 128, 2, false, true},
+    {"slices_64x64_w4", 64, 64, 4, 1, 128, 2, true, true},
     {"slices_64x64_w8", 64, 64, 8, 1, 128, 2, true, true},
 };
 constexpr int kFp8Policies_n = sizeof(kFp8Policies) / sizeof(kFp8Policies[0]);
 constexpr int kFp8Direct = 3, kFp8Slices = 5;
 
-// Estimated microseconds (launch_cost in gemm_kernel.h).  The direct classes are fitted to 350 shapes each, m 2 .. 8192, n 64 ..
-// 16384, k 256 .. 16384, weights from memory: on 115 others per class 3 % from the best policy of all measured, one in ten
-// more than 10 %, the worst 34 % (the table before the tiles' present order: [k,n] 7 %, 23 %, 64 %).  The any-alignment class:
-// 240 shapes, m 1 .. 8192, 2 % on those, 3 to 4 % on others.
+// Estimated microseconds (launch_cost in gemm_kernel.h), fitted to 6100 shapes per direct class and 3200 of the other, m 1 .. 8192,
+// n 64 .. 16384, k 64 .. 16384, weights from memory: least squares, then moved so that the policies they choose are the fastest.
+// On 1500 (800) other shapes 0.6 % (0.5 %) from the best policy of all measured, one in ten more than 2 %, the worst 21 % (24 %).
+// A table fitted to k of 256 and more, which stood here before, lost 4 to 5 % (3 %), one in ten 12 to 14 % (8 %): 965 x 5456 x 96, B
+// [k,n], 10.4 us on 128 x 128 tiles where 64 x 64 take 7.8.
 constexpr TileCost kFp8Cost[3][kFp8Policies_n] = {
     {  // direct loads possible, B stored [K, N]
-     {5.397f, 0.987f, 1.885f, 8.612f, 5.243f},
-     {4.759f, 0.596f, 1.095f, 6.471f, 3.21f},
-     {5.059f, 0.806f, 0.561f, 1.5f, 0.f},  // (more than 256 tiles)
-     {4.011f, 0.668f, 0.532f, 2.909f, 1.888f},
-     {3.027f, 0.32f, 0.225f, 0.672f, 1.311f},
-     {3.021f, 0.388f, 0.18f, 0.286f, 1.294f},
-     {2.704f, 0.875f, 0.194f, 0.936f, 1.195f},
-     {1.231f, 2.745f, 0.246f, 1.699f, 1.428f},
-     {2.836f, 1.194f, 0.219f, 1.978f, 1.25f},
-     {3.775f, 0.84f, 0.303f, 3.027f, 1.032f},
-     {3.356f, 1.986f, 0.388f, 3.034f, 2.102f},
+     {7.4f, 0.974f, 1.068f, 9.869f, 8.691f},
+     {5.27f, 0.759f, 0.835f, 6.426f, 11.51f},
+     {3.83f, 0.888f, 0.745f, 1.616f, 0.024f},  // (more than 256 tiles)
+     {4.299f, 0.695f, 0.488f, 2.753f, 1.793f},
+     {3.311f, 0.326f, 0.3f, 0.355f, 1.468f},
+     {2.551f, 0.469f, 0.163f, 0.129f, 1.093f},
+     {1.394f, 1.516f, 0.262f, 1.148f, 1.31f},
+     {0.307f, 4.123f, 0.241f, 1.936f, 2.128f},
+     {2.035f, 1.596f, 0.203f, 2.081f, 1.276f},
+     {3.352f, 1.037f, 0.361f, 3.278f, 1.494f},
+     {2.437f, 2.515f, 0.399f, 3.198f, 3.169f},
     },
     {  // direct loads possible, B stored [N, K]
-     {5.026f, 0.989f, 1.517f, 9.792f, 7.747f},
-     {4.458f, 0.597f, 1.115f, 4.438f, 5.174f},
-     {4.782f, 0.947f, 0.545f, 1.329f, 0.f},
-     {3.78f, 0.644f, 0.521f, 2.042f, 2.495f},
-     {3.042f, 0.276f, 0.186f, 0.633f, 1.407f},
-     {3.188f, 0.302f, 0.097f, 0.445f, 0.511f},
-     {3.186f, 0.579f, 0.122f, 1.073f, 0.565f},
-     {2.224f, 1.9f, 0.159f, 1.916f, 0.857f},
-     {3.155f, 0.942f, 0.179f, 2.022f, 1.003f},
-     {3.749f, 0.766f, 0.282f, 2.87f, 0.995f},
-     {3.497f, 1.359f, 0.296f, 2.632f, 1.294f},
+     {7.227f, 0.979f, 1.902f, 9.457f, 9.902f},
+     {4.898f, 0.721f, 0.874f, 6.179f, 12.309f},
+     {3.75f, 0.975f, 0.746f, 1.457f, 0.067f},  // (more than 256 tiles)
+     {4.05f, 0.743f, 0.512f, 2.339f, 2.12f},
+     {3.03f, 0.346f, 0.3f, 0.434f, 1.062f},
+     {2.024f, 0.448f, 0.12f, 0.326f, 0.694f},
+     {2.501f, 0.816f, 0.16f, 1.159f, 0.756f},
+     {1.468f, 2.761f, 0.182f, 1.976f, 1.487f},
+     {2.671f, 0.858f, 0.188f, 2.071f, 1.393f},
+     {3.682f, 0.829f, 0.286f, 3.477f, 1.247f},
+     {2.793f, 1.62f, 0.256f, 3.124f, 2.311f},
     },
     {  // any alignment
      {},
      {},
      {},
-     {5.016f, 0.937f, 0.804f, 2.238f, 2.798f},
-     {3.469f, 0.413f, 0.383f, 0.587f, 1.429f},
-     {2.968f, 0.748f, 0.209f, 0.508f, 0.654f},
-     {2.344f, 1.551f, 0.231f, 1.4f, 0.511f},
-     {1.357f, 3.735f, 0.293f, 2.856f, 1.51f},
-     {2.231f, 2.238f, 0.341f, 2.558f, 0.921f},
-     {3.817f, 1.428f, 0.471f, 3.425f, 0.838f},
-     {3.23f, 3.795f, 0.64f, 3.87f, 1.223f},
+     {5.682f, 0.818f, 0.484f, 2.523f, 3.206f},
+     {3.202f, 0.464f, 0.36f, 0.586f, 1.811f},
+     {1.951f, 0.684f, 0.226f, 0.394f, 0.95f},
+     {2.952f, 1.299f, 0.315f, 1.144f, 1.562f},
+     {1.195f, 3.618f, 0.264f, 3.012f, 2.195f},
+     {2.128f, 1.501f, 0.318f, 2.545f, 1.62f},
+     {3.91f, 1.244f, 0.47f, 3.883f, 1.945f},
+     {3.065f, 3.612f, 0.521f, 4.207f, 2.525f},
     },
 };
 
 // The 128 x 128 tile where every CU has one at most (K steps of 128 bytes), B stored [K, N] / [N, K]; fitted with them.
-constexpr TileCost kFp8OnePerCu[2] = {{3.919f, 0.324f, 0.f, 0.f, 2.146f}, {3.689f, 0.29f, 0.f, 0.f, 3.007f}};
+constexpr TileCost kFp8OnePerCu[2] = {{4.287f, 0.509f, 0.016f, 0.f, 2.896f}, {4.124f, 0.487f, 0.055f, 0.f, 3.529f}};
 
 // Policies 3 and up; A is [M, K], b_mc: B stored [K, N].
 void launch_fp8_any(int policy, bool b_mc, Fp8Params& p, hipStream_t st);
