@@ -39,7 +39,8 @@ typedef __attribute__((address_space(3))) void* lds_void_ptr;
 constexpr int BS = 64;   // streamed rows per block
 constexpr int BO = 128;  // owner rows per work-group
 constexpr uint32_t kOob = 0x80000000u;
-constexpr int kNonTemporal = 2;  // cache policy of dS, written once and read once: 1079 -> 1034 us against the default ([8,32,2048,128] causal)
+// Cache policy of dS, written once and read once: 1079 -> 1034 us against the default ([8,32,2048,128] causal).
+constexpr int kNonTemporal = 2;
 constexpr float kLog2e = 1.4426950408889634f;
 
 template <typename F, int... I>
@@ -564,13 +565,16 @@ __device__ __forceinline__ void bwd_pass(const std::conditional_t<SAVE_DS, Saved
 }
 
 // Keys own, dS from memory: dK = scale dS^T Q, and with PV also dV = P^T dO, whose P it forms again from S.
-// What bounds the keys-own passes is the matrix pipe under the package's power limit: forming dS here takes two products
-// (S and dP) for the one that uses it, and the registers of a second owner operand, without which both accumulators fit at
-// two waves per SIMD.  The queries-own pass has dS at hand; it costs a write and a read of 2 bytes per score, hidden behind
-// the products: [8,32,2048,128] causal bf16 1255 -> 1034 us (dQ 482 -> 540, dK and dV 488 + 354 -> 490), without a mask
-// 2145 -> 1775; 600 x 300 causal heads of 128 95 -> 72; 64 x 2048 heads of 256 953 -> 703.  At heads of 64 the traffic
-// weighs twice as much and dK and dV share their products anyway: 180 -> 194 us, not used.  A work-group owns 128 keys and walks the queries in blocks of 32 through three LDS stages (two blocks
-// ahead, 75 KiB, two work-groups per CU).
+// Forming dS here takes two products (S and dP) for the one that uses it, and the registers of a second owner operand,
+// without which both accumulators fit at two waves per SIMD.  The queries-own pass has dS at hand; it costs a write and a
+// read of 2 bytes per score: [8,32,2048,128] causal bf16 1309 -> 1075 us (in one trace of both forms dQ 482 -> 540, dK and dV
+// 488 + 354 -> 490), without a mask 2145 -> 1775; 600 x 300 causal heads of 128 95 -> 72; 64 x 2048 heads of 256 953 -> 703.
+// At heads of 64 the traffic weighs twice as much and dK and dV share their products anyway: 180 -> 194 us, not used.
+// What bounds the two launches: by the counters of a first call the matrix pipe is busy 42 and 48 % of the cycles, the vector
+// port 42 and 27 %, a third of the waves' time is waits for an instruction to issue, and memory moves 3.9 and 4.2 TB/s: no
+// unit alone, at the clock that the package's power limit leaves (1.9 GHz in that call, 1.75 over a second of them).
+// A work-group owns 128 keys and walks the queries in blocks of 32 through three LDS stages (two blocks ahead, 75 KiB, two
+// work-groups per CU).
 constexpr int SBS = 32;
 template <int HP, bool PV> struct SavedLds {
   static constexpr int TILE = SBS * HP * 2, DSB = BO * SBS * 2, STAT = PV ? 4 * 256 : 0;
@@ -932,13 +936,14 @@ bool one_grid(const Args& a, uint64_t units) {
 
 // All units in one part run with fewer launches than without dS; what a part of them loses is its last, partly empty
 // rounds of 512 work-groups: 896 per part (32 x 16384, 7 units at a time) 8.2 -> 10.9 ms, 1408 (64 x 8192) 4.19 -> 4.02.
-// The one grid of a small problem fills the device with the work-groups of all passes; with dS kept each pass has to by itself.
-// One grid / dS kept, us, two work-groups per CU: 512 groups, 32 x 2048, causal 195 / 179, no mask 291 / 236; 384, 24 x 2048, 145 /
-// 150 and 235 / 197; 352, 352 x 180 34.6 / 32.3; 320, 10 x 4096, 278 / 264, but 269 x 61 causal 21.4 / 23.9, 277 x 46 20.2 / 22.1,
-// 280 groups of 1014 79 / 87.  Heads of more than 128: no mask 272 groups of 2154 353 / 418, 302 of 225 111 / 118, 348 of 471
-// 0.95; causal level at 256.  And where queries or keys are few, so is the work of one pass: 86 x 302 queries and 77 keys 26.0 /
-// 30.9, 48 x 54 and 884 29.9 / 39.2, 69 x 125 and 583, heads of 256, 72 / 98 (up to 160 rows of such heads: level).  Of 858 drawn sizes 4 lose more than 2 % by this
-// rule, the worst 3 %; with 256 work-groups of the longer side as the rule 49 did, up to 48 %.
+// The one grid of a small problem fills the device with the work-groups of all passes; with dS kept each pass has to by
+// itself.  One grid / dS kept, us, two work-groups per CU: 512 groups, 32 x 2048, causal 195 / 179, no mask 291 / 236; 384,
+// 24 x 2048, 145 / 150 and 235 / 197; 352, 352 x 180, 34.6 / 32.3; 320, 10 x 4096, 278 / 264, but 269 x 61 causal 21.4 / 23.9,
+// 277 x 46 20.2 / 22.1, 35 x 1014 79 / 87.  Heads of more than 128: no mask 272 groups of 2154 353 / 418, 302 of 225 111 / 118,
+// 348 of 471 5 % faster with it; causal level at 256.  And where queries or keys are few, so is the work of one pass: 86 x 302
+// queries and 77 keys 26.0 / 30.9, 48 x 54 and 884 29.9 / 39.2, 69 x 125 and 583, heads of 256, 72 / 98 (up to 160 rows of
+// such heads: level).  Of 858 drawn sizes 4 lose more than 2 % by this rule, the worst 3 %; with 256 work-groups of the
+// longer side as the rule 49 did, up to 48 %.
 uint64_t saved_units(const Args& a, uint64_t units, uint64_t bytes) {
   constexpr uint64_t kMost = (uint64_t)2 << 30, kPartGroups = 1280;
   auto groups = [&](uint64_t rows) { return units * ((rows + BO - 1) / BO); };

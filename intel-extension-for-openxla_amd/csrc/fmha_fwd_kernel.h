@@ -157,9 +157,9 @@ __device__ __forceinline__ float bias_value(u32x2 w, int e) {
 // first) as two 16-byte pieces, wherever they lie (the hardware takes global loads at any address), and hands the eight keys
 // that are the other lane's to it when they are used.  Pieces may reach past the row, into the next one (the caller masks
 // those keys); where they would reach past the whole bias (`whole` false; uniform over the wave) keys are read one by one, the
-// row's last one, `keys` - 1 after `at` (also where that is before it), in place of those past it.  (With a load for each element, waited for where it is used, the wave stood still:
-// 4 x 15 heads of 1907 x 256 fp16 2011 us against 355 so, 5 of 5413 x 40 bf16 1095 against 146, 16 of 2876 x 160 causal 680
-// against 127.)
+// row's last one, `keys` - 1 after `at` (also where that is before it), in place of those past it.  (With a load for each
+// element, waited for where it is used, the wave stood still: 4 x 15 heads of 1907 x 256 fp16 2011 us against 355 so, 5 of
+// 5413 x 40 bf16 1095 against 146, 16 of 2876 x 160 causal 680 against 127.)
 template <typename T>
 __device__ __forceinline__ void fetch_bias_keys(const T* at, bool whole, int keys, u32x4 (&b)[2]) {
   if (whole) {
@@ -801,7 +801,7 @@ void launch_cfg(FmhaParams p, uint64_t units, uint32_t F, bool causal, int bias,
   // TFLOP/s), more when a unit has so few query blocks that four units do not fill an XCD's 64 slots.
   p.ug = std::max(4, (64 + p.nqb - 1) / p.nqb);
   const dim3 grid((unsigned)(p.per_xcd * 8)), block(NW * 64);
-  // bias: 0 none, 1 element-wise from global memory, 2 staged through LDS
+  // bias: 0 none, 1 from global memory in 16-byte pieces (fetch_bias_keys), 2 staged through LDS
   if (causal) {
     if (bias == 2) hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, KS, HT, NW, WPS, true, 2>), grid, block, 0, st, p);
     else if (bias == 1) hipLaunchKernelGGL((fmha_fwd_kernel<T, HP, KS, HT, NW, WPS, true, 1>), grid, block, 0, st, p);

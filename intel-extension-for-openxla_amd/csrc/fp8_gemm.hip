@@ -276,7 +276,7 @@ __global__ __launch_bounds__(256) void fp8_gemm_generic_kernel(Fp8Params p, int 
 
 // Up to 256 tiles of 128 x 128 a CU has one work-group, which may then fill its LDS: K steps of 128 bytes in four stages
 // instead of 64.  Half the barriers, and whole cache lines from rows of k (268 instead of 366 MB at 256 x 16384 x 4096, B
-// [n,k]).  Microseconds: there 22.6 -> 20.6, B [k,n] 23.5 -> 20.4; 512 x 4096 x 4096 19.3 -> 15.0, 128 x 16384 x 4096 20.2 ->
+// [n,k]).  Microseconds: there 22.8 -> 19.6, B [k,n] 23.5 -> 20.4; 512 x 4096 x 4096 19.3 -> 15.0, 128 x 16384 x 4096 20.2 ->
 // 16.4.  (Three stages 25.2, five 20.9: neither the depth nor the barriers alone.)  With more tiles two work-groups share a CU,
 // which the small stages allow: 700 x 6000 x 2048 18.3 against 19.9.  The 256 x 128 tile on steps of 128 bytes, three stages:
 // 2048 x 4096 x 4096 37.9 -> 36.4 with B [n,k], 35.8 -> 36.8 with [k,n], 1024 x 8192 x 8192 74.9 -> 76.6: left alone.

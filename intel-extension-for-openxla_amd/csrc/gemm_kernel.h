@@ -751,13 +751,12 @@ enum : int { kClassKN = 0, kClassNK = 1, kClassRagged = 2, kClassF32 = 3 };
 // that rounded up; at least 1),
 //     start + step * KTw + fill * KT * min(tiles / 256, 1) / 8 + (L - 1) * (more_step * KT + more).
 // Least-squares fits (non-negative, relative error) to 380 shapes per class, m 1 .. 8192, n and k 64 .. 16384 at
-// random, every policy: mean error 5 - 12 %; on those shapes the policy that this picks is on average 2 % (fp32: 4 %)
-// slower than the best of all measured, where tile rate x occupancy x inside area, the rule before, lost 7 - 26 %.
-// On other shapes of the range (280 and 140 per storage order, m up to 2048, the weights rotating so that they come from
-// memory) it is 3 % slower than the best tile without a K split (any alignment 2 %, fp32 4 %; one in ten by more than 5 to
-// 9 %, the worst by 56 %), and with scratch 5 % slower than the best tile and split (6 % and 7 %; one in ten by more than
-// 10 to 20 %): it expects too much of the slices kernels where a few rows meet weights of 100 MB (16 x 16384 x 4096 31 us where
-// the 64 x 64 tile takes 27), and too little of a split of 128 rows (128 x 4096 x 4096 25 us, 18 on four slices).
+// random, every policy: mean error 5 - 12 %.  They are older than the fourth stage of the 128 x 128 tile and the present tile
+// order.  With these, on 1100 to 1250 other shapes per class, the weights from memory, the policy that this picks is without a
+// K split 3.2 % slower than the best of all ([k,n]; [n,k] 3.1 %, any alignment 1.7 %, fp32 1.9 %), one in ten by more than 5 to
+// 7 %, the worst by 78 % (609 x 1568 x 6968; the streaming kernel for [n,k] apart: 4 x 13536 x 80 takes it 14 us, a tile 4).
+// With scratch, against every tile on 1 to 8 slices, 500 to 730 shapes per class, it is level on aligned operands (copies and
+// streams are no tiles), any alignment and fp32 3 %, one in ten by more than 7 to 10 %, the worst by 34 %.
 // Looking all candidates over takes the host 0.15 to 0.65 us per call.
 struct TileCost {
   float start, step, more_step, more, fill;

@@ -236,9 +236,9 @@ XMK_PY(fmha_forward) {
 }
 
 // Whether `bytes` of scratch that a call can do without are to be asked for: the allocator holds that much in whole unused
-// segments, or the device has twice as much left.  A request that fails is no answer to that: torch then gives back every cached block and waits for the
-// device, in each such call of a program whose memory is nearly full.  Under stream capture nothing is queried (the memory is the
-// graph's, and asked for once).
+// segments, or the device has twice as much left.  A request that fails is no answer to that: torch then gives back every
+// cached block and waits for the device, in each such call of a program whose memory is nearly full.  Under stream capture
+// nothing is queried (the memory is the graph's, and asked for once).
 bool spare_memory(const at::Tensor& like, int64_t bytes, void* st) {
   if (!like.is_cuda()) return false;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
