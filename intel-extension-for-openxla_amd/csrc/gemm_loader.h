@@ -111,13 +111,17 @@ struct AnyLoader {
     }
     advance(1);
   }
-  __device__ __forceinline__ void store(char* tile, Regs& r) const {
+  // Moves what was read from before an operand's end into place.
+  __device__ __forceinline__ void shift_ends(Regs& r) const {
     if constexpr (MIS) {
       if (reach > r.limit) {  // only at the operand's end
 #pragma unroll
         for (int i = 0; i < NL; ++i) r.g[i] = shift_bytes(r.g[i], (uint32_t)max((int32_t)off[i] - r.limit, 0));
       }
     }
+  }
+  __device__ __forceinline__ void store(char* tile, Regs& r) const {
+    shift_ends(r);
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       // (KC: the XOR counts pairs of rows modulo 16 rows)

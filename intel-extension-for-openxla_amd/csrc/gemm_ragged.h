@@ -1,39 +1,42 @@
 // MFMA GEMM for operands of any alignment: 16-bit ones whose rows do not start on 16-byte boundaries or do not
 // hold whole 16-byte chunks (odd leading dimensions, odd K or N; the direct-to-LDS loads of gemm_kernel.h cannot
-// take them), and all fp32 ones.
+// take them), and fp32 ones on the small tile (on the large one: gemm_split.h, which comes here for what it cannot take).
 //
 // What bounds it: 16-bit, the load path (gemm_loader.h); fp32, the matrix instructions (256 flop per cycle and CU).
 // A K step's chunks are loaded one or two whole steps before they are written to LDS, so that two LDS stages suffice
-// and two work-groups of the large tile share a CU.  fp32 has eight waves on the large tile, so that the SIMDs have
-// a second wave to run while one waits for LDS or the barrier (four: 77 us where eight take 71).
+// and two work-groups of the large tile share a CU.
 // Measured, microseconds (element-wise gathers -> here): bf16 1023 x 5003 x 2047 421 -> 56 (52 on operands that stay in
 // the caches), 496 x 1331 x 13447 2930 -> 73, with scratch for a K split 59, 4001 x 4001 x 4001 189; fp32
-// 2048 x 2048 x 1024 123 -> 71 (121 TFLOP/s), 4096 x 4096 x 1024 252 (136 TFLOP/s of 157).
+// 2048 x 2048 x 1024 123 -> 71 on the large tile (121 TFLOP/s).
 #pragma once
 #include "gemm_loader.h"
 
 namespace gemm_impl {
 
-// BT x BT tile, 2 x WGN waves, K step of 128 bytes, two LDS stages.
-template <typename T, bool OutF32, bool A_MC, bool B_MC, int BT, int WGN, bool MIS>
-__global__ __launch_bounds__(2 * WGN * 64) void gemm_ragged_kernel(typename AnyType<T>::Params p) {
+// Every wave's LDS stores are done and its reads have returned (global loads stay in flight).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+constexpr int ragged_lds_bytes(int bt) { return 4 * bt * 128; }
+
+// The products of a BT x BT tile at (m0, n0): 2 x WGN waves, K step of 128 bytes, two LDS stages.
+// acc[i][j][e] is out[m][n], m = m0 + 32 TM wm + 32 i + lane % 32, n = n0 + 32 TN wn + 32 j + 8 (e / 4) + 4 (lane / 32) + e % 4.
+template <typename T, bool A_MC, bool B_MC, int BT, int WGN, bool MIS>
+__device__ __forceinline__ void ragged_products(const typename AnyType<T>::Params& p, int m0, int n0, int64_t bz, int tid, char* lds,
+                                                floatx16 (&acc)[BT / 64][BT / WGN / 32]) {
   constexpr int BK = 128 / sizeof(T), KS = AnyType<T>::KS;
   constexpr int NT = 2 * WGN * 64, TM = BT / 64, TN = BT / WGN / 32;
   constexpr int OP_BYTES = BT * 128, STAGE = 2 * OP_BYTES;
+  static_assert(ragged_lds_bytes(BT) == 2 * STAGE, "two stages");
   typedef typename Elem<T>::vec8 V8;
   typedef AnyLoader<T, A_MC, BT, NT, MIS> LoaderA;
   typedef AnyLoader<T, B_MC, BT, NT, MIS> LoaderB;
-  __shared__ __attribute__((aligned(1024))) char lds[2 * STAGE];
-
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
-
-  request_first_args(p);
-  const TileAt tile = tile_at(blockIdx.x, p.order);
-  const int m0 = tile.m * BT, n0 = tile.n * BT;
-
-  const int64_t bz = blockIdx.z;
   const int64_t k0 = bz * p.kslice;  // K slices (kslice > 0): grid member z takes k0 .. k0 + kslice - 1
   const int K = p.kslice ? min(p.K - (int)k0, p.kslice) : p.K;
   LoaderA la;
@@ -41,7 +44,6 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_ragged_kernel(typename AnyT
   la.init(reinterpret_cast<const T*>(p.a) + bz * p.sa, p.lda, m0, p.M, k0, p.K, tid);
   lb.init(reinterpret_cast<const T*>(p.b) + bz * p.sb, p.ldb, n0, p.N, k0, p.K, tid);
 
-  floatx16 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -64,17 +66,11 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_ragged_kernel(typename AnyT
     la.store(stage, g.a);
     lb.store(stage + OP_BYTES, g.b);
   };
-  // Every wave's LDS stores are done and its reads have returned (global loads stay in flight).
-  auto barrier = [&] {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-  };
   load(even);
   if (TWO && KT > 1) load(odd);
   store(even, lds);
   if (KT > (TWO ? 2 : 1)) load(even);
-  barrier();
+  lds_barrier();
 
   AnyFrag<T, A_MC, BT, TM> faddr;
   AnyFrag<T, B_MC, BT, TN> fbddr;
@@ -97,7 +93,7 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_ragged_kernel(typename AnyT
       if constexpr (ks + 1 < KS) {
         read_frags(cur, ks + 1, (ks + 1) & 1);
       } else {
-        barrier();
+        lds_barrier();
         read_frags(nxt, 0, KS & 1);
       }
       mma_block<T, TM, TN>(acc, fa[ks & 1], fb[ks & 1]);
@@ -122,9 +118,25 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_ragged_kernel(typename AnyT
     for (int j = 0; j < TN; ++j) mask_fragment<T>(fb[ks & 1][j], ks, lane, tail);
     mma_block<T, TM, TN>(acc, fa[ks & 1], fb[ks & 1]);
   });
+}
 
-  // acc[i][j][e] is out[m][n], m = m0 + 32 TM wm + 32 i + lane % 32, n = n0 + 32 TN wn + 32 j + 8 (e / 4) + 4 (lane / 32) + e % 4.
-  barrier();  // every wave has read its last fragments
+// The same tile as a kernel of its own.
+template <typename T, bool OutF32, bool A_MC, bool B_MC, int BT, int WGN, bool MIS>
+__global__ __launch_bounds__(2 * WGN * 64) void gemm_ragged_kernel(typename AnyType<T>::Params p) {
+  constexpr int TM = BT / 64, TN = BT / WGN / 32;
+  __shared__ __attribute__((aligned(1024))) char lds[ragged_lds_bytes(BT)];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WGN, wn = wave % WGN;
+
+  request_first_args(p);
+  const TileAt tile = tile_at(blockIdx.x, p.order);
+  const int m0 = tile.m * BT, n0 = tile.n * BT;
+  const int64_t bz = blockIdx.z;
+  floatx16 acc[TM][TN];
+  ragged_products<T, A_MC, B_MC, BT, WGN, MIS>(p, m0, n0, bz, tid, lds, acc);
+
+  lds_barrier();  // every wave has read its last fragments
   typename AnyType<T>::template Epilogue<OutF32> epi(p, bz);
   store_tile<typename AnyType<T>::Out, OutF32>(epi, acc, lds + wave * (TN * 4096), member_out(p, bz), p.ldc, bz * p.sc, p.M, p.N, m0 + wm * 32 * TM,
                         n0 + wn * 32 * TN, lane);
@@ -136,15 +148,14 @@ void launch_ragged_tile(typename AnyType<T>::Params& p, int batch, int tile, hip
   p.tiles_n = (int)xmk::ceil_div(p.N, tile);
   p.order = tile_order((uint32_t)p.tiles_m, (uint32_t)p.tiles_n, p.K);
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n), 1, (unsigned)batch);
-  constexpr int WGN = sizeof(T) == 4 ? 4 : 2;
   if constexpr (sizeof(T) != 2) {  // (16-bit operands without misaligned rows take the direct kernels)
     if (!p.misaligned) {
-      if (tile == 128) hipLaunchKernelGGL((gemm_ragged_kernel<T, OutF32, A_MC, B_MC, 128, WGN, false>), grid, dim3(WGN * 128), 0, st, p);
+      if (tile == 128) hipLaunchKernelGGL((gemm_ragged_kernel<T, OutF32, A_MC, B_MC, 128, 2, false>), grid, dim3(256), 0, st, p);
       else hipLaunchKernelGGL((gemm_ragged_kernel<T, OutF32, A_MC, B_MC, 64, 2, false>), grid, dim3(256), 0, st, p);
       return;
     }
   }
-  if (tile == 128) hipLaunchKernelGGL((gemm_ragged_kernel<T, OutF32, A_MC, B_MC, 128, WGN, true>), grid, dim3(WGN * 128), 0, st, p);
+  if (tile == 128) hipLaunchKernelGGL((gemm_ragged_kernel<T, OutF32, A_MC, B_MC, 128, 2, true>), grid, dim3(256), 0, st, p);
   else hipLaunchKernelGGL((gemm_ragged_kernel<T, OutF32, A_MC, B_MC, 64, 2, true>), grid, dim3(256), 0, st, p);
 }
 
