@@ -430,10 +430,10 @@ __device__ __forceinline__ void bwd_pass(const std::conditional_t<SAVE_DS, Saved
     }
     float bs[BIAS ? 2 : 1][16];
     if constexpr (BIAS) load_bias(t0, bs);
-    // The dK launch of the larger head sizes holds both owner operands, the accumulators and the scores of
-    // a whole block only with spills (30 registers): it goes through the block's two halves one after the
-    // other, so that one half's scores are dead before the other's are made.
-    constexpr bool BY_HALF = DS && ((OWNER_K && HP >= 128) || HP > 128);
+    // With both owner operands and the accumulators of the larger head sizes there are registers for the scores of half a
+    // block: one half's are dead before the other's are made.  (A whole block's: the dK launch spills 30 registers, the
+    // dQ launch has none left in which to read fragments ahead of their products, 526 -> 499 us at [8,32,2048,128] causal.)
+    constexpr bool BY_HALF = DS && HP >= 128;
     floatx16 sc[2], dp[2];
     if constexpr (!BY_HALF) {
       scores(c1, of1, sc);
@@ -516,14 +516,17 @@ __device__ __forceinline__ void bwd_pass(const std::conditional_t<SAVE_DS, Saved
   };
 
   if (b0 < b1) {
-    issue_tile(Str1, b0 * BS, s1 + (b0 & 1) * TILE);
-    issue_tile(Str2, b0 * BS, s2 + (b0 & 1) * TILE);
-    if constexpr (OWNER_K) issue_stats(b0 * BS, sst + (b0 & 1) * STATS);
+    issue_tile(Str1, b0 * BS, s1);
+    issue_tile(Str2, b0 * BS, s2);
+    if constexpr (OWNER_K) issue_stats(b0 * BS, sst);
     __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(0));
     __builtin_amdgcn_s_barrier();
-    for (int it = b0; it < b1; ++it) {
-      if (it & 1) block(it, s1 + TILE, s2 + TILE, sst + STATS, s1, s2, sst);
-      else block(it, s1, s2, sst, s1 + TILE, s2 + TILE, sst + STATS);
+    // Two blocks a turn: with the stages picked by a block's parity instead, the two copies of the block met at every turn, and
+    // the accumulators were moved from one's registers to the other's (64 moves a block; 4 heads of 4096 x 128 154 -> 129 us
+    // together with the half blocks, 16 x 2048 heads of 64 157 -> 146, 32 x 4096 of 160 913 -> 821).
+    for (int it = b0; it < b1; it += 2) {
+      block(it, s1, s2, sst, s1 + TILE, s2 + TILE, sst + STATS);
+      if (it + 1 < b1) block(it + 1, s1 + TILE, s2 + TILE, sst + STATS, s1, s2, sst);
     }
   }
 
