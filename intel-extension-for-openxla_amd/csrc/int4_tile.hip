@@ -16,20 +16,28 @@
 // work-group expands them again, and they are kept in registers for all row tiles.  The activations come in through LDS
 // (two buffers, one step of 128 WK k each), the weights two steps ahead in registers.
 //
-// What bounds it: a wave's step is 24 RT matrix instructions (16 RT of them the product, 8 RT the sums of a) and 128 vector
-// instructions for the expansion, 64 RT for scales and zero points; with one wave per SIMD the two add up unless interleaved
-// (kPipe), and two hardly overlap them either (512 x 4096 x 16384: matrix pipe busy 59 % of the launch, vector instructions
-// issuing 54 %, the waves wait 48 % of their time to issue).  Microseconds a call, weights from memory, group 128, against
-// passes of 32 rows, each of which expands all weights, and against writing the fp16 weights out and the dense product on
-// them, all on one device: k 4096, n 16384: 64 rows 22.2 / 25.8 / 52.5, 96 27.6 / 38.4 / 54.5, 128 28.9 / 50.6 / 55.9,
-// 256 49.4 / 100 / 68.8, 512 86.7 / 199 / 93.3; k 16384, n 4096: 64 rows 32.3 / 41.6 / 76.4, 128 36.9 / 80.7 / 84.0.
+// What bounds it: a wave's step of 128 k is 16 RT matrix instructions of 32 cycles, 128 vector instructions for the expansion
+// (in the shadow of the former: up to six per matrix instruction cost nothing) and 32 RT for the scales.  The sums of a were
+// 8 RT more matrix instructions of 32 cycles, whose 32 columns were all the same, and 32 RT more vector instructions took zero
+// points off; now they are 16 RT of four by four, 8 cycles each and four in a row, since a change from one length to another costs
+// ten cycles (one beside each product: 53 cycles a pair, no gain left), and one fp32 matrix instruction per two groups and 32 x 32
+// results.  Their sums over the four waves that share rows, each a quarter of them, through LDS: no faster (82 us against 81).
+// 512 x 4096 x 16384 at group 128 / 64 / 32: 91 -> 81 us, 104 -> 92, 163 -> 111; of the 81, 12 go with the power limit (69 on
+// zeros) and 11 with staged activations, 8 are the launch, its first loads and its end.  Microseconds a call, weights from memory,
+// group 128, against passes of 32 rows, each of which expands all weights, and against writing the fp16 weights out and the dense
+// product on them: k 4096, n 16384: 64 rows 21.4 / 25.8 / 52.5, 128 29.6 / 50.6 / 55.9, 256 46.6 / 100 / 68.8, 512 81 / 199 / 93.3;
+// k 16384, n 4096: 64 rows 33.2 / 41.6 / 76.4.
 #include "int4_tile.h"
+
+#include <type_traits>
+#include <utility>
 
 #include "common.h"
 
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -41,6 +49,14 @@ constexpr uint32_t kOob = 0x80000000u;
 constexpr int kStepK = 128;  // k a wave takes per step
 constexpr int vmcnt_imm(int n) { return (n & 0xf) | ((n >> 4) << 14) | (0x7 << 4) | (0xf << 8); }
 
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(static_cast<F&&>(f), std::make_integer_sequence<int, N>{});
+}
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
 }
@@ -48,13 +64,10 @@ __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t r, char* lds,
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_ptr)lds, 16, voff, 0, 0, 0);
 }
 
-// The eight nibbles of a word as fp16 16 + q, in the order of k: times 2^6 + 2^18, a byte has its low nibble in bits 6 to 9 of
+// Two nibbles of a word, k = 2 i and 2 i + 1, as fp16 16 + q: times 2^6 + 2^18, a byte has its low nibble in bits 6 to 9 of
 // the lower half and its high nibble in those of the upper one, where 0x4c00 | q << 6 is 16 + q.
-__device__ __forceinline__ half8 expand(uint32_t w, uint32_t magic) {
-  uint32_t h[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) h[i] = (__umul24((w >> (8 * i)) & 0xff, 0x00040040u) & 0x03c003c0u) | magic;
-  return __builtin_bit_cast(half8, u32x4{h[0], h[1], h[2], h[3]});
+__device__ __forceinline__ uint32_t expand(uint32_t w, int i, uint32_t magic) {
+  return (__umul24((w >> (8 * i)) & 0xff, 0x00040040u) & 0x03c003c0u) | magic;
 }
 __device__ __forceinline__ float half_of(uint32_t pair, int c) {
   return (float)__builtin_bit_cast(_Float16, (uint16_t)(pair >> (16 * c)));
@@ -114,7 +127,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 || (RT == 2 && WN > 1 && GS > 32) 
   constexpr int RPL = 4 * NW, NI = BM / RPL;  // a staging load of all waves covers RPL rows: NI loads per wave and 128 of K
   constexpr int NSUB = kStepK / GS;        // scale groups per step
   constexpr int SPG = GS / 16;             // matrix instructions per scale group and tile
-  constexpr bool kPipe = WN == 1 && NW == 4;
+  constexpr bool kDefer = RT == 1;
   constexpr int kWeightLoads = 8 + 2 * NSUB;
   static_assert(BM % RPL == 0, "whole loads");
   __shared__ StageOrSums<STAGE, NW> s0;
@@ -174,16 +187,13 @@ __global__ __launch_bounds__(NW * 64, NW == 8 || (RT == 2 && WN > 1 && GS > 32) 
       o.w[s] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r_w, voff_w + (uint32_t)(k0 / 8 + 2 * s) * (uint32_t)N * 4, 0, 0));
   };
 
+  const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   floatx16 acc[RT][2];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[rt][c][e] = 0.f;
+  for (int rt = 0; rt < RT; ++rt) acc[rt][0] = acc[rt][1] = zero;
   uint32_t magic = 0x4c004c00u;
   asm volatile("" : "+v"(magic));  // (a value the compiler cannot see through: (x & m) | magic is then one instruction)
-  const half8 ones = __builtin_bit_cast(half8, u32x4{0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u});
+  const half4 ones = __builtin_bit_cast(half4, u32x2{0x3c003c00u, 0x3c003c00u});
 
   // fragment of k-step s, row tile rt: row lane % 32, chunk 2 s + lane / 32
   const int frow = lane % 32;
@@ -201,90 +211,116 @@ __global__ __launch_bounds__(NW * 64, NW == 8 || (RT == 2 && WN > 1 && GS > 32) 
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // A chain of matrix instructions ends in 32 sums per lane that go into acc with two multiply-adds each.
-  const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  struct Chain {
-    floatx16 d[2], sum;
-    float sc[2], zz[2];
-  } last{{zero, zero}, zero, {0.f, 0.f}, {0.f, 0.f}};
-  auto fix_up = [&](int rt, int from, int to) {
+  // A scale group's matrix instructions are a chain per row tile and column set; its sums go into acc with a multiply-add each.
+  // What the offset and the zero point added to them comes off acc after every second group: an fp32 product of the row sums of two
+  // groups, even and odd, with their s (16 + z).  acc holds it for two groups at most, so that next to nothing of its precision goes
+  // to sums that cancel.  kDefer (32 rows): a chain's sums are worked in beside the next chain; 64 rows have no registers for that.
+  floatx16 d[kDefer ? 2 : 1][RT][2];
+  float sc[2][2], zz[2][2];  // of an even and an odd group: the scales, and -s (16 + z)
+  float rows[2][RT];         // row sums over the lane's half of each k-step (a lane's column of a four by four product is its own,
+                             // so that an infinite activation stays in its row)
+  if constexpr (kDefer) {
+    d[1][0][0] = d[1][0][1] = zero;
+    sc[1][0] = sc[1][1] = 0.f;
+  }
+  auto fix_up = [&](auto P, auto E) {  // element E of the chains of parity P
+    constexpr int par = decltype(P)::value, e = decltype(E)::value;
 #pragma unroll
-    for (int e = from; e < to; ++e)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int c = 0; c < 2; ++c) acc[rt][c][e] = fmaf(last.sc[c], fmaf(last.zz[c], last.sum[e], last.d[c][e]), acc[rt][c][e]);
+      for (int c = 0; c < 2; ++c) acc[rt][c][e] = fmaf(sc[par][c], d[kDefer ? par : 0][rt][c][e], acc[rt][c][e]);
   };
 
-  // kPipe (one wave per SIMD): the arithmetic between matrix instructions is spread over the chains -- the weights of a
-  // k-step are expanded in front of its first use, a chain's sums are worked in during the next one -- since there is no
-  // second wave to fill the gaps.
-  auto step = [&](int i, char* cur, char* next, Weights& w) {
+  auto step = [&](auto ODD, int i, char* cur, char* next, Weights& w) {
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(kWeightLoads));  // this step's activations have landed; the next step's weights may be out
     __builtin_amdgcn_s_barrier();                         // for every wave, and the other buffer has been read
     __builtin_amdgcn_sched_barrier(0);
+    half8 a[2][RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) a[0][rt] = fragment(cur, 0, rt);
     stage(i + 1, next);
     asm volatile("" : "+v"(magic) : : "memory");
     __builtin_amdgcn_sched_barrier(0);
-    float sc[NSUB][2], zz[NSUB][2];
+    uint32_t b[2][2][4];
 #pragma unroll
-    for (int u = 0; u < NSUB; ++u)
+    for (int x = 0; x < 8; ++x) b[0][x / 4][x % 4] = expand(w.w[0][x / 4], x % 4, magic);
+    static_for<NSUB>([&](auto U) {
+      constexpr int u = decltype(U)::value, par = NSUB > 1 ? u & 1 : decltype(ODD)::value;
+      floatx4 sum[2][RT];
+      if constexpr (!kDefer) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) sc[par][c] = half_of(w.s[u], c);
+      }
+      static_for<SPG>([&](auto J) {
+        constexpr int j = decltype(J)::value, s = u * SPG + j;
+        static_for<2 * RT>([&](auto R) {
+          constexpr int r = decltype(R)::value, rt = r / 2, c = r % 2;
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (s < 7 && c == 0) a[(s + 1) & 1][rt] = fragment(cur, s + 1, rt);
+          auto& to = d[kDefer ? par : 0][rt][c];
+          to = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[s & 1][rt], __builtin_bit_cast(half8, u32x4{b[s & 1][c][0], b[s & 1][c][1], b[s & 1][c][2], b[s & 1][c][3]}),
+                                                      j == 0 ? zero : to, 0, 0, 0);
+          if constexpr (s < 7) {
+#pragma unroll
+            for (int x = 4 * r / RT; x < 4 * (r + 1) / RT; ++x) b[(s + 1) & 1][x / 4][x % 4] = expand(w.w[s + 1][x / 4], x % 4, magic);
+          }
+          if constexpr (kDefer) {
+            constexpr int slot = j * 2 * RT + r, slots = SPG * 2 * RT;
+            static_for<16>([&](auto E) {
+              constexpr int e = decltype(E)::value;
+              if constexpr (e >= 16 * slot / slots && e < 16 * (slot + 1) / slots) fix_up(std::integral_constant<int, 1 - par>{}, E);
+            });
+          }
+        });
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          const half8 v = a[s & 1][rt];
+          const floatx4 none = {0.f, 0.f, 0.f, 0.f};
+          sum[0][rt] = __builtin_amdgcn_mfma_f32_4x4x4f16(ones, __builtin_shufflevector(v, v, 0, 1, 2, 3), j == 0 ? none : sum[0][rt], 0, 0, 0);
+          sum[1][rt] = __builtin_amdgcn_mfma_f32_4x4x4f16(ones, __builtin_shufflevector(v, v, 4, 5, 6, 7), j == 0 ? none : sum[1][rt], 0, 0, 0);
+        }
+      });
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
-        sc[u][c] = half_of(w.s[u], c);
-        zz[u][c] = -16.f - half_of(w.z[u], c);
-        asm volatile("" : "+v"(sc[u][c]), "+v"(zz[u][c]));  // (in registers of their own before the fetch below reuses w)
+        if constexpr (kDefer) sc[par][c] = half_of(w.s[u], c);
+        zz[par][c] = fmaf(-half_of(w.s[u], c), half_of(w.z[u], c), -16.f * half_of(w.s[u], c));
+        asm volatile("" : "+v"(sc[par][c]), "+v"(zz[par][c]));  // (in registers of their own before the fetch below reuses w)
       }
-    half8 b[8][2];
-    if constexpr (!kPipe) {
 #pragma unroll
-      for (int s = 0; s < 8; ++s)
+      for (int rt = 0; rt < RT; ++rt) rows[par][rt] = sum[0][rt][0] + sum[1][rt][0];
+      if constexpr (u == NSUB - 1) fetch_pinned(i + 2, w);
+      if constexpr (par == 1) {
+        float off[2];
 #pragma unroll
-        for (int c = 0; c < 2; ++c) b[s][c] = expand(w.w[s][c], magic);
-      fetch_pinned(i + 2, w);
-    }
-    // chain q: scale group q / RT, row tile q % RT
-    half8 a = fragment(cur, 0, 0);
+        for (int c = 0; c < 2; ++c) off[c] = lane < 32 ? zz[0][c] : zz[1][c];
 #pragma unroll
-    for (int q = 0; q < NSUB * RT; ++q) {
-      const int u = q / RT, rt = q % RT, before = (q + RT - 1) % RT;
-      floatx16 d0 = zero, d1 = zero, sum = zero;
+        for (int rt = 0; rt < RT; ++rt) {
+          // The upper lanes' half of the even group for the lower lanes' half of the odd one: the even group's sum then lies
+          // in the lower lanes, the odd one's in the upper lanes.
+          asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(rows[0][rt]), "+v"(rows[1][rt]));
+          const float both = rows[0][rt] + rows[1][rt];
 #pragma unroll
-      for (int j = 0; j < SPG; ++j) {
-        const int s = u * SPG + j;
-        if constexpr (kPipe) {
-          if (rt == 0) {
-            b[s][0] = expand(w.w[s][0], magic);
-            b[s][1] = expand(w.w[s][1], magic);
-          }
-        }
-        const int nj = (j + 1) % SPG, nq = nj == 0 ? q + 1 : q;
-        const half8 now = a;
-        if (nq < NSUB * RT) a = fragment(cur, nq / RT * SPG + nj, nq % RT);
-        sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(now, ones, sum, 0, 0, 0);
-        d0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(now, b[s][0], d0, 0, 0, 0);
-        d1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(now, b[s][1], d1, 0, 0, 0);
-        if constexpr (kPipe) {
-          fix_up(before, j * 16 / SPG, (j + 1) * 16 / SPG);
-          __builtin_amdgcn_sched_barrier(0);
+          for (int c = 0; c < 2; ++c) acc[rt][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(both, off[c], acc[rt][c], 0, 0, 0);
         }
       }
-      last.d[0] = d0; last.d[1] = d1; last.sum = sum;
-#pragma unroll
-      for (int c = 0; c < 2; ++c) last.sc[c] = sc[u][c], last.zz[c] = zz[u][c];
-      if constexpr (!kPipe) fix_up(rt, 0, 16);
-    }
-    if constexpr (kPipe) fetch_pinned(i + 2, w);
+      if constexpr (!kDefer) static_for<16>([&](auto E) { fix_up(std::integral_constant<int, par>{}, E); });
+    });
   };
 
   Weights w0, w1;
   fetch(0, w0);
   stage(0, s0.stage);
   fetch_pinned(1, w1);
+  typedef std::integral_constant<int, 0> Even;
+  typedef std::integral_constant<int, 1> Odd;
   for (int i = 0; i < steps; i += 2) {  // (an odd count ends on a step of zeros)
-    step(i, s0.stage, s1, w0);
-    step(i + 1, s1, s0.stage, w1);
+    step(Even{}, i, s0.stage, s1, w0);
+    step(Odd{}, i + 1, s1, s0.stage, w1);
   }
-  if constexpr (kPipe) fix_up(RT - 1, 0, 16);
+  if constexpr (kDefer) static_for<16>([&](auto E) { fix_up(Odd{}, E); });
 
   // Sums over the waves that split K, in wave order, one row tile after the other through LDS; a thread then owns eight
   // columns of a row.
@@ -355,14 +391,14 @@ Shape choose(int64_t m, int64_t k, int64_t n, int64_t group) {
   auto pairs = [](int64_t r, double two, double one) { return (double)(r / 2) * two + (double)(r % 2) * one; };
   // 32 rows: few work-groups, so all eight waves on one reduction where there is a single round of them
   // (64 x 16384 x 4096: 32.1 us against 37.2; two rounds, 256 x 4096 x 4096: 22.7 against 19.2)
-  // Scales and zero points of groups of 32 are four times the work of those of 128: 1.15 to 1.6 times the whole, the wide
-  // shapes most (214 x 7264 x 5768: 83 us where groups of 128 take 51).
-  const double g8 = group == 32 ? 1.15 : 1.0, g4 = group == 32 ? 1.35 : 1.0, gw = group == 32 ? 1.6 : 1.0;
-  Shape best = slim == 1 && k > 1024 ? Shape{Shape::kSlim8, 5.0 + 1.95 * g8 * steps(1024)}
-                                     : Shape{Shape::kSlim4, 4.0 + 1.03 * g4 * steps(512) * (double)slim};
-  const Shape others[] = {wide == 1 && k > 512 ? Shape{Shape::kWide8, 5.4 + 2.85 * gw * steps(512)}
-                                               : Shape{Shape::kWide4, 4.6 + gw * steps(256) * pairs(wide, 2.7, 1.65)},
-                          Shape{Shape::kBroad4, 4.6 + gw * steps(128) * pairs(broad, 2.6, 1.7)}};
+  // Scales and zero points of groups of 32 are four times the work of those of 128 (512 x 4096 x 16384: 111 us where groups of
+  // 128 take 81), the wide shapes' the most.
+  const double g8 = group == 32 ? 1.15 : 1.0, g4 = group == 32 ? 1.25 : 1.0, gw = group == 32 ? 1.35 : group == 64 ? 1.1 : 1.0;
+  Shape best = slim == 1 && k > 1024 ? Shape{Shape::kSlim8, 5.0 + 1.84 * g8 * steps(1024)}
+                                     : Shape{Shape::kSlim4, 4.0 + 0.98 * g4 * steps(512) * (double)slim};
+  const Shape others[] = {wide == 1 && k > 512 ? Shape{Shape::kWide8, 5.4 + 2.65 * gw * steps(512)}
+                                               : Shape{Shape::kWide4, 4.6 + gw * steps(256) * pairs(wide, 2.5, 1.45)},
+                          Shape{Shape::kBroad4, 4.6 + gw * steps(128) * pairs(broad, 2.35, 1.4)}};
   for (const Shape& s : others)
     if (s.us < best.us) best = s;
   return best;
