@@ -236,7 +236,7 @@ int elem_size(int dtype) {
 
 // What runs a policy's tile: the kernels that take any alignment have names of their own.
 const char* kernel_name(int policy, bool any_alignment) {
-  if (!any_alignment || policy >= kSlicesPolicy) return kPolicies[policy].name;
+  if (!any_alignment || is_slices(policy)) return kPolicies[policy].name;
   return kPolicies[policy].bm == 128 ? "ragged_128x128" : "ragged_64x64";
 }
 // Whether an operand is long enough for the loaders of those kernels, which read 16 bytes at a time.
@@ -635,7 +635,7 @@ int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int p
       else if (dout == XMK_F32) f(_Float16{}, std::true_type{});
       else f(_Float16{}, std::false_type{});
     };
-    if (pol >= kSlicesPolicy) {
+    if (is_slices(pol)) {
       typed([&](auto t, auto o) { launch_slices<decltype(t), decltype(o)::value>(a_mc, b_mc, pol - kSlicesPolicy, p, batch, st); });
       return xmk::check_launch("gemm");
     }

@@ -694,10 +694,16 @@ constexpr Policy kPolicies[] = {
     {"slices_32x64_w8", 32, 64, 8, 1, 64, 2, true, true},
     {"slices_64x64_w4", 64, 64, 4, 1, 64, 2, false, true},
     {"slices_64x64_w8", 64, 64, 8, 1, 64, 2, true, true},
+    // between the 128 x 128 and the 256 x 128 tile, for outputs that those leave CUs idle or nearly empty rounds with:
+    // 1152 x 4096 x 4096 47.8 -> 40.7 us, 768 x 8192 x 4096 (B [n,k]) 60.6 -> 52.6, 1024 x 5056 x 2048 28.9 -> 26.7
+    {"mfma_192x128x64_w2x2_s4", 192, 128, 2, 2, 64, 4, true, false},
 };
 constexpr int kNumPolicies = sizeof(kPolicies) / sizeof(kPolicies[0]);
 constexpr int kRowsPolicy = 5;
 constexpr int kSlicesPolicy = 6;        // first of the slices variants
+constexpr int kNumSlices = 6;
+constexpr bool is_slices(int policy) { return policy >= kSlicesPolicy && policy < kSlicesPolicy + kNumSlices; }
+constexpr int k192Policy = 12;
 constexpr int kRowsMaxM = 8;            // rows the streaming kernel takes
 constexpr int kRowsMinBN = 64;          // its output columns per work-group: 64, 128, 256 or 512
 constexpr int kRowsEnoughBlocks = 192;  // work-groups from which on a launch pulls the memory system's rate
@@ -757,6 +763,8 @@ enum : int { kClassKN = 0, kClassNK = 1, kClassRagged = 2, kClassF32 = 3 };
 // 7 %, the worst by 78 % (609 x 1568 x 6968; the streaming kernel for [n,k] apart: 4 x 13536 x 80 takes it 14 us, a tile 4).
 // With scratch, against every tile on 1 to 8 slices, 500 to 730 shapes per class, it is level on aligned operands (copies and
 // streams are no tiles), any alignment and fp32 3 %, one in ten by more than 7 to 10 %, the worst by 34 %.
+// The 192 x 128 tile's rows: chosen for what they pick beside the others, on 855 shapes of more than 100 tiles of 128 x 128 (taken for
+// 200 of them, which it makes 13 % faster on average, nine 2 to 5 % slower).
 // Looking all candidates over takes the host 0.15 to 0.65 us per call.
 struct TileCost {
   float start, step, more_step, more, fill;
@@ -775,6 +783,7 @@ constexpr TileCost kTileCost[4][kNumPolicies] = {
      {2.953f, 1.099f, 0.213f, 2.398f, 1.076f},
      {3.747f, 0.862f, 0.313f, 3.855f, 1.603f},
      {3.11f, 1.488f, 0.285f, 3.156f, 1.679f},
+     {4.669f, 0.509f, 0.831f, 4.313f, 1.555f},
     },
     {  // 16-bit direct, B stored [N, K]
      {8.272f, 0.959f, 1.836f, 11.842f, 5.729f},
@@ -789,6 +798,7 @@ constexpr TileCost kTileCost[4][kNumPolicies] = {
      {2.982f, 1.019f, 0.208f, 2.326f, 1.129f},
      {3.735f, 0.806f, 0.31f, 3.754f, 1.666f},
      {2.945f, 1.596f, 0.302f, 3.078f, 2.018f},
+     {4.41f, 0.482f, 0.815f, 3.821f, 1.96f},
     },
     {  // 16-bit, any alignment
      {},
@@ -824,7 +834,11 @@ constexpr float kSplitCost = 4.0f, kSplitFloor = 8.0f;
 
 // kt: K steps of 128 bytes.
 inline float launch_cost(const Policy& P, const TileCost& c, bool slices, uint32_t m, uint32_t n, uint32_t kt, uint32_t batch) {
-  auto blocks = [](uint32_t v, int b) { return (v + b - 1) >> __builtin_ctz((unsigned)b); };  // b: a power of two
+  auto blocks = [](uint32_t v, int b) {  // b: a power of two, or three times one
+    const int shift = __builtin_ctz((unsigned)b);
+    const uint32_t units = (v + (1u << shift) - 1) >> shift;
+    return b >> shift == 3 ? (units + 2) / 3 : units;
+  };
   const uint64_t tiles = (uint64_t)blocks(m, P.bm) * blocks(n, P.bn) * batch;
   const float load = (float)tiles * (1.0f / 256);
   const uint32_t ktw = slices ? blocks(kt, P.wgm) : kt;
@@ -846,7 +860,12 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
     for (int pol = 0; pol < kNumPolicies; ++pol) {
       if (pol == kRowsPolicy || (!direct && !kPolicies[pol].any_alignment)) continue;
       const uint32_t kt = (uint32_t)(((k + s - 1) / s + kstep - 1) / kstep);
-      const float cost = std::max(launch_cost(kPolicies[pol], kTileCost[cls][pol], pol >= kSlicesPolicy, (uint32_t)m, (uint32_t)n, kt,
+      // The 192 x 128 tile is not for short reductions, whose time is the output's (7102 x 1408 x 64 11 % slower), nor for long ones
+      // where the 256-row tile takes as many: the last of that one's tile rows is the emptier, which gives the others clock and
+      // load path (560 x 10240 x 12288 141 us against 159; 560 x 10240 x 2048 30.1 against 27.3).
+      // With K slices its estimate is too low (161 x 3553 x 12725 62.8 us, with it 72.4).
+      if (pol == k192Policy && (s > 1 || kt < 6 || (kt > 32 && xmk::ceil_div(m, 192) == xmk::ceil_div(m, 256)))) continue;
+      const float cost = std::max(launch_cost(kPolicies[pol], kTileCost[cls][pol], is_slices(pol), (uint32_t)m, (uint32_t)n, kt,
                                               (uint32_t)(batch * s)) + extra, least);
       if (cost < best.us) best = {pol, s, cost};
     }
@@ -884,6 +903,7 @@ void launch_mfma(const GemmParams& p, int batch, hipStream_t st) {
 
 template <typename T, bool OutF32, bool A_MC, bool B_MC>
 void launch_policy(int pol, GemmParams& p, int batch, hipStream_t st) {
+  if (A_MC && pol == k192Policy) pol = 4;  // (rows of 192 elements are no whole number of loads)
   p.tiles_m = (int)xmk::ceil_div(p.M, kPolicies[pol].bm);
   p.tiles_n = (int)xmk::ceil_div(p.N, kPolicies[pol].bn);
   p.order = tile_order((uint32_t)p.tiles_m, (uint32_t)p.tiles_n, p.K);
@@ -892,6 +912,9 @@ void launch_policy(int pol, GemmParams& p, int batch, hipStream_t st) {
     case 1: launch_mfma<T, OutF32, A_MC, B_MC, 128, 128, 2, 2, 64, 4>(p, batch, st); break;
     case 2: launch_mfma<T, OutF32, A_MC, B_MC, 128, 64, 2, 2, 64, 4>(p, batch, st); break;
     case 4: launch_mfma<T, OutF32, A_MC, B_MC, 256, 128, 2, 2, 64, 3>(p, batch, st); break;
+    case k192Policy:
+      if constexpr (!A_MC) launch_mfma<T, OutF32, A_MC, B_MC, 192, 128, 2, 2, 64, 4>(p, batch, st);
+      break;
     default: launch_mfma<T, OutF32, A_MC, B_MC, 64, 64, 2, 2, 64, 4>(p, batch, st); break;
   }
 }
