@@ -182,7 +182,14 @@ __global__ __launch_bounds__(NW * 64) void int4_gemm_kernel(Int4Problem p0, Int4
   // which are half a grid apart -- the ones that end up sharing a CU -- belong to different products
   // and every CU gets the same share of the longer reduction.
   const bool second = (SK && mixed) ? (((int)blockIdx.x + (int)(blockIdx.y >> 1)) & 1) != 0 : (int)blockIdx.x >= blocks0;
-  const int bx = (SK && mixed) ? (int)blockIdx.x >> 1 : (int)blockIdx.x - (second ? blocks0 : 0);
+  int bx = (SK && mixed) ? (int)blockIdx.x >> 1 : (int)blockIdx.x - (second ? blocks0 : 0);
+  // Blocks of one or two words per lane cover 64 or 128 bytes of a row of weights and share cache lines with their
+  // neighbours: two neighbours go to one XCD (sixteen blocks at a time; what is left keeps its order).  2 x 12544 x 4056 12.6
+  // -> 10.6 us, 4 x 3584 x 7192 6.7 -> 6.1, 150 drawn sizes 2 % on the mean.
+  if constexpr (W < 4 && !SK) {
+    const int blocks = second ? (int)gridDim.x - blocks0 : blocks0;
+    if ((bx | 15) < blocks) bx = (bx & ~15) | (bx & 7) << 1 | (bx >> 3 & 1);
+  }
   const _Float16* __restrict__ act = second ? p1.act : p0.act;
   const uint32_t* __restrict__ qw = second ? p1.qw : p0.qw;
   const _Float16* __restrict__ scales = second ? p1.scales : p0.scales;
@@ -682,10 +689,10 @@ int prepare(const xmk::Int4Call& c, int64_t m, int64_t group, Config* cfg) {
   if (!xmk::aligned(c.act, 16) || !xmk::aligned(c.qweight, 16) || !xmk::aligned(c.scales, 8) ||
       !xmk::aligned(c.zeros, 8) || !xmk::aligned(c.out, 2))
     return xmk::fail(XMK_INVALID_ARGUMENT, "int4_gemm: act, qweight must be 16-byte and scales, zeros 8-byte aligned");
-  // Words per lane: the widest load that still yields about one block per CU.
-  cfg->w = 4;
-  if (n / 64 < 192) cfg->w = 2;
-  if (n / 32 < 192) cfg->w = 1;
+  // Words per lane: the fewest whose blocks still are one round of the 256 CUs.  (With as many words as leave 192 blocks, 260 to
+  // 380 blocks ran in two rounds, or in work-groups of four waves which have too few loads in flight: 16 x 9728 x 4424
+  // 18.6 -> 12.8 us, 5 x 6656 x 5544 in groups of 32 19.9 -> 12.5, 1 x 10368 x 10152 23.2 -> 18.1.)
+  cfg->w = n <= 256 * 16 ? 1 : n <= 256 * 32 ? 2 : 4;
   cfg->nw = 16;
   if (forced_tile()) {
     int ew = 0, enw = 0;

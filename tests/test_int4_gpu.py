@@ -310,3 +310,20 @@ def test_int4_errors(xmk):
     with pytest.raises(xmk.XmkError) as e:
         xmk.int4_gemm_ws(a2, qw, sz, sz, out2, ws, group=8)
     assert e.value.code == xmk.UNIMPLEMENTED
+
+
+@pytest.mark.parametrize("m", [1, 3, 7, 16, 20])
+@pytest.mark.parametrize("n", [8, 232, 240, 256, 272, 504, 1032, 4096, 4104, 4608, 8192, 8200])
+def test_int4_gemm_every_block_once(xmk, m, n):
+    """Numbers of column blocks on both sides of the lines between block widths, and of sixteen: whole numbers with scale 1 and
+    zero point 0, whose sums (below 64 * 15) fp16 holds exactly."""
+    k, group = 64, 32
+    g = torch.Generator(device="cuda").manual_seed(n + m)
+    act = torch.randint(-1, 2, (m, k), generator=g, device="cuda").half()
+    qw = torch.randint(-2 ** 31, 2 ** 31, (k // 8, n), generator=g, device="cuda", dtype=torch.int32)
+    s, z = torch.ones((k // group, n), device="cuda").half(), torch.zeros((k // group, n), device="cuda").half()
+    out = torch.full((m, n), float("nan"), device="cuda", dtype=torch.float16)
+    xmk.int4_gemm(act, qw, s, z, out, group=group)
+    shifts = torch.arange(0, 32, 4, device="cuda", dtype=torch.int32)
+    q = ((qw[:, None, :] >> shifts[None, :, None]) & 15).reshape(k, n)
+    assert torch.equal(out.double().cpu(), act.double().cpu() @ q.double().cpu())
