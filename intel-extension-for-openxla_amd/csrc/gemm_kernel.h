@@ -67,6 +67,13 @@ __device__ __forceinline__ float gelu_tanh(float x) {
   const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
   return x / (1.0f + __expf(-2.0f * u));
 }
+// The same for results of 16 bits, which do not show the reciprocal's last bit (error against float64 the same to seven digits):
+// eight instructions, where the division alone takes ten.  A large tile has one wave per SIMD and nothing beside its epilogue:
+// 1659 x 11592 x 120 47.4 -> 36.8 us, 6870 x 3856 x 936 89.6 -> 78.7, 1023 x 5003 x 2047 with scratch 42.9 -> 38.5.
+__device__ __forceinline__ float gelu_tanh_16(float x) {
+  constexpr float k1 = -2.0f * 0.7978845608028654f * 1.4426950408889634f;
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * __builtin_fmaf(0.044715f * k1, x * x, k1)));
+}
 
 __device__ __forceinline__ float apply_act(float v, int act) {
   if (act == ACT_RELU) return fmaxf(v, 0.0f);
@@ -395,7 +402,7 @@ struct GemmEpilogue {
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[u][e] = gelu_tanh(v[u][e]);
+        for (int e = 0; e < 8; ++e) v[u][e] = OutF32 || sizeof(T) == 4 ? gelu_tanh(v[u][e]) : gelu_tanh_16(v[u][e]);
     }
   }
 };
