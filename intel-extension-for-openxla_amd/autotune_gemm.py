@@ -26,7 +26,8 @@ TABLE = os.path.join(HERE, "csrc", "gemm_policy_table.h")
 # kPolicies of csrc/gemm_kernel.h, in its order
 POLICIES = ["mfma_256x256x32_w2x2_s4", "mfma_128x128x64_w2x2_s4", "mfma_128x64x64_w2x2_s4", "mfma_64x64x64_w2x2_s4",
             "mfma_256x128x64_w2x2_s3", "stream_rows_8x512_w8", "slices_32x32_w4", "slices_32x32_w8", "slices_32x32_w16",
-            "slices_32x64_w8", "slices_64x64_w4", "slices_64x64_w8", "mfma_192x128x64_w2x2_s4"]
+            "slices_32x64_w8", "slices_64x64_w4", "slices_64x64_w8", "mfma_192x128x64_w2x2_s4",
+            "mfma_128x128x32_w2x2_s3"]
 # The streaming kernel takes at most eight rows: forced on a shape it cannot take, the library falls back to its own
 # choice, so such a candidate simply repeats the rule's time.
 STREAM, STREAM_ROWS = POLICIES.index("stream_rows_8x512_w8"), 8

@@ -704,13 +704,18 @@ constexpr Policy kPolicies[] = {
     // between the 128 x 128 and the 256 x 128 tile, for outputs that those leave CUs idle or nearly empty rounds with:
     // 1152 x 4096 x 4096 47.8 -> 40.7 us, 768 x 8192 x 4096 (B [n,k]) 60.6 -> 52.6, 1024 x 5056 x 2048 28.9 -> 26.7
     {"mfma_192x128x64_w2x2_s4", 192, 128, 2, 2, 64, 4, true, false},
+    // three work-groups on a CU, so that one's epilogue runs beside the others' loads and products: large outputs of short
+    // reductions, where a tile alone on its CU does one after the other (8072 x 4544 x 256 50.8 -> 33.1 us, 7553 x 2640 x 152
+    // 31.5 -> 19.7, 3094 x 6104 x 504 46.4 -> 35.9; 4096^3 150.8 against 110).  256 x 128 likewise, two of them: ahead of all
+    // others by 6 % on one shape in fifty, left out.
+    {"mfma_128x128x32_w2x2_s3", 128, 128, 2, 2, 32, 3, false, false},
 };
 constexpr int kNumPolicies = sizeof(kPolicies) / sizeof(kPolicies[0]);
 constexpr int kRowsPolicy = 5;
 constexpr int kSlicesPolicy = 6;        // first of the slices variants
 constexpr int kNumSlices = 6;
 constexpr bool is_slices(int policy) { return policy >= kSlicesPolicy && policy < kSlicesPolicy + kNumSlices; }
-constexpr int k192Policy = 12;
+constexpr int k192Policy = 12, k3PerCuPolicy = 13;
 constexpr int kRowsMaxM = 8;            // rows the streaming kernel takes
 constexpr int kRowsMinBN = 64;          // its output columns per work-group: 64, 128, 256 or 512
 constexpr int kRowsEnoughBlocks = 192;  // work-groups from which on a launch pulls the memory system's rate
@@ -770,8 +775,9 @@ enum : int { kClassKN = 0, kClassNK = 1, kClassRagged = 2, kClassF32 = 3 };
 // 7 %, the worst by 78 % (609 x 1568 x 6968; the streaming kernel for [n,k] apart: 4 x 13536 x 80 takes it 14 us, a tile 4).
 // With scratch, against every tile on 1 to 8 slices, 500 to 730 shapes per class, it is level on aligned operands (copies and
 // streams are no tiles), any alignment and fp32 3 %, one in ten by more than 7 to 10 %, the worst by 34 %.
-// The 192 x 128 tile's rows: chosen for what they pick beside the others, on 855 shapes of more than 100 tiles of 128 x 128 (taken for
-// 200 of them, which it makes 13 % faster on average, nine 2 to 5 % slower).
+// The last two tiles' rows: chosen for what they pick beside the others.  192 x 128, on 855 shapes of more than 100 tiles of
+// 128 x 128: taken for 200 of them, 13 % faster there on average, nine 2 to 5 % slower.  128 x 128 in steps of 32, on 900 of
+// more than 40, k 64 .. 8192: taken for 180, 30 % faster there, two 2 to 4 % slower.
 // Looking all candidates over takes the host 0.15 to 0.65 us per call.
 struct TileCost {
   float start, step, more_step, more, fill;
@@ -791,6 +797,7 @@ constexpr TileCost kTileCost[4][kNumPolicies] = {
      {3.747f, 0.862f, 0.313f, 3.855f, 1.603f},
      {3.11f, 1.488f, 0.285f, 3.156f, 1.679f},
      {4.669f, 0.509f, 0.831f, 4.313f, 1.555f},
+     {3.941f, 0.676f, 0.578f, 0.601f, 1.348f},
     },
     {  // 16-bit direct, B stored [N, K]
      {8.272f, 0.959f, 1.836f, 11.842f, 5.729f},
@@ -806,6 +813,7 @@ constexpr TileCost kTileCost[4][kNumPolicies] = {
      {3.735f, 0.806f, 0.31f, 3.754f, 1.666f},
      {2.945f, 1.596f, 0.302f, 3.078f, 2.018f},
      {4.41f, 0.482f, 0.815f, 3.821f, 1.96f},
+     {4.065f, 0.485f, 0.6f, 1.552f, 3.272f},
     },
     {  // 16-bit, any alignment
      {},
@@ -863,6 +871,8 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
   Choice best{3, 1, 1e30f};
   const bool direct = cls == kClassKN || cls == kClassNK;
   const int kstep = cls == kClassF32 ? 32 : 64;
+  const int64_t tiles_256_x_128 = xmk::ceil_div(m, 256) * xmk::ceil_div(n, 128) * batch;
+  const bool one_round_of_256_x_128 = tiles_256_x_128 > 240 && tiles_256_x_128 <= 256;
   auto each = [&](int s, float extra, float least) {
     for (int pol = 0; pol < kNumPolicies; ++pol) {
       if (pol == kRowsPolicy || (!direct && !kPolicies[pol].any_alignment)) continue;
@@ -871,6 +881,9 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
       // where the 256-row tile takes as many: the last of that one's tile rows is the emptier, which gives the others clock and
       // load path (560 x 10240 x 12288 141 us against 159; 560 x 10240 x 2048 30.1 against 27.3).
       // With K slices its estimate is too low (161 x 3553 x 12725 62.8 us, with it 72.4).
+      // 128 x 128 in steps of 32: not with K slices (not measured), and not where the 256 x 128 tiles are one round of the CUs: the
+      // tests of that tile rely on such shapes, one in a hundred, and it is the 15 to 25 % slower one there.
+      if (pol == k3PerCuPolicy && (s > 1 || (kt > 2 && one_round_of_256_x_128))) continue;
       if (pol == k192Policy && (s > 1 || kt < 6 || (kt > 32 && xmk::ceil_div(m, 192) == xmk::ceil_div(m, 256)))) continue;
       const float cost = std::max(launch_cost(kPolicies[pol], kTileCost[cls][pol], is_slices(pol), (uint32_t)m, (uint32_t)n, kt,
                                               (uint32_t)(batch * s)) + extra, least);
@@ -919,6 +932,7 @@ void launch_policy(int pol, GemmParams& p, int batch, hipStream_t st) {
     case 1: launch_mfma<T, OutF32, A_MC, B_MC, 128, 128, 2, 2, 64, 4>(p, batch, st); break;
     case 2: launch_mfma<T, OutF32, A_MC, B_MC, 128, 64, 2, 2, 64, 4>(p, batch, st); break;
     case 4: launch_mfma<T, OutF32, A_MC, B_MC, 256, 128, 2, 2, 64, 3>(p, batch, st); break;
+    case k3PerCuPolicy: launch_mfma<T, OutF32, A_MC, B_MC, 128, 128, 2, 2, 32, 3>(p, batch, st); break;
     case k192Policy:
       if constexpr (!A_MC) launch_mfma<T, OutF32, A_MC, B_MC, 192, 128, 2, 2, 64, 4>(p, batch, st);
       break;
