@@ -223,6 +223,12 @@ __global__ __launch_bounds__(NW * 64, NW == 8 || (RT == 2 && WN > 1 && GS > 32) 
     d[1][0][0] = d[1][0][1] = zero;
     sc[1][0] = sc[1][1] = 0.f;
   }
+  // An infinite scale stands as 2^60, which makes infinite fp16 results of any finite difference of the two sums; with infinity the
+  // sums, which come into acc one after the other, would be infinity less infinity.
+  auto scale_of = [&](uint32_t pair, int c) {
+    constexpr float kMost = 0x1p60f;
+    return __builtin_elementwise_minimum(__builtin_elementwise_maximum(half_of(pair, c), -kMost), kMost);
+  };
   auto fix_up = [&](auto P, auto E) {  // element E of the chains of parity P
     constexpr int par = decltype(P)::value, e = decltype(E)::value;
 #pragma unroll
@@ -250,7 +256,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 || (RT == 2 && WN > 1 && GS > 32) 
       floatx4 sum[2][RT];
       if constexpr (!kDefer) {
 #pragma unroll
-        for (int c = 0; c < 2; ++c) sc[par][c] = half_of(w.s[u], c);
+        for (int c = 0; c < 2; ++c) sc[par][c] = scale_of(w.s[u], c);
       }
       static_for<SPG>([&](auto J) {
         constexpr int j = decltype(J)::value, s = u * SPG + j;
@@ -285,8 +291,8 @@ __global__ __launch_bounds__(NW * 64, NW == 8 || (RT == 2 && WN > 1 && GS > 32) 
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
-        if constexpr (kDefer) sc[par][c] = half_of(w.s[u], c);
-        zz[par][c] = fmaf(-half_of(w.s[u], c), half_of(w.z[u], c), -16.f * half_of(w.s[u], c));
+        if constexpr (kDefer) sc[par][c] = scale_of(w.s[u], c);
+        zz[par][c] = fmaf(-sc[par][c], half_of(w.z[u], c), -16.f * sc[par][c]);
         asm volatile("" : "+v"(sc[par][c]), "+v"(zz[par][c]));  // (in registers of their own before the fetch below reuses w)
       }
 #pragma unroll

@@ -327,3 +327,29 @@ def test_int4_gemm_every_block_once(xmk, m, n):
     shifts = torch.arange(0, 32, 4, device="cuda", dtype=torch.int32)
     q = ((qw[:, None, :] >> shifts[None, :, None]) & 15).reshape(k, n)
     assert torch.equal(out.double().cpu(), act.double().cpu() @ q.double().cpu())
+
+
+@pytest.mark.parametrize("m,k,n,group", [(65, 1056, 72, 32), (128, 640, 16328, 128), (64, 768, 200, 64), (310, 512, 16400, 64), (49, 512, 200, 128)])
+def test_int4_gemm_row_tiles_infinite_scales(xmk, m, k, n, group):
+    """Infinite and NaN scales and zero points: their columns come out as from the kernel for 32 rows and fewer, which forms a
+    group's difference of sums before it is scaled (groups of 256 in two parts, whose infinities may cancel: left out); the other
+    columns are as they are without them."""
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    act = torch.randn((m, k), generator=g, device="cuda").half()
+    qw = torch.randint(-2 ** 31, 2 ** 31, (k // 8, n), generator=g, device="cuda", dtype=torch.int32)
+    s = torch.empty((k // group, n), device="cuda", dtype=torch.float16).uniform_(0.001, 0.02, generator=g)
+    z = torch.empty_like(s).uniform_(0.0, 15.0, generator=g)
+    plain = torch.empty((m, n), dtype=torch.float16, device="cuda")
+    xmk.int4_gemm(act, qw, s, z, plain, group=group)
+    inf = float("inf")
+    s[0, 3], s[k // group - 1, 8], s[1, 20], z[1, 33], z[0, 40] = inf, -inf, float("nan"), inf, -inf
+    bad = [3, 8, 20, 33, 40]
+    tiles, direct = torch.empty_like(plain), torch.empty_like(plain)
+    xmk.int4_gemm(act, qw, s, z, tiles, group=group)
+    for m0 in range(0, m, 32):
+        xmk.int4_gemm(act[m0:m0 + 32], qw, s, z, direct[m0:m0 + 32], group=group)
+    keep = torch.ones(n, dtype=torch.bool, device="cuda")
+    keep[bad] = False
+    assert torch.equal(tiles[:, keep], plain[:, keep])
+    assert not bool(direct[:, bad].isfinite().any())
+    assert torch.equal(tiles[:, bad].nan_to_num(nan=7.0), direct[:, bad].nan_to_num(nan=7.0))
