@@ -35,7 +35,9 @@ __global__ __launch_bounds__(256) void dp_sum_kernel(const T* __restrict__ o, co
   const int lane = threadIdx.x & 63;
   const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + lane / LPR;
   const int c = (lane % LPR) * 8;
-  float s = 0.f;
+  float s = 0.f, row_lse = 0.f;
+  // (asked for with the rows: behind the sum it was a second round trip to memory)
+  if (row < rows && lse2) row_lse = lse[row];
   if (row < rows && c < H) {
     const u32x4 a = *reinterpret_cast<const u32x4*>(o + row * H + c);
     const u32x4 b = *reinterpret_cast<const u32x4*>(d_o + row * H + c);
@@ -48,7 +50,7 @@ __global__ __launch_bounds__(256) void dp_sum_kernel(const T* __restrict__ o, co
   for (int off = LPR / 2; off >= 1; off >>= 1) s += __shfl_xor(s, off);
   if (row < rows && lane % LPR == 0) {
     dsum[row] = s;
-    if (lse2) lse2[row] = lse[row] * 1.4426950408889634f;
+    if (lse2) lse2[row] = row_lse * 1.4426950408889634f;
   }
 }
 
