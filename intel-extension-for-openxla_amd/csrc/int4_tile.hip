@@ -73,9 +73,39 @@ __device__ __forceinline__ float half_of(uint32_t pair, int c) {
   return (float)__builtin_bit_cast(_Float16, (uint16_t)(pair >> (16 * c)));
 }
 
+// Results of a finite row that are NaN, in columns with infinite scales: those come into the accumulators with a group's two
+// sums one after the other, infinity less infinity, and are to come with their difference.  Formed again from the groups
+// whose scale or zero point is not finite (the others do not matter beside them), in parts of 128 as the products are.
+__device__ __forceinline__ void mend_columns(const xmk::Int4TileArgs& p, int m, int n, const half8& old, const float (&bias)[8]) {
+  const _Float16* const a = p.act + (size_t)m * p.K;
+  const int part = min(p.group, kStepK);
+#pragma unroll 1
+  for (int j = 0; j < 8; ++j) {
+    if (old[j] == old[j]) continue;
+    bool found = false;
+    float sum = 0.f;
+#pragma unroll 1
+    for (int k0 = 0; k0 < p.K && sum == sum; k0 += part) {
+      const size_t sz = (size_t)(k0 / p.group) * p.N + n + j;
+      const float s = (float)p.scales[sz], z = (float)p.zeros[sz];
+      if (fabsf(s) <= 65504.f && fabsf(z) <= 65504.f) continue;
+      found = true;
+      // (with an infinite zero point the weights do not matter)
+      const bool far = !(fabsf(z) <= 65504.f);
+      float diff = 0.f;
+#pragma unroll 1
+      for (int k = k0; k < k0 + part; ++k) {
+        const float q = (float)((p.qw[(size_t)(k / 8) * p.N + n + j] >> (4 * (k % 8))) & 15);
+        diff = fmaf((float)a[k], far ? 1.f : q - z, diff);
+      }
+      sum = fmaf(s, far ? -z * diff : diff, sum);
+    }
+    if (found) p.out[(size_t)m * p.N + n + j] = (_Float16)(sum + bias[j]);
+  }
+}
+
 // An infinite activation makes both sums of its group infinite and their difference NaN, whatever the weights.  Eight results
-// of a row that holds one, formed again weight by weight: the finite activations do not matter beside the others.  Left as
-// they are where the row is finite (the NaN then comes from scales or zero points).
+// of a row that holds one, formed again weight by weight: the finite activations do not matter beside the others.
 __device__ __forceinline__ void mend_row(const xmk::Int4TileArgs& p, int m, int n, const float (&bias)[8]) {
   _Float16* const out = p.out + (size_t)m * p.N + n;
   const half8 old = *reinterpret_cast<const half8*>(out);
@@ -106,7 +136,7 @@ __device__ __forceinline__ void mend_row(const xmk::Int4TileArgs& p, int m, int 
       for (int j = 0; j < 8; ++j) open |= sum[j] == sum[j];
     }
   }
-  if (!found) return;
+  if (!found) return mend_columns(p, m, n, old, bias);
   half8 o;
 #pragma unroll
   for (int j = 0; j < 8; ++j) o[j] = (_Float16)(sum[j] + bias[j]);
@@ -223,12 +253,6 @@ __global__ __launch_bounds__(NW * 64, NW == 8 || (RT == 2 && WN > 1 && GS > 32) 
     d[1][0][0] = d[1][0][1] = zero;
     sc[1][0] = sc[1][1] = 0.f;
   }
-  // An infinite scale stands as 2^60, which makes infinite fp16 results of any finite difference of the two sums; with infinity the
-  // sums, which come into acc one after the other, would be infinity less infinity.
-  auto scale_of = [&](uint32_t pair, int c) {
-    constexpr float kMost = 0x1p60f;
-    return __builtin_elementwise_minimum(__builtin_elementwise_maximum(half_of(pair, c), -kMost), kMost);
-  };
   auto fix_up = [&](auto P, auto E) {  // element E of the chains of parity P
     constexpr int par = decltype(P)::value, e = decltype(E)::value;
 #pragma unroll
@@ -256,7 +280,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 || (RT == 2 && WN > 1 && GS > 32) 
       floatx4 sum[2][RT];
       if constexpr (!kDefer) {
 #pragma unroll
-        for (int c = 0; c < 2; ++c) sc[par][c] = scale_of(w.s[u], c);
+        for (int c = 0; c < 2; ++c) sc[par][c] = half_of(w.s[u], c);
       }
       static_for<SPG>([&](auto J) {
         constexpr int j = decltype(J)::value, s = u * SPG + j;
@@ -291,7 +315,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 || (RT == 2 && WN > 1 && GS > 32) 
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
-        if constexpr (kDefer) sc[par][c] = scale_of(w.s[u], c);
+        if constexpr (kDefer) sc[par][c] = half_of(w.s[u], c);
         zz[par][c] = fmaf(-sc[par][c], half_of(w.z[u], c), -16.f * sc[par][c]);
         asm volatile("" : "+v"(sc[par][c]), "+v"(zz[par][c]));  // (in registers of their own before the fetch below reuses w)
       }

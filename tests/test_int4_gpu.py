@@ -353,3 +353,41 @@ def test_int4_gemm_row_tiles_infinite_scales(xmk, m, k, n, group):
     assert torch.equal(tiles[:, keep], plain[:, keep])
     assert not bool(direct[:, bad].isfinite().any())
     assert torch.equal(tiles[:, bad].nan_to_num(nan=7.0), direct[:, bad].nan_to_num(nan=7.0))
+
+
+@pytest.mark.parametrize("m,k,n,group", [(65, 1056, 72, 32), (64, 768, 200, 64), (49, 512, 200, 128), (310, 512, 16400, 64), (70, 1024, 136, 256)])
+def test_int4_gemm_row_tiles_infinite_scales_without_a_sum(xmk, m, k, n, group):
+    """Infinite scales on differences of zero (rows of zero activations, groups whose weights are their zero points) and on groups
+    whose infinities have opposite signs: NaN.  Whole numbers, so that every sum is exact, against the formula group by group (in
+    parts of 128, as the products are formed), which the kernel for 32 rows and fewer gives too."""
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    act = torch.randint(-3, 4, (m, k), generator=g, device="cuda").half()
+    act[[0, 33, m - 1]] = 0
+    act[5, :group] = 0
+    qw = torch.randint(-2 ** 31, 2 ** 31, (k // 8, n), generator=g, device="cuda", dtype=torch.int32)
+    qw[group // 8:2 * group // 8, 12] = 0x44444444
+    s = torch.full((k // group, n), 0.5, device="cuda", dtype=torch.float16)
+    z = torch.randint(0, 16, s.shape, generator=g, device="cuda").half()
+    z[1, 12] = 4
+    inf = float("inf")
+    s[0, 3] = s[1, 12] = s[0, 20] = s[1, 20] = s[0, 41] = s[0, 50] = s[0, 51] = inf
+    s[1, 41] = s[k // group - 1, 60] = -inf
+    z[1, 50], z[0, 51], z[1, 61] = -inf, inf, inf
+    bias = torch.randint(-3, 4, (n,), generator=g, device="cuda").half()
+    out, few = (torch.empty((m, n), dtype=torch.float16, device="cuda") for _ in range(2))
+    xmk.int4_gemm(act, qw, s, z, out, group=group, bias=bias)
+    for m0 in range(0, m, 32):
+        xmk.int4_gemm(act[m0:m0 + 32], qw, s, z, few[m0:m0 + 32], group=group, bias=bias)
+    shifts = torch.arange(0, 32, 4, device="cuda", dtype=torch.int32)
+    q = ((qw[:, None, :] >> shifts[None, :, None]) & 15).reshape(k, n).double().cpu()
+    a, s, z, ref = act.double().cpu(), s.double().cpu(), z.double().cpu(), bias.double().cpu().expand(m, n)
+    part = min(group, 128)
+    for k0 in range(0, k, part):
+        rows, gr = slice(k0, k0 + part), k0 // group
+        diff = a[:, rows] @ q[rows] - a[:, rows].sum(1, keepdim=True) * z[gr]
+        ref = ref + diff * s[gr]
+    ref = ref.half()
+    assert bool(ref[:, [3, 12, 20, 41]].isnan().any(0).all()) and bool(ref[:, [3, 20, 41]].isinf().any(0).all())
+    for got in (out.cpu(), few.cpu()):
+        assert torch.equal(got.isnan(), ref.isnan())
+        assert torch.equal(got.nan_to_num(nan=7.0), ref.nan_to_num(nan=7.0))
