@@ -871,8 +871,6 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
   Choice best{3, 1, 1e30f};
   const bool direct = cls == kClassKN || cls == kClassNK;
   const int kstep = cls == kClassF32 ? 32 : 64;
-  const int64_t tiles_256_x_128 = xmk::ceil_div(m, 256) * xmk::ceil_div(n, 128) * batch;
-  const bool one_round_of_256_x_128 = tiles_256_x_128 > 240 && tiles_256_x_128 <= 256;
   auto each = [&](int s, float extra, float least) {
     for (int pol = 0; pol < kNumPolicies; ++pol) {
       if (pol == kRowsPolicy || (!direct && !kPolicies[pol].any_alignment)) continue;
@@ -881,9 +879,9 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
       // where the 256-row tile takes as many: the last of that one's tile rows is the emptier, which gives the others clock and
       // load path (560 x 10240 x 12288 141 us against 159; 560 x 10240 x 2048 30.1 against 27.3).
       // With K slices its estimate is too low (161 x 3553 x 12725 62.8 us, with it 72.4).
-      // 128 x 128 in steps of 32: not with K slices (not measured), and not where the 256 x 128 tiles are one round of the CUs: the
-      // tests of that tile rely on such shapes, one in a hundred, and it is the 15 to 25 % slower one there.
-      if (pol == k3PerCuPolicy && (s > 1 || (kt > 2 && one_round_of_256_x_128))) continue;
+      // 128 x 128 in steps of 32: not with K slices, of which it is the slowest tile (1024 x 1024 x 8192 on four 39.0 us, in steps
+      // of 64 30.3; 2048 x 2048 x 4096 on two 61 and 64, unsplit 35).
+      if (pol == k3PerCuPolicy && s > 1) continue;
       if (pol == k192Policy && (s > 1 || kt < 6 || (kt > 32 && xmk::ceil_div(m, 192) == xmk::ceil_div(m, 256)))) continue;
       const float cost = std::max(launch_cost(kPolicies[pol], kTileCost[cls][pol], is_slices(pol), (uint32_t)m, (uint32_t)n, kt,
                                               (uint32_t)(batch * s)) + extra, least);
