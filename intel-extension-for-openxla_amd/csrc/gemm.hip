@@ -283,7 +283,7 @@ extern "C" const char* xmk_gemm_policy_name(int64_t m, int64_t n, int64_t k, int
     if (!rhs_transpose && n % 8 == 0) rows_kind = kRowsMC;
     if (rhs_transpose && k <= kColsMaxK) rows_kind = kRowsKC;
   }
-  return kernel_name(select_policy(m, n, k, 1, rows_kind, cls), any_alignment);
+  return kernel_name(select_policy(m, n, k, 1, rows_kind, cls, false), any_alignment);
 }
 
 namespace {
@@ -648,7 +648,8 @@ int run_gemm(const xmk_gemm_desc* d, void* out1, void* out2, void* stream, int p
     // an operand take the tile one of them would: the results are then the same bits)
     const int pol = (forced_policy() < 0 && policy >= 0 && policy < kNumPolicies &&
                      (policy != kRowsPolicy || rows_kind != kRowsNone))
-                        ? policy : select_policy(m, n, k, qkv ? 1 : batch, qkv ? kRowsNone : rows_kind, din == XMK_F32 ? kClassF32 : ragged ? kClassRagged : b_mc ? kClassKN : kClassNK);
+                        ? policy : select_policy(m, n, k, qkv ? 1 : batch, qkv ? kRowsNone : rows_kind,
+                                        din == XMK_F32 ? kClassF32 : ragged ? kClassRagged : b_mc ? kClassKN : kClassNK, a_mc);
     xmk::trace("gemm m=%lld n=%lld k=%lld batch=%lld lhs_t=%d rhs_t=%d epilogue=%d beta=%g -> %s",
                (long long)m, (long long)n, (long long)k, (long long)d->batch_size, lhs.transpose,
                rhs.transpose, d->epilogue, d->beta, kernel_name(pol, ragged));

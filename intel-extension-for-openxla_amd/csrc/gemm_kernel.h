@@ -866,14 +866,14 @@ struct Choice {
   int policy, slices;
   float us;
 };
-// The cheapest policy and number of K slices (1 unless may_split).
-inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, bool may_split) {
+// The cheapest policy and number of K slices (1 unless may_split).  a_mc: A is stored [K, M].
+inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, bool may_split, bool a_mc = false) {
   Choice best{3, 1, 1e30f};
   const bool direct = cls == kClassKN || cls == kClassNK;
   const int kstep = cls == kClassF32 ? 32 : 64;
   auto each = [&](int s, float extra, float least) {
     for (int pol = 0; pol < kNumPolicies; ++pol) {
-      if (pol == kRowsPolicy || (!direct && !kPolicies[pol].any_alignment)) continue;
+      if (pol == kRowsPolicy || (!direct && !kPolicies[pol].any_alignment) || (a_mc && pol == k192Policy)) continue;
       const uint32_t kt = (uint32_t)(((k + s - 1) / s + kstep - 1) / kstep);
       // The 192 x 128 tile is not for short reductions, whose time is the output's (7102 x 1408 x 64 11 % slower), nor for long ones
       // where the 256-row tile takes as many: the last of that one's tile rows is the emptier, which gives the others clock and
@@ -898,11 +898,11 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
 
 // rows_kind: which streaming kernel the operands allow (gemm_rows_applicable); it is never chosen otherwise.
 // The tuned table applies to the layout it was measured with (direct operands, B stored [K, N]).
-inline int select_policy(int64_t m, int64_t n, int64_t k, int64_t batch, int rows_kind, int cls) {
+inline int select_policy(int64_t m, int64_t n, int64_t k, int64_t batch, int rows_kind, int cls, bool a_mc) {
   const bool rows_ok = rows_kind != kRowsNone;
   const bool direct = cls == kClassKN || cls == kClassNK;
   auto usable = [&](int v) {
-    return v >= 0 && v < kNumPolicies && (v != kRowsPolicy || rows_ok) && (direct || kPolicies[v].any_alignment);
+    return v >= 0 && v < kNumPolicies && (v != kRowsPolicy || rows_ok) && (direct || kPolicies[v].any_alignment) && !(a_mc && v == k192Policy);
   };
   const int forced = forced_policy();
   if (usable(forced)) return forced;
@@ -910,7 +910,7 @@ inline int select_policy(int64_t m, int64_t n, int64_t k, int64_t batch, int row
     if (const TunedShape* t = tuned_shape(m, n, k); t && t->ksplit <= 1 && usable(t->policy)) return t->policy;
   // A few rows against a very wide matrix: stream it.
   if (batch == 1 && rows_streams_by_default(rows_kind, m, n)) return kRowsPolicy;
-  return cheapest(m, n, k, batch, cls, false).policy;
+  return cheapest(m, n, k, batch, cls, false, a_mc).policy;
 }
 
 template <typename T, bool OutF32, bool A_MC, bool B_MC, int BM, int BN, int WGM, int WGN, int BK, int NSTAGE>
@@ -921,7 +921,6 @@ void launch_mfma(const GemmParams& p, int batch, hipStream_t st) {
 
 template <typename T, bool OutF32, bool A_MC, bool B_MC>
 void launch_policy(int pol, GemmParams& p, int batch, hipStream_t st) {
-  if (A_MC && pol == k192Policy) pol = 4;  // (rows of 192 elements are no whole number of loads)
   p.tiles_m = (int)xmk::ceil_div(p.M, kPolicies[pol].bm);
   p.tiles_n = (int)xmk::ceil_div(p.N, kPolicies[pol].bn);
   p.order = tile_order((uint32_t)p.tiles_m, (uint32_t)p.tiles_n, p.K);
@@ -931,7 +930,7 @@ void launch_policy(int pol, GemmParams& p, int batch, hipStream_t st) {
     case 2: launch_mfma<T, OutF32, A_MC, B_MC, 128, 64, 2, 2, 64, 4>(p, batch, st); break;
     case 4: launch_mfma<T, OutF32, A_MC, B_MC, 256, 128, 2, 2, 64, 3>(p, batch, st); break;
     case k3PerCuPolicy: launch_mfma<T, OutF32, A_MC, B_MC, 128, 128, 2, 2, 32, 3>(p, batch, st); break;
-    case k192Policy:
+    case k192Policy:  // (not for A stored [K, M], whose LDS rows of 192 elements are no whole number of loads)
       if constexpr (!A_MC) launch_mfma<T, OutF32, A_MC, B_MC, 192, 128, 2, 2, 64, 4>(p, batch, st);
       break;
     default: launch_mfma<T, OutF32, A_MC, B_MC, 64, 64, 2, 2, 64, 4>(p, batch, st); break;
