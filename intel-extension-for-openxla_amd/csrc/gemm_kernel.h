@@ -777,7 +777,9 @@ enum : int { kClassKN = 0, kClassNK = 1, kClassRagged = 2, kClassF32 = 3 };
 // streams are no tiles), any alignment and fp32 3 %, one in ten by more than 7 to 10 %, the worst by 34 %.
 // The last two tiles' rows: chosen for what they pick beside the others.  192 x 128, on 855 shapes of more than 100 tiles of
 // 128 x 128: taken for 200 of them, 13 % faster there on average, nine 2 to 5 % slower.  128 x 128 in steps of 32, on 900 of
-// more than 40, k 64 .. 8192: taken for 180, 30 % faster there, two 2 to 4 % slower.
+// more than 40, k 64 .. 8192: taken for 180, 30 % faster there.  Both on 1520 others of more than 200 and k 64 .. 3000, either
+// storage order of both operands, against the choice without the two: 10 % faster on average, eight of the 1520 more than 3 %
+// slower (1656 x 4760 x 552 with B [n,k] 21.8 us against 19.0, the others 6 % and less).
 // Looking all candidates over takes the host 0.15 to 0.65 us per call.
 struct TileCost {
   float start, step, more_step, more, fill;
@@ -871,6 +873,7 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
   Choice best{3, 1, 1e30f};
   const bool direct = cls == kClassKN || cls == kClassNK;
   const int kstep = cls == kClassF32 ? 32 : 64;
+  const int64_t tiles_256_x_256 = xmk::ceil_div(m, 256) * xmk::ceil_div(n, 256) * batch;
   auto each = [&](int s, float extra, float least) {
     for (int pol = 0; pol < kNumPolicies; ++pol) {
       if (pol == kRowsPolicy || (!direct && !kPolicies[pol].any_alignment) || (a_mc && pol == k192Policy)) continue;
@@ -881,7 +884,9 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
       // With K slices its estimate is too low (161 x 3553 x 12725 62.8 us, with it 72.4).
       // 128 x 128 in steps of 32: not with K slices, of which it is the slowest tile (1024 x 1024 x 8192 on four 39.0 us, in steps
       // of 64 30.3; 2048 x 2048 x 4096 on two 61 and 64, unsplit 35).
-      if (pol == k3PerCuPolicy && s > 1) continue;
+      // Nor, above six K steps, where the 256 x 256 tiles are more than a round and a half: they load half as much, and the estimate
+      // did not see it (5400 x 15512 x 840 202 us where they take 168, 6936 x 8152 x 560 with B [n,k] 109 against 93).
+      if (pol == k3PerCuPolicy && (s > 1 || (kt > 6 && tiles_256_x_256 > 384))) continue;
       if (pol == k192Policy && (s > 1 || kt < 6 || (kt > 32 && xmk::ceil_div(m, 192) == xmk::ceil_div(m, 256)))) continue;
       const float cost = std::max(launch_cost(kPolicies[pol], kTileCost[cls][pol], is_slices(pol), (uint32_t)m, (uint32_t)n, kt,
                                               (uint32_t)(batch * s)) + extra, least);

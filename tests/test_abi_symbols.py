@@ -177,6 +177,14 @@ def test_short_reductions_take_three_tiles_per_cu(lib, m, n, k):
     assert xmk.gemm_policy_name(m, n, k) == "mfma_128x128x32_w2x2_s3"
 
 
+@pytest.mark.parametrize("m,n,k,rhs_t", [(5400, 15512, 840, 0), (6936, 8152, 560, 1), (5352, 11304, 656, 0), (3088, 10936, 1200, 0)])
+def test_many_large_tiles_stay_large(lib, m, n, k, rhs_t):
+    """More than a round and a half of 256 x 256 tiles: three small ones per CU take 11 to 21 % longer there."""
+    import importlib
+    xmk = importlib.import_module("intel-extension-for-openxla_amd")
+    assert xmk.gemm_policy_name(m, n, k, bool(rhs_t)) == "mfma_256x256x32_w2x2_s4"
+
+
 def test_decode_attention_needs_a_workspace_tensor():
     """A forgotten workspace is refused: only fmha_decode_static may use the library's built-in array, on which calls
     on two streams would race.  (The refusal comes before any device work: host tensors, and a shape the library
