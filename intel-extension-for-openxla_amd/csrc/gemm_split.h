@@ -43,6 +43,11 @@ struct SplitLoader : AnyLoader<float, MC, ROWS, NT, MIS> {
     Base::init(op, ld, row0, rows, k0, depth, tid);
     const int row = tid / Base::CPR, c = tid % Base::CPR;
     at = row * RB + (((c >> 1) ^ swz<MC, ROWS, 32>(row)) << 4) + (c & 1) * 8;
+    // (MC: chunks past the last column repeat the last one, as rows past the end do)
+    if constexpr (MC) {
+#pragma unroll
+      for (int i = 0; i < Base::NL; ++i) this->off[i] -= 16 * max(c - (rows - 1 - row0) / 4, 0);
+    }
   }
   // As the base's, with the lanes' offsets bounded in 32 bits (the compiler would do it in 64).
   __device__ __forceinline__ void load(Regs& r) {
@@ -57,6 +62,18 @@ struct SplitLoader : AnyLoader<float, MC, ROWS, NT, MIS> {
       else r.g[i] = *reinterpret_cast<const u32x4*>(from + o);
     }
     this->advance(1);
+  }
+  // Zeroes what is no number of this tile: k from kleft on, (MC) columns from cleft on.  Chunks reach past both, into the padding
+  // between a row's end and the next one or into the next row, and what lies there is neither looked at nor multiplied.
+  __device__ __forceinline__ void clip(Regs& r, int kleft, int cleft) const {
+    if (kleft >= Base::BK && (!MC || cleft >= ROWS)) return;  // (uniform)
+    const int lrow = (int)threadIdx.x / Base::CPR, c = 4 * ((int)threadIdx.x % Base::CPR);
+#pragma unroll
+    for (int i = 0; i < Base::NL; ++i) {
+      const int n = !MC ? kleft - c : lrow + i * Base::RPL < kleft ? cleft - c : 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r.g[i][e] = e < n ? r.g[i][e] : 0u;
+    }
   }
   // The numbers of a Regs on their way to LDS.  Pair q (elements 2 q and 2 q + 1) passes through six steps, one after
   // the other; split_step<t>() runs step t - q of every pair that has it, so that a step's instructions do not wait for each other.
@@ -91,9 +108,10 @@ struct SplitLoader : AnyLoader<float, MC, ROWS, NT, MIS> {
       }
     });
   }
-  __device__ __forceinline__ void store(char* tile, Regs& r, uint32_t& least) const {
+  __device__ __forceinline__ void store(char* tile, Regs& r, uint32_t& least, int kleft, int cleft) const {
     Split s;
     this->shift_ends(r);
+    clip(r, kleft, cleft);
     static_for<STEPS>([&](auto S) { split_step<decltype(S)::value>(tile, r, s, least); });
   }
 };
@@ -131,7 +149,8 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_split_kernel(GemmParams p) 
   // Between the barriers of two K steps lie the second half of one step's matrix instructions and the first half of the
   // next one's: A of the step after that is split beside the former, B beside the latter, each into the stage that the
   // barrier has freed.  Loads are sent as soon as the registers are free, two K steps ahead; those past the end of K
-  // come from the operand's last 16 bytes, and what they bring is not used.
+  // come from the operand's last 16 bytes, and zeros are split in their place.
+  const int cols_a = p.M - m0, cols_b = p.N - n0;
   typename LoaderA::Regs ga[2];  // K steps of even and odd number
   typename LoaderB::Regs gb[2];
   uint32_t least = 0xffffffffu;
@@ -140,11 +159,11 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_split_kernel(GemmParams p) 
     la.load(ga[i]);
     lb.load(gb[i]);
   }
-  la.store(lds, ga[0], least);
+  la.store(lds, ga[0], least, K, cols_a);
   la.load(ga[0]);
-  lb.store(lds + OP_BYTES, gb[0], least);
+  lb.store(lds + OP_BYTES, gb[0], least, K, cols_b);
   lb.load(gb[0]);
-  la.store(lds + STAGE, ga[1], least);
+  la.store(lds + STAGE, ga[1], least, K - BK, cols_a);
   la.load(ga[1]);
   lds_barrier();
 
@@ -171,11 +190,12 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_split_kernel(GemmParams p) 
   };
   // Half a K step: its products, the reads of the next half's fragments (from the stage `frags`), and an operand's split numbers on
   // their way to LDS, in slots of one matrix instruction each.
-  auto half = [&](auto KSI, const char* frags, auto& ld, auto& regs, char* to) {
+  auto half = [&](auto KSI, auto CLIP, const char* frags, auto& ld, auto& regs, char* to, int kleft, int cleft) {
     constexpr int ks = decltype(KSI)::value;
     typedef std::remove_reference_t<decltype(ld)> L;
     typename L::Split s;
     ld.shift_ends(regs);
+    if constexpr (decltype(CLIP)::value) ld.clip(regs, kleft, cleft);
     static_for<NMFMA>([&](auto R) {
       constexpr int r = decltype(R)::value;
       __builtin_amdgcn_sched_barrier(0);
@@ -197,33 +217,28 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_split_kernel(GemmParams p) 
   static_for<READ_SLABS>([&](auto F) { read_frag(F, lds, 0); });
   typedef std::integral_constant<int, 0> First;
   typedef std::integral_constant<int, 1> Second;
-  auto step = [&](auto ODD) {
+  auto step = [&](auto ODD, auto CLIP, int kt) {
     constexpr int odd = decltype(ODD)::value, cur = odd * STAGE, nxt = STAGE - cur;
-    half(First{}, lds + cur, lb, gb[1 - odd], lds + nxt + OP_BYTES);
+    half(First{}, CLIP, lds + cur, lb, gb[1 - odd], lds + nxt + OP_BYTES, K - (kt + 1) * BK, cols_b);
     lds_barrier();
-    half(Second{}, lds + nxt, la, ga[odd], lds + cur);
+    half(Second{}, CLIP, lds + nxt, la, ga[odd], lds + cur, K - (kt + 2) * BK, cols_a);
   };
-    int kt = 0;
-  for (; kt + 2 < KT; kt += 2) {
-    step(First{});
-    step(Second{});
+  // Clipping costs 2 to 6 % of a step, so only the steps that split the last one's numbers do it (and all of a tile whose
+  // last chunk of columns reaches past the end).
+  const bool cut = (A_MC && cols_a < BT && cols_a % 4) || (B_MC && cols_b < BT && cols_b % 4);
+  const int inside = cut ? 0 : (K - 2 * BK) / BK;  // whole K steps, two steps ago
+  int kt = 0;
+  for (; kt + 1 < inside; kt += 2) {
+    step(First{}, std::false_type{}, kt);
+    step(Second{}, std::false_type{}, kt + 1);
   }
-  if (kt + 1 < KT) step(First{});
+  for (; kt + 1 < KT; kt += 2) {
+    step(First{}, std::true_type{}, kt);
+    if (kt + 2 < KT) step(Second{}, std::true_type{}, kt + 1);
+  }
   const int cur = (KT - 1) % 2 * STAGE;
-  // The last K step, of which only some k may exist.
-  const int tail = K - (KT - 1) * BK;
   static_for<READ_SLABS>([&](auto F) { read_frag(F, lds + cur, 1); });
-  static_for<KS>([&](auto KSI) {
-    constexpr int ks = decltype(KSI)::value;
-#pragma unroll
-    for (int pl = 0; pl < 3; ++pl) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i) mask_fragment<__bf16>(fa[ks][pl][i], ks, lane, tail);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) mask_fragment<__bf16>(fb[ks][pl][j], ks, lane, tail);
-    }
-    static_for<NMFMA>([&](auto R) { mma(R, KSI); });
-  });
+  static_for<KS>([&](auto KSI) { static_for<NMFMA>([&](auto R) { mma(R, KSI); }); });
   bool redo = least < kSplitLeast - 1u;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
