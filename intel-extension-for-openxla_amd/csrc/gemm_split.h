@@ -7,10 +7,12 @@
 // running sum of the large one bias it.  The large products of even and of odd halves of the K steps and the five small ones
 // therefore have accumulators of their own, added at the end.
 //
-// What the split does not hold for is found, and the tile is then formed again by the fp32 instructions (gemm_ragged.h):
-//   a number above 2^127 (h may be infinite) or infinite: l is a NaN, and so is a sum; a NaN shows the same way; a sum that
-//       overflows is not finite either.
-//   a nonzero number below 2^-102: l would lie below the smallest normal bf16.  Looked for in every number that is split.
+// Range.  Numbers are split times 2^23, which makes 2^-149, fp32's smallest, the smallest normal bf16: the parts of every number,
+// however small, are normal or zero, and no product of them is lost.  (Numbers below 2^-102, which softmax weights and gradients have,
+// were looked for before and their tiles formed again by the fp32 instructions: 2048 x 2048 x 1024 115 to 126 us.)  At the other end
+// a number above 2^104 (h may be infinite) or an infinite one has a NaN for l, and so has a sum; a NaN shows the same way; a sum above
+// 2^82 is not finite either.  The tile is then formed again by the fp32 instructions (gemm_ragged.h; all tiles of 2048 x 2048 x 1024
+// 122 us).
 //
 // What bounds it: matrix and vector instructions, which share the issue port: 24 products per wave and K step stand beside
 // 110 vector instructions (6.5 per split number: each work-group splits what it loads), and the matrix pipe is busy 53 %
@@ -27,7 +29,7 @@
 
 namespace gemm_impl {
 
-constexpr uint32_t kSplitLeast = (127u - 102u) << 24;  // 2^-102, shifted by its sign
+constexpr float kSplitScale = 0x1p23f, kSplitUnscale = 0x1p-46f;
 
 // AnyLoader's chunks of four floats, written to LDS as 3 planes of bf16: [row][32 k] (KC) or [k][rows] (MC), laid out and
 // read as the 16-bit kernels' tiles with BK = 32.
@@ -75,44 +77,45 @@ struct SplitLoader : AnyLoader<float, MC, ROWS, NT, MIS> {
       for (int e = 0; e < 4; ++e) r.g[i][e] = e < n ? r.g[i][e] : 0u;
     }
   }
-  // The numbers of a Regs on their way to LDS.  Pair q (elements 2 q and 2 q + 1) passes through six steps, one after
+  // The numbers of a Regs on their way to LDS.  Pair q (elements 2 q and 2 q + 1) passes through seven steps, one after
   // the other; split_step<t>() runs step t - q of every pair that has it, so that a step's instructions do not wait for each other.
-  static constexpr int PAIRS = 2 * Base::NL, STEPS = PAIRS + 5;
+  static constexpr int PAIRS = 2 * Base::NL, STEPS = PAIRS + 6;
   struct Split {
     uint32_t part[3][PAIRS];
   };
-  // least: the smallest number seen, as its bits shifted by the sign, less one (a zero counts as the largest).
   template <int STEP>
-  __device__ __forceinline__ void split_step(char* tile, Regs& r, Split& s, uint32_t& least) const {
+  __device__ __forceinline__ void split_step(char* tile, Regs& r, Split& s) const {
     typedef __bf16 v2 __attribute__((ext_vector_type(2)));
     static_for<PAIRS>([&](auto Q) {
       constexpr int q = decltype(Q)::value, step = STEP - q, i = q / 2, e = 2 * (q & 1);
-      const uint32_t w0 = r.g[i][e], w1 = r.g[i][e + 1];
-      const float x0 = __builtin_bit_cast(float, w0), x1 = __builtin_bit_cast(float, w1);
-      if constexpr (step == 0) least = min(min((w0 << 1) - 1u, (w1 << 1) - 1u), least);
-      if constexpr (step == 0 || step == 2 || step == 4) {
+      const float x0 = __builtin_bit_cast(float, (uint32_t)r.g[i][e]), x1 = __builtin_bit_cast(float, (uint32_t)r.g[i][e + 1]);
+      if constexpr (step == 0) {
+        r.g[i][e] = __builtin_bit_cast(uint32_t, x0 * kSplitScale);
+        r.g[i][e + 1] = __builtin_bit_cast(uint32_t, x1 * kSplitScale);
+      }
+      if constexpr (step == 1 || step == 3 || step == 5) {
         s.part[step / 2][q] = __builtin_bit_cast(uint32_t, v2{(__bf16)x0, (__bf16)x1});
         asm("" : "+v"(s.part[step / 2][q]));  // (the compiler would convert x1 once more to have it alone)
       }
-      if constexpr (step == 1 || step == 3) {  // what is left: exact
-        const uint32_t h = s.part[step / 2][q];
+      if constexpr (step == 2 || step == 4) {  // what is left: exact
+        const uint32_t h = s.part[step / 2 - 1][q];
         const float y0 = x0 - __builtin_bit_cast(float, h << 16);
         const float y1 = x1 - __builtin_bit_cast(float, h & 0xffff0000u);
         r.g[i][e] = __builtin_bit_cast(uint32_t, y0);
         r.g[i][e + 1] = __builtin_bit_cast(uint32_t, y1);
       }
-      if constexpr (step == 5 && (q & 1)) {
+      if constexpr (step == 6 && (q & 1)) {
 #pragma unroll
         for (int pl = 0; pl < 3; ++pl)
           *reinterpret_cast<u32x2*>(tile + pl * PLANE + at + i * Base::RPL * RB) = u32x2{s.part[pl][q - 1], s.part[pl][q]};
       }
     });
   }
-  __device__ __forceinline__ void store(char* tile, Regs& r, uint32_t& least, int kleft, int cleft) const {
+  __device__ __forceinline__ void store(char* tile, Regs& r, int kleft, int cleft) const {
     Split s;
     this->shift_ends(r);
     clip(r, kleft, cleft);
-    static_for<STEPS>([&](auto S) { split_step<decltype(S)::value>(tile, r, s, least); });
+    static_for<STEPS>([&](auto S) { split_step<decltype(S)::value>(tile, r, s); });
   }
 };
 
@@ -153,17 +156,16 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_split_kernel(GemmParams p) 
   const int cols_a = p.M - m0, cols_b = p.N - n0;
   typename LoaderA::Regs ga[2];  // K steps of even and odd number
   typename LoaderB::Regs gb[2];
-  uint32_t least = 0xffffffffu;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     la.load(ga[i]);
     lb.load(gb[i]);
   }
-  la.store(lds, ga[0], least, K, cols_a);
+  la.store(lds, ga[0], K, cols_a);
   la.load(ga[0]);
-  lb.store(lds + OP_BYTES, gb[0], least, K, cols_b);
+  lb.store(lds + OP_BYTES, gb[0], K, cols_b);
   lb.load(gb[0]);
-  la.store(lds + STAGE, ga[1], least, K - BK, cols_a);
+  la.store(lds + STAGE, ga[1], K - BK, cols_a);
   la.load(ga[1]);
   lds_barrier();
 
@@ -207,7 +209,7 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_split_kernel(GemmParams p) 
       });
       constexpr int s0 = L::STEPS * r / SSLOTS, s1 = L::STEPS * (r + 1) / SSLOTS;
       static_for<L::STEPS>([&](auto S) {
-        if constexpr (decltype(S)::value >= s0 && decltype(S)::value < s1) ld.template split_step<decltype(S)::value>(to, regs, s, least);
+        if constexpr (decltype(S)::value >= s0 && decltype(S)::value < s1) ld.template split_step<decltype(S)::value>(to, regs, s);
       });
       if constexpr (r == NMFMA - 1) ld.load(regs);
     });
@@ -239,7 +241,7 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_split_kernel(GemmParams p) 
   const int cur = (KT - 1) % 2 * STAGE;
   static_for<READ_SLABS>([&](auto F) { read_frag(F, lds + cur, 1); });
   static_for<KS>([&](auto KSI) { static_for<NMFMA>([&](auto R) { mma(R, KSI); }); });
-  bool redo = least < kSplitLeast - 1u;
+  bool redo = false;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -247,6 +249,7 @@ __global__ __launch_bounds__(2 * WGN * 64) void gemm_split_kernel(GemmParams p) 
       acc[i][j] += acc1[i][j] + low[i][j];
 #pragma unroll
       for (int e = 0; e < 16; ++e) redo |= !(fabsf(acc[i][j][e]) <= 3.402823466e38f);
+      acc[i][j] *= kSplitUnscale;
     }
   if (__syncthreads_or(redo)) ragged_products<float, A_MC, B_MC, BT, WGN, MIS>(p, m0, n0, bz, tid, lds, acc);
 
