@@ -432,8 +432,9 @@ __device__ __forceinline__ void bwd_pass(const std::conditional_t<SAVE_DS, Saved
     if constexpr (BIAS) load_bias(t0, bs);
     // With both owner operands and the accumulators of the larger head sizes there are registers for the scores of half a
     // block: one half's are dead before the other's are made.  (A whole block's: the dK launch spills 30 registers, the
-    // dQ launch has none left in which to read fragments ahead of their products, 526 -> 499 us at [8,32,2048,128] causal.)
-    constexpr bool BY_HALF = DS && HP >= 128;
+    // dQ launch has none left in which to read fragments ahead of their products, 526 -> 499 us at [8,32,2048,128] causal; with a
+    // bias, whose loads the second half then waits for, it is faster whole: 40 heads of 459 x 128 94.6 us, by halves 101.3.)
+    constexpr bool BY_HALF = DS && HP >= 128 && (OWNER_K || !BIAS || HP > 128);
     floatx16 sc[2], dp[2];
     if constexpr (!BY_HALF) {
       scores(c1, of1, sc);
@@ -527,8 +528,9 @@ __device__ __forceinline__ void bwd_pass(const std::conditional_t<SAVE_DS, Saved
     // Heads above 128: up to four blocks go one a turn, since leaving such a turn in its middle moves accumulators, which a
     // short pass has nothing to set against (30 heads of 187 x 256 causal 27.2 -> 24.9 us).  With the short loop in front the compiler
     // also finds better registers for the long one: 32 x 1024 heads of 256 causal 163.6 -> 138.5, of 160 105.8 -> 96.8.
-    // So do all passes of small heads with a bias (128 heads of 1024 x 64 218 us, with two blocks a turn 242).
-    if ((HP > 128 && b1 - b0 <= 4) || (BIAS && HP <= 64)) {
+    // So do all passes of heads up to 128 with a bias (128 heads of 1024 x 64 218 us, with two blocks a turn 242; 40 of 459 x 80 85.2
+    // and 89.6; over 70 drawn sizes of heads of 80 to 128 level on the mean, from 10 % slower to 8 % faster).
+    if ((HP > 128 && b1 - b0 <= 4) || (BIAS && HP <= 128)) {
       for (int it = b0; it < b1; ++it) {
         if ((it - b0) & 1) block(it, s1 + TILE, s2 + TILE, sst + STATS, s1, s2, sst);
         else block(it, s1, s2, sst, s1 + TILE, s2 + TILE, sst + STATS);
