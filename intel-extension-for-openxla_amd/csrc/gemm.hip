@@ -17,10 +17,10 @@
 // holding four consecutive output columns of one row.
 //
 // 16-bit operands whose strides or sizes the direct loads cannot take and all fp32 operands run gemm_ragged_kernel
-// (gemm_ragged.h; fp32 on the large tile gemm_split_kernel, gemm_split.h), products of few tiles gemm_slices_kernel (gemm_slices.h), int8 operands the int8 MFMA kernel
-// (gemm_s8.hip); what is left (operands of less than 16 bytes, int8 products into an unaligned output) runs
-// gemm_generic_kernel, a plain LDS-tiled kernel.  This is where the reference falls back to oneDNN
-// (onednn_matmul_utils.cc:394-491).
+// (gemm_ragged.h; fp32 on the large tile gemm_split_kernel, gemm_split.h), products of few tiles gemm_slices_kernel
+// (gemm_slices.h), int8 operands the int8 MFMA kernel (gemm_s8.hip); what is left (operands of less than 16 bytes, int8
+// products into an unaligned output) runs gemm_generic_kernel, a plain LDS-tiled kernel.  This is where the reference
+// falls back to oneDNN (onednn_matmul_utils.cc:394-491).
 #include <algorithm>
 
 #include "gemm_kernel.h"

@@ -779,7 +779,8 @@ enum : int { kClassKN = 0, kClassNK = 1, kClassRagged = 2, kClassF32 = 3 };
 // 128 x 128: taken for 200 of them, 13 % faster there on average, nine 2 to 5 % slower.  128 x 128 in steps of 32, on 900 of
 // more than 40, k 64 .. 8192: taken for 180, 30 % faster there.  Both on 1520 others of more than 200 and k 64 .. 3000, either
 // storage order of both operands, against the choice without the two: 10 % faster on average, eight of the 1520 more than 3 %
-// slower (1656 x 4760 x 552 with B [n,k] 21.8 us against 19.0, the others 6 % and less).
+// slower (1656 x 4760 x 552 with B [n,k] 21.8 us against 19.0, the others 6 % and less); of 500 more with k 256 .. 3000 six
+// (528 x 12400 x 1328 36.4 against 26.9: 291 tiles of 192 x 128 are a second round of 35, which the estimate takes for less).
 // Looking all candidates over takes the host 0.15 to 0.65 us per call.
 struct TileCost {
   float start, step, more_step, more, fill;

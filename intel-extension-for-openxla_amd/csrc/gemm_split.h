@@ -1,7 +1,7 @@
 // fp32 GEMM on the bf16 matrix instructions.  An fp32 number is the sum of three bf16 ones, exactly:
 //     x = h + m + l,   h = bf16(x), m = bf16(x - h), l = x - h - m     (8 + 8 + 8 significant bits)
-// and a product of two is h h' + (h m' + m h') + (h l' + m m' + l h') up to 2^-25 of itself, half an fp32 rounding.  Six bf16
-// matrix instructions take the time of 3/8 of the fp32 ones: the device does 2.5 PFLOP/s in bf16 and 157 TFLOP/s in fp32.
+// and a product of two is h h' + (h m' + m h') + (h l' + m m' + l h') up to 2^-24 of itself, an fp32 rounding.  Six bf16 matrix
+// instructions take the time of 3/8 of the fp32 ones: the device does 2.5 PFLOP/s in bf16 and 157 TFLOP/s in fp32.
 //
 // Error.  The bf16 instructions truncate what they align to the largest term, so that five small products added into the
 // running sum of the large one bias it.  The large products of even and of odd halves of the K steps and the five small ones
@@ -14,16 +14,25 @@
 // 2^82 is not finite either.  The tile is then formed again by the fp32 instructions (gemm_ragged.h; all tiles of 2048 x 2048 x 1024
 // 122 us).
 //
-// What bounds it: matrix and vector instructions, which share the issue port: 24 products per wave and K step stand beside
-// 110 vector instructions (6.5 per split number: each work-group splits what it loads), and the matrix pipe is busy 53 %
-// of a launch of one tile per CU.  They are interleaved by hand in slots of one product, and a number's steps are spread
+// What bounds it: no unit alone.  24 products per wave and K step stand beside 110 vector instructions (6.5 per split number: each
+// work-group splits what it loads), which share the issue port.  In a launch of one tile per CU the matrix pipe is busy 54 %
+// of the time, vector and matrix instructions issue 44 %, LDS is busy 36 %, and the waves wait 29 % of theirs to issue and 31 % for
+// data or the barrier.  Products and the rest are interleaved by hand in slots of one product, and a number's steps are spread
 // over the slots, since what converts or subtracts has to wait for the one before.  The residuals by a shift or mask and a
 // subtraction; v_dot2_f32_bf16, which does both at once, issues in ten cycles (1024 x 1024 x 4096 149 us, 122 without).
 // Eight waves of 64 x 32; four of 64 x 64 read a third less from LDS and leave a SIMD with nothing beside a wait (165 us).
 // 2048 x 2048 x 1024 71 -> 53 us (162 TFLOP/s where the fp32 instructions' peak is 157), 4096 x 4096 x 1024 252 -> 192,
-// 3926 x 924 x 2976 192 -> 130.  Error against 64 bits, normal operands, k = 64 / 1024 / 4096: 4.9e-8 / 1.3e-7 / 2.7e-7 of the
-// result in the 2-norm; fp32 instructions on this tile 1.4e-7 / 5.7e-7 / 1.1e-6, on tiles whose waves split K 1.1e-7 / 1.6e-7 /
-// 4.1e-7.
+// 3926 x 924 x 2976 192 -> 128.
+//
+// Error against 64 bits, of the result in the 2-norm, here / fp32 instructions on this tile:
+//     k                        64               1024             4096             16384
+//     normal                   4.4e-8 / 1.4e-7  1.3e-7 / 5.8e-7  2.7e-7 / 1.2e-6  5.8e-7 / 2.3e-6
+//     uniform in 0 .. 1        4.0e-8 / 1.2e-7  8.6e-8 / 4.3e-7  1.6e-7 / 8.4e-7  3.0e-7 / 1.7e-6
+//     normal, negatives 0      3.3e-8 / 6.5e-8  6.8e-8 / 2.5e-7  1.5e-7 / 4.9e-7  3.3e-7 / 9.9e-7
+//     softmax x normal         6.5e-8 / 1.4e-7  1.5e-7 / 5.0e-7  2.8e-7 / 9.1e-7
+// (on tiles whose waves split K the fp32 instructions reach 1.1e-7 / 1.6e-7 / 4.1e-7 for the first three of the first line).  Sums that
+// one or two products make up are the other way round, as a truncated last place is twice a rounded one: e^(4 x), x normal, k 64
+// and 256 6.9e-8 / 3.3e-8 and 1.1e-7 / 7.6e-8 (all elements alike, 8.9e-8 / 1.3e-7 and 1.0e-7 / 3.4e-7).
 #pragma once
 #include "gemm_ragged.h"
 
