@@ -779,8 +779,7 @@ enum : int { kClassKN = 0, kClassNK = 1, kClassRagged = 2, kClassF32 = 3 };
 // 128 x 128: taken for 200 of them, 13 % faster there on average, nine 2 to 5 % slower.  128 x 128 in steps of 32, on 900 of
 // more than 40, k 64 .. 8192: taken for 180, 30 % faster there.  Both on 1520 others of more than 200 and k 64 .. 3000, either
 // storage order of both operands, against the choice without the two: 10 % faster on average, eight of the 1520 more than 3 %
-// slower (1656 x 4760 x 552 with B [n,k] 21.8 us against 19.0, the others 6 % and less); of 500 more with k 256 .. 3000 six
-// (528 x 12400 x 1328 36.4 against 26.9: 291 tiles of 192 x 128 are a second round of 35, which the estimate takes for less).
+// slower (1656 x 4760 x 552 with B [n,k] 12 %, the others 6 % and less).
 // Looking all candidates over takes the host 0.15 to 0.65 us per call.
 struct TileCost {
   float start, step, more_step, more, fill;
@@ -875,6 +874,7 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
   const bool direct = cls == kClassKN || cls == kClassNK;
   const int kstep = cls == kClassF32 ? 32 : 64;
   const int64_t tiles_256_x_256 = xmk::ceil_div(m, 256) * xmk::ceil_div(n, 256) * batch;
+  const int64_t tiles_192_x_128 = xmk::ceil_div(m, 192) * xmk::ceil_div(n, 128) * batch;
   auto each = [&](int s, float extra, float least) {
     for (int pol = 0; pol < kNumPolicies; ++pol) {
       if (pol == kRowsPolicy || (!direct && !kPolicies[pol].any_alignment) || (a_mc && pol == k192Policy)) continue;
@@ -889,8 +889,12 @@ inline Choice cheapest(int64_t m, int64_t n, int64_t k, int64_t batch, int cls, 
       // did not see it (5400 x 15512 x 840 202 us where they take 168, 6936 x 8152 x 560 with B [n,k] 109 against 93).
       if (pol == k3PerCuPolicy && (s > 1 || (kt > 6 && tiles_256_x_256 > 384))) continue;
       if (pol == k192Policy && (s > 1 || kt < 6 || (kt > 32 && xmk::ceil_div(m, 192) == xmk::ceil_div(m, 256)))) continue;
-      const float cost = std::max(launch_cost(kPolicies[pol], kTileCost[cls][pol], is_slices(pol), (uint32_t)m, (uint32_t)n, kt,
-                                              (uint32_t)(batch * s)) + extra, least);
+      float us = launch_cost(kPolicies[pol], kTileCost[cls][pol], is_slices(pol), (uint32_t)m, (uint32_t)n, kt, (uint32_t)(batch * s));
+      // A second round of fewer than a hundred 192 x 128 tiles takes longer than the estimate's share of one: 5 % on it gives such
+      // sizes to others (568 x 11568 x 1112 33.6 -> 24.2 us, 528 x 12400 x 1328 36.3 -> 27; over 700 sizes of 257 to 384 of the
+      // tiles 0.4 % on the mean, and the worst loss against having no such tile 12 % where it was 39).
+      if (pol == k192Policy && tiles_192_x_128 > 256 && tiles_192_x_128 <= 352) us *= 1.05f;
+      const float cost = std::max(us + extra, least);
       if (cost < best.us) best = {pol, s, cost};
     }
   };
