@@ -529,8 +529,10 @@ __device__ __forceinline__ void bwd_pass(const std::conditional_t<SAVE_DS, Saved
     // short pass has nothing to set against (30 heads of 187 x 256 causal 27.2 -> 24.9 us).  With the short loop in front the compiler
     // also finds better registers for the long one: 32 x 1024 heads of 256 causal 163.6 -> 138.5, of 160 105.8 -> 96.8.
     // So do all passes of heads up to 128 with a bias (128 heads of 1024 x 64 218 us, with two blocks a turn 242; 40 of 459 x 80 85.2
-    // and 89.6; over 70 drawn sizes of heads of 80 to 128 level on the mean, from 10 % slower to 8 % faster).
-    if ((HP > 128 && b1 - b0 <= 4) || (BIAS && HP <= 128)) {
+    // and 89.6; over 70 drawn sizes of heads of 80 to 128 level on the mean, from 10 % slower to 8 % faster), and those of heads above
+    // 160 with a bias and no mask (38 heads of 148 x 192 77.9 us, with both loops 81.4; 34 sizes 2 % on the mean; causal ones
+    // and heads of 160 are 5 to 8 % faster with both).
+    if ((HP > 128 && b1 - b0 <= 4) || (BIAS && (HP <= 128 || (HP > 160 && !CAUSAL)))) {
       for (int it = b0; it < b1; ++it) {
         if ((it - b0) & 1) block(it, s1 + TILE, s2 + TILE, sst + STATS, s1, s2, sst);
         else block(it, s1, s2, sst, s1 + TILE, s2 + TILE, sst + STATS);
